@@ -8,6 +8,7 @@ OUT = os.path.join(HERE, "libelmo_xmc.so")
 
 SRC_HEAVY = os.path.join(HERE, "csrc", "xmc_fp8_role_heavy.hip")
 SRC_PLAIN = os.path.join(HERE, "csrc", "xmc_fp8_role_plain.hip")
+SRC_CLUSTER = [os.path.join(HERE, "csrc", "xmc_cluster_%s.hip" % t) for t in ("bf16", "sim", "fp8")]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-munsafe-fp-atomics",
@@ -56,10 +57,11 @@ def build(verbose=False):
     digest = source_hash()
     tmp = OUT + ".tmp%d" % os.getpid()
     extra = ["-Rpass-analysis=kernel-resource-usage"] if verbose else []
-    objs = [tmp + ".main.o", tmp + ".heavy.o", tmp + ".plain.o"]
+    objs = [tmp + ".main.o", tmp + ".heavy.o", tmp + ".plain.o"] + [tmp + ".cluster%d.o" % i for i in range(len(SRC_CLUSTER))]
     cmds = [[hipcc] + HIPCC_FLAGS + extra + [f'-DXMC_SOURCE_HASH="{digest}"', "-c", SRC, "-o", objs[0]],
             [hipcc] + HIPCC_FLAGS + HEAVY_FLAGS + extra + ["-c", SRC_HEAVY, "-o", objs[1]],
             [hipcc] + HIPCC_FLAGS + PLAIN_FLAGS + extra + ["-c", SRC_PLAIN, "-o", objs[2]]]
+    cmds += [[hipcc] + HIPCC_FLAGS + PLAIN_FLAGS + extra + ["-c", src, "-o", obj] for src, obj in zip(SRC_CLUSTER, objs[3:])]
     procs = [subprocess.Popen(c, stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True) for c in cmds]   # side by side
     outs = [p.communicate() for p in procs]
     log = "".join(o[0] + o[1] for o in outs)

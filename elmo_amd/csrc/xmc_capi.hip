@@ -5,6 +5,7 @@
 #include "xmc_fp8_quad.hip"
 #include "xmc_fp8_role.hip"
 #include "xmc_tiled.hip"
+#include "xmc_cluster_aux.hip"
 #include "xmc_topk.hip"
 #include "xmc_dropout.hip"
 #include <stdlib.h>
@@ -24,7 +25,7 @@ static __device__ __align__(256) unsigned char scratch[FWD_STATIC_BYTES];
 
 namespace {
 
-struct DeviceInfo { int ok; int cus; unsigned char* scratch_ptr; };
+struct DeviceInfo { int ok; int cus; unsigned char* scratch_ptr; int* failure_word; };
 
 // Filled once per device, by the first call on it; std::call_once makes concurrent first calls of several host threads
 // wait for the one that fills the slot, and publishes the finished slot to all of them.
@@ -32,7 +33,7 @@ DeviceInfo g_device_info[64];
 std::once_flag g_device_once[64];
 
 void fill_device_info(int dev) {
-  DeviceInfo di = {-1, 0, nullptr};
+  DeviceInfo di = {-1, 0, nullptr, nullptr};
   hipDeviceProp_t prop;
   if (hipGetDeviceProperties(&prop, dev) != hipSuccess) { g_device_info[dev] = di; return; }
   di.cus = prop.multiProcessorCount;
@@ -40,9 +41,25 @@ void fill_device_info(int dev) {
   // this device's copy of the static scratch array (device `dev` is current here); stays null if the lookup fails
   void* sp = nullptr;
   di.scratch_ptr = (di.ok == 1 && hipGetSymbolAddress(&sp, HIP_SYMBOL(scratch)) == hipSuccess) ? (unsigned char*)sp : nullptr;
+  // the word of host memory in which the kernels of this device announce a failed step; lives until the process ends.  A
+  // caller may be capturing a graph: the allocation is none of that graph's business
+  if (di.ok == 1) {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool swapped = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    void* fw = nullptr;
+    if (hipHostMalloc(&fw, 64, hipHostMallocMapped) == hipSuccess) {
+      *(int*)fw = 0;
+      di.failure_word = (int*)fw;
+    }
+    if (swapped) (void)hipThreadExchangeStreamCaptureMode(&mode);
+  }
   // opt in to the full 160 KiB of LDS once per device
   role_plain_set_lds();
   role_heavy_set_lds();
+  cluster_set_lds_bf16();
+  cluster_set_lds_sim();
+  cluster_set_lds_fp8();
+  (void)hipFuncSetAttribute((const void*)cluster_prep_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (MAX_POS + 256) * 4);
   (void)hipFuncSetAttribute((const void*)fp8_forward_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, FWD_LDS);
   (void)hipFuncSetAttribute((const void*)fp8_forward_select_kernel<0>, hipFuncAttributeMaxDynamicSharedMemorySize, SEL_LDS);
   (void)hipFuncSetAttribute((const void*)fp8_forward_select_kernel<1>, hipFuncAttributeMaxDynamicSharedMemorySize, SEL_LDS);
@@ -109,6 +126,16 @@ int check_common(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, co
 // plain 16-byte-per-lane copy: the known-size reference against which memory counters are calibrated
 __global__ __launch_bounds__(256) void copy_probe_kernel(const uint4* __restrict__ src, uint4* __restrict__ dst, size_t n16) {
   for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n16; i += (size_t)gridDim.x * 256) dst[i] = src[i];
+}
+
+// stride of the order in which a chunk's n tiles are visited: about 0.618 n, coprime to n
+int tile_stride(int n) {
+  if (n < 3) return 1;
+  for (int s = (int)(0.618 * n);; s++) {
+    int a = s, b = n;
+    while (b) { const int t = a % b; a = b; b = t; }
+    if (a == 1) return s;   // (n - 1 at the latest)
+  }
 }
 
 int launch_status() { return hipGetLastError() == hipSuccess ? XMC_OK : XMC_ERR_LAUNCH; }
@@ -295,7 +322,7 @@ static int fused_step(void* const* chunk_ptrs, int num_chunks, int rows_per_chun
     if (g_prof_stop) (void)hipEventRecord(g_prof_stop, stream);
     g_prof_start = g_prof_stop = nullptr;
     reduce_gx_role_kernel<<<192, 128, 0, stream>>>((const floatx4*)(ws + WS_PARTIAL), qgrid, scale_w, grad_x_f32,
-                                                 (unsigned short*)grad_x_bf16, batch, (int*)(ws + WS_FLAGS), dp);
+                                                 (unsigned short*)grad_x_bf16, batch, (int*)(ws + WS_FLAGS), di.failure_word, dp);
   }
   return launch_status();
 }
@@ -555,8 +582,15 @@ size_t xmc_tiled_workspace_bytes_ex(int num_chunks, int rows_per_chunk, int max_
   const size_t halves = (size_t)tiled_halves(max_batch), pairs = (halves + 1) / 2;
   const size_t rows_buf = (size_t)tiled_group(num_chunks, rows_per_chunk) * rows_pad;   // rows of one launch
   // per batch half G in both orientations; tile_ptr per pair of halves (padded to 64 entries); two loss shares per tile
-  return tiled_layout((int)halves, features).g + halves * 2 * rows_buf * BP * 2 + pairs * ((tiles + 1 + 63) / 64 * 64 * 4) + (tiles * 8 + 255) / 256 * 256;
+  const size_t three = TW_HEAD + tiled_layout((int)halves, features).g + halves * 2 * rows_buf * BP * 2 + pairs * ((tiles + 1 + 63) / 64 * 64 * 4) + (tiles * 8 + 255) / 256 * 256;
+  const size_t one = features == D ? cluster_layout(num_chunks, rows_per_chunk, max_batch).bytes : 0;
+  return three > one ? three : one;
 }
+
+int* xmc_failure_word(void) { return device_info().failure_word; }
+
+size_t xmc_tiled_error_offset(void) { return TW_ERR; }
+size_t xmc_tiled_sticky_error_offset(void) { return TW_ERR + 4; }
 
 int xmc_tiled_step(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, int rows_last_chunk, int weight_type,
                    const void* x_bf16, int batch, int features, const int32_t* labels_coo, int nnz, float lr,
@@ -569,6 +603,81 @@ int xmc_tiled_step(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, 
 }
 
 }  // extern "C"
+
+// The one-pass form of the step (xmc_cluster.hip): 768 features, no compensated head, no loss, no weight decay (options
+// that would have to stay in its main loop, whose registers are full).  Within these it was the faster form at every size
+// tried, from 2 K to 8.6 M labels and 1 to 512 batch rows.  The arguments have been checked by the caller.
+static int cluster_step(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, int rows_last_chunk, int weight_type,
+                        const void* x_bf16, int batch, const int32_t* labels_coo, int nnz, float lr, const uint32_t* seeds,
+                        int round_mode, int quantize_x, int saturate, const DropoutParams& dp, void* grad_x_bf16, float* grad_x_f32,
+                        unsigned char* ws, int cus, int* failure_word, hipStream_t stream) {
+  const bool bf16 = weight_type == W_BF16, fp8 = !bf16 && quantize_x;
+  const int c = cluster_size(batch, fp8), nbk = cluster_blocks(batch, fp8), bp = c * 16 * nbk, pairs = (bp + 255) / 256;
+  const ClusterLayout lay = cluster_layout(num_chunks, rows_per_chunk, bp);
+  const int tile_rows = fp8 && c < 8 ? 64 : 32;
+  const int tpc64 = (rows_per_chunk + TL - 1) / TL;
+  int n_pad = 0;
+  if (nnz > 0) { n_pad = 64; while (n_pad < nnz) n_pad <<= 1; }
+  // a sort key keeps 24 bits for the label: larger label spaces are taken in segments of whole chunks
+  int seg_chunks = ((1 << 24) - 2) / rows_per_chunk;
+  if (seg_chunks > num_chunks) seg_chunks = num_chunks;
+  if (seg_chunks < 1) return XMC_ERR_RANGE;
+  int* err = (int*)(ws + TW_ERR);
+  unsigned* keys = (unsigned*)(ws + lay.keys);
+  int* tile_ptr = (int*)(ws + lay.tile_ptr);
+  float* gx_total = (float*)(ws + lay.gx);
+  const ClusterVariant var = bf16 ? cluster_variant_bf16(c, nbk, round_mode) : fp8 ? cluster_variant_fp8(c, nbk, round_mode) : cluster_variant_sim(c, nbk, round_mode);
+  for (int c0 = 0; c0 < num_chunks; c0 += seg_chunks) {
+    const int nch = c0 + seg_chunks <= num_chunks ? seg_chunks : num_chunks - c0;
+    const bool last = c0 + nch == num_chunks;
+    const int sort_blocks = n_pad / 64, prep_blocks = (bp * (D / 4) + 255) / 256;
+    cluster_prep_kernel<<<sort_blocks * pairs + prep_blocks, 256, (size_t)(n_pad + 256) * 4, stream>>>(
+        labels_coo, nnz, n_pad, batch, c0 * rows_per_chunk, nch * rows_per_chunk, keys, sort_blocks, pairs, (const unsigned short*)x_bf16, bp,
+        bf16 ? 0 : fp8 ? 2 : 1, ws + lay.xq, (unsigned short*)(ws + lay.xt), (int*)(ws + lay.flags), err, dp);
+    cluster_tile_ptr_kernel<<<dim3((nch * tpc64 + 1 + 255) / 256, pairs), 256, 0, stream>>>(keys, n_pad, rows_per_chunk, tpc64, nch * tpc64, tile_ptr,
+                                                                                         lay.tp_stride);
+    ClusterParams p;
+    for (int k = 0; k < MAX_CHUNKS; k++) {
+      p.chunk[k] = k < nch ? (unsigned char*)chunk_ptrs[c0 + k] : nullptr;
+      p.seed[k] = k < nch && seeds ? (round_mode == XMC_ROUND_SR_FAST ? fast_seed(seeds[c0 + k]) : seeds[c0 + k]) : 0u;
+    }
+    p.nchunks = nch;
+    p.rows_per_chunk = rows_per_chunk;
+    p.rows_last = last ? rows_last_chunk : rows_per_chunk;
+    p.tpc = (rows_per_chunk + tile_rows - 1) / tile_rows;
+    p.tpc_last = (p.rows_last + tile_rows - 1) / tile_rows;
+    p.perm = tile_stride(p.tpc);
+    p.perm_last = tile_stride(p.tpc_last);
+    p.tpc64 = tpc64;
+    p.ntiles = (nch - 1) * p.tpc + p.tpc_last;
+    const int most = (cus < CLU_MAXWG ? cus : CLU_MAXWG) / 8 / c * 8;   // whole clusters on every XCD
+    if (most < 8) return XMC_ERR_DEVICE;
+    p.nclusters = p.ntiles < most ? p.ntiles : most;
+    p.label0_seg = 0u;
+    p.label0 = (unsigned)c0 * (unsigned)rows_per_chunk;
+    p.xq = ws + lay.xq;
+    p.xt = (const bf16x8*)(ws + lay.xt);
+    for (int q = 0; q < 2; q++) {
+      const int pr = q < pairs ? q : 0;
+      p.keys[q] = keys + (size_t)pr * MAX_POS;
+      p.tile_ptr[q] = tile_ptr + pr * lay.tp_stride;
+    }
+    p.partial = (floatx4*)(ws + lay.partial);
+    p.exch = ws + lay.exch;
+    p.flags = (int*)(ws + lay.flags);
+    p.xcc = (int*)(ws + lay.xcc);
+    p.err = err;
+    p.lr = lr;
+    p.flush = bf16 ? 1 : 0;   // the reference rounds each chunk's sum where the weights are bf16
+    p.saturate = saturate;
+    p.spin_limit = g_spin_limit.load(std::memory_order_relaxed);
+    var.fn<<<(p.nclusters + 7) / 8 * 8 * c, CLU_NT, var.lds, stream>>>(p);
+    const ClusterReduce rd = {p.partial, c, nbk, p.nclusters, p.ntiles, p.tpc, nch, p.flush, p.xcc, err, failure_word, gx_total, c0 > 0 ? 1 : 0, last ? 1 : 0, batch,
+                              (unsigned short*)grad_x_bf16, grad_x_f32};
+    cluster_reduce_kernel<<<c * nbk * 6 * 8, 256, 0, stream>>>(rd, dp);
+  }
+  return launch_status();
+}
 
 // xmc_tiled_step_ex for DD features (768 or 1024)
 template <int DD>
@@ -604,7 +713,10 @@ static int tiled_step_t(void* const* chunk_ptrs, int num_chunks, int rows_per_ch
   DeviceInfo di = device_info();
   if (di.ok != 1) return XMC_ERR_DEVICE;
   hipStream_t stream = (hipStream_t)stream_;
-  unsigned char* ws = (unsigned char*)workspace;
+  if (DD == D && kahan_type == 0 && !loss_out && weight_decay == 0.f)
+    return cluster_step(chunk_ptrs, num_chunks, rows_per_chunk, rows_last_chunk, weight_type, x_bf16, batch, labels_coo, nnz, lr, seeds,
+                        round_mode, quantize_x, saturate, dp, grad_x_bf16, grad_x_f32, (unsigned char*)workspace, di.cus, di.failure_word, stream);
+  unsigned char* ws = (unsigned char*)workspace + TW_HEAD;
 
   const int rows_pad = (rows_per_chunk + TL - 1) / TL * TL;
   const int tiles_per_chunk = rows_pad / TL;
@@ -642,7 +754,7 @@ static int tiled_step_t(void* const* chunk_ptrs, int num_chunks, int rows_per_ch
   const bool split_update = weight_type == W_E4M3 && halves == 2 && kahan_type == 0 && DD == D;
   tiled_prep_x_kernel<DD><<<(halves * BP * DD + 255) / 256, 256, 0, stream>>>((const unsigned short*)x_bf16, batch, halves, quantize_x,
                                                                         fp8_logits ? 1 : 0, split_update ? 1 : 0, xb, xT, gx_total,
-                                                                        loss_part, loss_out ? 2 * num_tiles : 0, dp);
+                                                                        loss_part, loss_out ? 2 * num_tiles : 0, (int*)((unsigned char*)workspace + TW_ERR), dp);
   for (int c = 0; c < num_chunks; c += group) {
     const int seg0 = c / seg_chunks * seg_chunks;   // first chunk of the segment
     if (c == seg0) {

@@ -1,0 +1,789 @@
+// One-pass training step of the extreme-classifier layers for gfx950 (MI355X): logits, G = sigmoid - targets, grad_X,
+// grad_W and the in-place update of one tile of label rows after the other, every weight read from HBM once and written
+// once.  It covers the modes that keep bf16 temporaries (bf16 weights, src/xmc_classifiers/chunked.py:85-131; simulated FP8,
+// chunked_fp8xmc_clf.py:98-99,110,115-116) and the true-FP8 arithmetic for batches of more than 128 rows (:81-123).
+//
+// A cluster of C workgroups (one per compute unit, all on one XCD) walks a sequence of tiles of T label rows.  Every
+// member loads the whole tile into LDS (from HBM once, then from the XCD's L2) and
+//   * computes the logits and G of its own slice of the batch (64 rows; 32 for small batches) and accumulates
+//     grad_X[slice x 768] += G^T W in registers (96 of them per lane for 64 rows), and
+//   * computes A^T = X^T G^T over the whole batch for its own 768 / C features and updates those weights.
+// The members exchange G (T x 64 bf16 per member and tile) through the XCD's L2.  A batch of up to 64 rows is a cluster
+// of one: no exchange, no waiting.  C = 2, 4, 8 take batches of 128, 256, 512.  Whatever C is, a compute unit keeps the
+// X operand of its slice's logits (48 registers), the X^T operand of its features (48 - 64) and the accumulators (96)
+// resident, and a tile costs it 3 x 2 x T x 64 x 768 flops.
+//
+// Why this split: the three-kernel form reads the weights three times and passes G through HBM in two layouts, and the
+// vector work of the update (up to 170 clocks per 64 weights with the reference's Philox recipe) runs when the matrix
+// cores and the memory system are idle.  Here the four overlap.  The batch slice bounds the registers, not the label
+// rows, so one geometry serves every batch size.
+//
+// What bounds it: bf16 with a small batch the HBM stream (131 K labels, batch 32, round to nearest: 214 us before, 113 now,
+// 3.6 TB/s of weights); the Philox modes the vector units (143 clocks of the SIMD per 64 weights; 501 K labels, batch 128,
+// bf16: 1142 us before, 809 now; 500 K, e4m3: 1086 / 821; 131 K, batch 512: 882 / 601); true FP8 with batch 256 the length
+// of an iteration's dependent phases, about 40 % of whose cycles issue something (8.6 M labels: 11.07 ms before, 10.00 now).
+#include "xmc_common.h"
+
+namespace xmc {
+
+enum CluWeight { CLU_E4M3 = 0, CLU_BF16 = 1 };
+constexpr int CLU_NT = 512;               // eight wavefronts, two per SIMD, 256 registers each
+constexpr int CLU_MAXWG = 256;            // most workgroups of a launch
+constexpr int CLU_FLAG_INTS = CLU_MAXWG * 8;   // tiles-published counters: [cluster][member][wavefront]
+constexpr int CLU_SLOTS = 2;              // exchange slots: a member publishes tile i after every partner has taken tile i - 2
+
+struct ClusterParams {
+  unsigned char* chunk[MAX_CHUNKS];       // first row of every chunk of the launch
+  unsigned seed[MAX_CHUNKS];
+  int nchunks;
+  int rows_per_chunk, rows_last;          // rows of a chunk, of the last one
+  int tpc, tpc_last;                      // tiles of T rows of a chunk, of the last one
+  int perm, perm_last;                    // stride of the order in which a chunk's tiles are visited, coprime to the tile count
+  int tpc64;                              // entries of tile_ptr per chunk (64-row tiles)
+  int ntiles, nclusters;
+  unsigned label0_seg;                    // first label of the launch as the sorted keys count it
+  unsigned label0;                        // ... and in the whole label space (random words of the fast rounding)
+  const unsigned char* xq;                // operand image of X for the logits
+  const bf16x8* xt;                       // operand image of X^T
+  const unsigned* keys[2];                // sorted positives of batch rows 0..255 and 256..511: label * 256 + row
+  const int* tile_ptr[2];                 // first key of every 64-row tile
+  floatx4* partial;                       // grad_X sums, [slot][member][16-row block][feature block][wavefront][lane]
+  unsigned char* exch;                    // [cluster][member][CLU_SLOTS] G slices
+  int* flags;                             // tiles-published counters
+  int* xcc;                               // XCC id of every workgroup
+  int* err;                               // error word: bit 0 = a bounded wait expired
+  float lr;
+  int flush;                              // grad_X sums are stored per chunk (bf16 weights: each chunk's sum is rounded)
+  int saturate;                           // e4m3: casts saturate at +-448 (true FP8) instead of giving NaN above 464
+  int spin_limit;
+};
+
+template <int WT, int QX, int C, int NBK> struct CluGeom {
+  static constexpr int WB = WT == CLU_BF16 ? 2 : 1;            // bytes of a weight
+  static constexpr int T = QX && C < 8 ? 64 : 32;              // label rows of a tile
+  static constexpr int RB = T / 16, KT = T / 32;               // row blocks; K steps of grad_X
+  static constexpr int RS = D * WB;                            // bytes of a weight row
+  static constexpr int LS = RS + 32;                           // stride of a row in LDS (see clu_slot)
+  static constexpr int IMG = T * LS;                           // one tile in LDS
+  static constexpr int SL = 16 * NBK;                          // batch rows of a member
+  static constexpr int GSL = T * SL * 2;                       // its part of G
+  static constexpr int KS = C * NBK / 2;                       // K steps (32 batch rows) of A^T
+  static constexpr int FBN = 48 / C;                           // feature blocks (16 features) of a member
+  static constexpr int ORS = FBN * 16 * WB;                    // bytes of a row of the image of updated weights
+  static constexpr int OIMG = T * ORS;
+  static constexpr int ONC = ORS / 16;
+  static constexpr int OSW = (ONC & -ONC) < 16 ? (ONC & -ONC) - 1 : 15;   // chunk swizzle of that image
+  static constexpr int NBLK = C == 1 ? 6 : C == 2 ? 3 : C == 4 ? 2 : 1;   // feature blocks whose X^T operand a wavefront keeps
+  static constexpr int L_W = 0;
+  static constexpr int NOWN = C > 1 ? 2 : 1;
+  static constexpr int L_OWN = L_W + 2 * IMG;                  // own G of this tile (and of the one before: it is updated one tile behind)
+  static constexpr int L_PART = L_OWN + NOWN * GSL;            // the partners' G of one tile
+  static constexpr int L_OUT = L_PART + (C - 1) * GSL;         // updated weights
+  static constexpr int L_PS = L_OUT + OIMG;                    // partial logits (the K range is split between two wavefronts)
+  static constexpr int L_MISC = L_PS + (QX ? 0 : 8192);        // see below
+  static constexpr int LDS = L_MISC + 64 + 256;                // abort word; at + 16 the range of positives of two tiles; at + 64 a
+                                                               // copy of the cluster's counters
+  static constexpr int WPIECES = T * WB / 8;                   // direct-to-LDS loads of a wavefront per tile: 768 bytes each
+  static constexpr int GPIECES = (C - 1) * GSL / 1024;         // ... of all wavefronts for the partners' G
+  static constexpr int OPIECES = OIMG / 1024;                  // wave-wide stores of updated weights
+  static constexpr int PSLOT = NBK * 6 * 8 * 64;               // floatx4 values of a member's grad_X sum
+  static_assert(LDS <= 160 * 1024, "LDS budget");
+};
+
+typedef __attribute__((address_space(3))) unsigned char clds_u8;
+template <int N> struct CluInt { static constexpr int value = N; };
+typedef unsigned cux2 __attribute__((ext_vector_type(2)));
+typedef short cshortx4 __attribute__((ext_vector_type(4)));
+typedef short cshortx8 __attribute__((ext_vector_type(8)));
+
+// LDS row that holds row r of a tile.  Loads must stay whole runs of consecutive bytes: with the 16-byte chunks of a row
+// permuted (an XOR swizzle) a load of 1 KiB took 100 clocks of the compute unit's memory path instead of a quarter of that.
+// So the rows are permuted instead (bits 2 and 3 trade places) and padded by two chunks.  ds_read_b128 serves lanes 0-3,
+// 12-15, 20-23, 24-27 together (then 4-11, 16-19, 28-31, and the upper half alike), the 8-byte reads 32 lanes: the operand
+// reads of sixteen rows at chunks k, k + 1 and the transposing reads of 32 bytes of rows 8k..8k+3 (bf16) are then free of
+// bank conflicts, those of 16 bytes of rows 8k..8k+7 (e4m3) two-way.
+__host__ __device__ constexpr int clu_slot(int r) { return (r & ~12) | ((r & 4) << 1) | ((r & 8) >> 1); }
+// chunk swizzle of the 64-byte rows of G (four chunks; q = row / 4 % 4) for the same reads
+__device__ __forceinline__ int clu_gswz(int q) { return -q & 3; }
+
+__device__ __forceinline__ void clu_lds_load16(const unsigned char* base, unsigned off, unsigned ldsoff_) {
+  const unsigned ldsoff = __builtin_amdgcn_readfirstlane(ldsoff_);
+  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(ldsoff), "v"(off), "s"(base) : "memory", "m0");
+}
+// at device scope: never served by this compute unit's L1, which may hold an exchange slot's previous contents
+__device__ __forceinline__ void clu_lds_load16_l2(const unsigned char* base, unsigned off, unsigned ldsoff_) {
+  const unsigned ldsoff = __builtin_amdgcn_readfirstlane(ldsoff_);
+  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2 sc1" : : "s"(ldsoff), "v"(off), "s"(base) : "memory", "m0");
+}
+
+// 4 bytes per lane at device scope into LDS at ldsoff + 4 * lane
+__device__ __forceinline__ void clu_lds_load4_l2(const void* g, unsigned ldsoff_) {
+  const unsigned ldsoff = __builtin_amdgcn_readfirstlane(ldsoff_);
+  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, off sc1" : : "s"(ldsoff), "v"(g) : "memory", "m0");
+}
+
+__device__ __forceinline__ bf16x8 clu_widen8(intx2 raw) {   // eight e4m3 codes as bf16, exact
+  bf16x2 c0 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(raw.x, 1.0f, false), c1 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(raw.x, 1.0f, true);
+  bf16x2 c2 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(raw.y, 1.0f, false), c3 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(raw.y, 1.0f, true);
+  return bf16x8{c0.x, c0.y, c1.x, c1.y, c2.x, c2.y, c3.x, c3.y};
+}
+
+// Four consecutive features of one row: t = w - lr a, rounded (definitions: the comment in front of tiled_update_kernel).
+// a is rounded to bf16 first with bf16 weights.
+template <int WT, int MODE>
+__device__ __forceinline__ void clu_update4(floatx4 a, const unsigned (&wr)[WT == CLU_BF16 ? 2 : 1], float lr, unsigned off0, unsigned fidx,
+                                            unsigned seed, unsigned (&wo)[WT == CLU_BF16 ? 2 : 1]) {
+  float w[4], t[4];
+  if constexpr (WT == CLU_BF16) {
+    w[0] = __uint_as_float(wr[0] << 16); w[1] = __uint_as_float(wr[0] & 0xFFFF0000u);
+    w[2] = __uint_as_float(wr[1] << 16); w[3] = __uint_as_float(wr[1] & 0xFFFF0000u);
+    const unsigned a01 = bf16_pack2(a[0], a[1]), a23 = bf16_pack2(a[2], a[3]);
+    a[0] = __uint_as_float(a01 << 16); a[1] = __uint_as_float(a01 & 0xFFFF0000u);
+    a[2] = __uint_as_float(a23 << 16); a[3] = __uint_as_float(a23 & 0xFFFF0000u);
+  } else {
+    floatx2 w01 = __builtin_amdgcn_cvt_pk_f32_fp8((int)wr[0], false), w23 = __builtin_amdgcn_cvt_pk_f32_fp8((int)wr[0], true);
+    w[0] = w01.x; w[1] = w01.y; w[2] = w23.x; w[3] = w23.y;
+  }
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    t[e] = __builtin_fmaf(-lr, a[e], w[e]);
+    if (MODE == ROUND_SR_PHILOX) {
+      const unsigned r = philox_word0(off0 + (unsigned)e, seed, 0u);
+      const unsigned mask = WT == CLU_BF16 ? 0xFFFFu : 0xFFFFFu;
+      unsigned tb = __float_as_uint(t[e]) + (r & mask);
+      if (WT == CLU_E4M3) tb &= ~mask;   // (bf16: the lower half is dropped by the pack below)
+      asm volatile("" : "+v"(off0), "+v"(tb));   // one chain of ten rounds at a time: no registers for four
+      t[e] = __uint_as_float(tb);
+    }
+  }
+  if constexpr (WT == CLU_BF16) {
+    if (MODE == ROUND_SR_PHILOX) {
+      wo[0] = __builtin_amdgcn_perm(__float_as_uint(t[1]), __float_as_uint(t[0]), 0x07060302u);
+      wo[1] = __builtin_amdgcn_perm(__float_as_uint(t[3]), __float_as_uint(t[2]), 0x07060302u);
+    } else if (MODE == ROUND_SR_FAST) {
+      const unsigned h = fast_mix(fidx, seed);
+      bf16x2 lo = {}, hi = {};
+      lo = __builtin_amdgcn_cvt_sr_bf16_f32(lo, t[0], fast_word(h, 0), false);
+      lo = __builtin_amdgcn_cvt_sr_bf16_f32(lo, t[1], fast_word(h, 1), true);
+      hi = __builtin_amdgcn_cvt_sr_bf16_f32(hi, t[2], fast_word(h, 2), false);
+      hi = __builtin_amdgcn_cvt_sr_bf16_f32(hi, t[3], fast_word(h, 3), true);
+      wo[0] = __builtin_bit_cast(unsigned, lo);
+      wo[1] = __builtin_bit_cast(unsigned, hi);
+    } else {
+      wo[0] = bf16_pack2(t[0], t[1]);
+      wo[1] = bf16_pack2(t[2], t[3]);
+    }
+  } else {
+    int packed = 0;   // saturating or not: MODE.FP16_OVFL, set once per launch
+    if (MODE == ROUND_SR_FAST) {
+      const unsigned h = fast_mix(fidx, seed);
+      packed = __builtin_amdgcn_cvt_sr_fp8_f32(t[0], fast_word(h, 0), packed, 0);
+      packed = __builtin_amdgcn_cvt_sr_fp8_f32(t[1], fast_word(h, 1), packed, 1);
+      packed = __builtin_amdgcn_cvt_sr_fp8_f32(t[2], fast_word(h, 2), packed, 2);
+      packed = __builtin_amdgcn_cvt_sr_fp8_f32(t[3], fast_word(h, 3), packed, 3);
+    } else {
+      packed = __builtin_amdgcn_cvt_pk_fp8_f32(t[0], t[1], packed, false);
+      packed = __builtin_amdgcn_cvt_pk_fp8_f32(t[2], t[3], packed, true);
+    }
+    wo[0] = (unsigned)packed;
+  }
+}
+
+#define CFENCE() __builtin_amdgcn_sched_barrier(0)   // nothing is scheduled across this point
+// the compiler takes `x` for a new value: what depends on it is computed where it is used instead of being kept in
+// registers over the whole loop (256 registers hold the resident operands and the accumulators and little else)
+#define COPAQUE(x) asm volatile("" : "+v"(x))
+// the lane number, without a register that holds it
+__device__ __forceinline__ int clu_lane() { return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); }
+
+// A tile of the sequence (wave-uniform).
+struct CluTile { unsigned char* base; int c, row0, rows_valid; unsigned seed; };
+
+// The launch parameters are read from the kernel argument segment where they are needed (scalar loads that hit the
+// constant cache) instead of occupying scalar registers over the whole loop.
+typedef const __attribute__((address_space(4))) ClusterParams* clu_cparams;
+
+template <int WT, int QX, int C, int NBK, int MODE>
+__global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterParams) {
+  typedef CluGeom<WT, QX, C, NBK> G;
+  constexpr int T = G::T, RB = G::RB, KT = G::KT, RS = G::RS, KS = G::KS, WDW = WT == CLU_BF16 ? 2 : 1;
+  clu_cparams kp = (clu_cparams)__builtin_amdgcn_kernarg_segment_ptr();
+#define p (*kp)
+  extern __shared__ __attribute__((aligned(16))) unsigned char clu_lds[];
+  clds_u8* lds = (clds_u8*)clu_lds;
+  const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, kg = lane >> 4;
+  int v = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // members of cluster j: workgroups ((j / 8) C + m) 8 + j % 8, which share an XCD (workgroup g runs on XCD g % 8) and are
+  // dispatched one behind the other on it
+  const int g = blockIdx.x;
+  int m = (g >> 3) % C, j = ((g >> 3) / C) * 8 + (g & 7);
+  if (j >= p.nclusters) return;
+  if (WT == CLU_E4M3 && p.saturate) asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 23, 1), 1");
+  if (C > 1 && tid == 0) {
+    p.xcc[g] = (int)(__builtin_amdgcn_s_getreg((3 << 11) | 20) & 15);   // XCC_ID
+    *(__attribute__((address_space(3))) int*)(lds + G::L_MISC) = 0;
+  }
+  if (C > 1 && tid < 64) *(__attribute__((address_space(3))) int*)(lds + G::L_MISC + 64 + 4 * tid) = 0;
+  const int v0 = (int)((long long)j * p.ntiles / p.nclusters), v1 = (int)((long long)(j + 1) * p.ntiles / p.nclusters);
+  const int n_it = v1 - v0;
+
+  const float lr = p.lr;
+  const int rpc = p.rows_per_chunk, nchunks = p.nchunks;
+  const unsigned label0 = p.label0;
+  unsigned char* exq = p.exch + (size_t)j * C * CLU_SLOTS * G::GSL;   // this cluster's exchange slots
+  int* cflags = p.flags + j * C * 8;                                  // ... and counters
+  const int* ctptr = p.tile_ptr[C == 8 ? m >> 2 : 0];
+  const int tpc64 = p.tpc64;
+  // ---- the sequence: positions v0 .. v1-1 of the chunks' tiles laid one behind the other, the tiles of a chunk in the
+  //      order 0, perm, 2 perm, ... (modulo their count), which spreads the label-sorted positives over the clusters
+  int sc = v0 / p.tpc;                       // chunk, position within it and tile of the next position to be read
+  int sp = v0 - sc * p.tpc;
+  int sn, ss, srows;                         // of that chunk: tiles, stride of their order, rows
+  unsigned char* sbase;
+  unsigned sseed;
+  auto enter_chunk = [&]() {
+    const bool last = sc == p.nchunks - 1;
+    sn = last ? p.tpc_last : p.tpc;
+    ss = last ? p.perm_last : p.perm;
+    srows = last ? p.rows_last : p.rows_per_chunk;
+    sbase = p.chunk[sc];
+    sseed = p.seed[sc];
+  };
+  enter_chunk();
+  int st = (int)((long long)sp * ss % sn);
+  auto next_tile = [&]() {
+    CluTile q;
+    q.c = sc;
+    q.row0 = st * T;
+    q.base = sbase + (size_t)q.row0 * RS;
+    q.rows_valid = min(T, srows - q.row0);
+    q.seed = sseed;
+    st += ss;
+    if (st >= sn) st -= sn;
+    if (++sp == sn && sc + 1 < nchunks) { sp = 0; st = 0; sc++; enter_chunk(); }
+    return q;
+  };
+
+  // ---- loads of a tile: 48 lanes x 16 bytes = a row of e4m3 or half a row of bf16 weights each, so that no lane computes an
+  //      address (a reload of an offset from scratch memory would make the compiler wait for every load issued before)
+  auto load_pieces = [&](const CluTile& q, int slot, int s0, int s1) {
+    const int ln = clu_lane();
+    // (the range of positives travels with the tile: as a scalar load it would make the next wait for an LDS read wait for it)
+    if (s0 == 0 && v == 7 && ln < 2) clu_lds_load4_l2(ctptr + (q.c * tpc64 + (q.row0 >> 6)) + ln, (unsigned)(G::L_MISC + 16 + slot * 8));
+    if (ln < 48) {
+#pragma unroll
+      for (int s = s0; s < s1; s++) {
+        const int row = v * (T / 8) + s / G::WB, src = min(row, q.rows_valid - 1);   // rows past the end re-read the last valid one
+        clu_lds_load16(q.base + src * RS + (s % G::WB) * 768, (unsigned)ln * 16u, (unsigned)(G::L_W + slot * G::IMG + clu_slot(row) * G::LS + (s % G::WB) * 768));
+      }
+    }
+  };
+  auto load_tile = [&](const CluTile& q, int slot) { load_pieces(q, slot, 0, G::WPIECES); };
+  CluTile cur = next_tile(), prev = cur, prev2 = cur, nxt = cur;
+  if (n_it > 0) load_tile(cur, 0);
+
+  // ---- resident operands
+  // Logits: with FP8 products wavefront v takes batch block v % 4 and half of the tile's row blocks; with bf16 products the
+  // K range is split in two instead (a wavefront's share of X is then half as large) and the partial sums go through LDS.
+  // 64-row slices: batch block v % 4, K half v / 4, both row blocks, of which it finishes one; 32-row slices: batch block
+  // v % 2, row block (v / 2) % 2, K half v / 4, finished by the lower half.
+  int b = NBK == 4 ? (v & 3) : (v & 1), hi4 = v >> 2;
+  bf16x8 xr[QX ? 1 : 12];
+  intx8 xq8[QX ? 6 : 1];
+  {
+    const int bg = m * NBK + b;
+    if constexpr (QX) {
+#pragma unroll
+      for (int ks = 0; ks < 6; ks++) xq8[ks] = *(const intx8*)(p.xq + ((size_t)(bg * 6 + ks) * 64 + lane) * 32);
+    } else {
+#pragma unroll
+      for (int k = 0; k < 12; k++) {
+        const int ks = WT == CLU_BF16 ? 12 * hi4 + k : 2 * (2 * (k >> 1) + hi4) + (k & 1);
+        xr[k] = *(const bf16x8*)(p.xq + ((size_t)(bg * 24 + ks) * 64 + lane) * 16);
+      }
+    }
+  }
+  // A^T: feature blocks of this wavefront (within the member's FBN) and the row blocks it takes of each
+  //   C = 1, 2: 6 or 3 blocks, every row block;  C = 4: wavefronts v and v + 4 take one block whole and half of the row blocks of
+  //   a third;  C = 8: wavefronts 0-3 one block whole, 4-7 half of the row blocks of one (six blocks in all)
+  auto block_of = [&](int k) {
+    if (C == 1) return 6 * v + k;
+    if (C == 2) return 3 * v + k;
+    if (C == 4) return k == 0 ? 3 * (v & 3) + hi4 : 3 * (v & 3) + 2;
+    return v < 4 ? v : 4 + ((v - 4) >> 1);
+  };
+  // the row blocks in the order in which the wavefront takes them, the ones it takes of every block first
+  auto row_block = [&](int n) { return C <= 2 ? n : C == 4 ? (n + hi4 * (RB / 2)) & (RB - 1) : v < 4 ? n : v & 1; };
+  auto takes = [&](int k, int n) { return C <= 2 || (C == 4 ? k == 0 || n < RB / 2 : n == 0 || v < 4); };   // (wave-uniform)
+  bf16x8 xt[G::NBLK][KS];
+#pragma unroll
+  for (int k = 0; k < G::NBLK; k++)
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++)   // (the batch slices in the order own, next member's, ...)
+      xt[k][ks] = p.xt[(size_t)((m * G::FBN + block_of(k)) * KS + (ks + m * (G::SL / 32)) % KS) * 64 + lane];
+  floatx4 acc[NBK][6];   // grad_X[slice x 96 features]
+#pragma unroll
+  for (int mb = 0; mb < NBK; mb++)
+#pragma unroll
+    for (int nn = 0; nn < 6; nn++) acc[mb][nn] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+  // ---- per-lane parts of the LDS addresses, two to a register
+  constexpr int LS = G::LS;
+  unsigned pk_w, pk_g, pk_o;
+  {
+    // grad_X, W operand (transposing reads): row 8kg + l16 / 4 (bf16) or 8kg + l16 / 2;  logits: row l16, chunk kg
+    const unsigned wtr = WT == CLU_BF16 ? (unsigned)(clu_slot(8 * kg + (l16 >> 2)) * LS + (l16 & 3) * 8) : (unsigned)(clu_slot(8 * kg + (l16 >> 1)) * LS + (l16 & 1) * 8);
+    const unsigned wrow = (unsigned)(clu_slot(l16) * LS + kg * 16);
+    pk_w = wtr | (wrow << 16);
+    // A^T, G operand (transposing reads): batch rows 8kg + l16 / 4, labels 4 (l16 % 4)..;  own G: batch row 16b + l16, labels 4kg..
+    const unsigned gtr = (unsigned)((8 * kg + (l16 >> 2)) * 64 + ((((l16 >> 1) & 1) ^ (2 * (kg & 1))) * 16) + (l16 & 1) * 8);
+    const unsigned gout = (unsigned)((16 * b + l16) * 64 + ((kg >> 1) ^ clu_gswz(l16 >> 2)) * 16 + (kg & 1) * 8);
+    pk_g = gtr | (gout << 16);
+    // old weights: row l16, features 4kg.. of a block;  grad_X, G^T operand: batch row l16 of a block, labels 8kg..
+    const unsigned wold = (unsigned)(clu_slot(l16) * LS + 4 * kg * G::WB);
+    const unsigned ga = (unsigned)(l16 * 64 + (kg ^ clu_gswz(l16 >> 2)) * 16);
+    pk_o = wold | (ga << 16);
+  }
+  auto exch_slot = [&](int qm, int t) { return exq + (unsigned)((qm * CLU_SLOTS + (t & (CLU_SLOTS - 1))) * G::GSL); };
+
+  auto read_old = [&](unsigned wimg, int k, int rb, unsigned (&wr)[WDW]) {
+    const unsigned at = (pk_o & 0xFFFFu) + (wimg + (unsigned)(rb * 16 * LS + (m * G::FBN + block_of(k)) * 16 * G::WB));
+    if constexpr (WT == CLU_BF16) {
+      const cux2 q = *(const __attribute__((address_space(3))) cux2*)(lds + at);
+      wr[0] = q.x; wr[1] = q.y;
+    } else {
+      wr[0] = *(const __attribute__((address_space(3))) unsigned*)(lds + at);
+    }
+  };
+  unsigned wold[C > 1 ? G::NBLK : 1][C > 1 ? RB : 1][WDW];   // clusters of several: the weights the lagging update starts from
+
+  // A^T and update of the tile q whose G is complete in LDS (own part at gown), the result to the image of updated weights
+  // (row blocks n0 .. n1-1 in this wavefront's order; `between` runs once, in the middle of the last one's vector work)
+  auto update_tile = [&](const CluTile& q, unsigned gown, unsigned wimg, auto n0_c, auto n1_c, auto&& between) {
+    constexpr int n0 = decltype(n0_c)::value, n1 = decltype(n1_c)::value;
+    const unsigned seed = q.seed;
+    const unsigned grow0 = label0 + (unsigned)q.c * (unsigned)rpc + (unsigned)q.row0;
+#pragma unroll
+    for (int n = n0; n < n1; n++) {
+      const int rb = row_block(n);
+      if (C <= 4 || takes(0, n)) {
+        const int ln = clu_lane(), l16 = ln & 15, kg = ln >> 4;
+        const unsigned g_lane = ((pk_g & 0xFFFFu) ^ (unsigned)((rb & 1) * 32)) + (unsigned)((rb >> 1) * G::SL * 64);
+        // G operands one K step ahead of their products
+        bf16x8 bg[2];
+        auto rdg = [&](int ks) {
+          const int d = ks * 32 / G::SL, kk = ks - d * (G::SL / 32);   // slice: own, next member's, ...; K step within it
+          const unsigned a0 = g_lane + (d == 0 ? gown : (unsigned)(G::L_PART + (d - 1) * G::GSL));
+          cshortx4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) cshortx4*)(lds + a0 + kk * 32 * 64));
+          cshortx4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) cshortx4*)(lds + (a0 ^ 48u) + (kk * 32 + 4) * 64));
+          return __builtin_bit_cast(bf16x8, cshortx8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]});
+        };
+        floatx4 aa[G::NBLK];
+        bg[0] = rdg(0);
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+          if (ks + 1 < KS) bg[(ks + 1) & 1] = rdg(ks + 1);
+#pragma unroll
+          for (int k = 0; k < G::NBLK; k++)
+            if (takes(k, n)) aa[k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xt[k][ks], bg[ks & 1], ks == 0 ? floatx4{0.f, 0.f, 0.f, 0.f} : aa[k], 0, 0, 0);
+          CFENCE();
+        }
+        const unsigned row = (unsigned)(16 * rb + l16);
+        const unsigned orow = (unsigned)q.row0 + row;
+#pragma unroll
+        for (int k = 0; k < G::NBLK; k++) {
+          if (!takes(k, n)) continue;
+          const floatx4 a = aa[k];
+          unsigned wr[WDW], wo[WDW];
+          if constexpr (C == 1) {
+            read_old(wimg, k, rb, wr);
+          } else {
+#pragma unroll
+            for (int d = 0; d < WDW; d++) wr[d] = wold[k][n][d];
+          }
+          const int lb = block_of(k);
+          const unsigned col = (unsigned)((m * G::FBN + lb) * 16 + 4 * kg);
+          clu_update4<WT, MODE>(a, wr, lr, orow * (unsigned)D + col, (grow0 + row) * (unsigned)(D / 4) + (col >> 2), seed, wo);
+          if constexpr (WT == CLU_BF16) {
+            *(__attribute__((address_space(3))) cux2*)(lds + G::L_OUT + row * G::ORS + (unsigned)(((2 * lb + (kg >> 1)) ^ (l16 & G::OSW)) * 16 + 8 * (kg & 1))) = cux2{wo[0], wo[1]};
+          } else {
+            *(__attribute__((address_space(3))) unsigned*)(lds + G::L_OUT + row * G::ORS + (unsigned)((lb ^ (l16 & G::OSW)) * 16 + 4 * kg)) = wo[0];
+          }
+          CFENCE();
+          if (n == n1 - 1 && k == 0) between();
+        }
+      }
+    }
+  };
+  // the image of updated weights to memory, as whole 16-byte pieces of row segments; a full tile takes the same number of
+  // stores in every wavefront up to one (counted below), a partial one may take fewer
+  auto store_out = [&](const CluTile& q) {
+    int ln = clu_lane();
+    COPAQUE(ln);
+    auto piece = [&](int pc, bool all) {
+      const int ch = pc * 64 + ln, row = ch / G::ONC, c = ch - row * G::ONC;
+      const intx4 ov = *(const __attribute__((address_space(3))) intx4*)(lds + G::L_OUT + row * G::ORS + ((c ^ (row & 15 & G::OSW)) * 16));
+      if (all || row < q.rows_valid) *(intx4*)(q.base + (unsigned)(row * RS + m * G::ORS + c * 16)) = ov;
+    };
+    if (q.rows_valid == T) {
+#pragma unroll
+      for (int s = 0; s < (G::OPIECES + 7) / 8; s++)
+        if (v + 8 * s < G::OPIECES) piece(v + 8 * s, true);
+    } else {
+      for (int s = v; s < G::OPIECES; s += 8) piece(s, false);
+    }
+  };
+  auto store_acc = [&](int slot) {
+    unsigned char* dst = (unsigned char*)(p.partial + (size_t)(slot * C + m) * G::PSLOT + v * 64);   // (wave-uniform)
+    unsigned off = (unsigned)clu_lane() * 16u;
+    COPAQUE(off);
+#pragma unroll
+    for (int mb = 0; mb < NBK; mb++)
+#pragma unroll
+      for (int nn = 0; nn < 6; nn++) {
+        *(floatx4*)(dst + off) = acc[mb][nn];
+        acc[mb][nn] = floatx4{0.f, 0.f, 0.f, 0.f};
+        off += 8192u;
+        COPAQUE(off);
+      }
+  };
+
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0);   // (a wait the compiler knows of: nothing it loaded is outstanding in the loop)
+
+  bool aborted = false;
+  const int last = C > 1 ? n_it + 1 : n_it;   // clusters of several update one tile behind
+#pragma unroll 1
+  for (int i = 0; i < last; i++) {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __syncthreads();   // tile i has landed; the image of updated weights is complete
+    const bool do_a = C == 1 || i < n_it;
+    asm volatile("" : "+s"(kp), "+s"(v), "+s"(m), "+s"(j), "+s"(b), "+s"(hi4));
+    // (the operands count as used here, or the register allocator spills them in favour of short-lived values)
+#pragma unroll
+    for (int k = 0; k < G::NBLK; k++)
+#pragma unroll
+      for (int ks = 0; ks < KS; ks++) COPAQUE(xt[k][ks]);
+    if constexpr (QX) {
+#pragma unroll
+      for (int ks = 0; ks < 6; ks++) COPAQUE(xq8[ks]);
+    } else {
+#pragma unroll
+      for (int k = 0; k < 12; k++) COPAQUE(xr[k]);
+    }
+    COPAQUE(pk_w); COPAQUE(pk_g); COPAQUE(pk_o);
+    if (i + 1 < n_it) nxt = next_tile();
+    if (C == 1) {
+      if (i + 1 < n_it) load_tile(nxt, (i + 1) & 1);
+      if (i > 0) store_out(prev);
+    }
+    const int p0 = __builtin_amdgcn_readfirstlane(*(const __attribute__((address_space(3))) int*)(lds + G::L_MISC + 16 + (i & 1) * 8));
+    const int p1 = __builtin_amdgcn_readfirstlane(*(const __attribute__((address_space(3))) int*)(lds + G::L_MISC + 20 + (i & 1) * 8));
+    if (C > 1 && i > 0) {
+      // the partners' G of tile i-1: normally they had published it when the counters were read at the end of the
+      // iteration before
+      constexpr unsigned long long ALL = C == 8 ? ~0ull : (1ull << (8 * C)) - 1ull;
+      const int seen = *(const __attribute__((address_space(3))) int*)(lds + G::L_MISC + 64 + 4 * (clu_lane() & (8 * C - 1)));
+      if ((__builtin_amdgcn_ballot_w64(seen >= i) & ALL) != ALL) {
+        for (int spin = 0;; spin++) {
+          const int fv = __hip_atomic_load(cflags + (clu_lane() & (8 * C - 1)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          if ((__builtin_amdgcn_ballot_w64(fv >= i) & ALL) == ALL) break;
+          if (spin >= p.spin_limit || ((spin & 1023) == 1023 && __hip_atomic_load(p.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
+            // give up: partners that wait for this workgroup see the error word and give up too
+            if (clu_lane() == 0) {
+              __hip_atomic_fetch_or(p.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+              *(__attribute__((address_space(3))) int*)(lds + G::L_MISC) = 1;
+            }
+            break;
+          }
+          __builtin_amdgcn_s_sleep(1);
+        }
+      }
+#pragma unroll
+      for (int s = 0; s < (G::GPIECES + 7) / 8; s++) {
+        const int pc = v + 8 * s;
+        if (pc < G::GPIECES) {
+          const int d = pc / (G::GSL / 1024), part = pc - d * (G::GSL / 1024), qm = (m + 1 + d) & (C - 1);
+          clu_lds_load16_l2(exch_slot(qm, i - 1) + part * 1024, (unsigned)clu_lane() * 16u, (unsigned)(G::L_PART + pc * 1024));
+        }
+      }
+    }
+    const unsigned wimg = (unsigned)(G::L_W + (i & 1) * G::IMG), gown = (unsigned)(G::L_OWN + (C > 1 ? i & 1 : 0) * G::GSL);
+    constexpr int ZN = QX ? RB / 2 : NBK == 4 ? 2 : 1;   // row blocks of the products
+    constexpr int FN = QX ? RB / 2 : 1;                  // row blocks this wavefront finishes
+    floatx4 z[ZN];
+    if (do_a) {
+#pragma unroll
+      for (int n = 0; n < ZN; n++) z[n] = floatx4{0.f, 0.f, 0.f, 0.f};
+      const unsigned rb0 = QX ? (unsigned)(hi4 * (RB / 2) * 16 * LS) : NBK == 4 ? 0u : (unsigned)(((v >> 1) & 1) * 16 * LS);
+      const unsigned abase = wimg + (pk_w >> 16) + rb0 + (QX ? 0u : (unsigned)(hi4 * (WT == CLU_BF16 ? 768 : 64)));
+      // operands are read three steps ahead of their products
+      if constexpr (QX) {
+        constexpr int NS = 6 * ZN;
+        intx4 lo[2], hi[2];
+        auto rd = [&](int t) {
+          const int ks = t / ZN, n = t - ks * ZN;
+          lo[t & 1] = *(const __attribute__((address_space(3))) intx4*)(lds + abase + ks * 128 + n * 16 * LS);
+          hi[t & 1] = *(const __attribute__((address_space(3))) intx4*)(lds + abase + ks * 128 + 64 + n * 16 * LS);
+        };
+        rd(0);
+#pragma unroll
+        for (int t = 0; t < NS; t++) {
+          if (t + 1 < NS) rd(t + 1);
+          const intx4 l = lo[t & 1], h = hi[t & 1];
+          z[t % ZN] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(intx8{l[0], l[1], l[2], l[3], h[0], h[1], h[2], h[3]}, xq8[t / ZN], z[t % ZN], 0, 0, 0, 0, 0, 0);
+          CFENCE();
+        }
+      } else if constexpr (WT == CLU_BF16) {
+        constexpr int NS = 12 * ZN;
+        bf16x8 wv[4];
+        auto rd = [&](int t) {
+          const int k = t / ZN, n = t - k * ZN;
+          wv[t & 3] = *(const __attribute__((address_space(3))) bf16x8*)(lds + abase + k * 64 + n * 16 * LS);
+        };
+        rd(0); rd(1); rd(2);
+#pragma unroll
+        for (int t = 0; t < NS; t++) {
+          if (t + 3 < NS) rd(t + 3);
+          z[t % ZN] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[t & 3], xr[t / ZN], z[t % ZN], 0, 0, 0);
+          CFENCE();
+        }
+      } else {
+        constexpr int NS = 6 * ZN;
+        intx4 wv[4];
+        auto rd = [&](int t) {
+          const int k2 = t / ZN, n = t - k2 * ZN;
+          wv[t & 3] = *(const __attribute__((address_space(3))) intx4*)(lds + abase + k2 * 128 + n * 16 * LS);
+        };
+        rd(0); rd(1); rd(2);
+#pragma unroll
+        for (int t = 0; t < NS; t++) {
+          if (t + 3 < NS) rd(t + 3);
+          const intx4 w4 = wv[t & 3];
+          z[t % ZN] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(clu_widen8(intx2{w4.x, w4.y}), xr[2 * (t / ZN)], z[t % ZN], 0, 0, 0);
+          z[t % ZN] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(clu_widen8(intx2{w4.z, w4.w}), xr[2 * (t / ZN) + 1], z[t % ZN], 0, 0, 0);
+          CFENCE();
+        }
+      }
+      if constexpr (!QX) {
+        // the other K half's row block (64-row slices) or the upper half's sum (32-row slices) to the wavefront that finishes it
+        if (NBK == 4 || hi4 == 1)
+          *(__attribute__((address_space(3))) floatx4*)(lds + G::L_PS + v * 1024 + clu_lane() * 16) = NBK == 4 ? (hi4 ? z[0] : z[ZN - 1]) : z[0];
+      }
+    }
+    if (C > 1) {
+      if (i > 1) store_out(prev2);   // the weights updated in the iteration before
+      // the partners' G has landed (younger than its loads: those stores)
+      if (i > 1 && prev2.rows_valid == T) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(G::OPIECES / 8) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    if (!QX || C > 1) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __syncthreads();   // the partial logits and the partners' G of tile i-1 are visible; the image of updated weights has been read
+    }
+    if (C > 1) {
+      if (__builtin_amdgcn_readfirstlane(*(const __attribute__((address_space(3))) int*)(lds + G::L_MISC)) != 0) { aborted = true; break; }
+    }
+    if (do_a && (QX || NBK == 4 || hi4 == 0)) {
+      if constexpr (!QX) {
+        const floatx4 o = *(const __attribute__((address_space(3))) floatx4*)(lds + G::L_PS + (v ^ 4) * 1024 + clu_lane() * 16);
+        const floatx4 own = NBK == 4 ? (hi4 ? z[ZN - 1] : z[0]) : z[0];
+        z[0] = NBK == 4 && hi4 ? o + own : own + o;   // lower K half first
+      }
+      const float nlog2e = -1.44269504088896340736f;
+#pragma unroll
+      for (int n = 0; n < FN; n++) {
+        const int rb = QX ? hi4 * (RB / 2) + n : NBK == 4 ? hi4 : (v >> 1) & 1;   // row block (wave-uniform)
+        const unsigned z01 = bf16_pack2(z[n][0], z[n][1]), z23 = bf16_pack2(z[n][2], z[n][3]);
+        const float zf[4] = {__uint_as_float(z01 << 16), __uint_as_float(z01 & 0xFFFF0000u), __uint_as_float(z23 << 16), __uint_as_float(z23 & 0xFFFF0000u)};
+        float s[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) s[e] = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(zf[e] * nlog2e));
+        unsigned s01 = bf16_pack2(s[0], s[1]), s23 = bf16_pack2(s[2], s[3]);
+        // positives of the enclosing 64-row tile (set semantics: a repeated key counts once), eight keys at a time through
+        // the scalar path; a key costs vector instructions only if it lies in this wavefront's block.  Up to seven keys
+        // behind the tile's last are read and ignored; the buffer behind the keys belongs to the workspace.
+        if (p1 > p0) {
+          float sg[4] = {__uint_as_float(s01 << 16), __uint_as_float(s01 & 0xFFFF0000u), __uint_as_float(s23 << 16), __uint_as_float(s23 & 0xFFFF0000u)};
+          const __attribute__((address_space(4))) unsigned* ckeys = (const __attribute__((address_space(4))) unsigned*)p.keys[C == 8 ? m >> 2 : 0];
+          typedef unsigned c_keysx8 __attribute__((ext_vector_type(8), aligned(4)));
+          const unsigned brow0 = (unsigned)(((m * G::SL) & 255) + 16 * b);   // first batch row of this wavefront's block within the key's 256
+          const unsigned lbase = p.label0_seg + (unsigned)cur.c * (unsigned)p.rows_per_chunk + (unsigned)(cur.row0 + 16 * rb);
+          unsigned before = p0 > 0 ? ckeys[p0 - 1] : ~ckeys[p0];
+          for (int e0 = p0; e0 < p1; e0 += 8) {
+            const c_keysx8 kk = *(const __attribute__((address_space(4))) c_keysx8*)(ckeys + e0);
+#pragma unroll
+            for (int jj = 0; jj < 8; jj++) {
+              const int ln = clu_lane();
+              const unsigned key = kk[jj];
+              const unsigned lrel = (key >> 8) - lbase, br = (key & 255u) - brow0;
+              if (e0 + jj < p1 && key != before && lrel < 16u && br < 16u) {
+                const bool mine = (unsigned)ln == 16u * (lrel >> 2) + br;
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                  if ((lrel & 3u) == (unsigned)e) sg[e] = mine ? bf16_rt(sg[e] - 1.0f) : sg[e];
+              }
+              before = key;
+            }
+          }
+          s01 = bf16_pack2(sg[0], sg[1]);
+          s23 = bf16_pack2(sg[2], sg[3]);
+        }
+        if (cur.rows_valid < T) {   // rows past the end of the chunk contribute nothing
+          const int r0 = 16 * rb + 4 * (clu_lane() >> 4);
+          if (r0 >= cur.rows_valid) s01 &= 0xFFFF0000u;
+          if (r0 + 1 >= cur.rows_valid) s01 &= 0x0000FFFFu;
+          if (r0 + 2 >= cur.rows_valid) s23 &= 0xFFFF0000u;
+          if (r0 + 3 >= cur.rows_valid) s23 &= 0x0000FFFFu;
+        }
+        const unsigned goff = ((pk_g >> 16) ^ (unsigned)(32 * (rb & 1))) + (unsigned)((rb >> 1) * G::SL * 64);
+        const cux2 sv = cux2{s01, s23};
+        *(__attribute__((address_space(3))) cux2*)(lds + gown + goff) = sv;
+        if constexpr (C > 1) {
+          unsigned char* slot = exch_slot(m, i);
+          asm volatile("global_store_dwordx2 %0, %1, %2" : : "v"(goff), "v"(sv), "s"(slot) : "memory");
+        }
+      }
+    }
+    // ---- first half of grad_W and update of the tile before (it only needs the partners' G): vector work beside the latencies
+    //      of the sigmoid
+    const unsigned gprev = (unsigned)(G::L_OWN + (C > 1 ? (i - 1) & 1 : 0) * G::GSL);
+    if constexpr (C > 1) {
+      if (i > 0) update_tile(prev, gprev, 0u, CluInt<0>{}, CluInt<RB / 2>{}, [] {});
+      if (do_a) {
+        // this wavefront's part of G(i) has reached the L2 by now: tell the partners
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if (clu_lane() == 0) __hip_atomic_store(cflags + m * 8 + v, i + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __syncthreads();   // own G of tile i is visible
+    // ---- Two jobs are left: grad_X of tile i (matrix instructions) and (the second half of) grad_W and update of this tile
+    //      (cluster of one) or of the one before (vector instructions).  The two wavefronts of a SIMD take them in opposite
+    //      order, so that each runs in the gaps of the other - except with the Philox recipe, where the vector work is several
+    //      times the matrix work and keeping in step measured 2-6 % faster.
+    constexpr bool OPPOSITE = MODE != ROUND_SR_PHILOX;
+    auto update_part = [&] {
+      if constexpr (C == 1) {
+        update_tile(cur, gown, wimg, CluInt<0>{}, CluInt<RB>{}, [] {});
+      } else {
+        auto snapshot = [&] {   // the counters as they are now go to LDS, looked at in the next iteration
+          const int ln = clu_lane();
+          if (v == 0 && ln < 8 * C) clu_lds_load4_l2(cflags + ln, (unsigned)(G::L_MISC + 64));
+        };
+        if (i > 0) update_tile(prev, gprev, 0u, CluInt<RB / 2>{}, CluInt<RB>{}, snapshot);
+        else snapshot();
+      }
+    };
+    auto gradx_part = [&](bool load) {   // load: request the next tile on the way
+      if (!do_a) return;
+      const unsigned wtr_lane = (pk_w & 0xFFFFu) + wimg + (unsigned)(96 * G::WB * v), ga_lane = pk_o >> 16;
+#pragma unroll
+      for (int kt = 0; kt < KT; kt++) {
+        bf16x8 ga[NBK];
+#pragma unroll
+        for (int mb = 0; mb < NBK; mb++)
+          ga[mb] = *(const __attribute__((address_space(3))) bf16x8*)(lds + gown + ga_lane + kt * G::SL * 64 + mb * 1024);
+        // the W operand of a feature block is read one block ahead of its products
+        auto rdw = [&](int nn) {
+          if constexpr (WT == CLU_BF16) {
+            cshortx4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) cshortx4*)(lds + wtr_lane + kt * 32 * LS + nn * 32));
+            cshortx4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) cshortx4*)(lds + wtr_lane + kt * 32 * LS + 8 * LS + nn * 32));
+            return __builtin_bit_cast(bf16x8, cshortx8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]});
+          } else {
+            return __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) intx2*)(lds + wtr_lane + kt * 32 * LS + nn * 16));
+          }
+        };
+        decltype(rdw(0)) wraw[2];
+        wraw[0] = rdw(0);
+#pragma unroll
+        for (int nn = 0; nn < 6; nn++) {
+          if (nn + 1 < 6) wraw[(nn + 1) & 1] = rdw(nn + 1);
+          bf16x8 wb;
+          if constexpr (WT == CLU_BF16) wb = wraw[nn & 1];
+          else wb = clu_widen8(wraw[nn & 1]);
+#pragma unroll
+          for (int mb = 0; mb < NBK; mb++) acc[mb][nn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ga[mb], wb, acc[mb][nn], 0, 0, 0);
+          // the next tile, spread over the products: issued together the loads of eight wavefronts fill the memory pipeline's
+          // queue and block them
+          if (C > 1 && kt == 0 && nn < 4 && load && i + 1 < n_it) load_pieces(nxt, (i + 1) & 1, nn * (G::WPIECES / 4), (nn + 1) * (G::WPIECES / 4));
+          CFENCE();
+        }
+      }
+      if (i + 1 == n_it || (p.flush && nxt.c != cur.c)) store_acc(p.flush ? j + cur.c : j);
+    };
+    if constexpr (OPPOSITE) {
+      if (C > 1 && hi4 && i + 1 < n_it) load_tile(nxt, (i + 1) & 1);
+#pragma unroll 1
+      for (int ph = 0; ph < 2; ph++) {
+        asm volatile("" : "+s"(kp), "+s"(v), "+s"(m), "+s"(j), "+s"(b), "+s"(hi4));
+        COPAQUE(pk_w); COPAQUE(pk_g); COPAQUE(pk_o);
+        if (ph == hi4) gradx_part(hi4 == 0);
+        else update_part();
+      }
+    } else {
+      gradx_part(true);
+      update_part();
+    }
+    if constexpr (C > 1) {
+      if (do_a) {
+#pragma unroll
+        for (int k = 0; k < G::NBLK; k++)
+#pragma unroll
+          for (int n = 0; n < RB; n++)
+            if (takes(k, n)) read_old(wimg, k, row_block(n), wold[k][n]);
+      }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // tile i+1 has landed
+    prev2 = prev;
+    prev = cur;
+    cur = nxt;
+  }
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+  __syncthreads();
+  // the last tile's image; prev is the tile of the last iteration (cluster of one) or a repetition of it (the iteration
+  // behind the last tile)
+  if (!aborted && n_it > 0) store_out(C > 1 ? prev2 : prev);
+#undef p
+}
+
+// The variants, one translation unit per arithmetic (bf16 weights; e4m3 weights with bf16 products; e4m3 with FP8 logits).
+// c: workgroups of a cluster (1, 2, 4, 8; FP8 logits: 2, 4, 8), nbk: 16-row batch blocks of a member (4, or 2 with c = 1).
+typedef void (*clu_kernel_t)(const ClusterParams);
+struct ClusterVariant { clu_kernel_t fn; int lds; };
+ClusterVariant cluster_variant_bf16(int c, int nbk, int round_mode);
+ClusterVariant cluster_variant_sim(int c, int nbk, int round_mode);
+ClusterVariant cluster_variant_fp8(int c, int nbk, int round_mode);
+void cluster_set_lds_bf16();
+void cluster_set_lds_sim();
+void cluster_set_lds_fp8();
+
+#ifdef CLU_VARIANT   // a translation unit of variants: CLU_VARIANT(function suffix) with CLU_WT, CLU_QX
+#define CLU_PICK(C, NBK)                                                                                                         \
+  do {                                                                                                                           \
+    if (round_mode == ROUND_RTN) return {cluster_step_kernel<CLU_WT, CLU_QX, C, NBK, ROUND_RTN>, CluGeom<CLU_WT, CLU_QX, C, NBK>::LDS};            \
+    if (round_mode == ROUND_SR_FAST) return {cluster_step_kernel<CLU_WT, CLU_QX, C, NBK, ROUND_SR_FAST>, CluGeom<CLU_WT, CLU_QX, C, NBK>::LDS};    \
+    return {cluster_step_kernel<CLU_WT, CLU_QX, C, NBK, ROUND_SR_PHILOX>, CluGeom<CLU_WT, CLU_QX, C, NBK>::LDS};                                 \
+  } while (0)
+#define CLU_CAT2(a, b) a##b
+#define CLU_CAT(a, b) CLU_CAT2(a, b)
+ClusterVariant CLU_CAT(cluster_variant_, CLU_VARIANT)(int c, int nbk, int round_mode) {
+#if !CLU_QX
+  if (c == 1 && nbk == 2) CLU_PICK(1, 2);
+  if (c == 1) CLU_PICK(1, 4);
+#endif
+  if (c == 2) CLU_PICK(2, 4);
+  if (c == 4) CLU_PICK(4, 4);
+  CLU_PICK(8, 4);
+}
+void CLU_CAT(cluster_set_lds_, CLU_VARIANT)() {   // opt in to the LDS size, once per device
+  for (int c = CLU_QX ? 2 : 1; c <= 8; c *= 2)
+    for (int nbk = c == 1 ? 2 : 4; nbk <= 4; nbk += 2)
+      for (int mode = 0; mode < 3; mode++) {
+        const ClusterVariant v = CLU_CAT(cluster_variant_, CLU_VARIANT)(c, nbk, mode);
+        (void)hipFuncSetAttribute((const void*)v.fn, hipFuncAttributeMaxDynamicSharedMemorySize, v.lds);
+      }
+}
+#endif
+
+}  // namespace xmc

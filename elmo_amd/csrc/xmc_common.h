@@ -57,6 +57,18 @@ __host__ __device__ inline bool quad_xcc_mismatch(const int* xcc_ids, int quad) 
          xcc_ids[quad_member_workgroup(quad, 3)] != id0;
 }
 
+// The end of a step, one thread of its last kernel: the step's error word joins the sticky word, which no kernel clears (a
+// caller that looks at it only now and then still learns of every failed step), and as long as the sticky word is not zero
+// every step changes the failure word in host memory (to an odd clock reading), which the host can watch without a copy,
+// an event or a wait: a step that went well costs two loads here and nothing on the host.
+__device__ __forceinline__ void report_step_error(const int* err, int* sticky, int* failure_word) {
+  const int e = __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const int before = __hip_atomic_load(sticky, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (e != 0) __hip_atomic_fetch_or(sticky, e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if ((e | before) != 0 && failure_word)
+    __hip_atomic_store(failure_word, (int)__builtin_amdgcn_s_memrealtime() | 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 __device__ __forceinline__ float bf16_rt(float f) { return (float)(__bf16)f; }
 
 // bf16(a) in the low half, bf16(b) in the high half (round to nearest even), one conversion instruction

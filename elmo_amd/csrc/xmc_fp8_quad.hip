@@ -140,14 +140,10 @@ __device__ __forceinline__ QTile q_desc_full(q_cdesc* desc, int t) {
 // threads, (n_pad + 256) * 4 bytes of LDS.
 // Labels are taken relative to label_base, and those outside [label_base, label_base + label_count) are dropped: a
 // label space of 2^24 labels and more is sorted in segments of whole chunks (a key keeps 24 bits for the label).
-__global__ __launch_bounds__(256) void quad_sort_kernel(const int* coo, int nnz, int n_pad, int batch, int row0, int label_base,
-                                                        int label_count, unsigned* keys, int* flags) {
+__device__ __forceinline__ void quad_sort_block(int block, const int* coo, int nnz, int n_pad, int batch, int row0, int label_base,
+                                                int label_count, unsigned* keys) {
   extern __shared__ unsigned sk[];
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63;
-  if (blockIdx.x == 0 && flags)
-    for (int i = tid; i < QF_WORDS; i += 256)
-      if (i != QF_STICKY) flags[i] = 0;
-  if (n_pad == 0) return;
   // eight (row, label) pairs per thread in flight at a time: the loads miss every cache
   const int2* coo2 = (const int2*)coo;
   for (int i0 = tid; i0 < n_pad; i0 += 8 * 256) {
@@ -166,7 +162,7 @@ __global__ __launch_bounds__(256) void quad_sort_kernel(const int* coo, int nnz,
     }
   }
   __syncthreads();
-  const int i0 = blockIdx.x * 64;
+  const int i0 = block * 64;
   const unsigned mine = sk[i0 + l];
   const int quarter = n_pad >> 2;
   // keys in front of the workgroup's own 64 precede on <=, keys behind them on <, the own 64 by position; each part
@@ -197,6 +193,13 @@ __global__ __launch_bounds__(256) void quad_sort_kernel(const int* coo, int nnz,
   part[tid] = (unsigned)rank;
   __syncthreads();
   if (w == 0) keys[part[l] + part[64 + l] + part[128 + l] + part[192 + l]] = mine;
+}
+__global__ __launch_bounds__(256) void quad_sort_kernel(const int* coo, int nnz, int n_pad, int batch, int row0, int label_base,
+                                                        int label_count, unsigned* keys, int* flags) {
+  if (blockIdx.x == 0 && flags)
+    for (int i = threadIdx.x; i < QF_WORDS; i += 256)
+      if (i != QF_STICKY) flags[i] = 0;
+  if (n_pad != 0) quad_sort_block((int)blockIdx.x, coo, nnz, n_pad, batch, row0, label_base, label_count, keys);
 }
 
 __device__ __forceinline__ void prep_x_quad_thread(int i, const unsigned short* x, int batch, float inv_scale_x, unsigned char* xq,

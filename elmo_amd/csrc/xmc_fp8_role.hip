@@ -773,18 +773,14 @@ __global__ __launch_bounds__(QNT, 1) void fp8_step_role_kernel(const QuadParams 
 // grad_X = scale * sum over quads of the member partials; writes fp32 and bf16 [batch, 768].  192 workgroups of 128
 // threads: workgroup (block, m, part) covers lanes 128 part.. of the 256 B-wavefront lanes of a step workgroup.
 __global__ __launch_bounds__(128) void reduce_gx_role_kernel(const floatx4* partial, int nwg, float scale, float* gx_f32,
-                                                             unsigned short* gx_bf16, int batch, int* flags, const DropoutParams dp) {
+                                                             unsigned short* gx_bf16, int batch, int* flags, int* failure_word,
+                                                             const DropoutParams dp) {
   // placement check: the members of a quad exchanged G through the L2 of one XCD, which holds only if all four ran there
   if (blockIdx.x == 0) {
     if ((int)threadIdx.x < (nwg >> 2) && quad_xcc_mismatch(flags + QF_XCC, (int)threadIdx.x))
       __hip_atomic_fetch_or(flags + QF_ERR, 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
-    // the error word of this step joins the sticky word, which no kernel clears: a caller that looks at it only now and
-    // then still learns of every failed step
-    if (threadIdx.x == 0) {
-      const int e = __hip_atomic_load(flags + QF_ERR, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (e != 0) __hip_atomic_fetch_or(flags + QF_STICKY, e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    if (threadIdx.x == 0) report_step_error(flags + QF_ERR, flags + QF_STICKY, failure_word);
   }
   const int blk = blockIdx.x >> 3, m = (blockIdx.x >> 1) & 3;   // blk = mb*3+nn
   const int t = (blockIdx.x & 1) * 128 + threadIdx.x, s = t >> 6, lane = t & 63, l16 = lane & 15, kg = lane >> 4;

@@ -85,8 +85,9 @@ __device__ __forceinline__ bf16x8 t_load_w8(const void* w, size_t idx) {
 template <int DD>
 __global__ void tiled_prep_x_kernel(const unsigned short* x, int batch, int halves, int quantize, int fp8_image, int xt_split,
                                     unsigned short* xb, unsigned short* xT, float* gx_total, float* loss_part, int n_loss,
-                                    const DropoutParams dp) {
+                                    int* err, const DropoutParams dp) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i == 0) *err = 0;   // these kernels do not wait for one another: their steps cannot fail
   if (i >= halves * BP * DD) return;
   gx_total[i] = 0.f;
   for (int j = i; j < n_loss; j += halves * BP * DD) loss_part[j] = 0.f;
@@ -116,11 +117,6 @@ __global__ void tiled_prep_x_kernel(const unsigned short* x, int batch, int halv
   } else {
     xT[(size_t)half * BP * DD + ((size_t)(blk * (BP / 32) + (bh >> 5)) * 64 + (4 * kgk + e) + 16 * ((bh >> 3) & 3)) * 8 + (bh & 7)] = v;
   }
-}
-
-__global__ void tiled_zero_kernel(float* p, int n) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = 0.f;
 }
 
 // ---- logits, sigmoid minus targets.  Persistent workgroups of 8 wavefronts; wavefront v keeps the X operand of batch

@@ -7,7 +7,7 @@ from . import _lib
 
 FEATURES = 768
 MAX_BATCH = 128          # fused step
-MAX_BATCH_TILED = 512    # three-kernel step: up to four halves of 128 rows
+MAX_BATCH_TILED = 512    # tiled step
 
 
 def _stream_ptr():
@@ -241,7 +241,7 @@ def dropout_quantize(x, p, seed):
 WEIGHT_TYPES = {"e4m3": 0, "bf16": 1}
 
 
-TILED_FEATURES = (768, 1024)   # input widths of the three-kernel path
+TILED_FEATURES = (768, 1024)   # input widths of the tiled step
 
 
 def tiled_workspace_bytes(num_chunks, rows_per_chunk, max_batch=MAX_BATCH, features=FEATURES):
@@ -252,15 +252,34 @@ def tiled_workspace_bytes(num_chunks, rows_per_chunk, max_batch=MAX_BATCH, featu
 
 
 def alloc_tiled_workspace(num_chunks, rows_per_chunk, device, max_batch=MAX_BATCH, features=FEATURES):
-    return torch.empty(tiled_workspace_bytes(num_chunks, rows_per_chunk, max_batch, features), dtype=torch.uint8,
-                       device=device)
+    ws = torch.empty(tiled_workspace_bytes(num_chunks, rows_per_chunk, max_batch, features), dtype=torch.uint8, device=device)
+    off = tiled_sticky_error_offset()       # as in alloc_workspace
+    ws[off:off + 4].zero_()
+    return ws
+
+
+def tiled_error_offset():
+    """Byte offset of the tiled step's error word (int32) inside its workspace."""
+    return int(_lib.load().xmc_tiled_error_offset())
+
+
+def tiled_sticky_error_offset():
+    """Byte offset of its sticky error word (int32): the error words of all steps since it was last zeroed."""
+    return int(_lib.load().xmc_tiled_sticky_error_offset())
+
+
+def sticky_error_words(workspace=None, tiled_workspace=None):
+    """The sticky error words of a layer's workspaces as int32 device tensors of one element."""
+    pairs = ((workspace, step_sticky_error_offset()), (tiled_workspace, tiled_sticky_error_offset()))
+    return [ws[off:off + 4].view(torch.int32) for ws, off in pairs if ws is not None]
 
 
 def tiled_step(chunk_views, rows_per_chunk, weight_type, x, labels, lr, seeds=None, round_mode="rtn", workspace=None,
                grad_out=None, want_f32=False, quantize_x=False, saturate=False, kahan=None, num_head=0, loss_out=None,
                weight_decay=0.0, dropout_p=0.0, dropout_seed=0):
     """One training step of the bf16 layer (chunked.py:76-133) or of the simulated-FP8 mode of the FP8 layer
-    (chunked_fp8xmc_clf.py:98-99,110,115-116), three kernels per chunk.  `chunk_views` are contiguous [rows, d]
+    (chunked_fp8xmc_clf.py:98-99,110,115-116): one kernel over all chunks, or three per chunk (1024 features, `kahan`,
+    `loss_out`, weight decay).  `chunk_views` are contiguous [rows, d]
     tensors with d = 768 or 1024 (views of one weight tensor, or the FP8 layer's chunk parameters): all have rows_per_chunk rows except the
     last, which may be shorter.  Updated in place; returns grad_input (bf16) or (grad_input, grad_x_fp32).
     e4m3 weights: quantize_x / saturate select the true-FP8 arithmetic (logits from e4m3(X), saturating cast) instead of

@@ -36,7 +36,7 @@ CONFIGS = {
     "cfg3_simfp8_500k": StepConfig("cfg3_simfp8_500k", 500000, 128, 768, 65536, 4.8, 1.05, 3, "e4m3"),
     "cfg4_fp8_3m": StepConfig("cfg4_fp8_3m", 2812281, 128, 768, 131072, 36.0, 0.9, 4, "e4m3"),
     "cfg5_fp8_8m6": StepConfig("cfg5_fp8_8m6", 8600000, 256, 768, 262144, 8.0, 1.1, 5, "e4m3"),
-    # the first and the third workload with an encoder of 1024 features (three-kernel path)
+    # the first and the third workload with an encoder of 1024 features (tiled step)
     "cfg1_bf16_131k_d1024": StepConfig("cfg1_bf16_131k_d1024", 131072, 32, 1024, 16384, 5.0, 1.1, 0, "bf16"),
     "cfg3_simfp8_500k_d1024": StepConfig("cfg3_simfp8_500k_d1024", 500000, 128, 1024, 65536, 4.8, 1.05, 3, "e4m3"),
 }

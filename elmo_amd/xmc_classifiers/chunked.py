@@ -4,7 +4,8 @@ Mirror of the reference's XMCBCECHUNKEDLayer (src/xmc_classifiers/chunked.py): s
 (`xfc_forward`, `xfc_forward_backward`), attributes (`xfc_weight` - ONE [num_labels, 768] tensor, a plain attribute and
 not a Parameter, as there - `grad_input`, `_dtype`, `num_labels`, `num_chunks`, `chunk_size`, `iteration`, `loss`) and
 error convention.  The reference's per-chunk sequence (matmul, sigmoid, index_put, matmul, mm, sgd_update with
-stochastic rounding; chunked.py:97-127) is one call into the C ABI, three kernels per chunk.
+stochastic rounding; chunked.py:97-127) is one call into the C ABI: one kernel over all
+chunks (three per chunk with 1,024 features or when the loss is asked for).
 
 The bf16 weight type - the one the reference's stochastic-rounding kernel serves (chunked.py:125-127) - runs on the
 gfx950 kernels.  As in the reference's bf16 path, weight decay and momentum are not applied there
@@ -23,6 +24,7 @@ import torch
 from torch import nn
 
 from .. import ops
+from ..step_errors import StepErrors
 
 dtype_map = {'float16': torch.float16, 'bfloat16': torch.bfloat16, 'float32': torch.float32,
              'float8': torch.float8_e4m3fn}
@@ -80,6 +82,7 @@ class XMCBCECHUNKEDLayer(nn.Module):
             self._workspace = ops.alloc_tiled_workspace(self.num_chunks, self.chunk_size, self.device,
                                                         min(max(int(cfg.data.batch_size), ops.MAX_BATCH), ops.MAX_BATCH_TILED),
                                                         features)
+            self._errors = StepErrors(self.device, ops.sticky_error_words(tiled_workspace=self._workspace))
 
     def _chunks(self):
         w = self.xfc_weight
@@ -132,6 +135,7 @@ class XMCBCECHUNKEDLayer(nn.Module):
         lab = labels if labels.dtype == torch.int32 else labels.to(torch.int32)
         lab = lab.contiguous()
         loss = 0
+        self._errors.check()      # a failure of an earlier step, without waiting
         views = self._chunks()
         # one seed per chunk from the global CPU generator, as the reference draws them (chunked.py:126)
         seeds = [torch.randint(0, 1000000, (1,)).item() for _ in range(len(views))]
@@ -142,6 +146,11 @@ class XMCBCECHUNKEDLayer(nn.Module):
         if loss_out is not None:
             loss = loss_out.item()
         return loss
+
+    def check_steps(self):
+        """Waits for the steps enqueued so far and raises if any of them failed.  Not part of the reference's interface."""
+        if self._workspace is not None:
+            self._errors.check_now()
 
     def _dense_step(self, embed, labels, xmc_lr, skip_loss):
         """fp32 / fp16 weights: chunked.py:85-124 operation by operation (library GEMMs and elementwise operations in the

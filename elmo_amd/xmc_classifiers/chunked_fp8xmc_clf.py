@@ -26,6 +26,7 @@ import torch
 from torch import nn
 
 from .. import ops
+from ..step_errors import StepErrors
 
 dtype_map = {'float16': torch.float16, 'bfloat16': torch.bfloat16, 'float32': torch.float32,
              'float8': torch.float8_e4m3fn}
@@ -60,7 +61,7 @@ class Fp8XMCBCEChunkedLayer(nn.Module):
         assert self.device.type == "cuda", "Fp8XMCBCEChunkedLayer needs a GPU device: there is no CPU path"
         self.features = features
         # The fused step and the inference kernels are built for 768 features.  A layer of 1,024 trains on the
-        # three-kernel path (same arithmetic, rounding modes and random words) and takes its inference logits from a
+        # tiled step (same arithmetic, rounding modes and random words) and takes its inference logits from a
         # library GEMM per chunk on the exactly widened operands, as the reference does (:52-55).
         self._other_width = features != ops.FEATURES
 
@@ -78,7 +79,7 @@ class Fp8XMCBCEChunkedLayer(nn.Module):
             assert self.xfc_weight[i].shape[0] == self.num_labels_i
         assert n_labels == self.num_labels
 
-        # simulated FP8 (:98-99,115-116) runs on the three-kernel path, which rounds with the reference's recipe
+        # simulated FP8 (:98-99,115-116) runs on the tiled step, which rounds with the reference's recipe
         self.rounding = _opt(cfg.training.xmc, "rounding", "sr_philox" if self.fake_fp8_matmul else "sr_fast")
         assert self.rounding in (("sr_philox", "rtn") if self.fake_fp8_matmul else ("sr_fast", "sr_philox", "rtn"))
         self.scale_w = float(_opt(cfg.training.xmc, "scale_w", 1.0))
@@ -94,22 +95,12 @@ class Fp8XMCBCEChunkedLayer(nn.Module):
         self._workspace = (None if self._other_width else
                            ops.alloc_workspace(self.num_chunks, self.num_labels_i, self.device))
         self._tiled_workspace = None
-        self._fused_ran = False      # the error word in the workspace is defined once a fused step has run
-        # After every fused step the workspace's sticky error word (the error words of all steps since it was last
-        # zeroed, OR-ed together by the kernels) is copied to pinned host memory on the step's stream, without waiting;
-        # later calls look at the copies that have arrived (see _check_previous_steps).  A ring of slots, so that a copy
-        # still in flight is never overwritten by the next one.
-        off = ops.step_sticky_error_offset()
-        self._err_dev = None if self._other_width else self._workspace[off:off + 4].view(torch.int32)
-        self._err_slots = 4
-        self._err_host = torch.zeros(self._err_slots, dtype=torch.int32).pin_memory()
-        self._err_events = [None] * self._err_slots
-        self._err_next = 0
-        # batches of more than 128 rows (up to 512) also run on the three-kernel path, with the true-FP8 arithmetic
+        self._last = None            # workspace of the last step: its error word is defined from then on
+        # batches of more than 128 rows (up to 512) also run on the tiled step, with the true-FP8 arithmetic
         self._max_batch = int(_opt(cfg.data, "batch_size", ops.MAX_BATCH))
         if self.fake_fp8_matmul:
             assert self.scale_w == 1.0 and self.scale_x == 1.0, "simulated FP8 has no per-tensor scales"
-        # the fused kernel's sort keys hold 24 bits of label: larger label spaces run on the three-kernel path, which sorts
+        # the fused kernel's sort keys hold 24 bits of label: larger label spaces run on the tiled step, which sorts
         # the positives per segment of the label space
         self._wide = self.num_labels >= (1 << 24) - 1
         if self._other_width:
@@ -118,6 +109,7 @@ class Fp8XMCBCEChunkedLayer(nn.Module):
             self._tiled_workspace = ops.alloc_tiled_workspace(self.num_chunks, self.num_labels_i, self.device,
                                                               min(max(self._max_batch, ops.MAX_BATCH), ops.MAX_BATCH_TILED),
                                                               features)
+        self._errors = StepErrors(self.device, ops.sticky_error_words(self._workspace, self._tiled_workspace))
 
     def _chunks(self):
         return [w.data for w in self.xfc_weight]
@@ -181,7 +173,7 @@ class Fp8XMCBCEChunkedLayer(nn.Module):
         Computes activation gradients for the XMC layer fused with BCE Loss and applies the SGD update.
         Args:
             embed: Encoder or bottleneck layer output, bf16 [B, 768] or [B, 1024], B a multiple of 16 and <= 512 (the
-                   fused kernel takes up to 128 rows of 768 features, everything else runs on the three-kernel path).
+                   fused kernel takes up to 128 rows of 768 features, everything else runs on the tiled step).
             labels: Positive labels in sparse format, int32 [Nb, 2] = (row in batch, label id).
             xmc_lr: list of learning rates, only [0] is used.
             skip_loss: ignored, as in the reference's FP8 layer; the return value is 0.
@@ -197,6 +189,7 @@ class Fp8XMCBCEChunkedLayer(nn.Module):
         lab = labels if labels.dtype == torch.int32 else labels.to(torch.int32)
         lab = lab.contiguous()
         loss = 0
+        self._check_previous_steps()
         # one seed per chunk from the global CPU generator, exactly as the reference draws them (:113)
         seeds = [torch.randint(0, 1000000, (1,)).item() for _ in range(self.num_chunks)]
         extra = dict(weight_decay=self.weight_decay)
@@ -205,65 +198,52 @@ class Fp8XMCBCEChunkedLayer(nn.Module):
         if self.fake_fp8_matmul:
             self.grad_input = ops.tiled_step(self._chunks(), self.num_labels_i, "e4m3", x, lab, xmc_lr[0], seeds=seeds,
                                              round_mode=self.rounding, workspace=self._tiled_workspace, **extra)
+            self._last = self._tiled_workspace
         elif embed.shape[0] > ops.MAX_BATCH or self._wide or self._other_width:
-            # the fused kernel holds 128 batch rows; larger batches take the three-kernel path with the same arithmetic
+            # the fused kernel holds 128 batch rows; larger batches take the tiled step with the same arithmetic
             # (logits from e4m3(X), saturating cast) and the same rounding modes and random words
             assert self.scale_w == 1.0 and self.scale_x == 1.0, "per-tensor scales need a batch of at most 128 rows of 768 features"
             self.grad_input = ops.tiled_step(self._chunks(), self.num_labels_i, "e4m3", x, lab, xmc_lr[0], seeds=seeds,
                                              round_mode=self.rounding, workspace=self._tiled_workspace, quantize_x=True,
                                              saturate=True, **extra)
+            self._last = self._tiled_workspace
         else:
-            self._check_previous_steps()
             self.grad_input = ops.fp8_step(self._chunks(), x, lab, xmc_lr[0], seeds=seeds, round_mode=self.rounding,
                                            scale_w=self.scale_w, scale_x=self.scale_x, workspace=self._workspace, **extra)
-            self._fused_ran = True
-            # the sticky error word follows the step on the stream into pinned host memory; nobody waits for it here
-            slot = self._err_next
-            if self._err_events[slot] is not None:
-                self._err_events[slot].synchronize()      # that copy was enqueued four steps ago
-                self._raise_on_error(int(self._err_host[slot]))
-            self._err_host[slot:slot + 1].copy_(self._err_dev, non_blocking=True)
-            ev = torch.cuda.Event()
-            ev.record()
-            self._err_events[slot] = ev
-            self._err_next = (slot + 1) % self._err_slots
+            self._last = self._workspace
         self.iteration += 1
         return loss
 
-    def _raise_on_error(self, word):
-        if word != 0:
-            self._err_dev.zero_()                 # on the stream, behind every step enqueued so far
-            self._err_host.zero_()
-            self._err_events = [None] * self._err_slots
-            raise RuntimeError(
-                f"a fused classifier step failed (error word {word}): "
-                + ("a workgroup gave up waiting for its partners (another stream kept the device busy?); " if word & 1 else "")
-                + ("the workgroups of a quad were not placed on one XCD; " if word & 2 else "")
-                + "the weights and grad_input of that step are incomplete")
+    @property
+    def _err_dev(self):
+        """The sticky error word of the fused step's workspace."""
+        return self._errors.words[0]
+
+    @property
+    def _err_host(self):
+        """Non-zero if a step on the device has announced a failure that this layer has not looked into."""
+        return torch.tensor([int(self._errors.pending())])
 
     def _check_previous_steps(self):
-        """Raises if a fused step reported a failure and a copy of the sticky error word taken behind it has reached the
-        host.  Never waits: a copy that is still on its way is looked at by a later call.  The word is sticky, so a
-        failure is not lost when later, clean steps have run in between."""
-        for slot in range(self._err_slots):
-            ev = self._err_events[slot]
-            if ev is not None and ev.query():
-                self._err_events[slot] = None
-                self._raise_on_error(int(self._err_host[slot]))
+        """Raises if a step of this layer has reported a failure.  Never waits unless some step on the device has.  The
+        word behind it is sticky, so a failure is not lost when later, clean steps have run in between."""
+        self._errors.check()
 
     def check_steps(self):
         """Waits for the steps enqueued so far and raises if any of them failed (the end of a run, a checkpoint).  Not
         part of the reference's interface."""
-        if self._fused_ran:
-            torch.cuda.current_stream().synchronize()
-            self._raise_on_error(int(self._err_dev.item()))
+        if self._last is not None:
+            self._errors.check_now()
 
     def last_step_error(self):
-        """Error word of the last fused step (0 = fine; non-zero = a workgroup gave up waiting for its partners, e.g.
+        """Error word of the last step (0 = fine; non-zero = a workgroup gave up waiting for its partners, e.g.
         because another stream kept the device busy, and that step's results are invalid).  Synchronises the stream.
         Not part of the reference's interface."""
-        if not self._fused_ran:
+        if self._last is None:
             return 0
+        if self._last is self._tiled_workspace:
+            off = ops.tiled_error_offset()
+            return int(self._last[off:off + 4].view(torch.int32).item())
         return ops.step_error_word(self._workspace, self.num_chunks, self.xfc_weight[0].shape[0])
 
     def filter_non_local_inds(self, rows, cols, start, end):

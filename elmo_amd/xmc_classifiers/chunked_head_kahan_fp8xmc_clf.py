@@ -9,7 +9,7 @@ Without the compensation buffer (using_head_kahan false) and without simulated F
 Fp8XMCBCEChunkedLayer.  With the buffer the step is the fused kernel as well (ops.fp8_kahan_step: the tiles that hold
 head rows run first, in a variant of the kernel that carries the Kahan recurrence of fuse_kernel.py:202-262 for the
 first num_head rows of chunk 0; the other tiles follow in the plain kernel) whenever the batch is a multiple of 16;
-any other batch runs on the three-kernel path in the same true-FP8 arithmetic (logits from e4m3(X), saturating cast).
+any other batch runs on the tiled step in the same true-FP8 arithmetic (logits from e4m3(X), saturating cast).
 As in the reference, simulated FP8 takes precedence over the compensation (:122-124).
 
 Optional, not in the reference: training.xmc.rounding ("sr_philox" default with simulated FP8, else "sr_fast"; "rtn").
@@ -18,6 +18,7 @@ import torch
 from torch import nn
 
 from .. import ops
+from ..step_errors import StepErrors
 from .chunked_fp8xmc_clf import _opt
 
 dtype_map = {'float16': torch.float16, 'bfloat16': torch.bfloat16, 'float32': torch.float32,
@@ -43,7 +44,7 @@ class Fp8XMCBCEChunkedHeadKahanLayer(nn.Module):
         features = cfg.model.xmc.input_features
         assert features in ops.TILED_FEATURES, f"the gfx950 kernels are built for {ops.TILED_FEATURES} input features"
         self.features = features
-        # 768 features: fused step and inference kernel; 1,024: three-kernel path (same arithmetic) and a library GEMM per
+        # 768 features: fused step and inference kernel; 1,024: tiled step (same arithmetic) and a library GEMM per
         # chunk on the exactly widened operands for inference, as the reference does (:64-67)
         self._other_width = features != ops.FEATURES
         assert self.device.type == "cuda", "Fp8XMCBCEChunkedHeadKahanLayer needs a GPU device: there is no CPU path"
@@ -77,6 +78,7 @@ class Fp8XMCBCEChunkedHeadKahanLayer(nn.Module):
         self._workspace = None if self._other_width else ops.alloc_workspace(self.num_chunks, self.num_labels_i, self.device)
         self._tiled_workspace = (ops.alloc_tiled_workspace(self.num_chunks, self.num_labels_i, self.device, ops.MAX_BATCH,
                                                            features) if self._tiled else None)
+        self._errors = StepErrors(self.device, ops.sticky_error_words(self._workspace, self._tiled_workspace))
 
     def _chunks(self):
         return [w.data for w in self.xfc_weight]
@@ -122,6 +124,7 @@ class Fp8XMCBCEChunkedHeadKahanLayer(nn.Module):
         lab = labels if labels.dtype == torch.int32 else labels.to(torch.int32)
         lab = lab.contiguous()
         loss = 0
+        self._errors.check()      # a failure of an earlier step, without waiting
         seeds = [torch.randint(0, 1000000, (1,)).item() for _ in range(self.num_chunks)]      # :120
         if self.fake_fp8_matmul:
             self.grad_input = ops.tiled_step(self._chunks(), self.num_labels_i, "e4m3", x, lab, xmc_lr[0], seeds=seeds,
@@ -142,6 +145,10 @@ class Fp8XMCBCEChunkedHeadKahanLayer(nn.Module):
                                            workspace=self._workspace)
         self.iteration += 1
         return loss
+
+    def check_steps(self):
+        """Waits for the steps enqueued so far and raises if any of them failed.  Not part of the reference's interface."""
+        self._errors.check_now()
 
     def filter_non_local_inds(self, rows, cols, start, end):
         mask = (cols >= start) & (cols < end)

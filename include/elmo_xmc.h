@@ -244,6 +244,13 @@ int xmc_tiled_step_ex(void* const* chunk_ptrs, int num_chunks, int rows_per_chun
                       int num_head, float weight_decay, float dropout_p, unsigned long long dropout_seed, void* grad_x_bf16,
                       float* grad_x_f32, float* loss_out, void* workspace, size_t workspace_bytes, void* stream);
 
+/* Byte offsets, inside the workspace of xmc_tiled_step, of its error word and its sticky error word (one int32 each; no
+ * counterpart in the reference).  With 768 features, without a compensated head, a loss or weight decay, the step is one
+ * persistent kernel; for batches of more than 64 rows the workgroups that share a tile sequence wait for one another as
+ * those of xmc_fp8_step do, with the same bounds, bits and consequences (see there and xmc_step_sticky_error_offset). */
+size_t xmc_tiled_error_offset(void);
+size_t xmc_tiled_sticky_error_offset(void);
+
 /* Measurement aid (no counterpart in the reference): copies `bytes` (a multiple of 16) from src to dst with a plain
  * grid-stride kernel.  Memory-traffic counters are calibrated against this launch of known size. */
 int xmc_copy_probe(void* dst, const void* src, size_t bytes, void* stream);
@@ -261,10 +268,16 @@ size_t xmc_step_error_offset(void);
 
 /* Byte offset of the sticky error word (one int32) inside the workspace (no counterpart in the reference): the last
  * kernel of every fused step ORs the step's error word into it, and no kernel ever clears it.  It is for callers that
- * do not want to synchronise after every step: zero the word once after allocating the workspace, copy it to pinned
- * host memory behind any step (or every few steps) without waiting, and look at a copy whenever one has arrived - a
- * failure of any step since the word was last zeroed is still in it.  Zero it again after handling a failure. */
+ * do not want to synchronise after every step: zero the word once after allocating the workspace and look at it now and
+ * then (xmc_failure_word tells when) - a failure of any step since the word was last zeroed is still in it.  Zero it again
+ * after handling a failure. */
 size_t xmc_step_sticky_error_offset(void);
+
+/* A word of host memory of the current device, there until the process ends (NULL without a usable device; no counterpart
+ * in the reference): it changes whenever a step on the device (fused or tiled) ends while its workspace's sticky error
+ * word is not zero.  Remember its value; when it has changed, wait for the device and look at the sticky word of your own
+ * workspace: the failure may be another's. */
+int* xmc_failure_word(void);
 
 /* Diagnostics of the placement assumption of the fused kernel (no counterpart in the reference).  The kernel builds
  * quads out of workgroups g with equal g % 8 and expects them on one XCD; every workgroup records the XCC id it really

@@ -1,0 +1,108 @@
+"""The one-pass step (bf16 weights, simulated FP8, true FP8 above 128 batch rows) at the sizes where its split changes: the
+cluster sizes' batch limits, partial tiles and chunks, fewer tiles than clusters, chunk boundaries within a cluster's range.
+Oracle and tolerances as in test_tiled_gpu.py."""
+import numpy as np
+import pytest
+
+import helpers as H
+from oracle import codecs as C
+from oracle import step as O
+from test_tiled_gpu import bf16_case, check_bf16_weights, check_gx, run_bf16
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("kind,nc,rows,batch,mode", [
+    ("bf16", 1, 1, 1, "rtn"),                # one label, one row: a cluster of one, 32 batch rows
+    ("bf16", 3, 33, 32, "sr_philox"),        # chunks of one tile and a row
+    ("bf16", 2, 31, 33, "sr_fast"),          # 64 batch rows
+    ("bf16", 40, 320, 64, "rtn"),            # more tiles than clusters, several chunks to a cluster
+    ("bf16", 1, 65, 65, "sr_fast"),          # clusters of two, fewer tiles than clusters
+    ("bf16", 3, 4100, 128, "sr_philox"),
+    ("bf16", 2, 545, 129, "rtn"),            # clusters of four
+    ("bf16", 60, 96, 257, "sr_philox"),      # clusters of eight, a chunk boundary at every third tile
+    ("bf16", 2, 2000, 511, "sr_fast"),
+    ("sim", 2, 48, 32, "sr_philox"),
+    ("sim", 3, 4112, 64, "rtn"),
+    ("sim", 2, 2064, 100, "sr_philox"),
+    ("sim", 2, 1040, 250, "rtn"),
+    ("sim", 1, 16, 512, "sr_philox"),
+    ("fp8", 7, 208, 96, "sr_fast"),          # clusters of two, tiles of 64 rows
+    ("fp8", 1, 16, 144, "rtn"),              # clusters of four, a single partial tile
+    ("fp8", 3, 3088, 256, "sr_philox"),
+    ("fp8", 2, 1040, 272, "sr_fast"),        # clusters of eight, tiles of 32 rows
+    ("fp8", 5, 848, 512, "rtn"),
+])
+def test_one_pass_step_matches_the_oracle(gpu, kind, nc, rows, batch, mode):
+    from elmo_amd import ops
+    seeds = None if mode == "rtn" else [77 + 31 * c for c in range(nc)]
+    L = nc * rows - (nc - 1 if kind == "bf16" else 0)      # bf16: the last chunk is shorter
+    edges = np.array([[batch - 1, L - 1], [0, 0], [0, 0], [batch // 2, min(rows, L - 1)], [batch // 2, rows - 1]], np.int32)
+    if kind == "bf16":
+        x, w, labels = bf16_case(L, batch, 500 + batch)
+        labels = np.concatenate([edges, labels])
+        new, gf, gb = run_bf16(x, w, labels, nc, gpu, mode, seeds)
+        sr = {"rtn": "rtn", "sr_philox": "reference", "sr_fast": "fast"}[mode]
+        ref_w, ref_gx, _ = O.bf16_step(w, x, labels, 0.05, nc, seeds=seeds, sr_mode=sr)
+        check_bf16_weights(new, ref_w, w, x)
+        check_gx(gf, gb, ref_gx, tol=4e-3)
+        return
+    case = H.make_case(nc, rows, batch, 500 + batch, extra_labels=edges.tolist())
+    chunks, x, labels = H.to_device_case(case, gpu)
+    true_fp8 = kind == "fp8"
+    g, gf = ops.tiled_step(chunks, rows, "e4m3", x, labels, 0.05, seeds=seeds, round_mode=mode, want_f32=True,
+                           quantize_x=true_fp8, saturate=true_fp8)
+
+    def rand_fn(c, offs):
+        return C.fast_sr_words(seeds[c], c * rows + offs // 768, offs % 768)
+
+    kw = dict(sr_mode="exact", rand_fn=rand_fn) if mode == "sr_fast" else dict(sr_mode="rtn" if mode == "rtn" else "reference", seeds=seeds)
+    ref_codes, ref_gx, _ = O.fp8_step(case["chunks"], case["x"], case["labels"], 0.05, simulated=not true_fp8, **kw)
+    dist = np.concatenate([H.e4m3_ulp_distance(a, b).ravel() for a, b in zip(H.chunks_to_numpy(chunks), ref_codes)])
+    assert dist.max() <= 1 and (dist != 0).mean() < 5e-3, (dist.max(), (dist != 0).mean())
+    check_gx(gf.cpu().numpy(), g.float().cpu().numpy(), ref_gx)
+
+
+def test_one_pass_step_gives_up_cleanly(gpu):
+    """A polling limit of 0, set from the host: a wait that is not satisfied at once ends the workgroup's walk.  Every kernel
+    ends, the error words say so, no weight is updated from missing data, the layer raises, and the next step is clean."""
+    import torch
+    from elmo_amd import ops
+    from test_host_cpu import make_cfg
+    from xmc_classifiers.chunked_fp8xmc_clf import Fp8XMCBCEChunkedLayer
+    nc, rows, batch = 2, 8192, 256
+    cfg = make_cfg("cuda:0", nc * rows - 16, nc, rounding="rtn")
+    cfg.data.batch_size = batch
+    xfc = Fp8XMCBCEChunkedLayer(cfg)
+    assert xfc.xfc_weight[0].shape[0] == rows
+    # every label of six tiles positive for the batch rows of the first member: its partners have to wait for it there
+    dense = [[b, 1024 * t + l] for t in range(6) for l in range(64) for b in range(64)]
+    case = H.make_case(nc, rows, batch, 611, extra_labels=dense)
+    chunks, x, labels = H.to_device_case(case, gpu)
+    ref_codes, _, _ = O.fp8_step(case["chunks"], case["x"], case["labels"], 0.05, sr_mode="rtn")
+    prev = ops.debug_spin_limit(0)
+    try:
+        raised = False
+        for attempt in range(8):              # whether a wait finds its counter at once depends on timing
+            for wt, c in zip(xfc.xfc_weight, chunks):
+                wt.data.copy_(c.view(torch.float8_e4m3fn))
+            try:
+                xfc.xfc_forward_backward(x, labels, [0.05])
+                xfc.check_steps()
+            except RuntimeError as e:
+                raised = "gave up waiting" in str(e)
+            assert xfc.last_step_error() == int(raised)
+            for wt, old, ref in zip(xfc.xfc_weight, case["chunks"], ref_codes):
+                new = wt.data.view(torch.uint8).cpu().numpy()
+                # the unit of the update is a member's quarter of the features of a row
+                same_old = (new == old).reshape(-1, 4, 192).all(axis=2)
+                good = (H.e4m3_ulp_distance(new, ref) <= 1).reshape(-1, 4, 192).all(axis=2)
+                assert np.all(same_old | good), "weights were updated from incomplete data"
+            if raised:
+                break
+        assert raised, "no wait expired in eight steps with a polling limit of 0"
+    finally:
+        ops.debug_spin_limit(prev)
+    xfc.xfc_forward_backward(x, labels, [0.05])
+    xfc.check_steps()
+    assert xfc.last_step_error() == 0
