@@ -20,7 +20,7 @@
 //
 // What bounds it: bf16 with a small batch the HBM stream (131 K labels, batch 32, round to nearest: 214 us before, 113 now,
 // 3.6 TB/s of weights); the Philox modes the vector units (143 clocks of the SIMD per 64 weights; 501 K labels, batch 128,
-// bf16: 1142 us before, 809 now; 500 K, e4m3: 1086 / 821; 131 K, batch 512: 882 / 601); true FP8 with batch 256 the length
+// bf16: 1142 us before, 780 now; 500 K, e4m3: 1086 / 784; 131 K, batch 512: 882 / 600); true FP8 with batch 256 the length
 // of an iteration's dependent phases, about 40 % of whose cycles issue something (8.6 M labels: 11.07 ms before, 10.00 now).
 #include "xmc_common.h"
 
@@ -129,10 +129,10 @@ __device__ __forceinline__ bf16x8 clu_widen8(intx2 raw) {   // eight e4m3 codes 
 }
 
 // Four consecutive features of one row: t = w - lr a, rounded (definitions: the comment in front of tiled_update_kernel).
-// a is rounded to bf16 first with bf16 weights.
-template <int WT, int MODE>
+// a is rounded to bf16 first with bf16 weights.  rw: the Philox words, if they have been computed before (PRE).
+template <int WT, int MODE, bool PRE>
 __device__ __forceinline__ void clu_update4(floatx4 a, const unsigned (&wr)[WT == CLU_BF16 ? 2 : 1], float lr, unsigned off0, unsigned fidx,
-                                            unsigned seed, unsigned (&wo)[WT == CLU_BF16 ? 2 : 1]) {
+                                            unsigned seed, const unsigned (&rw)[WT == CLU_BF16 ? 2 : 4], unsigned (&wo)[WT == CLU_BF16 ? 2 : 1]) {
   float w[4], t[4];
   if constexpr (WT == CLU_BF16) {
     w[0] = __uint_as_float(wr[0] << 16); w[1] = __uint_as_float(wr[0] & 0xFFFF0000u);
@@ -148,11 +148,11 @@ __device__ __forceinline__ void clu_update4(floatx4 a, const unsigned (&wr)[WT =
   for (int e = 0; e < 4; e++) {
     t[e] = __builtin_fmaf(-lr, a[e], w[e]);
     if (MODE == ROUND_SR_PHILOX) {
-      const unsigned r = philox_word0(off0 + (unsigned)e, seed, 0u);
+      const unsigned r = !PRE ? philox_word0(off0 + (unsigned)e, seed, 0u) : WT == CLU_E4M3 ? rw[e & (WT == CLU_BF16 ? 1 : 3)] : e & 1 ? rw[e >> 1] >> 16 : rw[e >> 1];
       const unsigned mask = WT == CLU_BF16 ? 0xFFFFu : 0xFFFFFu;
       unsigned tb = __float_as_uint(t[e]) + (r & mask);
       if (WT == CLU_E4M3) tb &= ~mask;   // (bf16: the lower half is dropped by the pack below)
-      asm volatile("" : "+v"(off0), "+v"(tb));   // one chain of ten rounds at a time: no registers for four
+      if (!PRE) asm volatile("" : "+v"(off0), "+v"(tb));   // one chain of ten rounds at a time: no registers for four
       t[e] = __uint_as_float(tb);
     }
   }
@@ -357,6 +357,48 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
   };
   unsigned wold[C > 1 ? G::NBLK : 1][C > 1 ? RB : 1][WDW];   // clusters of several: the weights the lagging update starts from
 
+  // ---- The words of the Philox recipe, the larger part of the update's vector work, depend on nothing but the element's
+  //      place: up to three blocks' words per half of the update are computed between the matrix instructions of the logits
+  //      (first half) and of grad_X (second half), whose operand reads and pipeline leave the vector units idle.  Only where
+  //      the words' registers do not make the loop spill.  With the falling priorities: 501 K labels, bf16, batch 128 812 us
+  //      without, 780 with; 500 K, e4m3 824 / 784.
+  constexpr bool EARLY = MODE == ROUND_SR_PHILOX && !QX && (C == 2 || (C == 1 && (WT == CLU_BF16 || NBK == 2))), EARLY2 = EARLY && (NBK == 2 || (WT == CLU_E4M3 && C == 2));
+  constexpr int NBE = G::NBLK < 3 ? G::NBLK : 3, EP = 8 * NBE;   // blocks; pieces (half an evaluation each)
+  constexpr int RWN = WT == CLU_BF16 ? 2 : 4;                    // registers of four words (bf16 weights take 16 bits of each)
+  unsigned rw[C == 1 ? 2 : 1][EARLY ? NBE : 1][RWN];
+  // In long stretches of vector work the priority falls with the progress, so that the wavefront of a SIMD that is behind
+  // goes first: otherwise the older one finishes early and waits, and one wavefront alone issues at half the rate of two.
+  auto priority = [](int level) {
+    if (level == 3) __builtin_amdgcn_s_setprio(3);
+    else if (level == 2) __builtin_amdgcn_s_setprio(2);
+    else if (level == 1) __builtin_amdgcn_s_setprio(1);
+    else __builtin_amdgcn_s_setprio(0);
+  };
+  PhiloxState ps;
+  auto element_lanes = [&] { const int ln = clu_lane(); return (unsigned)((ln & 15) * D + 4 * (ln >> 4)); };   // a lane's part of the place
+  auto words = [&](const CluTile& q, auto half_c, unsigned lanes, int p0, int p1) {
+    constexpr int half = decltype(half_c)::value, n = half * (RB / 2);
+    if constexpr (half == 0 ? EARLY : EARLY2) {
+#pragma unroll
+      for (int pc = p0; pc < p1; pc++) {
+        const int k = pc >> 3, e = (pc >> 1) & 3;
+        if (pc % (EP / 4) == 0) priority(3 - pc / (EP / 4));
+        if (!takes(k, n)) continue;
+        if (pc & 1) {
+          philox_rounds<5, 10>(ps, q.seed, 0u);
+          unsigned (&w)[RWN] = rw[C == 1 ? half : 0][k];
+          if (WT == CLU_E4M3) w[e & (RWN - 1)] = ps.c0;
+          else if (e & 1) w[e >> 1] = __builtin_amdgcn_perm(ps.c0, w[e >> 1], 0x05040100u);
+          else w[e >> 1] = ps.c0;
+          COPAQUE(w[WT == CLU_E4M3 ? e & (RWN - 1) : e >> 1]);   // (or the compiler moves the evaluation to the word's use)
+        } else {
+          ps = PhiloxState{lanes + (unsigned)((q.row0 + 16 * row_block(n)) * D + (m * G::FBN + block_of(k)) * 16 + e), 0u, 0u, 0u};
+          philox_rounds<0, 5>(ps, q.seed, 0u);
+        }
+      }
+    }
+  };
+
   // A^T and update of the tile q whose G is complete in LDS (own part at gown), the result to the image of updated weights
   // (row blocks n0 .. n1-1 in this wavefront's order; `between` runs once, in the middle of the last one's vector work)
   auto update_tile = [&](const CluTile& q, unsigned gown, unsigned wimg, auto n0_c, auto n1_c, auto&& between) {
@@ -393,6 +435,7 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
 #pragma unroll
         for (int k = 0; k < G::NBLK; k++) {
           if (!takes(k, n)) continue;
+          if ((MODE == ROUND_SR_PHILOX || QX) && G::NBLK > 1) priority((G::NBLK - 1 - k) * 4 / G::NBLK);
           const floatx4 a = aa[k];
           unsigned wr[WDW], wo[WDW];
           if constexpr (C == 1) {
@@ -403,7 +446,10 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
           }
           const int lb = block_of(k);
           const unsigned col = (unsigned)((m * G::FBN + lb) * 16 + 4 * kg);
-          clu_update4<WT, MODE>(a, wr, lr, orow * (unsigned)D + col, (grow0 + row) * (unsigned)(D / 4) + (col >> 2), seed, wo);
+          if (EARLY && k < NBE && (n == 0 || (EARLY2 && n == RB / 2)))
+            clu_update4<WT, MODE, true>(a, wr, lr, 0u, 0u, seed, rw[C == 1 ? n / (RB / 2) : 0][k < NBE ? k : 0], wo);
+          else
+            clu_update4<WT, MODE, false>(a, wr, lr, orow * (unsigned)D + col, (grow0 + row) * (unsigned)(D / 4) + (col >> 2), seed, {}, wo);
           if constexpr (WT == CLU_BF16) {
             *(__attribute__((address_space(3))) cux2*)(lds + G::L_OUT + row * G::ORS + (unsigned)(((2 * lb + (kg >> 1)) ^ (l16 & G::OSW)) * 16 + 8 * (kg & 1))) = cux2{wo[0], wo[1]};
           } else {
@@ -482,7 +528,7 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
     if (C > 1 && i > 0) {
       // the partners' G of tile i-1: normally they had published it when the counters were read at the end of the
       // iteration before
-      constexpr unsigned long long ALL = C == 8 ? ~0ull : (1ull << (8 * C)) - 1ull;
+      constexpr unsigned long long ALL = C == 8 ? ~0ull : (1ull << (8 * C & 63)) - 1ull;
       const int seen = *(const __attribute__((address_space(3))) int*)(lds + G::L_MISC + 64 + 4 * (clu_lane() & (8 * C - 1)));
       if ((__builtin_amdgcn_ballot_w64(seen >= i) & ALL) != ALL) {
         for (int spin = 0;; spin++) {
@@ -517,6 +563,8 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
       for (int n = 0; n < ZN; n++) z[n] = floatx4{0.f, 0.f, 0.f, 0.f};
       const unsigned rb0 = QX ? (unsigned)(hi4 * (RB / 2) * 16 * LS) : NBK == 4 ? 0u : (unsigned)(((v >> 1) & 1) * 16 * LS);
       const unsigned abase = wimg + (pk_w >> 16) + rb0 + (QX ? 0u : (unsigned)(hi4 * (WT == CLU_BF16 ? 768 : 64)));
+      unsigned lanes = EARLY ? element_lanes() : 0u;
+      if (EARLY) COPAQUE(lanes);
       // operands are read three steps ahead of their products
       if constexpr (QX) {
         constexpr int NS = 6 * ZN;
@@ -532,6 +580,7 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
           if (t + 1 < NS) rd(t + 1);
           const intx4 l = lo[t & 1], h = hi[t & 1];
           z[t % ZN] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(intx8{l[0], l[1], l[2], l[3], h[0], h[1], h[2], h[3]}, xq8[t / ZN], z[t % ZN], 0, 0, 0, 0, 0, 0);
+          if constexpr (EARLY) words(C == 1 ? cur : prev, CluInt<0>{}, lanes, t * EP / NS, (t + 1) * EP / NS);
           CFENCE();
         }
       } else if constexpr (WT == CLU_BF16) {
@@ -546,6 +595,7 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
         for (int t = 0; t < NS; t++) {
           if (t + 3 < NS) rd(t + 3);
           z[t % ZN] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[t & 3], xr[t / ZN], z[t % ZN], 0, 0, 0);
+          if constexpr (EARLY) words(C == 1 ? cur : prev, CluInt<0>{}, lanes, t * EP / NS, (t + 1) * EP / NS);
           CFENCE();
         }
       } else {
@@ -562,6 +612,7 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
           const intx4 w4 = wv[t & 3];
           z[t % ZN] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(clu_widen8(intx2{w4.x, w4.y}), xr[2 * (t / ZN)], z[t % ZN], 0, 0, 0);
           z[t % ZN] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(clu_widen8(intx2{w4.z, w4.w}), xr[2 * (t / ZN) + 1], z[t % ZN], 0, 0, 0);
+          if constexpr (EARLY) words(C == 1 ? cur : prev, CluInt<0>{}, lanes, t * EP / NS, (t + 1) * EP / NS);
           CFENCE();
         }
       }
@@ -570,6 +621,8 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
         if (NBK == 4 || hi4 == 1)
           *(__attribute__((address_space(3))) floatx4*)(lds + G::L_PS + v * 1024 + clu_lane() * 16) = NBK == 4 ? (hi4 ? z[0] : z[ZN - 1]) : z[0];
       }
+    } else {
+      if constexpr (EARLY) words(prev, CluInt<0>{}, element_lanes(), 0, EP);
     }
     if (C > 1) {
       if (i > 1) store_out(prev2);   // the weights updated in the iteration before
@@ -676,7 +729,12 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
       }
     };
     auto gradx_part = [&](bool load) {   // load: request the next tile on the way
-      if (!do_a) return;
+      if (!do_a) {
+        if constexpr (EARLY) words(prev, CluInt<1>{}, element_lanes(), 0, EP);
+        return;
+      }
+      unsigned lanes = EARLY ? element_lanes() : 0u;
+      if (EARLY2) COPAQUE(lanes);
       const unsigned wtr_lane = (pk_w & 0xFFFFu) + wimg + (unsigned)(96 * G::WB * v), ga_lane = pk_o >> 16;
 #pragma unroll
       for (int kt = 0; kt < KT; kt++) {
@@ -704,6 +762,7 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
           else wb = clu_widen8(wraw[nn & 1]);
 #pragma unroll
           for (int mb = 0; mb < NBK; mb++) acc[mb][nn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ga[mb], wb, acc[mb][nn], 0, 0, 0);
+          if constexpr (EARLY) words(C == 1 ? cur : prev, CluInt<1>{}, lanes, (6 * kt + nn) * EP / (6 * KT), (6 * kt + nn + 1) * EP / (6 * KT));
           // the next tile, spread over the products: issued together the loads of eight wavefronts fill the memory pipeline's
           // queue and block them
           if (C > 1 && kt == 0 && nn < 4 && load && i + 1 < n_it) load_pieces(nxt, (i + 1) & 1, nn * (G::WPIECES / 4), (nn + 1) * (G::WPIECES / 4));

@@ -96,18 +96,22 @@ __device__ __forceinline__ unsigned xor3(unsigned a, unsigned b, unsigned c) { r
 // vector registers (4.2 against 2.4 clocks), so two of them cost 1.5 x one v_bitop3_b32 (4.2).  Measured, clocks per
 // evaluation and wavefront with 2 wavefronts per SIMD: 145 (189 with pairs of v_xor_b32, which is what the compiler makes of
 // a ^ b ^ c; 283 with separate high and low products).
-__device__ __forceinline__ unsigned philox_word0(unsigned off, unsigned k0, unsigned k1) {
-  unsigned c0 = off, c1 = 0, c2 = 0, c3 = 0;
+struct PhiloxState { unsigned c0, c1, c2, c3; };
+template <int R0, int R1> __device__ __forceinline__ void philox_rounds(PhiloxState& s, unsigned k0, unsigned k1) {   // rounds R0 .. R1-1
 #pragma unroll
-  for (int r = 0; r < 10; r++) {
+  for (int r = R0; r < R1; r++) {
     // one 32 x 32 -> 64 bit multiply per product (both halves are needed)
-    const unsigned long long p0 = (unsigned long long)0xD2511F53u * (unsigned long long)c0;
-    const unsigned long long p1 = (unsigned long long)0xCD9E8D57u * (unsigned long long)c2;
+    const unsigned long long p0 = (unsigned long long)0xD2511F53u * (unsigned long long)s.c0;
+    const unsigned long long p1 = (unsigned long long)0xCD9E8D57u * (unsigned long long)s.c2;
     const unsigned hi0 = (unsigned)(p0 >> 32), lo0 = (unsigned)p0, hi1 = (unsigned)(p1 >> 32), lo1 = (unsigned)p1;
-    c0 = xor3(hi1, c1, k0); c1 = lo1; c2 = xor3(hi0, c3, k1); c3 = lo0;
-    k0 += 0x9E3779B9u; k1 += 0xBB67AE85u;
+    s.c0 = xor3(hi1, s.c1, k0 + (unsigned)r * 0x9E3779B9u); s.c1 = lo1;
+    s.c2 = xor3(hi0, s.c3, k1 + (unsigned)r * 0xBB67AE85u); s.c3 = lo0;
   }
-  return c0;
+}
+__device__ __forceinline__ unsigned philox_word0(unsigned off, unsigned k0, unsigned k1) {
+  PhiloxState s = {off, 0u, 0u, 0u};
+  philox_rounds<0, 10>(s, k0, k1);
+  return s.c0;
 }
 
 // Counter hash of the fast stochastic-rounding mode: one 32-bit mix per 4 consecutive weights of a row; the first
