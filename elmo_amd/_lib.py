@@ -104,6 +104,7 @@ def load():
 
 
 XMC_ERR_RANGE = -4
+XMC_ERR_WORKSPACE = -5
 
 
 def check(status, what):

@@ -64,7 +64,7 @@ void fill_device_info(int dev) {
   (void)hipFuncSetAttribute((const void*)fp8_forward_select_kernel<0>, hipFuncAttributeMaxDynamicSharedMemorySize, SEL_LDS);
   (void)hipFuncSetAttribute((const void*)fp8_forward_select_kernel<1>, hipFuncAttributeMaxDynamicSharedMemorySize, SEL_LDS);
   (void)hipFuncSetAttribute((const void*)quad_sort_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (MAX_POS + 256) * 4);
-  (void)hipFuncSetAttribute((const void*)quad_desc_prep_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (MAX_POS + 257) * 4);
+  (void)hipFuncSetAttribute((const void*)quad_prep_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (MAX_POS + 256) * 4);
 #define XMC_TILED_ATTR(DD)                                                                                                                        \
   (void)hipFuncSetAttribute((const void*)tiled_gradx_kernel<W_BF16, 1, DD>, hipFuncAttributeMaxDynamicSharedMemorySize, TgxGeom<W_BF16, 1, DD>::LDS); \
   (void)hipFuncSetAttribute((const void*)tiled_gradx_kernel<W_E4M3, 1, DD>, hipFuncAttributeMaxDynamicSharedMemorySize, TgxGeom<W_E4M3, 1, DD>::LDS); \
@@ -210,9 +210,9 @@ const char* xmc_error_string(int status) {
 size_t xmc_workspace_bytes(int num_chunks, int rows_per_chunk) {
   if (num_chunks <= 0 || num_chunks > MAX_CHUNKS || rows_per_chunk <= 0) return 0;
   size_t tiles = (size_t)num_chunks * ((rows_per_chunk + TL - 1) / TL);
-  // tile_ptr, then 32-byte tile descriptors, one run per quad (up to MAX_WG / 4 runs, each rounded up to whole entries)
-  // (two tables with a compensated head)
-  return WS_TILEPTR + ((tiles + 1) * 4 + 255) / 256 * 256 + (tiles + MAX_WG / 2) * 32;
+  // 32-byte tile descriptors, one run per quad (up to MAX_WG / 4 runs, each rounded up to whole entries; two tables with a
+  // compensated head)
+  return WS_DESC + (tiles + MAX_WG / 2) * 32;
 }
 
 int xmc_fp8_step(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, const void* x_bf16, int batch,
@@ -276,10 +276,9 @@ static int fused_step(void* const* chunk_ptrs, int num_chunks, int rows_per_chun
     p.xq = ws + WS_XQ;
     p.xt = (const bf16x8*)(ws + WS_XT);
     p.keys = (const unsigned*)(ws + WS_KEYS);
-    p.tile_ptr = (const int*)(ws + WS_TILEPTR);
     p.partial = (floatx4*)(ws + WS_PARTIAL);
     p.exch = ws + WS_EXCH;
-    uint4* desc = (uint4*)(ws + WS_TILEPTR + ((size_t)(num_tiles + 1) * 4 + 255) / 256 * 256);
+    uint4* desc = (uint4*)(ws + WS_DESC);
     p.desc = desc;
     p.flags = (int*)(ws + WS_FLAGS);
     p.zscale = scale_w * scale_x;
@@ -299,12 +298,10 @@ static int fused_step(void* const* chunk_ptrs, int num_chunks, int rows_per_chun
     p.cnt_base = 0;
     p.acc_init = 0;
     p.spin_limit = g_spin_limit.load(std::memory_order_relaxed);
-    quad_sort_kernel<<<n_pad > 0 ? n_pad / 64 : 1, 256, (size_t)(n_pad + 256) * 4, stream>>>(
-        labels_coo, nnz, n_pad, batch, 0, 0, num_chunks * rows_per_chunk, (unsigned*)(ws + WS_KEYS), (int*)(ws + WS_FLAGS));
-    const int desc_blocks = (num_tiles + 1 + 255) / 256;
-    quad_desc_prep_kernel<<<desc_blocks + (BP * (D / 4) + 255) / 256, 256, (size_t)(n_pad + 257) * 4, stream>>>(
-        p, n_pad, (int*)(ws + WS_TILEPTR), desc, desc_blocks, (const unsigned short*)x_bf16, 1.0f / scale_x, ws + WS_XQ,
-        (unsigned short*)(ws + WS_XT), dp);
+    const int sort_blocks = n_pad > 0 ? n_pad / 64 : 1, desc_blocks = (num_tiles + 255) / 256;
+    quad_prep_kernel<<<sort_blocks + desc_blocks + (BP * (D / 4) + 255) / 256, 256, (size_t)(n_pad + 256) * 4, stream>>>(
+        p, labels_coo, nnz, n_pad, (unsigned*)(ws + WS_KEYS), desc, sort_blocks, desc_blocks, (const unsigned short*)x_bf16, 1.0f / scale_x,
+        ws + WS_XQ, (unsigned short*)(ws + WS_XT), dp);
     if (g_prof_start) (void)hipEventRecord(g_prof_start, stream);
     QuadParams ph = p;   // the head's launch
     ph.run_tiles = head_tiles;
@@ -321,7 +318,7 @@ static int fused_step(void* const* chunk_ptrs, int num_chunks, int rows_per_chun
     }
     if (g_prof_stop) (void)hipEventRecord(g_prof_stop, stream);
     g_prof_start = g_prof_stop = nullptr;
-    reduce_gx_role_kernel<<<192, 128, 0, stream>>>((const floatx4*)(ws + WS_PARTIAL), qgrid, scale_w, grad_x_f32,
+    reduce_gx_role_kernel<<<(batch + 15) / 16 * 48, 256, 0, stream>>>((const floatx4*)(ws + WS_PARTIAL), qgrid, scale_w, grad_x_f32,
                                                  (unsigned short*)grad_x_bf16, batch, (int*)(ws + WS_FLAGS), di.failure_word, dp);
   }
   return launch_status();
@@ -630,12 +627,11 @@ static int cluster_step(void* const* chunk_ptrs, int num_chunks, int rows_per_ch
   for (int c0 = 0; c0 < num_chunks; c0 += seg_chunks) {
     const int nch = c0 + seg_chunks <= num_chunks ? seg_chunks : num_chunks - c0;
     const bool last = c0 + nch == num_chunks;
-    const int sort_blocks = n_pad / 64, prep_blocks = (bp * (D / 4) + 255) / 256;
-    cluster_prep_kernel<<<sort_blocks * pairs + prep_blocks, 256, (size_t)(n_pad + 256) * 4, stream>>>(
-        labels_coo, nnz, n_pad, batch, c0 * rows_per_chunk, nch * rows_per_chunk, keys, sort_blocks, pairs, (const unsigned short*)x_bf16, bp,
-        bf16 ? 0 : fp8 ? 2 : 1, ws + lay.xq, (unsigned short*)(ws + lay.xt), (int*)(ws + lay.flags), err, dp);
-    cluster_tile_ptr_kernel<<<dim3((nch * tpc64 + 1 + 255) / 256, pairs), 256, 0, stream>>>(keys, n_pad, rows_per_chunk, tpc64, nch * tpc64, tile_ptr,
-                                                                                         lay.tp_stride);
+    const int sort_blocks = n_pad / 64, ptr_blocks = (nch * tpc64 + 1 + 255) / 256, prep_blocks = (bp * (D / 4) + 255) / 256;
+    const ClusterPrep pp = {labels_coo, nnz, n_pad, batch, c0 * rows_per_chunk, nch * rows_per_chunk, pairs, rows_per_chunk, tpc64, nch * tpc64,
+                            sort_blocks, ptr_blocks, keys, tile_ptr, lay.tp_stride, (const unsigned short*)x_bf16, bp, bf16 ? 0 : fp8 ? 2 : 1,
+                            ws + lay.xq, (unsigned short*)(ws + lay.xt), (int*)(ws + lay.flags), err};
+    cluster_prep_kernel<<<(sort_blocks + ptr_blocks) * pairs + prep_blocks, 256, (size_t)(n_pad + 256) * 4, stream>>>(pp, dp);
     ClusterParams p;
     for (int k = 0; k < MAX_CHUNKS; k++) {
       p.chunk[k] = k < nch ? (unsigned char*)chunk_ptrs[c0 + k] : nullptr;
@@ -674,7 +670,7 @@ static int cluster_step(void* const* chunk_ptrs, int num_chunks, int rows_per_ch
     var.fn<<<(p.nclusters + 7) / 8 * 8 * c, CLU_NT, var.lds, stream>>>(p);
     const ClusterReduce rd = {p.partial, c, nbk, p.nclusters, p.ntiles, p.tpc, nch, p.flush, p.xcc, err, failure_word, gx_total, c0 > 0 ? 1 : 0, last ? 1 : 0, batch,
                               (unsigned short*)grad_x_bf16, grad_x_f32};
-    cluster_reduce_kernel<<<c * nbk * 6 * 8, 256, 0, stream>>>(rd, dp);
+    cluster_reduce_kernel<<<c * nbk * 6 * 8, CLU_RW * 64, 0, stream>>>(rd, dp);
   }
   return launch_status();
 }
@@ -765,7 +761,7 @@ static int tiled_step_t(void* const* chunk_ptrs, int num_chunks, int rows_per_ch
         if (n_pad > 0)
           quad_sort_kernel<<<n_pad / 64, 256, (size_t)(n_pad + 256) * 4, stream>>>(labels_coo, nnz, n_pad, batch, 256 * pr,
                                                                                 seg0 * rows_per_chunk, seg_n * rows_per_chunk,
-                                                                                keys + (size_t)pr * MAX_POS, nullptr);
+                                                                                keys + (size_t)pr * MAX_POS);
         tile_ptr_kernel<<<(seg_n * tiles_per_chunk + 1 + 255) / 256, 256, 0, stream>>>(
             keys + (size_t)pr * MAX_POS, n_pad, rows_per_chunk, tiles_per_chunk, seg_n * tiles_per_chunk,
             tile_ptr + pr * tp_stride + seg0 * tiles_per_chunk);

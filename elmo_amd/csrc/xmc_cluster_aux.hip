@@ -78,30 +78,36 @@ __device__ __forceinline__ void cluster_prep_thread(int i, const unsigned short*
   }
 }
 
-// First launch of a step: blocks below sort_blocks * pairs sort the positives (sort_blocks per 256 batch rows), the others
-// prepare X.
-__global__ __launch_bounds__(256) void cluster_prep_kernel(const int* coo, int nnz, int n_pad, int batch, int label_base, int label_count,
-                                                           unsigned* keys, int sort_blocks, int pairs, const unsigned short* x, int bp, int kind,
-                                                           unsigned char* xq, unsigned short* xt, int* flags, int* err, const DropoutParams dp) {
-  const int blk = blockIdx.x;
-  if (blk < sort_blocks * pairs) {
-    const int pr = blk / sort_blocks;
-    quad_sort_block(blk - pr * sort_blocks, coo, nnz, n_pad, batch, 256 * pr, label_base, label_count, keys + (size_t)pr * MAX_POS);
+// The launch in front of the step kernel, 256 threads a block: sort_blocks blocks per 256 batch rows sort the positives,
+// ptr_blocks write the first key of every 64-row tile (first_keys_block), the others prepare X.
+struct ClusterPrep {
+  const int* coo; int nnz, n_pad, batch, label_base, label_count, pairs, rows_per_chunk, tiles_per_chunk, num_tiles, sort_blocks, ptr_blocks;
+  unsigned* keys; int* tile_ptr; size_t tp_stride;
+  const unsigned short* x; int bp, kind;
+  unsigned char* xq; unsigned short* xt; int* flags; int* err;
+};
+__global__ __launch_bounds__(256) void cluster_prep_kernel(const ClusterPrep p, const DropoutParams dp) {
+  int blk = blockIdx.x;
+  if (blk < p.sort_blocks * p.pairs) {
+    const int pr = blk / p.sort_blocks;
+    quad_sort_block(blk - pr * p.sort_blocks, p.coo, p.nnz, p.n_pad, p.batch, 256 * pr, p.label_base, p.label_count, p.keys + (size_t)pr * MAX_POS);
     return;
   }
-  cluster_prep_thread((blk - sort_blocks * pairs) * 256 + (int)threadIdx.x, x, batch, bp, kind, xq, xt, flags, err, dp);
-}
-
-// tile_ptr of every pair of batch halves in one launch (y = pair)
-__global__ void cluster_tile_ptr_kernel(const unsigned* keys, int n_pad, int rows_per_chunk, int tiles_per_chunk, int num_tiles, int* tile_ptr,
-                                        size_t tp_stride) {
-  tile_ptr_entry(blockIdx.x * blockDim.x + threadIdx.x, keys + (size_t)blockIdx.y * MAX_POS, n_pad, rows_per_chunk, tiles_per_chunk, num_tiles,
-                 tile_ptr + blockIdx.y * tp_stride);
+  blk -= p.sort_blocks * p.pairs;
+  if (blk < p.ptr_blocks * p.pairs) {
+    const int pr = blk / p.ptr_blocks, t0 = (blk - pr * p.ptr_blocks) * 256, t = t0 + (int)threadIdx.x;
+    int p0, p1;
+    first_keys_block(t0, p.coo, p.nnz, p.batch, 256 * pr, p.label_base, p.label_count, p.rows_per_chunk, 1.0f / (float)p.rows_per_chunk,
+                     p.tiles_per_chunk, &p0, &p1);
+    if (t <= p.num_tiles) p.tile_ptr[pr * p.tp_stride + t] = p0;
+    return;
+  }
+  cluster_prep_thread((blk - p.ptr_blocks * p.pairs) * 256 + (int)threadIdx.x, p.x, p.batch, p.bp, p.kind, p.xq, p.xt, p.flags, p.err, dp);
 }
 
 // grad_X = sum of the members' partials in a fixed order.  A block handles 64 positions (floatx4 values) of the partial
-// layout; its four wavefronts take a share of the slots each: a quarter of them, or with `flush` the chunks ck = wavefront,
-// wavefront + 4, ..., each chunk's sum rounded to bf16 by itself (chunked.py:116).  The first block checks that the members
+// layout; its wavefronts take a share of the slots each: equal shares, or with `flush` the chunks ck = wavefront, wavefront +
+// CLU_RW, ... (fewer chunks than wavefronts: several wavefronts share a chunk's slots), each chunk's sum rounded to bf16 by itself (chunked.py:116).  The first block checks that the members
 // of every cluster ran on one XCD and passes the error word on to the sticky one.
 //   add: continue from gx_total;  final: write grad_X (with the dropout's backward) instead of gx_total
 struct ClusterReduce {
@@ -110,7 +116,8 @@ struct ClusterReduce {
   float* gx_total; int add, final_out, batch;
   unsigned short* gx_bf16; float* gx_f32;
 };
-__global__ __launch_bounds__(256) void cluster_reduce_kernel(const ClusterReduce r, const DropoutParams dp) {
+constexpr int CLU_RW = 8;   // wavefronts of a block
+__global__ __launch_bounds__(CLU_RW * 64) void cluster_reduce_kernel(const ClusterReduce r, const DropoutParams dp) {
   const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
   if (blockIdx.x == 0) {
     if (r.c > 1 && tid < r.nclusters)
@@ -120,7 +127,7 @@ __global__ __launch_bounds__(256) void cluster_reduce_kernel(const ClusterReduce
     __syncthreads();
     if (tid == 0) report_step_error(r.err, r.err + 1, r.failure_word);
   }
-  __shared__ floatx4 sh[4][64];
+  __shared__ floatx4 sh[CLU_RW][64];
   const int pslot = r.nbk * 6 * 8 * 64;
   const int pos = blockIdx.x * 64 + lane, m = pos / pslot, q = pos - m * pslot;
   auto sum_slots = [&](int s0, int s1) {
@@ -136,23 +143,36 @@ __global__ __launch_bounds__(256) void cluster_reduce_kernel(const ClusterReduce
     for (; k < s1; k++) s += r.partial[(size_t)(k * r.c + m) * pslot + q];
     return s;
   };
+  const int per = r.flush && r.nchunks < CLU_RW ? CLU_RW / r.nchunks : 1;   // wavefronts of a chunk
   floatx4 tot = {0.f, 0.f, 0.f, 0.f};
   if (r.flush) {
     // cluster that walks tile t (see the partition in cluster_step_kernel): the last one whose range starts at or before t
     auto owner = [&](int t) { return (int)((((long long)t + 1) * r.nclusters - 1) / r.ntiles); };
-    for (int ck = wv; ck < r.nchunks; ck += 4) {
+    for (int ck = wv / per; ck < r.nchunks; ck += CLU_RW) {
       const int t1 = ck == r.nchunks - 1 ? r.ntiles : (ck + 1) * r.tpc;
-      const floatx4 s = sum_slots(owner(ck * r.tpc) + ck, owner(t1 - 1) + ck + 1);
+      const int s0 = owner(ck * r.tpc) + ck, ns = owner(t1 - 1) + ck + 1 - s0, q = wv % per;
+      const floatx4 s = sum_slots(s0 + ns * q / per, s0 + ns * (q + 1) / per);
 #pragma unroll
-      for (int e = 0; e < 4; e++) tot[e] += bf16_rt(s[e]);
+      for (int e = 0; e < 4; e++) tot[e] += per > 1 ? s[e] : bf16_rt(s[e]);
     }
   } else {
-    tot = sum_slots(r.nclusters * wv / 4, r.nclusters * (wv + 1) / 4);
+    tot = sum_slots(r.nclusters * wv / CLU_RW, r.nclusters * (wv + 1) / CLU_RW);
   }
   sh[wv][lane] = tot;
   __syncthreads();
   if (wv != 0) return;
-  tot = (sh[0][lane] + sh[1][lane]) + (sh[2][lane] + sh[3][lane]);
+  if (per > 1) {
+    tot = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int ck = 0; ck < r.nchunks; ck++) {
+      floatx4 s = sh[ck * per][lane];
+      for (int q = 1; q < per; q++) s += sh[ck * per + q][lane];
+#pragma unroll
+      for (int e = 0; e < 4; e++) tot[e] += bf16_rt(s[e]);
+    }
+  } else {
+#pragma unroll
+    for (int q = 1; q < CLU_RW; q++) tot += sh[q][lane];
+  }
   // position -> ((16-row block * 6 + feature block) * 8 + wavefront) * 64 + lane of cluster_step_kernel
   const int fv = (q >> 6) & 7, bk = q >> 9, mb = bk / 6, nn = bk - mb * 6;
   const int col = 96 * fv + 16 * nn + (lane & 15);

@@ -31,7 +31,7 @@ constexpr size_t WS_KEYS = WS_XT + (size_t)BP * D * 2;        // sorted positive
 constexpr size_t WS_FLAGS = WS_KEYS + (size_t)MAX_POS * 4;    // 4096 ints: counters, XCC ids, error words (below)
 constexpr size_t WS_PARTIAL = WS_FLAGS + 16384;               // MAX_WG * 12 * 512 * 16 bytes of grad_X partials
 constexpr size_t WS_EXCH = WS_PARTIAL + (size_t)MAX_WG * 12 * 512 * 16;     // G exchange ring: 64 quads x 8 slots x 20 KiB
-constexpr size_t WS_TILEPTR = WS_EXCH + (size_t)(MAX_WG / 4) * 8 * 20480;   // tile_ptr[num_tiles + 1], then the tile descriptors
+constexpr size_t WS_DESC = WS_EXCH + (size_t)(MAX_WG / 4) * 8 * 20480;      // the tile descriptors
 
 // Layout of the 4096 ints at WS_FLAGS (all but the sticky word cleared at the start of every step):
 //   [0, 1024)             tiles-published counters of the persistent step kernel: sixteen per quad

@@ -47,8 +47,9 @@ __global__ void prep_x_kernel(const unsigned short* x, int batch, float inv_scal
 }
 
 // tile_ptr[t] = first key whose label >= first label of tile t; tile_ptr[num_tiles] = first key past the last tile
-__device__ __forceinline__ void tile_ptr_entry(int t, const unsigned* keys, int n_pad, int rows_per_chunk, int tiles_per_chunk, int num_tiles,
-                                               int* tile_ptr) {
+__global__ void tile_ptr_kernel(const unsigned* keys, int n_pad, int rows_per_chunk, int tiles_per_chunk, int num_tiles,
+                                int* tile_ptr) {
+  int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t > num_tiles) return;
   unsigned long long label0;
   if (t == num_tiles) {
@@ -64,10 +65,6 @@ __device__ __forceinline__ void tile_ptr_entry(int t, const unsigned* keys, int 
     if ((unsigned long long)keys[mid] < bound) lo = mid + 1; else hi = mid;
   }
   tile_ptr[t] = lo;
-}
-__global__ void tile_ptr_kernel(const unsigned* keys, int n_pad, int rows_per_chunk, int tiles_per_chunk, int num_tiles,
-                                int* tile_ptr) {
-  tile_ptr_entry(blockIdx.x * blockDim.x + threadIdx.x, keys, n_pad, rows_per_chunk, tiles_per_chunk, num_tiles, tile_ptr);
 }
 
 // Inference logits: out[b, label - col0] = bf16(zscale * sum_k Xq[b,k] W[label,k]) for the 32-label tiles

@@ -765,14 +765,18 @@ __global__ __launch_bounds__(QNT, 1) void fp8_step_role_kernel(const QuadParams 
   floatx4* dst = p.partial + (size_t)g * 24 * 256;
 #pragma unroll
   for (int mb = 0; mb < 8; mb++)
+    if (16 * mb < p.batch) {   // (blocks of zero rows are not read)
 #pragma unroll
-    for (int nn = 0; nn < 3; nn++) dst[(mb * 3 + nn) * 256 + s * 64 + lane] = acc2[mb][nn];
+      for (int nn = 0; nn < 3; nn++) dst[(mb * 3 + nn) * 256 + s * 64 + lane] = acc2[mb][nn];
+    }
 }
 
 #ifndef XMC_HEAVY_TU   // compiled once, in the library's main translation unit
-// grad_X = scale * sum over quads of the member partials; writes fp32 and bf16 [batch, 768].  192 workgroups of 128
-// threads: workgroup (block, m, part) covers lanes 128 part.. of the 256 B-wavefront lanes of a step workgroup.
-__global__ __launch_bounds__(128) void reduce_gx_role_kernel(const floatx4* partial, int nwg, float scale, float* gx_f32,
+// grad_X = scale * sum over quads of the member partials; writes fp32 and bf16 [batch, 768].  Workgroup (16-row batch block,
+// feature block, member, B wavefront of the step) sums the 64 values of that wavefront; its four wavefronts take a quarter
+// of the quads each, all loads of a wavefront in flight at once: the kernel is bound by the latency of a few rounds of loads
+// (7.0 us with two wavefronts' worth of loads one behind the other and all blocks of 128 batch rows, whatever the batch).
+__global__ __launch_bounds__(256) void reduce_gx_role_kernel(const floatx4* partial, int nwg, float scale, float* gx_f32,
                                                              unsigned short* gx_bf16, int batch, int* flags, int* failure_word,
                                                              const DropoutParams dp) {
   // placement check: the members of a quad exchanged G through the L2 of one XCD, which holds only if all four ran there
@@ -782,18 +786,24 @@ __global__ __launch_bounds__(128) void reduce_gx_role_kernel(const floatx4* part
     __syncthreads();
     if (threadIdx.x == 0) report_step_error(flags + QF_ERR, flags + QF_STICKY, failure_word);
   }
-  const int blk = blockIdx.x >> 3, m = (blockIdx.x >> 1) & 3;   // blk = mb*3+nn
-  const int t = (blockIdx.x & 1) * 128 + threadIdx.x, s = t >> 6, lane = t & 63, l16 = lane & 15, kg = lane >> 4;
-  // the workgroups of member m, in a fixed order; eight loads in flight at a time
+  const int blk = blockIdx.x >> 4, m = (blockIdx.x >> 2) & 3, s = blockIdx.x & 3;   // blk = mb*3+nn
+  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, l16 = lane & 15, kg = lane >> 4;
+  // the workgroups of member m of quads nq wv / 4 .. nq (wv + 1) / 4 - 1 (quad 8 j + x), in a fixed order
   floatx4 sum = {0.f, 0.f, 0.f, 0.f};
   const int nq = nwg >> 5;   // quads per XCD
-  for (int jq = 0; jq < nq; jq++) {
+  for (int jq = nq * wv >> 2; jq < nq * (wv + 1) >> 2; jq++) {
     floatx4 pv[8];
 #pragma unroll
-    for (int x = 0; x < 8; x++) pv[x] = partial[((size_t)(((jq * 4 + m) << 3) + x) * 24 + blk) * 256 + t];
+    for (int x = 0; x < 8; x++) pv[x] = partial[((size_t)(((jq * 4 + m) << 3) + x) * 24 + blk) * 256 + s * 64 + lane];
 #pragma unroll
     for (int x = 0; x < 8; x++) sum += pv[x];
   }
+  __shared__ floatx4 part[3][64];
+  if (wv > 0) part[wv - 1][lane] = sum;
+  __syncthreads();
+  if (wv > 0) return;
+#pragma unroll
+  for (int q = 0; q < 3; q++) sum += part[q][lane];
   const int mb = blk / 3, nn = blk - mb * 3;
   const int col = QCOLS * m + 48 * s + 16 * nn + l16;
 #pragma unroll

@@ -6,23 +6,30 @@ import torch
 from . import _lib
 
 FEATURES = 768
+_CODE_TYPES = (torch.float8_e4m3fn, torch.uint8)
 MAX_BATCH = 128          # fused step
 MAX_BATCH_TILED = 512    # tiled step
 
 
 def _stream_ptr():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    """The current stream's handle.  Without a Stream object around it, which costs 2.7 us of a 16 us call."""
+    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()))
+
+
+def draw_seeds(n):
+    """n seeds from the global CPU generator: the values and the generator state of n draws of one, as the reference makes
+    them (chunked.py:126), in one call."""
+    return torch.randint(0, 1000000, (n,)).tolist()
 
 
 def _chunk_array(chunks):
-    arr = (ctypes.c_void_p * len(chunks))()
     rows = chunks[0].shape[0]
-    for i, c in enumerate(chunks):
+    shape = (rows, FEATURES)
+    for c in chunks:
         assert c.is_cuda and c.is_contiguous(), "weight chunks must be contiguous device tensors"
-        assert c.dtype in (torch.float8_e4m3fn, torch.uint8) and c.shape == (rows, FEATURES), \
+        assert c.dtype in _CODE_TYPES and c.shape == shape, \
             "weight chunks must be equal-sized [rows, 768] e4m3fn tensors"
-        arr[i] = c.data_ptr()
-    return arr, rows
+    return (ctypes.c_void_p * len(chunks))(*[c.data_ptr() for c in chunks]), rows
 
 
 def workspace_bytes(num_chunks, rows_per_chunk):
@@ -300,16 +307,16 @@ def tiled_step(chunk_views, rows_per_chunk, weight_type, x, labels, lr, seeds=No
     assert labels.dim() == 2 and labels.shape[1] == 2
     assert round_mode in ("rtn", "sr_philox", "sr_fast"), \
         "the tiled path rounds to nearest, with the reference's Philox recipe or with the fast hardware mode"
-    wdt = (torch.bfloat16,) if weight_type == "bf16" else (torch.float8_e4m3fn, torch.uint8)
+    wdt = (torch.bfloat16,) if weight_type == "bf16" else _CODE_TYPES
     nc = len(chunk_views)
-    arr = (ctypes.c_void_p * nc)()
-    for i, c in enumerate(chunk_views):
-        assert c.is_cuda and c.is_contiguous() and c.dtype in wdt and c.dim() == 2 and c.shape[1] == feats
-        assert c.shape[0] == rows_per_chunk or (i == nc - 1 and 0 < c.shape[0] <= rows_per_chunk)
-        arr[i] = c.data_ptr()
+    full, last = (rows_per_chunk, feats), chunk_views[-1]
+    assert last.dim() == 2 and 0 < last.shape[0] <= rows_per_chunk and last.shape[1] == feats
+    for c in chunk_views:
+        assert c.is_cuda and c.is_contiguous() and c.dtype in wdt and (c.shape == full or c is last)
+    arr = (ctypes.c_void_p * nc)(*[c.data_ptr() for c in chunk_views])
     batch = x.shape[0]
     assert 0 < batch <= MAX_BATCH_TILED, "batch must be at most 512"
-    if workspace is None or workspace.numel() < tiled_workspace_bytes(nc, rows_per_chunk, batch, feats):
+    if workspace is None:
         workspace = alloc_tiled_workspace(nc, rows_per_chunk, x.device, batch, feats)
     if grad_out is None:
         grad_out = torch.empty(batch, feats, dtype=torch.bfloat16, device=x.device)
@@ -319,14 +326,16 @@ def tiled_step(chunk_views, rows_per_chunk, weight_type, x, labels, lr, seeds=No
         sarr = (ctypes.c_uint32 * nc)(*[int(s) & 0xFFFFFFFF for s in seeds])
     if loss_out is not None:
         assert loss_out.is_cuda and loss_out.dtype == torch.float32 and loss_out.numel() == 1
-    st = lib.xmc_tiled_step_ex(arr, nc, rows_per_chunk, chunk_views[-1].shape[0], WEIGHT_TYPES[weight_type], x.data_ptr(),
-                            batch, feats, labels.data_ptr() if labels.numel() else None, labels.shape[0], float(lr),
-                            sarr, _lib.ROUND_MODES[round_mode], int(bool(quantize_x)), int(bool(saturate)),
-                            kahan.data_ptr() if kahan is not None else None, ktype, int(num_head), float(weight_decay),
-                            float(dropout_p), int(dropout_seed) & 0xFFFFFFFFFFFFFFFF, grad_out.data_ptr(),
-                            gf.data_ptr() if gf is not None else None,
-                            loss_out.data_ptr() if loss_out is not None else None, workspace.data_ptr(), workspace.numel(),
-                            _stream_ptr())
+    args = (arr, nc, rows_per_chunk, last.shape[0], WEIGHT_TYPES[weight_type], x.data_ptr(),
+            batch, feats, labels.data_ptr() if labels.numel() else None, labels.shape[0], float(lr),
+            sarr, _lib.ROUND_MODES[round_mode], int(bool(quantize_x)), int(bool(saturate)),
+            kahan.data_ptr() if kahan is not None else None, ktype, int(num_head), float(weight_decay),
+            float(dropout_p), int(dropout_seed) & 0xFFFFFFFFFFFFFFFF, grad_out.data_ptr(),
+            gf.data_ptr() if gf is not None else None, loss_out.data_ptr() if loss_out is not None else None)
+    st = lib.xmc_tiled_step_ex(*args, workspace.data_ptr(), workspace.numel(), _stream_ptr())
+    if st == _lib.XMC_ERR_WORKSPACE:     # nothing has been launched: the workspace is for smaller batches
+        workspace = alloc_tiled_workspace(nc, rows_per_chunk, x.device, batch, feats)
+        st = lib.xmc_tiled_step_ex(*args, workspace.data_ptr(), workspace.numel(), _stream_ptr())
     _lib.check(st, "xmc_tiled_step")
     return (grad_out, gf) if want_f32 else grad_out
 

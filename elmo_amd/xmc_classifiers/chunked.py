@@ -87,12 +87,7 @@ class XMCBCECHUNKEDLayer(nn.Module):
     def _chunks(self):
         w = self.xfc_weight
         assert w.is_contiguous() and w.dtype == self._dtype and w.shape == (self.num_labels, self.features)
-        views = []
-        for c in range(self.num_chunks):
-            lo, hi = c * self.chunk_size, min((c + 1) * self.chunk_size, self.num_labels)
-            if lo < hi:
-                views.append(w[lo:hi])
-        return views
+        return w.split(self.chunk_size)
 
     @torch.no_grad()
     def xfc_forward(self, embed):
@@ -138,7 +133,7 @@ class XMCBCECHUNKEDLayer(nn.Module):
         self._errors.check()      # a failure of an earlier step, without waiting
         views = self._chunks()
         # one seed per chunk from the global CPU generator, as the reference draws them (chunked.py:126)
-        seeds = [torch.randint(0, 1000000, (1,)).item() for _ in range(len(views))]
+        seeds = ops.draw_seeds(len(views))
         loss_out = None if skip_loss else torch.zeros(1, dtype=torch.float32, device=x.device)
         self.grad_input = ops.tiled_step(views, self.chunk_size, "bf16", x, lab, xmc_lr[0], seeds=seeds,
                                          round_mode=self.rounding, workspace=self._workspace, loss_out=loss_out)

@@ -81,7 +81,7 @@ class Fp8XMCBCEChunkedHeadKahanLayer(nn.Module):
         self._errors = StepErrors(self.device, ops.sticky_error_words(self._workspace, self._tiled_workspace))
 
     def _chunks(self):
-        return [w.data for w in self.xfc_weight]
+        return list(self.xfc_weight._parameters.values())
 
     @torch.no_grad()
     def xfc_forward(self, embed):
@@ -125,7 +125,7 @@ class Fp8XMCBCEChunkedHeadKahanLayer(nn.Module):
         lab = lab.contiguous()
         loss = 0
         self._errors.check()      # a failure of an earlier step, without waiting
-        seeds = [torch.randint(0, 1000000, (1,)).item() for _ in range(self.num_chunks)]      # :120
+        seeds = ops.draw_seeds(self.num_chunks)      # :120
         if self.fake_fp8_matmul:
             self.grad_input = ops.tiled_step(self._chunks(), self.num_labels_i, "e4m3", x, lab, xmc_lr[0], seeds=seeds,
                                              round_mode=self.rounding, workspace=self._tiled_workspace)
