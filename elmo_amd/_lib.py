@@ -56,6 +56,8 @@ def load():
                                        ctypes.POINTER(ctypes.c_uint32), i32, vp, i32, i32, vp, vp, vp, sz, vp]
     lib.xmc_fp8_forward.restype = i32
     lib.xmc_fp8_forward.argtypes = [ctypes.POINTER(vp), i32, i32, vp, i32, i32, f32, f32, vp, ll, ll, vp, sz, vp]
+    lib.xmc_fp8_forward_rows.restype = i32
+    lib.xmc_fp8_forward_rows.argtypes = lib.xmc_fp8_forward.argtypes
     lib.xmc_fp8_forward_static.restype = i32
     lib.xmc_fp8_forward_static.argtypes = [ctypes.POINTER(vp), i32, i32, vp, i32, i32, f32, f32, vp, ll, ll, vp]
     lib.xmc_step_error_word.restype = i32
@@ -83,6 +85,8 @@ def load():
     lib.xmc_fp8_forward_topk_fused.restype = i32
     lib.xmc_fp8_forward_topk_fused.argtypes = [ctypes.POINTER(vp), i32, i32, vp, i32, i32, f32, f32, ctypes.c_longlong, i32, vp,
                                                vp, i32, vp, sz, vp, sz, vp, vp]
+    lib.xmc_fp8_forward_topk_fused_rows.restype = i32
+    lib.xmc_fp8_forward_topk_fused_rows.argtypes = lib.xmc_fp8_forward_topk_fused.argtypes
     lib.xmc_dropout_quantize.restype = i32
     lib.xmc_dropout_quantize.argtypes = [vp, i32, i32, i32, f32, ctypes.c_ulonglong, vp, vp]
     lib.xmc_step_error_offset.restype = sz

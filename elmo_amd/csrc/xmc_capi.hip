@@ -14,14 +14,11 @@
 
 using namespace xmc;
 
-// Operand images of X for xmc_fp8_forward_static, the entry point that takes no workspace: e4m3 X in MFMA operand order
-// (BP*D bytes), then the bf16 image the same preparation kernel writes (BP*D*2 bytes).  Every GPU the library runs on
-// holds its own copy of this array until the process ends.  In host code the name stands for the symbol only, never for
-// device memory: the address kernels get is the one hipGetSymbolAddress returned for the current device.
-constexpr size_t FWD_STATIC_XQ = 0;
-constexpr size_t FWD_STATIC_XT = (size_t)BP * D;
-constexpr size_t FWD_STATIC_BYTES = FWD_STATIC_XT + (size_t)BP * D * 2;   // 294,912
-static __device__ __align__(256) unsigned char scratch[FWD_STATIC_BYTES];
+// Operand image of X for xmc_fp8_forward_static, the entry point that takes no workspace: e4m3 X in MFMA operand order
+// (BP*D bytes).  Every GPU the library runs on holds its own copy of this array until the process ends.  In host code the name
+// stands for the symbol only, never for device memory: the address kernels get is the one hipGetSymbolAddress returned for the
+// current device.
+static __device__ __align__(256) unsigned char scratch[(size_t)BP * D];
 
 namespace {
 
@@ -108,9 +105,9 @@ thread_local hipEvent_t g_prof_start = nullptr, g_prof_stop = nullptr;
 inline bool aligned16(const void* q) { return ((uintptr_t)q & 15) == 0; }
 
 int check_common(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, const void* x, int batch, int features,
-                 const void* workspace, size_t workspace_bytes) {
+                 const void* workspace, size_t workspace_bytes, int batch_unit = 16) {
   if (!chunk_ptrs || !x || !workspace) return XMC_ERR_NULL;
-  if (features != D || batch <= 0 || batch > BP || batch % 16 != 0) return XMC_ERR_SHAPE;
+  if (features != D || batch <= 0 || batch > BP || batch % batch_unit != 0) return XMC_ERR_SHAPE;
   if (rows_per_chunk <= 0 || rows_per_chunk % 16 != 0) return XMC_ERR_SHAPE;
   if (num_chunks <= 0 || num_chunks > MAX_CHUNKS) return XMC_ERR_RANGE;
   if ((long long)num_chunks * rows_per_chunk > 0x7FFFFFFFLL) return XMC_ERR_RANGE;   // the fused step has a lower limit of its own
@@ -151,17 +148,22 @@ size_t topk_zbuf_bytes(int rows_per_chunk) {
   return ((size_t)BP * (size_t)topk_segment_rows(rows_per_chunk) * 2 + 255) / 256 * 256;
 }
 
+// the operand image of X for the batch blocks of 32 rows in use
+void prep_x(const void* x_bf16, int batch, float scale_x, unsigned char* xq, hipStream_t stream) {
+  const int n = (batch + 31) / 32 * 32 * (D / 4);
+  prep_x_kernel<<<n / 256, 256, 0, stream>>>((const unsigned short*)x_bf16, batch, n, 1.0f / scale_x, xq);
+}
+
 // The launches of the inference logits, shared by xmc_fp8_forward (operand images in the caller's workspace) and
 // xmc_fp8_forward_static (operand images in this device's copy of the static array); shapes are checked by the callers.
 int forward_launch(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, const void* x_bf16, int batch, float scale_w,
-                   float scale_x, void* out_bf16, long long out_stride, long long num_labels, unsigned char* xq,
-                   unsigned short* xt, hipStream_t stream) {
+                   float scale_x, void* out_bf16, long long out_stride, long long num_labels, unsigned char* xq, hipStream_t stream) {
   if (!out_bf16) return XMC_ERR_NULL;
   if (num_labels <= 0 || out_stride < num_labels || num_labels > (long long)num_chunks * rows_per_chunk) return XMC_ERR_SHAPE;
   if (!(scale_w > 0.f) || !(scale_x > 0.f)) return XMC_ERR_SHAPE;
   DeviceInfo di = device_info();
   if (di.ok != 1) return XMC_ERR_DEVICE;
-  prep_x_kernel<<<(BP * (D / 4) + 255) / 256, 256, 0, stream>>>((const unsigned short*)x_bf16, batch, 1.0f / scale_x, xq, xt);
+  prep_x(x_bf16, batch, scale_x, xq, stream);
   ForwardParams fp;
   for (int c = 0; c < MAX_CHUNKS; c++) fp.chunk[c] = c < num_chunks ? (const unsigned char*)chunk_ptrs[c] : nullptr;
   fp.rows_per_chunk = rows_per_chunk;
@@ -176,8 +178,8 @@ int forward_launch(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, 
   fp.col0 = 0;
   fp.num_labels = num_labels;
   fp.batch = batch;
-  const int grid = fp.tile_end < 2 * di.cus ? fp.tile_end : 2 * di.cus;   // two workgroups fit the LDS of a compute unit
-  fp8_forward_kernel<<<grid, NT, FWD_LDS, stream>>>(fp);
+  const int grid = fp.tile_end < di.cus ? fp.tile_end : di.cus;   // one workgroup fills the LDS of a compute unit
+  fp8_forward_kernel<<<grid, FNT, FWD_LDS, stream>>>(fp);
   return launch_status();
 }
 
@@ -345,20 +347,33 @@ int xmc_fp8_kahan_step(void* const* chunk_ptrs, int num_chunks, int rows_per_chu
                     workspace_bytes, stream_);
 }
 
+static int forward_checked(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, const void* x_bf16, int batch, int features,
+                           float scale_w, float scale_x, void* out_bf16, long long out_stride, long long num_labels, void* workspace,
+                           size_t workspace_bytes, void* stream_, int batch_unit) {
+  int st = check_common(chunk_ptrs, num_chunks, rows_per_chunk, x_bf16, batch, features, workspace, workspace_bytes, batch_unit);
+  if (st != XMC_OK) return st;
+  return forward_launch(chunk_ptrs, num_chunks, rows_per_chunk, x_bf16, batch, scale_w, scale_x, out_bf16, out_stride,
+                        num_labels, (unsigned char*)workspace + WS_XQ, (hipStream_t)stream_);
+}
+
 int xmc_fp8_forward(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, const void* x_bf16, int batch,
                     int features, float scale_w, float scale_x, void* out_bf16, long long out_stride,
                     long long num_labels, void* workspace, size_t workspace_bytes, void* stream_) {
-  int st = check_common(chunk_ptrs, num_chunks, rows_per_chunk, x_bf16, batch, features, workspace, workspace_bytes);
-  if (st != XMC_OK) return st;
-  unsigned char* ws = (unsigned char*)workspace;
-  return forward_launch(chunk_ptrs, num_chunks, rows_per_chunk, x_bf16, batch, scale_w, scale_x, out_bf16, out_stride,
-                        num_labels, ws + WS_XQ, (unsigned short*)(ws + WS_XT), (hipStream_t)stream_);
+  return forward_checked(chunk_ptrs, num_chunks, rows_per_chunk, x_bf16, batch, features, scale_w, scale_x, out_bf16, out_stride,
+                         num_labels, workspace, workspace_bytes, stream_, 16);
+}
+
+int xmc_fp8_forward_rows(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, const void* x_bf16, int batch,
+                         int features, float scale_w, float scale_x, void* out_bf16, long long out_stride,
+                         long long num_labels, void* workspace, size_t workspace_bytes, void* stream_) {
+  return forward_checked(chunk_ptrs, num_chunks, rows_per_chunk, x_bf16, batch, features, scale_w, scale_x, out_bf16, out_stride,
+                         num_labels, workspace, workspace_bytes, stream_, 1);
 }
 
 int xmc_fp8_forward_static(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, const void* x_bf16, int batch,
                            int features, float scale_w, float scale_x, void* out_bf16, long long out_stride,
                            long long num_labels, void* stream_) {
-  // the same checks as xmc_fp8_forward, without a workspace; the static array holds the operand images of at most
+  // the same checks as xmc_fp8_forward, without a workspace; the static array holds the operand image of at most
   // BP = 128 batch rows of D = 768 features, which is also the limit of xmc_fp8_forward
   if (!chunk_ptrs || !x_bf16) return XMC_ERR_NULL;
   if (features != D || batch <= 0 || batch > BP || batch % 16 != 0) return XMC_ERR_SHAPE;
@@ -373,8 +388,7 @@ int xmc_fp8_forward_static(void* const* chunk_ptrs, int num_chunks, int rows_per
   const DeviceInfo di = device_info();
   if (di.ok != 1 || !di.scratch_ptr) return XMC_ERR_DEVICE;
   return forward_launch(chunk_ptrs, num_chunks, rows_per_chunk, x_bf16, batch, scale_w, scale_x, out_bf16, out_stride,
-                        num_labels, di.scratch_ptr + FWD_STATIC_XQ, (unsigned short*)(di.scratch_ptr + FWD_STATIC_XT),
-                        (hipStream_t)stream_);
+                        num_labels, di.scratch_ptr, (hipStream_t)stream_);
 }
 
 size_t xmc_topk_scratch_bytes(int rows_per_chunk) {
@@ -399,17 +413,16 @@ int xmc_fp8_forward_topk(void* const* chunk_ptrs, int num_chunks, int rows_per_c
   DeviceInfo di = device_info();
   if (di.ok != 1) return XMC_ERR_DEVICE;
   hipStream_t stream = (hipStream_t)stream_;
-  unsigned char* ws = (unsigned char*)workspace;
+  unsigned char* xq = (unsigned char*)workspace + WS_XQ;
   unsigned short* zbuf = (unsigned short*)scratch;
   unsigned short* run_val = (unsigned short*)((unsigned char*)scratch + topk_zbuf_bytes(rows_per_chunk));
   int* run_idx = (int*)(run_val + (size_t)BP * 2 * TOPK_MAX);
-  prep_x_kernel<<<(BP * (D / 4) + 255) / 256, 256, 0, stream>>>((const unsigned short*)x_bf16, batch, 1.0f / scale_x, ws + WS_XQ,
-                                                              (unsigned short*)(ws + WS_XT));
+  prep_x(x_bf16, batch, scale_x, xq, stream);
   ForwardParams fp;
   for (int c = 0; c < MAX_CHUNKS; c++) fp.chunk[c] = c < num_chunks ? (const unsigned char*)chunk_ptrs[c] : nullptr;
   fp.rows_per_chunk = rows_per_chunk;
   fp.tiles_per_chunk = (rows_per_chunk + FT - 1) / FT;
-  fp.xq = ws + WS_XQ;
+  fp.xq = xq;
   fp.zscale = scale_w * scale_x;
   const int group = topk_group(rows_per_chunk);
   const long long seg_rows = topk_segment_rows(rows_per_chunk);
@@ -434,7 +447,7 @@ int xmc_fp8_forward_topk(void* const* chunk_ptrs, int num_chunks, int rows_per_c
     fp.tile_end = tile_end;
     fp.col0 = base;
     const int tiles = tile_end - tile_begin;
-    fp8_forward_kernel<<<tiles < 2 * di.cus ? tiles : 2 * di.cus, NT, FWD_LDS, stream>>>(fp);
+    fp8_forward_kernel<<<tiles < di.cus ? tiles : di.cus, FNT, FWD_LDS, stream>>>(fp);
     int done = 0;
     if (n > 32768) {          // two workgroups per row
       if (have[0] < k || have[1] < k) {
@@ -472,11 +485,10 @@ int xmc_fp8_forward_topk(void* const* chunk_ptrs, int num_chunks, int rows_per_c
   return launch_status();
 }
 
-// scratch of xmc_fp8_forward_topk_fused: group maxima, bounds, counts, candidate labels and keys
+// scratch of xmc_fp8_forward_topk_fused: group maxima, bounds, (512 bytes unused), candidate labels and keys
 constexpr size_t SELS_GMAX = 0;
 constexpr size_t SELS_BOUND = SELS_GMAX + (size_t)SEL_GROUPS * BP * 2;
-constexpr size_t SELS_COUNT = SELS_BOUND + 256;
-constexpr size_t SELS_LABEL = SELS_COUNT + (size_t)BP * 4;
+constexpr size_t SELS_LABEL = SELS_BOUND + 256 + (size_t)BP * 4;
 constexpr size_t SELS_KEY = SELS_LABEL + (size_t)BP * SEL_CAP * 4;
 constexpr size_t SELS_BYTES = SELS_KEY + (size_t)BP * SEL_CAP * 2;
 static_assert(SEL_CAP == TOPK_LIST && SEL_GROUPS == TOPK_GROUPS, "the two top-k kernels share these sizes");
@@ -491,11 +503,11 @@ static int topk_fused_step(int tiles, int k) {
   return tiles / step >= 4 * k ? step : 0;
 }
 
-int xmc_fp8_forward_topk_fused(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, const void* x_bf16, int batch,
-                               int features, float scale_w, float scale_x, long long num_labels, int k, void* out_val_bf16,
-                               void* out_idx, int idx_int64, void* workspace, size_t workspace_bytes, void* scratch,
-                               size_t scratch_bytes, int32_t* status, void* stream_) {
-  int st = check_common(chunk_ptrs, num_chunks, rows_per_chunk, x_bf16, batch, features, workspace, workspace_bytes);
+static int topk_fused(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, const void* x_bf16, int batch, int features,
+                      float scale_w, float scale_x, long long num_labels, int k, void* out_val_bf16, void* out_idx, int idx_int64,
+                      void* workspace, size_t workspace_bytes, void* scratch, size_t scratch_bytes, int32_t* status, void* stream_,
+                      int batch_unit) {
+  int st = check_common(chunk_ptrs, num_chunks, rows_per_chunk, x_bf16, batch, features, workspace, workspace_bytes, batch_unit);
   if (st != XMC_OK) return st;
   if (!out_val_bf16 || !out_idx || !scratch || !status) return XMC_ERR_NULL;
   if (((uintptr_t)scratch & 255) != 0 || ((uintptr_t)status & 3) != 0 || ((uintptr_t)out_idx & (idx_int64 ? 7 : 3)) != 0) return XMC_ERR_ALIGN;
@@ -513,18 +525,18 @@ int xmc_fp8_forward_topk_fused(void* const* chunk_ptrs, int num_chunks, int rows
   DeviceInfo di = device_info();
   if (di.ok != 1) return XMC_ERR_DEVICE;
   hipStream_t stream = (hipStream_t)stream_;
-  unsigned char* ws = (unsigned char*)workspace;
+  unsigned char* xq = (unsigned char*)workspace + WS_XQ;
   unsigned char* sc = (unsigned char*)scratch;
-  prep_x_kernel<<<(BP * (D / 4) + 255) / 256, 256, 0, stream>>>((const unsigned short*)x_bf16, batch, 1.0f / scale_x, ws + WS_XQ,
-                                                              (unsigned short*)(ws + WS_XT));
+  prep_x(x_bf16, batch, scale_x, xq, stream);
   for (int c = 0; c < MAX_CHUNKS; c++) sp.chunk[c] = c < num_chunks ? (const unsigned char*)chunk_ptrs[c] : nullptr;
-  sp.xq = ws + WS_XQ;
+  sp.xq = xq;
   sp.zscale = scale_w * scale_x;
   sp.num_labels = num_labels;
   sp.batch = batch;
   sp.gmax = (unsigned short*)(sc + SELS_GMAX);
   sp.bound = (const unsigned short*)(sc + SELS_BOUND);
-  sp.count = (unsigned*)(sc + SELS_COUNT);
+  // (the counters lie a cache line apart, in a part of the workspace that inference has no other use for)
+  sp.count = (unsigned*)((unsigned char*)workspace + WS_XT);
   sp.cand_label = (unsigned*)(sc + SELS_LABEL);
   sp.cand_key = (unsigned short*)(sc + SELS_KEY);
   // pass 1: the sampled tiles, one group of them per workgroup
@@ -540,6 +552,22 @@ int xmc_fp8_forward_topk_fused(void* const* chunk_ptrs, int num_chunks, int rows
   topk_pick_kernel<<<batch, TOPK_LIST, 0, stream>>>(sp.cand_label, sp.cand_key, sp.count, k, (unsigned short*)out_val_bf16, out_idx,
                                                     idx_int64 ? 1 : 0, status);
   return launch_status();
+}
+
+int xmc_fp8_forward_topk_fused(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, const void* x_bf16, int batch,
+                               int features, float scale_w, float scale_x, long long num_labels, int k, void* out_val_bf16,
+                               void* out_idx, int idx_int64, void* workspace, size_t workspace_bytes, void* scratch,
+                               size_t scratch_bytes, int32_t* status, void* stream_) {
+  return topk_fused(chunk_ptrs, num_chunks, rows_per_chunk, x_bf16, batch, features, scale_w, scale_x, num_labels, k, out_val_bf16,
+                    out_idx, idx_int64, workspace, workspace_bytes, scratch, scratch_bytes, status, stream_, 16);
+}
+
+int xmc_fp8_forward_topk_fused_rows(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, const void* x_bf16, int batch,
+                               int features, float scale_w, float scale_x, long long num_labels, int k, void* out_val_bf16,
+                               void* out_idx, int idx_int64, void* workspace, size_t workspace_bytes, void* scratch,
+                               size_t scratch_bytes, int32_t* status, void* stream_) {
+  return topk_fused(chunk_ptrs, num_chunks, rows_per_chunk, x_bf16, batch, features, scale_w, scale_x, num_labels, k, out_val_bf16,
+                    out_idx, idx_int64, workspace, workspace_bytes, scratch, scratch_bytes, status, stream_, 1);
 }
 
 int xmc_dropout_quantize(const void* x, int x_type, int rows, int cols, float p, unsigned long long seed, void* out_e4m3,

@@ -1,5 +1,5 @@
-// Inference logits of the FP8 extreme-classifier layer for gfx950 (MI355X), and two small kernels shared with the
-// training paths: the e4m3 operand image of X (prep_x_kernel) and the first positive of every tile (tile_ptr_kernel).
+// Inference logits of the FP8 extreme-classifier layer for gfx950 (MI355X), top-k of them without storing them, and a small
+// kernel of the training paths: the first positive of every tile (tile_ptr_kernel).
 //
 // Reference semantics: src/xmc_classifiers/chunked_fp8xmc_clf.py:45-60 (xfc_forward).
 #include "xmc_common.h"
@@ -14,36 +14,20 @@ __device__ __forceinline__ intx8 lds_read32(const unsigned char* q) {
   return intx8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
 }
 
-// Operand images of X for the inference kernel (xt: a bf16 image in matrix-operand order that the kernel does not read).
-//   xq: e4m3(X / scale_x) in v_mfma 16x16x128 B-operand order: [(w*2+nb)*6+ks][lane][32 bytes]
-//   xt: bf16 X^T in v_mfma 16x16x32 A-operand order: [(col/16)*4+ks][lane][8 bf16], lane = (col%16) + 16*kg,
-//       element j = X[32ks + 8kg + j][col]
-__global__ void prep_x_kernel(const unsigned short* x, int batch, float inv_scale_x, unsigned char* xq, unsigned short* xt) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;   // one thread per (b, k4) group of 4 features
-  if (i >= BP * (D / 4)) return;
-  int b = i / (D / 4), k = (i - b * (D / 4)) * 4;
-  float v[4] = {0.f, 0.f, 0.f, 0.f};
-  unsigned short raw[4] = {0, 0, 0, 0};
-  if (b < batch) {
-#pragma unroll
-    for (int q = 0; q < 4; q++) { raw[q] = x[(size_t)b * D + k + q]; v[q] = bf16_from_bits(raw[q]) * inv_scale_x; }
-  }
-  int packed = 0;
-  packed = __builtin_amdgcn_cvt_pk_fp8_f32(clamp448(v[0]), clamp448(v[1]), packed, false);
-  packed = __builtin_amdgcn_cvt_pk_fp8_f32(clamp448(v[2]), clamp448(v[3]), packed, true);
-  {
-    int w = b >> 5, nb = (b >> 4) & 1, n = b & 15;
-    int ks = k >> 7, kgq = (k >> 5) & 3, jq = k & 31;
-    size_t off = ((size_t)((w * 2 + nb) * 6 + ks) * 64 + (n + 16 * kgq)) * 32 + jq;
-    *(int*)(xq + off) = packed;
-  }
-#pragma unroll
-  for (int q = 0; q < 4; q++) {
-    int col = k + q;
-    int ks = b >> 5, kgq = (b >> 3) & 3, jq = b & 7;
-    size_t off = ((size_t)((col >> 4) * 4 + ks) * 64 + ((col & 15) + 16 * kgq)) * 8 + jq;
-    xt[off] = raw[q];
-  }
+// Operand image of X for the inference kernels: e4m3(X / scale_x) in v_mfma 16x16x128 B-operand order,
+// [(w*2+nb)*6+ks][lane][32 bytes]; one thread per four features, rows at or past `batch` are zero.  (Converted by every
+// workgroup from X itself instead, without this launch: 9 us more per pass at batch 128.)
+__global__ void prep_x_kernel(const unsigned short* x, int batch, int n, float inv_scale_x, unsigned char* xq) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int b = i / (D / 4), k = (i - b * (D / 4)) * 4;
+  uint2 raw = {0u, 0u};
+  if (b < batch) raw = *(const uint2*)(x + (size_t)b * D + k);
+  auto val = [&](unsigned bits) { return clamp448(__uint_as_float(bits) * inv_scale_x); };
+  int packed = __builtin_amdgcn_cvt_pk_fp8_f32(val(raw.x << 16), val(raw.x & 0xFFFF0000u), 0, false);
+  packed = __builtin_amdgcn_cvt_pk_fp8_f32(val(raw.y << 16), val(raw.y & 0xFFFF0000u), packed, true);
+  const int w = b >> 5, nb = (b >> 4) & 1, ks = k >> 7, kgq = (k >> 5) & 3, jq = k & 31;
+  *(int*)(xq + ((size_t)((w * 2 + nb) * 6 + ks) * 64 + ((b & 15) + 16 * kgq)) * 32 + jq) = packed;
 }
 
 // tile_ptr[t] = first key whose label >= first label of tile t; tile_ptr[num_tiles] = first key past the last tile
@@ -73,7 +57,7 @@ struct ForwardParams {
   const unsigned char* chunk[MAX_CHUNKS];
   int rows_per_chunk, tiles_per_chunk;
   int tile_begin, tile_end;
-  const unsigned char* xq;     // logits operands (prep kernel layout)
+  const unsigned char* xq;     // operand image of X
   float zscale;
   unsigned short* out;         // bf16 [batch][out_stride]
   long long out_stride;
@@ -82,127 +66,157 @@ struct ForwardParams {
   int batch;
 };
 
-constexpr int FT = 32;                    // labels per tile of the inference kernel
+constexpr int FT = 32;                    // labels per tile of the inference kernels
 constexpr int FB = FT * WS;               // one tile in LDS (rows of 48 + 1 pieces of 16 bytes)
-constexpr int FWD_LDS = 3 * FB;           // three tiles in flight per workgroup; two workgroups share a compute unit
-constexpr int FWD_DMA = 7;                // direct-to-LDS loads per wavefront and tile (8 rows x 49 pieces = 392 = 6 x 64 + 8)
+constexpr int FNT = 512;                  // eight wavefronts: four per half of a tile's labels, each with 32 batch rows
+constexpr int FBUF = 5;                   // tile buffers in LDS, one workgroup to a compute unit
 constexpr int ZS = FT * 2 + 16;           // LDS row stride of the staged logits [b][32 labels] bf16, bytes
+constexpr int ZB = BP * ZS;
+constexpr int FWD_LDS = FBUF * FB + 2 * ZB;
 
-// Every wavefront fetches 8 rows of the tile with exactly FWD_DMA instructions (the wait counts below rely on it).
-__device__ __forceinline__ void fwd_issue_tile(const unsigned char* gtile, int rows_valid, unsigned lds_off, int w, int lane) {
-  const int last_row = rows_valid - 1;
+// Each of WAVES wavefronts fetches its rows of the tile with exactly one instruction a row (fwd_wait relies on it), 48 lanes
+// wide, from a scalar row address: no lane computes one.
+template <int WAVES>
+__device__ __forceinline__ void fwd_issue_tile(const unsigned char* gtile, int rows_valid, unsigned lds_off, int v, int lane) {
+  if (lane < D / 16) {
 #pragma unroll
-  for (int j = 0; j < FWD_DMA; j++) {
-    const int pl = 64 * j + lane;
-    if (pl < 392) {
-      const int pc = 392 * w + pl;
-      int row = pc / 49, c = pc - row * 49;
-      row = row < last_row ? row : last_row;   // rows past the end and the pad piece re-read a valid address
-      c = c < 47 ? c : 47;
-      const unsigned char* g = gtile + row * D + c * 16;
-      const unsigned ldsoff = __builtin_amdgcn_readfirstlane(lds_off + (unsigned)(392 * w + 64 * j) * 16u);
-      asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(ldsoff), "v"(g) : "memory", "m0");
+    for (int j = 0; j < FT / WAVES; j++) {
+      const int row = FT / WAVES * v + j, src = min(row, rows_valid - 1);   // rows past the end re-read the last valid one
+      const unsigned ldsoff = __builtin_amdgcn_readfirstlane(lds_off + (unsigned)(row * WS));
+      asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(ldsoff), "v"(lane * 16), "s"(gtile + src * D) : "memory", "m0");
     }
   }
 }
 
-// One workgroup streams its tiles through three LDS buffers, the loads two tiles ahead of the matrix products.  The
-// accumulators go back through the buffer of the tile just used, so that a lane stores 16 consecutive bytes of one
-// batch row.  Memory operations complete in order: "all but the newest FWD_DMA" means the tile after this one has
-// landed and the stores of the tile before have left, whatever their number.
-__device__ __forceinline__ void fp8_forward_body(const ForwardParams& p, unsigned char* lds_raw, int block, int nblocks) {
-  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, l16 = lane & 15, kg = lane >> 4;
-  const unsigned lds0 = (unsigned)(size_t)(lds_u8*)lds_raw;
-  intx8 xq[2][6];
+// the logits operands of a wavefront: batch rows 32w .. 32w + 31
+__device__ __forceinline__ void fwd_load_x(const unsigned char* xq_image, int w, int lane, intx8 (&xq)[2][6]) {
 #pragma unroll
   for (int nb = 0; nb < 2; nb++)
 #pragma unroll
     for (int ks = 0; ks < 6; ks++)
-      xq[nb][ks] = *(const intx8*)(p.xq + ((size_t)((w * 2 + nb) * 6 + ks) * 64 + lane) * 32);
-  __builtin_amdgcn_s_waitcnt(0);
-  const int first = p.tile_begin + block;
-  auto issue = [&](int t, int buf) {
-    const int c = t / p.tiles_per_chunk, row0 = (t - c * p.tiles_per_chunk) * FT;
-    fwd_issue_tile(p.chunk[c] + (size_t)row0 * D, min(FT, p.rows_per_chunk - row0), lds0 + (unsigned)buf * FB, w, lane);
-  };
-  if (first >= p.tile_end) return;
-  issue(first, 0);
-  if (first + nblocks < p.tile_end) {
-    issue(first + nblocks, 1);
-    asm volatile("s_waitcnt vmcnt(%0)" : : "n"(FWD_DMA) : "memory");
-  } else {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  }
-  __syncthreads();
-  int buf = 0;
-  for (int t = first; t < p.tile_end; t += nblocks) {
-    const int c = t / p.tiles_per_chunk, row0 = (t - c * p.tiles_per_chunk) * FT;
-    const int rows_valid = min(FT, p.rows_per_chunk - row0);
-    const long long label0 = (long long)c * p.rows_per_chunk + row0;
-    unsigned char* wt = lds_raw + buf * FB;
-    const bool more = t + 2 * nblocks < p.tile_end;
-    if (more) issue(t + 2 * nblocks, buf == 0 ? 2 : buf - 1);
-    floatx4 z[2][2];
+      xq[nb][ks] = *(const intx8*)(xq_image + ((size_t)((w * 2 + nb) * 6 + ks) * 64 + lane) * 32);
+}
+
+// z[nb]: logits of 16 labels (tile rows from `rows` on) and batch rows 32w + 16nb ..  All operands are requested before the
+// first product: two wavefronts per SIMD do not hide an LDS read's latency in front of each of the six steps.  `between` runs
+// while they are on their way.
+template <class F>
+__device__ __forceinline__ void fwd_products(const unsigned char* rows, int l16, int kg, const intx8 (&xq)[2][6], floatx4 (&z)[2], F&& between) {
+  intx8 a[6];
 #pragma unroll
-    for (int rb = 0; rb < 2; rb++) { z[rb][0] = floatx4{0.f, 0.f, 0.f, 0.f}; z[rb][1] = floatx4{0.f, 0.f, 0.f, 0.f}; }
+  for (int ks = 0; ks < 6; ks++) a[ks] = lds_read32(rows + l16 * WS + ks * 128 + kg * 32);
+  __builtin_amdgcn_sched_barrier(0);
+  between();
+  z[0] = z[1] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int ks = 0; ks < 6; ks++)
-#pragma unroll
-      for (int rb = 0; rb < 2; rb++) {
-        intx8 a = lds_read32(wt + (16 * rb + l16) * WS + ks * 128 + kg * 32);
-        z[rb][0] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, xq[0][ks], z[rb][0], 0, 0, 0, 0, 0, 0);
-        z[rb][1] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, xq[1][ks], z[rb][1], 0, 0, 0, 0, 0, 0);
-      }
-    __syncthreads();   // the weight tile has been read: its buffer now stages the logits
-#pragma unroll
-    for (int rb = 0; rb < 2; rb++)
-#pragma unroll
-      for (int nb = 0; nb < 2; nb++) {
-        const int b = 32 * w + 16 * nb + l16;
-        uint2 v;
-        v.x = bf16_pack2(z[rb][nb][0] * p.zscale, z[rb][nb][1] * p.zscale);
-        v.y = bf16_pack2(z[rb][nb][2] * p.zscale, z[rb][nb][3] * p.zscale);
-        *(uint2*)(wt + b * ZS + (16 * rb + 4 * kg) * 2) = v;
-      }
-    if (more) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(FWD_DMA) : "memory");
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();   // the next tile has landed for every wavefront; the staged logits are visible
-    long long left = p.num_labels - label0;
-    const int nvalid = (int)(left < rows_valid ? (left < 0 ? 0 : left) : rows_valid);
-#pragma unroll
-    for (int q = 0; q < 2; q++) {
-      const int piece = tid + NT * q, b = piece >> 2, seg = piece & 3;
-      if (b < p.batch) {
-        unsigned short* orow = p.out + (size_t)b * p.out_stride + (label0 - p.col0);
-        const unsigned short* zrow = (const unsigned short*)(wt + b * ZS);
-        const int s = (int)((8u - (unsigned)(((uintptr_t)orow >> 1) & 7u)) & 7u);   // elements before a 16-byte boundary
-        const int a = s + 8 * seg;
-        if (a + 8 <= nvalid) {
-          uint4 v;
-          if (s == 0) {
-            v = *(const uint4*)(zrow + a);
-          } else {
-            v.x = zrow[a] | ((unsigned)zrow[a + 1] << 16);
-            v.y = zrow[a + 2] | ((unsigned)zrow[a + 3] << 16);
-            v.z = zrow[a + 4] | ((unsigned)zrow[a + 5] << 16);
-            v.w = zrow[a + 6] | ((unsigned)zrow[a + 7] << 16);
-          }
-          *(uint4*)(orow + a) = v;
-        } else {
-          for (int e = a; e < nvalid && e < a + 8; e++) orow[e] = zrow[e];
-        }
-        if (seg == 0)
-          for (int e = 0; e < s && e < nvalid; e++) orow[e] = zrow[e];
-      }
-    }
-    __syncthreads();   // the staged logits have been read: the buffer is free for the tile three ahead
-    buf = buf == 2 ? 0 : buf + 1;
+  for (int ks = 0; ks < 6; ks++) {
+    z[0] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a[ks], xq[0][ks], z[0], 0, 0, 0, 0, 0, 0);
+    z[1] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a[ks], xq[1][ks], z[1], 0, 0, 0, 0, 0, 0);
   }
 }
 
-__global__ __launch_bounds__(NT) void fp8_forward_kernel(const ForwardParams p) {
+// Place of a tile in the chunk list: chunk c, tile r within it.
+struct FwdPlace {
+  int c, r;
+  __device__ __forceinline__ FwdPlace(int t, int tiles_per_chunk) : c(t / tiles_per_chunk), r(t - c * tiles_per_chunk) {}
+  // n tiles on (no division in the loop)
+  __device__ __forceinline__ void advance(int n, int tiles_per_chunk) {
+    r += n;
+    while (r >= tiles_per_chunk) { r -= tiles_per_chunk; c++; }
+  }
+};
+
+// The next tile has landed: all loads but those of the AHEAD tiles behind it are complete.  Loads complete in order; stores
+// in between only make the wait stricter.  `full`: AHEAD tiles have been requested behind it.
+template <int WAVES, int AHEAD>
+__device__ __forceinline__ void fwd_wait(bool full) {
+  if (full) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(AHEAD * FT / WAVES) : "memory");
+  else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
+// One workgroup streams its tiles through FBUF LDS buffers, the loads four tiles ahead of the matrix products, with one
+// barrier per tile: behind it a tile has landed for everyone, the buffer of the tile before is free for the load, and the
+// staged logits of the tile before (two stages in turn) leave as 16 consecutive bytes of a batch row per lane.
+// HBM bound: 131 K labels, batch 40 (101 MB in, 10 MB out) 20.9 us = 5.3 TB/s; the same loads without anything else take 17.2.
+// Two workgroups of four wavefronts with three buffers and three barriers per tile took 23.2; a batch that is no multiple of
+// 16 also cost a padded copy of X and a copy of the logits (42 us the call, 25 now).
+__global__ __launch_bounds__(FNT, 2) void fp8_forward_kernel(const ForwardParams p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
-  fp8_forward_body(p, lds_raw, (int)blockIdx.x, (int)gridDim.x);
+  const int tid = threadIdx.x, v = __builtin_amdgcn_readfirstlane(tid >> 6), w = v & 3, half = v >> 2;
+  const int lane = tid & 63, l16 = lane & 15, kg = lane >> 4, nblocks = (int)gridDim.x;
+  const unsigned lds0 = (unsigned)(size_t)(lds_u8*)lds_raw;
+  const bool active = 32 * w < p.batch;   // (wave-uniform) a wavefront without batch rows only helps to load and store
+  intx8 xq[2][6];
+  if (active) fwd_load_x(p.xq, w, lane, xq);
+  __builtin_amdgcn_s_waitcnt(0);
+  const int first = p.tile_begin + (int)blockIdx.x;
+  int ahead = first;                      // next tile to be requested
+  FwdPlace at_ahead(first, p.tiles_per_chunk), at_store = at_ahead;   // its place, that of the next one to be stored
+  auto issue = [&](int buf) {
+    if (ahead < p.tile_end) {
+      const int row0 = at_ahead.r * FT;
+      fwd_issue_tile<FNT / 64>(p.chunk[at_ahead.c] + (size_t)row0 * D, min(FT, p.rows_per_chunk - row0), lds0 + (unsigned)buf * FB, v, lane);
+    }
+    ahead += nblocks;
+    at_ahead.advance(nblocks, p.tiles_per_chunk);
+  };
+  auto store = [&](const unsigned char* stage) {
+    const int row0 = at_store.r * FT;
+    const int rows_valid = min(FT, p.rows_per_chunk - row0);
+    const long long label0 = (long long)at_store.c * p.rows_per_chunk + row0, left = p.num_labels - label0;
+    const int nvalid = (int)(left < rows_valid ? (left < 0 ? 0 : left) : rows_valid);
+    at_store.advance(nblocks, p.tiles_per_chunk);
+    const int b = tid >> 2, seg = tid & 3;
+    if (b >= p.batch) return;
+    unsigned short* orow = p.out + (size_t)b * p.out_stride + (label0 - p.col0);
+    const unsigned short* zrow = (const unsigned short*)(stage + b * ZS);
+    const int s = (int)((8u - (unsigned)(((uintptr_t)orow >> 1) & 7u)) & 7u);   // elements before a 16-byte boundary
+    const int a = s + 8 * seg;
+    if (a + 8 <= nvalid) {
+      uint4 o;
+      if (s == 0) {
+        o = *(const uint4*)(zrow + a);
+      } else {
+        o.x = zrow[a] | ((unsigned)zrow[a + 1] << 16);
+        o.y = zrow[a + 2] | ((unsigned)zrow[a + 3] << 16);
+        o.z = zrow[a + 4] | ((unsigned)zrow[a + 5] << 16);
+        o.w = zrow[a + 6] | ((unsigned)zrow[a + 7] << 16);
+      }
+      *(uint4*)(orow + a) = o;
+    } else {
+      for (int e = a; e < nvalid && e < a + 8; e++) orow[e] = zrow[e];
+    }
+    if (seg == 0)
+      for (int e = 0; e < s && e < nvalid; e++) orow[e] = zrow[e];
+  };
+  for (int k = 0; k < FBUF - 1; k++) issue(k);
+  int buf = 0, par = 0, t = first;
+  for (; t < p.tile_end; t += nblocks) {
+    unsigned char* stage = lds_raw + FBUF * FB;
+    fwd_wait<FNT / 64, FBUF - 2>(t + (FBUF - 2) * nblocks < p.tile_end);
+    __syncthreads();
+    auto other = [&] {
+      issue(buf == 0 ? FBUF - 1 : buf - 1);
+      if (t != first) store(stage + (par ^ 1) * ZB);
+    };
+    if (!active) {
+      other();
+    } else {
+      floatx4 z[2];
+      fwd_products(lds_raw + buf * FB + 16 * half * WS, l16, kg, xq, z, other);
+#pragma unroll
+      for (int nb = 0; nb < 2; nb++) {
+        uint2 o;
+        o.x = bf16_pack2(z[nb][0] * p.zscale, z[nb][1] * p.zscale);
+        o.y = bf16_pack2(z[nb][2] * p.zscale, z[nb][3] * p.zscale);
+        *(uint2*)(stage + par * ZB + (32 * w + 16 * nb + l16) * ZS + (16 * half + 4 * kg) * 2) = o;
+      }
+    }
+    buf = buf == FBUF - 1 ? 0 : buf + 1;
+    par ^= 1;
+  }
+  __syncthreads();
+  if (t != first) store(lds_raw + FBUF * FB + (par ^ 1) * ZB);
 }
 
 
@@ -216,21 +230,28 @@ __global__ __launch_bounds__(NT) void fp8_forward_kernel(const ForwardParams p) 
 // kernel reports a row whose count exceeded it.
 constexpr int SEL_CAP = 1024;
 constexpr int SEL_GROUPS = 512;          // most workgroups of pass 1
-constexpr int SEL_QUEUE = 256;           // candidates a workgroup of pass 2 collects in LDS between two flushes
-constexpr int SEL_FLUSH = 8;             // tiles between two flushes
-constexpr int SEL_LDS = FWD_LDS + 16 + SEL_QUEUE * 8;
+// Here two workgroups of four wavefronts share a compute unit, with three tile buffers each: a wavefront that collects
+// candidates holds up the barrier of its own workgroup only.  Pass 2 over 670 K labels, batch 128, k = 100: 90 us = 5.7 TB/s
+// (the loads alone: 85), one workgroup of eight wavefronts and five buffers 110, one queue per workgroup with LDS atomics 113.
+constexpr int SEL_BUF = 3;
+constexpr int SEL_QUEUE = 128;           // candidates a wavefront of pass 2 collects in LDS
+constexpr int SEL_LDS = SEL_BUF * FB + NT / 64 * SEL_QUEUE * 8;
+// The rows' counters lie a cache line apart: next to each other 57 K atomics (670 K labels, batch 128, k = 100) on four lines
+// took 16 us where they came together.
+constexpr int SEL_COUNT_STRIDE = 32;
+static_assert(2 * SEL_LDS <= 160 * 1024 && FWD_LDS <= 160 * 1024, "LDS budget");
 
 struct SelectParams {
   const unsigned char* chunk[MAX_CHUNKS];
   int rows_per_chunk, tiles_per_chunk;
   int n_visit, tile_step;        // the launch visits tiles j * tile_step, j in [0, n_visit)
-  const unsigned char* xq;       // logits operands (prep kernel layout)
+  const unsigned char* xq;       // operand image of X
   float zscale;
   long long num_labels;          // labels at or past this one do not take part
   int batch;
   unsigned short* gmax;          // MODE 0: [gridDim.x][BP] keys
   const unsigned short* bound;   // MODE 1: [BP] keys
-  unsigned* count;               // MODE 1: [BP]
+  unsigned* count;               // MODE 1: [BP], SEL_COUNT_STRIDE apart
   unsigned* cand_label;          // MODE 1: [BP][SEL_CAP]
   unsigned short* cand_key;      // MODE 1: [BP][SEL_CAP]
 };
@@ -247,23 +268,22 @@ __device__ __forceinline__ unsigned key_pair(unsigned w) {
 }
 
 template <int MODE>
-__global__ __launch_bounds__(NT) void fp8_forward_select_kernel(const SelectParams p) {
+__global__ __launch_bounds__(NT, 2) void fp8_forward_select_kernel(const SelectParams p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
-  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, l16 = lane & 15, kg = lane >> 4;
-  const int block = blockIdx.x, nblocks = gridDim.x;
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63, l16 = lane & 15, kg = lane >> 4, block = blockIdx.x, nblocks = gridDim.x;
   const unsigned lds0 = (unsigned)(size_t)(lds_u8*)lds_raw;
+  const bool active = 32 * w < p.batch;   // (wave-uniform) a wavefront without batch rows only helps to load
   intx8 xq[2][6];
-#pragma unroll
-  for (int nb = 0; nb < 2; nb++)
-#pragma unroll
-    for (int ks = 0; ks < 6; ks++)
-      xq[nb][ks] = *(const intx8*)(p.xq + ((size_t)((w * 2 + nb) * 6 + ks) * 64 + lane) * 32);
+  if (active) fwd_load_x(p.xq, w, lane, xq);
   unsigned bkey[2] = {0xFFFFu, 0xFFFFu}, bm1[2] = {0xFFFEFFFEu, 0xFFFEFFFEu};
+  unsigned rows_in_use = 0u;              // bits 8half + 4nb + e of the batch blocks that this lane has a row of
   if (MODE == 1) {
 #pragma unroll
     for (int nb = 0; nb < 2; nb++) {
       const int b = 32 * w + 16 * nb + l16;
       if (b < p.batch) {
+        rows_in_use |= 0x0F0Fu << (4 * nb);
         unsigned t = p.bound[b];
         t = t < 1u ? 1u : t;
         bkey[nb] = t;
@@ -272,138 +292,136 @@ __global__ __launch_bounds__(NT) void fp8_forward_select_kernel(const SelectPara
     }
   }
   __builtin_amdgcn_s_waitcnt(0);
-  auto issue = [&](int j, int buf) {
-    const int t = j * p.tile_step;
-    const int c = t / p.tiles_per_chunk, row0 = (t - c * p.tiles_per_chunk) * FT;
-    fwd_issue_tile(p.chunk[c] + (size_t)row0 * D, min(FT, p.rows_per_chunk - row0), lds0 + (unsigned)buf * FB, w, lane);
+  int ahead = block;                      // next visit to be requested
+  FwdPlace at_ahead(block * p.tile_step, p.tiles_per_chunk), place = at_ahead;   // its place, that of the visit at hand
+  const int stride = nblocks * p.tile_step;
+  auto issue = [&](int buf) {
+    if (ahead < p.n_visit) {
+      const int row0 = at_ahead.r * FT;
+      fwd_issue_tile<NT / 64>(p.chunk[at_ahead.c] + (size_t)row0 * D, min(FT, p.rows_per_chunk - row0), lds0 + (unsigned)buf * FB, w, lane);
+    }
+    ahead += nblocks;
+    at_ahead.advance(stride, p.tiles_per_chunk);
   };
   unsigned mx[2] = {0u, 0u};
-  unsigned* q_cnt = (unsigned*)(lds_raw + FWD_LDS);
-  unsigned long long* q_ent = (unsigned long long*)(lds_raw + FWD_LDS + 16);
+  unsigned long long* q_ent = (unsigned long long*)(lds_raw + SEL_BUF * FB) + w * SEL_QUEUE;
   auto emit = [&](unsigned long long ent) {
     const unsigned b = (unsigned)(ent >> 48);
-    const unsigned slot = atomicAdd(p.count + b, 1u);
+    const unsigned slot = atomicAdd(p.count + b * SEL_COUNT_STRIDE, 1u);
     if (slot < (unsigned)SEL_CAP) {
       p.cand_label[(size_t)b * SEL_CAP + slot] = 0xFFFFFFFFu - (unsigned)ent;
       p.cand_key[(size_t)b * SEL_CAP + slot] = (unsigned short)(ent >> 32);
     }
   };
-  int since = 0;
-  if (MODE == 1) {
-    if (tid == 0) *q_cnt = 0u;   // visible to all after the first barrier below
-  }
-  if (block < p.n_visit) {
-    issue(block, 0);
-    if (block + nblocks < p.n_visit) {
-      issue(block + nblocks, 1);
-      asm volatile("s_waitcnt vmcnt(%0)" : : "n"(FWD_DMA) : "memory");
+  // The queue moves to the rows' lists when it is half full and at the end: the list slots come from atomics whose results a
+  // wavefront has to wait for, together with its outstanding tile loads.
+  int queued = 0;                         // (wave-uniform) entries, those that went to the list because the queue was full included
+  auto flush = [&] {
+    const int n = queued < SEL_QUEUE ? queued : SEL_QUEUE;
+    for (int i = lane; i < n; i += 64) emit(q_ent[i]);
+    queued = 0;
+  };
+  for (int k = 0; k < SEL_BUF - 1; k++) issue(k);
+  int buf = 0;
+  for (int j = block; j < p.n_visit; j += nblocks) {
+    const int row0 = place.r * FT;
+    const int rows_valid = min(FT, p.rows_per_chunk - row0);
+    const long long label0 = (long long)place.c * p.rows_per_chunk + row0;
+    const long long left = p.num_labels - label0;
+    const int nvalid = (int)(left < rows_valid ? (left < 0 ? 0 : left) : rows_valid);
+    fwd_wait<NT / 64, SEL_BUF - 2>(j + (SEL_BUF - 2) * nblocks < p.n_visit);
+    __syncthreads();   // the tile has landed for every wavefront, and the one before has been read by all
+    if (MODE == 1 && queued > SEL_QUEUE / 2) flush();
+    auto other = [&] { issue(buf == 0 ? SEL_BUF - 1 : buf - 1); };
+    if (!active) {
+      other();
     } else {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    }
-    __syncthreads();
-    int buf = 0;
-    for (int j = block; j < p.n_visit; j += nblocks) {
-      const int t = j * p.tile_step;
-      const int c = t / p.tiles_per_chunk, row0 = (t - c * p.tiles_per_chunk) * FT;
-      const int rows_valid = min(FT, p.rows_per_chunk - row0);
-      const long long label0 = (long long)c * p.rows_per_chunk + row0;
-      const long long left = p.num_labels - label0;
-      const int nvalid = (int)(left < rows_valid ? (left < 0 ? 0 : left) : rows_valid);
-      const unsigned char* wt = lds_raw + buf * FB;
-      const bool more = j + 2 * nblocks < p.n_visit;
-      // the buffer two ahead was read in the iteration before this one, which every wavefront has left (barrier below)
-      if (more) issue(j + 2 * nblocks, buf == 0 ? 2 : buf - 1);
-      floatx4 z[2][2];
+      // a lane holds, for batch rows 32w + 16nb + l16, the logits of tile rows 16half + 4kg + e (e = 0..3): the bf16
+      // values the dense kernel would store, two to a word, word 4half + 2nb + e / 2
+      unsigned wp[8];
 #pragma unroll
-      for (int rb = 0; rb < 2; rb++) { z[rb][0] = floatx4{0.f, 0.f, 0.f, 0.f}; z[rb][1] = floatx4{0.f, 0.f, 0.f, 0.f}; }
-#pragma unroll
-      for (int ks = 0; ks < 6; ks++)
-#pragma unroll
-        for (int rb = 0; rb < 2; rb++) {
-          intx8 a = lds_read32(wt + (16 * rb + l16) * WS + ks * 128 + kg * 32);
-          z[rb][0] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, xq[0][ks], z[rb][0], 0, 0, 0, 0, 0, 0);
-          z[rb][1] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, xq[1][ks], z[rb][1], 0, 0, 0, 0, 0, 0);
-        }
-      // a lane holds, for batch rows 32w + 16nb + l16, the logits of tile rows 16rb + 4kg + e (e = 0..3): the bf16
-      // values the dense kernel would store, two to a word
-      unsigned wp[2][2][2];
-#pragma unroll
-      for (int rb = 0; rb < 2; rb++)
+      for (int half = 0; half < 2; half++) {
+        floatx4 z[2];
+        const unsigned char* rows = lds_raw + buf * FB + 16 * half * WS;
+        if (half == 0) fwd_products(rows, l16, kg, xq, z, other);
+        else fwd_products(rows, l16, kg, xq, z, [] {});
 #pragma unroll
         for (int nb = 0; nb < 2; nb++) {
-          if (p.zscale != 1.0f) z[rb][nb] *= p.zscale;   // the same product as the dense kernel's
-          wp[rb][nb][0] = bf16_pack2(z[rb][nb][0], z[rb][nb][1]);
-          wp[rb][nb][1] = bf16_pack2(z[rb][nb][2], z[rb][nb][3]);
+          if (p.zscale != 1.0f) z[nb] *= p.zscale;   // the same product as the dense kernel's
+          wp[4 * half + 2 * nb] = bf16_pack2(z[nb][0], z[nb][1]);
+          wp[4 * half + 2 * nb + 1] = bf16_pack2(z[nb][2], z[nb][3]);
         }
+      }
       if (MODE == 0) {
 #pragma unroll
-        for (int rb = 0; rb < 2; rb++)
-#pragma unroll
-          for (int nb = 0; nb < 2; nb++)
-#pragma unroll
-            for (int hw = 0; hw < 2; hw++) {
-              unsigned kw = key_pair(wp[rb][nb][hw]);
-              if (nvalid < FT) {   // rows past the end of the chunk or of the labels do not count
-                const int r = 16 * rb + 4 * kg + 2 * hw;
-                kw &= (r < nvalid ? 0x0000FFFFu : 0u) | (r + 1 < nvalid ? 0xFFFF0000u : 0u);
-              }
-              mx[nb] = pk_max_u16(mx[nb], kw);
-            }
+        for (int q = 0; q < 8; q++) {
+          unsigned kw = key_pair(wp[q]);
+          if (nvalid < FT) {   // rows past the end of the chunk or of the labels do not count
+            const int r = 16 * (q >> 2) + 4 * kg + 2 * (q & 1);
+            kw &= (r < nvalid ? 0x0000FFFFu : 0u) | (r + 1 < nvalid ? 0xFFFF0000u : 0u);
+          }
+          mx[(q >> 1) & 1] = pk_max_u16(mx[(q >> 1) & 1], kw);
+        }
       } else {
-        unsigned hit[2][2][2], any = 0u, top = 0u;
+        unsigned hit[8], any = 0u, top = 0u;
 #pragma unroll
-        for (int rb = 0; rb < 2; rb++)
-#pragma unroll
-          for (int nb = 0; nb < 2; nb++)
-#pragma unroll
-            for (int hw = 0; hw < 2; hw++) {
-              hit[rb][nb][hw] = pk_max_u16(key_pair(wp[rb][nb][hw]), bm1[nb]) ^ bm1[nb];   // non-zero: a key above bound - 1
-              any |= hit[rb][nb][hw];
-              top = pk_max_u16(top, wp[rb][nb][hw]);                                      // a half above 0xFF80: a NaN with the sign bit
-            }
+        for (int q = 0; q < 8; q++) {
+          const unsigned below = bm1[(q >> 1) & 1];
+          hit[q] = pk_max_u16(key_pair(wp[q]), below) ^ below;   // non-zero: a key above bound - 1
+          any |= hit[q];
+          top = pk_max_u16(top, wp[q]);                          // a half above 0xFF80: a NaN with the sign bit
+        }
         const bool nan = pk_max_u16(top, 0xFF80FF80u) != 0xFF80FF80u;   // (a NaN without it has a key above every bound)
         if (__builtin_amdgcn_ballot_w64(any != 0u || nan) != 0) {
+          // Candidates go to the wavefront's queue in LDS, one of every lane that has any at a time; their places come from
+          // the lanes' ballot.  (One queue per workgroup, its places from an LDS atomic for each value, a move to the lists
+          // every eight tiles: all wavefronts waited at the next barrier for the one that was appending.)
+          unsigned mask = 0u;   // bit 2q + e of word q
 #pragma unroll
-          for (int rb = 0; rb < 2; rb++)
+          for (int q = 0; q < 8; q++) {
+            mask |= (hit[q] & 0xFFFFu) != 0u ? 1u << (2 * q) : 0u;
+            mask |= hit[q] >> 16 != 0u ? 2u << (2 * q) : 0u;
+          }
+          if (__builtin_amdgcn_ballot_w64(nan) != 0) {   // the exact keys decide
+            mask = 0u;
 #pragma unroll
-            for (int nb = 0; nb < 2; nb++) {
-              const int b = 32 * w + 16 * nb + l16;
+            for (int q = 0; q < 16; q++)
+              mask |= topk_key((unsigned short)(wp[q >> 1] >> (16 * (q & 1)))) >= bkey[(q >> 2) & 1] ? 1u << q : 0u;
+          }
+          mask &= rows_in_use;
+          if (nvalid < FT) {   // rows past the end of the chunk or of the labels do not count
 #pragma unroll
-              for (int hw = 0; hw < 2; hw++)
-                if ((hit[rb][nb][hw] != 0u || nan) && b < p.batch) {
-#pragma unroll
-                  for (int e = 0; e < 2; e++) {
-                    const int r = 16 * rb + 4 * kg + 2 * hw + e;
-                    const unsigned key = topk_key((unsigned short)(wp[rb][nb][hw] >> (16 * e)));
-                    if (key >= bkey[nb] && r < nvalid) {
-                      const unsigned long long ent = ((unsigned long long)b << 48) | ((unsigned long long)key << 32) |
-                                                     (unsigned long long)(0xFFFFFFFFu - (unsigned)(label0 + r));
-                      const unsigned qs = atomicAdd(q_cnt, 1u);
-                      if (qs < (unsigned)SEL_QUEUE) q_ent[qs] = ent;
-                      else emit(ent);   // queue full (many logits at the bound): straight to the list
-                    }
-                  }
-                }
+            for (int half = 0; half < 2; half++) {
+              const int n = nvalid - 16 * half - 4 * kg;
+              mask &= ~((n <= 0 ? 0xFFu : n >= 4 ? 0u : ((0xFu << n) & 0xFu) * 0x11u) << (8 * half));
             }
+          }
+          for (;;) {
+            const unsigned long long who = __builtin_amdgcn_ballot_w64(mask != 0u);
+            if (who == 0) break;
+            if (mask != 0u) {
+              const int q = __builtin_ctz(mask);
+              mask &= mask - 1u;
+              unsigned word = wp[0];
+#pragma unroll
+              for (int i = 1; i < 8; i++) word = q >> 1 == i ? wp[i] : word;
+              const unsigned key = topk_key((unsigned short)(q & 1 ? word >> 16 : word));
+              const unsigned b = (unsigned)(32 * w + 4 * (q & 4) + l16);
+              const unsigned label = (unsigned)label0 + (unsigned)(2 * (q & 8) + 4 * kg + (q & 3));
+              const unsigned long long ent = ((unsigned long long)((b << 16) | key) << 32) | (unsigned long long)(0xFFFFFFFFu - label);
+              const int at = queued + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(who >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)who, 0u));
+              if (at < SEL_QUEUE) q_ent[at] = ent;
+              else emit(ent);   // queue full (many logits at the bound): straight to the list
+            }
+            queued += __builtin_popcountll(who);
+          }
         }
       }
-      if (more) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(FWD_DMA) : "memory");
-      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      __syncthreads();   // the next tile has landed for every wavefront, and this one has been read by all
-      buf = buf == 2 ? 0 : buf + 1;
-      if (MODE == 1 && (++since == SEL_FLUSH || j + nblocks >= p.n_visit)) {
-        // Candidates wait in an LDS queue and move to the rows' lists every few tiles: the list slot comes from an
-        // atomic whose result a wavefront has to wait for, together with its outstanding tile loads.  Nobody adds to the
-        // queue between the barrier above and the one below.
-        since = 0;
-        const unsigned qn = *q_cnt < (unsigned)SEL_QUEUE ? *q_cnt : (unsigned)SEL_QUEUE;
-        for (unsigned i = tid; i < qn; i += NT) emit(q_ent[i]);
-        __syncthreads();
-        if (tid == 0) *q_cnt = 0u;
-        __syncthreads();
-      }
     }
+    buf = buf == SEL_BUF - 1 ? 0 : buf + 1;
+    place.advance(stride, p.tiles_per_chunk);
   }
+  if (MODE == 1) flush();
   if (MODE == 0) {
 #pragma unroll
     for (int nb = 0; nb < 2; nb++) {

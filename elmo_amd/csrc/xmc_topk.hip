@@ -347,7 +347,7 @@ __global__ __launch_bounds__(TOPK_GROUPS) void topk_bound_kernel(const unsigned 
   __shared__ unsigned wcnt[2 * (TOPK_GROUPS / 64)];
   const int b = blockIdx.x, g = threadIdx.x;
   if (g == 0) {
-    count[b] = 0u;
+    count[b * SEL_COUNT_STRIDE] = 0u;
     if (b == 0) *status = 0;
     if (b >= batch) bound[b] = 0xFFFFu;
   }
@@ -371,7 +371,7 @@ __global__ __launch_bounds__(TOPK_LIST) void topk_pick_kernel(const unsigned* ca
   __shared__ unsigned wcnt[2 * (TOPK_LIST / 64)];
   __shared__ unsigned s_m;
   const int b = blockIdx.x, tid = threadIdx.x;
-  const unsigned have = count[b];
+  const unsigned have = count[b * SEL_COUNT_STRIDE];
   const int n = have < (unsigned)TOPK_LIST ? (int)have : TOPK_LIST;
   if (tid == 0) {
     if (have > (unsigned)TOPK_LIST || n < k) atomicOr(status, have > (unsigned)TOPK_LIST ? 1 : 2);

@@ -114,9 +114,15 @@ def fp8_kahan_step(chunks, kahan, num_head, x, labels, lr, seeds=None, round_mod
     return (grad_out, gf) if want_f32 else grad_out
 
 
+def _aligned_rows(x):
+    """x, or, for a number of rows that is not a multiple of 16, a copy where its address (a view into a larger buffer) is
+    not a multiple of 16 bytes; the kernels refuse other misaligned rows."""
+    return x.clone() if x.shape[0] % 16 and x.data_ptr() % 16 else x
+
+
 def fp8_forward(chunks, x, num_labels, scale_w=1.0, scale_x=1.0, workspace=None):
     """Inference logits [B, num_labels] bf16 (reference: chunked_fp8xmc_clf.py:45-60).  Any batch size: rows are
-    processed in slices of at most 128, the last one padded to a multiple of 16."""
+    processed in slices of at most 128."""
     lib = _lib.load()
     assert x.is_cuda and x.dim() == 2 and x.shape[1] == FEATURES
     xb = x.to(torch.bfloat16).contiguous()      # exact for e4m3 input
@@ -131,20 +137,11 @@ def fp8_forward(chunks, x, num_labels, scale_w=1.0, scale_x=1.0, workspace=None)
     out = torch.empty(total, stride, dtype=torch.bfloat16, device=x.device)
     for lo in range(0, total, MAX_BATCH):
         hi = min(lo + MAX_BATCH, total)
-        n = hi - lo
-        npad = (n + 15) // 16 * 16
-        xs = xb[lo:hi]
-        if npad != n:
-            xs = torch.cat([xs, torch.zeros(npad - n, FEATURES, dtype=xb.dtype, device=xb.device)])
-            tmp = torch.empty(npad, stride, dtype=torch.bfloat16, device=x.device)
-        else:
-            tmp = out[lo:hi]
-        st = lib.xmc_fp8_forward(arr, nc, rows, xs.data_ptr(), npad, FEATURES, float(scale_w), float(scale_x),
-                                 tmp.data_ptr(), stride, num_labels, workspace.data_ptr(), workspace.numel(),
-                                 _stream_ptr())
-        _lib.check(st, "xmc_fp8_forward")
-        if npad != n:
-            out[lo:hi, :num_labels] = tmp[:n, :num_labels]
+        xs = _aligned_rows(xb[lo:hi])
+        st = lib.xmc_fp8_forward_rows(arr, nc, rows, xs.data_ptr(), hi - lo, FEATURES, float(scale_w), float(scale_x),
+                                      out[lo:hi].data_ptr(), stride, num_labels, workspace.data_ptr(), workspace.numel(),
+                                      _stream_ptr())
+        _lib.check(st, "xmc_fp8_forward_rows")
     return out[:, :num_labels]
 
 
@@ -189,34 +186,27 @@ def fp8_forward_topk(chunks, x, num_labels, k, scale_w=1.0, scale_x=1.0, workspa
     for si, lo in enumerate(range(0, total, MAX_BATCH)):
         hi = min(lo + MAX_BATCH, total)
         n = hi - lo
-        npad = (n + 15) // 16 * 16
-        xs = xb[lo:hi]
-        if npad != n:
-            # rows that pad the batch to a multiple of 16 repeat the last row (rows of zeros would tie on every label
-            # and overflow the two-pass path's candidate lists); their results are dropped below
-            xs = torch.cat([xs, xs[-1:].expand(npad - n, FEATURES)])
-            tv = torch.empty(npad, k, dtype=torch.bfloat16, device=x.device)
-        else:
-            tv = vals[lo:hi]                                               # written in place
+        xs = _aligned_rows(xb[lo:hi])
         done = False
         if fused:
             need = lib.xmc_topk_fused_scratch_bytes()
             if fused_scratch is None or fused_scratch.numel() < need:
                 fused_scratch = torch.empty(need, dtype=torch.uint8, device=x.device)
-            ti = idx[lo:hi] if npad == n else torch.empty(npad, k, dtype=torch.int64, device=x.device)
-            st = lib.xmc_fp8_forward_topk_fused(arr, nc, rows, xs.data_ptr(), npad, FEATURES, float(scale_w), float(scale_x),
-                                                int(num_labels), int(k), tv.data_ptr(), ti.data_ptr(), 1, workspace.data_ptr(),
-                                                workspace.numel(), fused_scratch.data_ptr(), fused_scratch.numel(),
-                                                status[si:].data_ptr(), _stream_ptr())
+            st = lib.xmc_fp8_forward_topk_fused_rows(arr, nc, rows, xs.data_ptr(), n, FEATURES, float(scale_w), float(scale_x),
+                                                     int(num_labels), int(k), vals[lo:hi].data_ptr(), idx[lo:hi].data_ptr(), 1,
+                                                     workspace.data_ptr(), workspace.numel(), fused_scratch.data_ptr(),
+                                                     fused_scratch.numel(), status[si:].data_ptr(), _stream_ptr())
             if st != _lib.XMC_ERR_RANGE:
-                _lib.check(st, "xmc_fp8_forward_topk_fused")
+                _lib.check(st, "xmc_fp8_forward_topk_fused_rows")
                 done = defer_check or int(status[si].item()) == 0
-                if done and npad != n:
-                    idx[lo:hi] = ti[:n]
         if not done:
             need = lib.xmc_topk_scratch_bytes(rows)
             if scratch is None or scratch.numel() < need:
                 scratch = torch.empty(need, dtype=torch.uint8, device=x.device)
+            npad = (n + 15) // 16 * 16      # rows that pad the batch repeat the last one; their results are dropped below
+            if npad != n:
+                xs = torch.cat([xs, xs[-1:].expand(npad - n, FEATURES)])
+            tv = vals[lo:hi] if npad == n else torch.empty(npad, k, dtype=torch.bfloat16, device=x.device)
             ti = torch.empty(npad, k, dtype=torch.int32, device=x.device)
             st = lib.xmc_fp8_forward_topk(arr, nc, rows, xs.data_ptr(), npad, FEATURES, float(scale_w), float(scale_x),
                                           int(num_labels), int(k), tv.data_ptr(), ti.data_ptr(), workspace.data_ptr(),
@@ -224,8 +214,8 @@ def fp8_forward_topk(chunks, x, num_labels, k, scale_w=1.0, scale_x=1.0, workspa
             _lib.check(st, "xmc_fp8_forward_topk")
             status[si] = 0
             idx[lo:hi] = ti[:n]
-        if npad != n:
-            vals[lo:hi] = tv[:n]
+            if npad != n:
+                vals[lo:hi] = tv[:n]
     if defer_check:
         return vals, idx, status
     return vals, idx

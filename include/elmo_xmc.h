@@ -117,10 +117,15 @@ int xmc_fp8_forward(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk,
                     int features, float scale_w, float scale_x, void* out_bf16, long long out_stride,
                     long long num_labels, void* workspace, size_t workspace_bytes, void* stream);
 
+/* xmc_fp8_forward for any batch of 1..128 rows (the last batch of an evaluation), not only multiples of 16. */
+int xmc_fp8_forward_rows(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, const void* x_bf16, int batch,
+                         int features, float scale_w, float scale_x, void* out_bf16, long long out_stride,
+                         long long num_labels, void* workspace, size_t workspace_bytes, void* stream);
+
 /* xmc_fp8_forward without a workspace argument.  It has no counterpart in the reference: it is for callers that cannot
  * allocate device memory for a workspace (code under HIP graph capture, serving loops and harnesses that forbid
- * hipMalloc).  The operand images of X that xmc_fp8_forward keeps in the caller's workspace live in a static device array
- * of the library instead (294,912 bytes per GPU, held until the process ends), so the limits are those of the array:
+ * hipMalloc).  The operand image of X that xmc_fp8_forward keeps in the caller's workspace lives in a static device array
+ * of the library instead (98,304 bytes per GPU, held until the process ends), so the limits are those of the array:
  * features == 768 and batch <= 128 (a multiple of 16); anything larger returns XMC_ERR_SHAPE.  The call allocates and
  * frees nothing.  Every call on a GPU uses that GPU's one array: calls that overlap on the same GPU (two streams, two
  * threads) race on it and must be serialised by the caller.  Outputs are bit-identical to xmc_fp8_forward's. */
@@ -165,6 +170,12 @@ int xmc_fp8_forward_topk_fused(void* const* chunk_ptrs, int num_chunks, int rows
                                int features, float scale_w, float scale_x, long long num_labels, int k, void* out_val_bf16,
                                void* out_idx, int idx_int64, void* workspace, size_t workspace_bytes, void* scratch,
                                size_t scratch_bytes, int32_t* status, void* stream);
+
+/* xmc_fp8_forward_topk_fused for any batch of 1..128 rows. */
+int xmc_fp8_forward_topk_fused_rows(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, const void* x_bf16, int batch,
+                                    int features, float scale_w, float scale_x, long long num_labels, int k, void* out_val_bf16,
+                                    void* out_idx, int idx_int64, void* workspace, size_t workspace_bytes, void* scratch,
+                                    size_t scratch_bytes, int32_t* status, void* stream);
 
 /* Dropout fused with the cast to e4m3 (the reference's prototype `_dropout` on the FP8 GEMM's A operand,
  * src/triton_kernels/tma_gemm.py:7-13,34-38): out[m][k] = e4m3(keep ? x[m][k] / (1 - p) : 0), keep = tl.rand(seed,

@@ -223,3 +223,38 @@ def test_dropout_quantize_matches_the_oracle(gpu, rows, cols, p, seed, as_e4m3):
     want = C.dropout_quantize(x, p, seed)
     got = out.view(torch.uint8).cpu().numpy()
     assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("nc,rows,batch,drop,hot", [
+    (3, 20016, 1, 0, 0),        # one batch row; chunks that end in half a tile; several tiles to every workgroup
+    (2, 30000, 33, 17, 32),     # one row in a wavefront of its own; labels end inside a tile; all rows share 32 best labels,
+    (2, 30000, 128, 5, 32),     # whose candidates come at once and overflow the queue of a wavefront
+    (1, 8208, 97, 1, 0),        # fewer tiles than two to a workgroup
+    (4, 16384, 40, 100, 16),
+])
+def test_forward_and_topk_any_batch(gpu, nc, rows, batch, drop, hot):
+    """Logits and the two-pass top-k for batches that are no multiple of 16 and for rows of X at any address, against a
+    float32 product of the same e4m3 operands (logits within one bf16 ulp of it) and the dense logits (top-k, exactly)."""
+    import torch
+    from elmo_amd import ops
+    gen = torch.Generator(device=gpu).manual_seed(nc * rows + batch)
+    L, k = nc * rows - drop, 40
+    base = torch.empty(batch * 768 + 4, dtype=torch.bfloat16, device=gpu)
+    x = base[4:] if batch % 16 else base[:-4]          # (8 bytes past an aligned address)
+    x = x.view(batch, 768)
+    common = torch.randn(768, generator=gen, device=gpu)
+    x.copy_(torch.randn(batch, 768, generator=gen, device=gpu) * 0.05 + common * 0.05)
+    chunks = [(torch.randn(rows, 768, generator=gen, device=gpu) * 0.02).to(torch.float8_e4m3fn) for _ in range(nc)]
+    if hot:
+        chunks[0][:hot] = (chunks[0][:hot].float() + 0.25 * common).to(torch.float8_e4m3fn)
+    out = ops.fp8_forward(chunks, x, L)
+    w = torch.cat([c.float() for c in chunks])[:L]
+    # the e4m3 products are exact in float32; the two differ in the order of 768 additions only
+    ref = (x.to(torch.float8_e4m3fn).cpu().double() @ w.cpu().double().T).to(torch.bfloat16).float()
+    H.assert_bf16_close(out.float().cpu().numpy(), ref.numpy())
+    dense = out.float().cpu().numpy()
+    vals, idx, status = ops.fp8_forward_topk(chunks, x, L, k, fused=True, defer_check=True)
+    assert int(status.max().item()) == 0
+    want_v, want_i = O.topk_of_logits(dense, k)
+    assert np.array_equal(vals.float().cpu().numpy(), want_v)
+    assert np.array_equal(idx.cpu().numpy(), want_i)
