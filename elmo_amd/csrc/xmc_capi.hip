@@ -658,7 +658,8 @@ static int cluster_step(void* const* chunk_ptrs, int num_chunks, int rows_per_ch
     const int sort_blocks = n_pad / 64, ptr_blocks = (nch * tpc64 + 1 + 255) / 256, prep_blocks = (bp * (D / 4) + 255) / 256;
     const ClusterPrep pp = {labels_coo, nnz, n_pad, batch, c0 * rows_per_chunk, nch * rows_per_chunk, pairs, rows_per_chunk, tpc64, nch * tpc64,
                             sort_blocks, ptr_blocks, keys, tile_ptr, lay.tp_stride, (const unsigned short*)x_bf16, bp, bf16 ? 0 : fp8 ? 2 : 1,
-                            ws + lay.xq, (unsigned short*)(ws + lay.xt), (int*)(ws + lay.flags), err};
+                            ws + lay.xq, (unsigned short*)(ws + lay.xt), (int*)(ws + lay.flags),
+                            c0 == 0 ? err : nullptr};   // (a failure in one segment stays visible behind the others)
     cluster_prep_kernel<<<(sort_blocks + ptr_blocks) * pairs + prep_blocks, 256, (size_t)(n_pad + 256) * 4, stream>>>(pp, dp);
     ClusterParams p;
     for (int k = 0; k < MAX_CHUNKS; k++) {

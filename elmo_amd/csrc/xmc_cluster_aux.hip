@@ -44,11 +44,11 @@ inline ClusterLayout cluster_layout(int num_chunks, int rows_per_chunk, int batc
 //                  element i of lane group q in step 2 j + u
 //           kind 2 (FP8 products): e4m3 codes, step of 128 features: lane group q holds bytes 16 q.. and 64 + 16 q..
 //   grad_W: X^T: block (16 features, 32 batch rows) of 64 lanes x 8: lane = feature % 16 + 16 (row / 8 % 4)
-// Also clears the counters and the error word.
+// Also clears the counters and, unless it is null, the error word.
 __device__ __forceinline__ void cluster_prep_thread(int i, const unsigned short* x, int batch, int bp, int kind, unsigned char* xq,
                                                     unsigned short* xt, int* flags, int* err, const DropoutParams& dp) {
   if (i < CLU_FLAG_INTS) flags[i] = 0;
-  if (i == 0) *err = 0;
+  if (i == 0 && err) *err = 0;
   if (i >= bp * (D / 4)) return;
   const int b = i / (D / 4), k = (i - b * (D / 4)) * 4;
   unsigned short raw[4] = {0, 0, 0, 0};
