@@ -676,7 +676,6 @@ static int cluster_step(void* const* chunk_ptrs, int num_chunks, int rows_per_ch
     p.tpc64 = tpc64;
     p.ntiles = (nch - 1) * p.tpc + p.tpc_last;
     const int most = (cus < CLU_MAXWG ? cus : CLU_MAXWG) / 8 / c * 8;   // whole clusters on every XCD
-    if (most < 8) return XMC_ERR_DEVICE;
     p.nclusters = p.ntiles < most ? p.ntiles : most;
     p.label0_seg = 0u;
     p.label0 = (unsigned)c0 * (unsigned)rows_per_chunk;
@@ -738,7 +737,9 @@ static int tiled_step_t(void* const* chunk_ptrs, int num_chunks, int rows_per_ch
   DeviceInfo di = device_info();
   if (di.ok != 1) return XMC_ERR_DEVICE;
   hipStream_t stream = (hipStream_t)stream_;
-  if (DD == D && kahan_type == 0 && !loss_out && weight_decay == 0.f)
+  // (a cluster needs its members on one XCD at the same time: a partition of the GPU too small for one keeps the three kernels)
+  const int cluster = cluster_size(batch, weight_type != W_BF16 && quantize_x);
+  if (DD == D && kahan_type == 0 && !loss_out && weight_decay == 0.f && di.cus / 8 / cluster >= 1)
     return cluster_step(chunk_ptrs, num_chunks, rows_per_chunk, rows_last_chunk, weight_type, x_bf16, batch, labels_coo, nnz, lr, seeds,
                         round_mode, quantize_x, saturate, dp, grad_x_bf16, grad_x_f32, (unsigned char*)workspace, di.cus, di.failure_word, stream);
   unsigned char* ws = (unsigned char*)workspace + TW_HEAD;
