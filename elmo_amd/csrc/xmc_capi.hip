@@ -261,8 +261,7 @@ static int fused_step(void* const* chunk_ptrs, int num_chunks, int rows_per_chun
   const int grid = di.cus < MAX_WG ? di.cus : MAX_WG;   // one workgroup per compute unit
   const int tiles_per_chunk = (rows_per_chunk + TL - 1) / TL;
   const int num_tiles = num_chunks * tiles_per_chunk;
-  int n_pad = 0;
-  if (nnz > 0) { n_pad = 64; while (n_pad < nnz) n_pad <<= 1; }
+  const int n_pad = (nnz + 63) / 64 * 64;   // whole blocks of the sort
 
   {
     QuadParams p;
@@ -641,8 +640,7 @@ static int cluster_step(void* const* chunk_ptrs, int num_chunks, int rows_per_ch
   const ClusterLayout lay = cluster_layout(num_chunks, rows_per_chunk, bp);
   const int tile_rows = fp8 && c < 8 ? 64 : 32;
   const int tpc64 = (rows_per_chunk + TL - 1) / TL;
-  int n_pad = 0;
-  if (nnz > 0) { n_pad = 64; while (n_pad < nnz) n_pad <<= 1; }
+  const int n_pad = (nnz + 63) / 64 * 64;   // whole blocks of the sort
   // a sort key keeps 24 bits for the label: larger label spaces are taken in segments of whole chunks
   int seg_chunks = ((1 << 24) - 2) / rows_per_chunk;
   if (seg_chunks > num_chunks) seg_chunks = num_chunks;
@@ -768,8 +766,7 @@ static int tiled_step_t(void* const* chunk_ptrs, int num_chunks, int rows_per_ch
   int* tile_ptr = (int*)(glb + halves * g_half);
   const size_t tp_stride = (size_t)(num_tiles + 1 + 63) / 64 * 64;   // entries of one pair's tile_ptr
   float* loss_part = (float*)(tile_ptr + pairs * tp_stride);         // one share per sub-tile of 32 rows
-  int n_pad = 0;
-  if (nnz > 0) { n_pad = 64; while (n_pad < nnz) n_pad <<= 1; }
+  const int n_pad = (nnz + 63) / 64 * 64;   // whole blocks of the sort
 
   // chunks per segment of the label space: a multiple of the launch group, fewer than 2^24 - 1 labels
   int seg_chunks = ((1 << 24) - 2) / rows_per_chunk / group * group;

@@ -140,10 +140,11 @@ __device__ __forceinline__ unsigned positive_key(int2 e, int batch, int row0, in
   return (r >= 0 && r < 256 && r + row0 < batch && e.y >= 0 && lab >= 0 && lab < label_count && lab < (1 << 24) - 1) ? (((unsigned)lab << 8) | (unsigned)r) : 0xFFFFFFFFu;
 }
 
-// Sorts the positives by rank.  Block b ranks keys 64b..64b+63 of the n_pad (a power of two, at least 64): every block
+// Sorts the positives by rank.  Block b ranks keys 64b..64b+63 of the n_pad (a multiple of 64): every block
 // builds all keys in LDS ((n_pad + 256) * 4 bytes), its four wavefronts each count the keys that precede the block's own
 // over a quarter of the set (equal keys: the one that comes first in the input precedes), and the sum of the four counts
-// is the key's position in the output.  256 threads.
+// is the key's position in the output.  256 threads.  (Padded to whole blocks only: up to the next power of two, the
+// preparation of a step with 4,608 positives took 28 us; 17 now.)
 __device__ __forceinline__ void quad_sort_block(int block, const int* coo, int nnz, int n_pad, int batch, int row0, int label_base,
                                                 int label_count, unsigned* keys) {
   // (aligned for the 16-byte reads below: behind a kernel's static LDS it would start at any word, and the sort of 4,608

@@ -204,3 +204,12 @@ def test_step_replays_in_a_captured_graph(gpu):
         assert torch.equal(gout.view(torch.int16), eager[k][1]), f"grad_input differs after replay {k}"
         scratch = torch.randn(1 << 20, device=gpu).sum().item()      # unrelated eager work between the replays
         assert scratch == scratch
+
+
+@pytest.mark.parametrize("nnz", [1, 63, 64, 65, 193, 1025, 4609])
+def test_sort_pads_the_positives_to_whole_blocks_only(gpu, nnz):
+    """Numbers of positives around the sort's block of 64 keys, in random order and with repetitions, against the oracle."""
+    case = H.make_case(2, 1040, 64, 90 + nnz)
+    rng = np.random.default_rng(nnz)
+    case["labels"] = np.stack([rng.integers(0, 64, nnz), rng.integers(0, 2 * 1040, nnz)], axis=1).astype(np.int32)
+    check_rtn(case, gpu)
