@@ -94,6 +94,8 @@ def load():
     lib.xmc_tiled_error_offset.restype = sz
     lib.xmc_tiled_sticky_error_offset.restype = sz
     lib.xmc_failure_word.restype = vp
+    lib.xmc_pass_on_error.restype = i32
+    lib.xmc_pass_on_error.argtypes = [vp, vp, vp, vp]
     lib.xmc_step_workgroups.restype = i32
     lib.xmc_step_xcc_ids.restype = i32
     lib.xmc_step_xcc_ids.argtypes = [vp, ctypes.POINTER(ctypes.c_int32), i32, vp]

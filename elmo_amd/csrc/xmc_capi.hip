@@ -38,14 +38,14 @@ void fill_device_info(int dev) {
   // this device's copy of the static scratch array (device `dev` is current here); stays null if the lookup fails
   void* sp = nullptr;
   di.scratch_ptr = (di.ok == 1 && hipGetSymbolAddress(&sp, HIP_SYMBOL(scratch)) == hipSuccess) ? (unsigned char*)sp : nullptr;
-  // the word of host memory in which the kernels of this device announce a failed step; lives until the process ends.  A
+  // the two words of host memory in which the kernels of this device announce failed steps; live until the process ends.  A
   // caller may be capturing a graph: the allocation is none of that graph's business
   if (di.ok == 1) {
     hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
     const bool swapped = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
     void* fw = nullptr;
     if (hipHostMalloc(&fw, 64, hipHostMallocMapped) == hipSuccess) {
-      *(int*)fw = 0;
+      ((int*)fw)[0] = ((int*)fw)[1] = 0;
       di.failure_word = (int*)fw;
     }
     if (swapped) (void)hipThreadExchangeStreamCaptureMode(&mode);
@@ -118,6 +118,20 @@ int check_common(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, co
   if (!aligned16(x) || ((uintptr_t)workspace & 255) != 0) return XMC_ERR_ALIGN;
   if (workspace_bytes < xmc_workspace_bytes(num_chunks, rows_per_chunk)) return XMC_ERR_WORKSPACE;
   return XMC_OK;
+}
+
+// The error word of a step that ran in a workspace which goes away with the call, passed on behind the step by one thread:
+// into the two words of a workspace that stays, or, without one, into the second failure word in host memory (a clock
+// reading, so that it changes with every failed step, and the error bits).
+__global__ void pass_on_error_kernel(const int* err, int* into_error, int* into_sticky, int* failure_word) {
+  const int e = __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (into_sticky) {
+    *into_error = e;
+    report_step_error(err, into_sticky, failure_word);
+  } else if (e != 0) {
+    __hip_atomic_store(failure_word + 1, (int)((unsigned)__builtin_amdgcn_s_memrealtime() << 2 | (unsigned)(e & 3)), __ATOMIC_RELEASE,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
+  }
 }
 
 // plain 16-byte-per-lane copy: the known-size reference against which memory counters are calibrated
@@ -612,6 +626,15 @@ size_t xmc_tiled_workspace_bytes_ex(int num_chunks, int rows_per_chunk, int max_
 }
 
 int* xmc_failure_word(void) { return device_info().failure_word; }
+
+int xmc_pass_on_error(const int32_t* error_word, int32_t* into_error, int32_t* into_sticky, void* stream_) {
+  if (!error_word || !into_error != !into_sticky) return XMC_ERR_NULL;
+  if ((((uintptr_t)error_word | (uintptr_t)into_error | (uintptr_t)into_sticky) & 3) != 0) return XMC_ERR_ALIGN;
+  const DeviceInfo di = device_info();
+  if (di.ok != 1 || !di.failure_word) return XMC_ERR_DEVICE;
+  pass_on_error_kernel<<<1, 1, 0, (hipStream_t)stream_>>>(error_word, into_error, into_sticky, di.failure_word);
+  return launch_status();
+}
 
 size_t xmc_tiled_error_offset(void) { return TW_ERR; }
 size_t xmc_tiled_sticky_error_offset(void) { return TW_ERR + 4; }

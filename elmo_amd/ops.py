@@ -4,6 +4,7 @@ import ctypes
 import torch
 
 from . import _lib
+from .step_errors import UnkeptStepErrors
 
 FEATURES = 768
 _CODE_TYPES = (torch.float8_e4m3fn, torch.uint8)
@@ -47,12 +48,36 @@ def alloc_workspace(num_chunks, rows_per_chunk, device):
     return ws
 
 
+_unkept = {}             # device index -> UnkeptStepErrors
+
+
+def _unkept_errors(device):
+    index = torch.cuda.current_device() if device.index is None else device.index
+    errors = _unkept.get(index)
+    return errors if errors is not None else _unkept.setdefault(index, UnkeptStepErrors(torch.device("cuda", index)))
+
+
+def check_steps(device="cuda"):
+    """Waits for the steps enqueued so far and raises RuntimeError if one of those that were given no workspace has failed
+    since the last report.  (The error words of the others are in their workspaces.)"""
+    _unkept_errors(torch.device(device)).check_now()
+
+
+def _pass_on_error(temporary, error_offset, kept=None):
+    """Behind a step in a workspace that goes away with the call: its error word, to the tiled step's words of the `kept`
+    workspace, or to the device's words for steps without one."""
+    into = (kept.data_ptr() + tiled_error_offset(), kept.data_ptr() + tiled_sticky_error_offset()) if kept is not None else (None, None)
+    _lib.check(_lib.load().xmc_pass_on_error(temporary.data_ptr() + error_offset, *into, _stream_ptr()), "xmc_pass_on_error")
+
+
 def fp8_step(chunks, x, labels, lr, seeds=None, round_mode="rtn", scale_w=1.0, scale_x=1.0, workspace=None,
              grad_out=None, want_f32=False, weight_decay=0.0, dropout_p=0.0, dropout_seed=0):
     """One fused training step (reference: chunked_fp8xmc_clf.py:81-123).  Updates `chunks` in place and returns
     grad_input (bf16 [B, 768]) or (grad_input, grad_x_fp32) when want_f32.  weight_decay, dropout_p, dropout_seed: the
     additions of xmc_fp8_step_ex (decay inside the update, dropout of the embedding inside the step); zero = the
-    reference's step."""
+    reference's step.
+    A step that fails (xmc_step_error_word) does not raise: its error words are in `workspace`.  Without one the next call
+    without one, or check_steps, raises."""
     lib = _lib.load()
     assert x.is_cuda and x.dtype == torch.bfloat16 and x.is_contiguous() and x.dim() == 2
     assert labels.is_cuda and labels.dtype == torch.int32 and labels.is_contiguous()
@@ -60,7 +85,9 @@ def fp8_step(chunks, x, labels, lr, seeds=None, round_mode="rtn", scale_w=1.0, s
     batch, feat = x.shape
     arr, rows = _chunk_array(chunks)
     nc = len(chunks)
-    if workspace is None:
+    kept = workspace is not None
+    if not kept:
+        _unkept_errors(x.device).check()
         workspace = alloc_workspace(nc, rows, x.device)
     if grad_out is None:
         grad_out = torch.empty(batch, feat, dtype=torch.bfloat16, device=x.device)
@@ -80,6 +107,8 @@ def fp8_step(chunks, x, labels, lr, seeds=None, round_mode="rtn", scale_w=1.0, s
                                  grad_out.data_ptr(), gf.data_ptr() if gf is not None else None,
                                  workspace.data_ptr(), workspace.numel(), _stream_ptr())
     _lib.check(st, "xmc_fp8_step")
+    if not kept:
+        _pass_on_error(workspace, step_error_offset())
     return (grad_out, gf) if want_f32 else grad_out
 
 
@@ -87,7 +116,7 @@ def fp8_kahan_step(chunks, kahan, num_head, x, labels, lr, seeds=None, round_mod
                    want_f32=False):
     """One fused step of the head-Kahan layer (reference: chunked_head_kahan_fp8xmc_clf.py:95-133): as fp8_step, and the
     first num_head rows of chunk 0 are updated with the compensation buffer `kahan` ([num_head, 768] bf16 or
-    float8_e5m2, updated in place)."""
+    float8_e5m2, updated in place).  Failures as in fp8_step."""
     lib = _lib.load()
     assert x.is_cuda and x.dtype == torch.bfloat16 and x.is_contiguous() and x.dim() == 2
     assert labels.is_cuda and labels.dtype == torch.int32 and labels.is_contiguous()
@@ -97,7 +126,9 @@ def fp8_kahan_step(chunks, kahan, num_head, x, labels, lr, seeds=None, round_mod
     nc = len(chunks)
     assert kahan.is_cuda and kahan.is_contiguous() and kahan.shape == (num_head, FEATURES)
     assert kahan.dtype in (torch.bfloat16, torch.float8_e5m2) and 0 < num_head <= rows
-    if workspace is None:
+    kept = workspace is not None
+    if not kept:
+        _unkept_errors(x.device).check()
         workspace = alloc_workspace(nc, rows, x.device)
     if grad_out is None:
         grad_out = torch.empty(batch, feat, dtype=torch.bfloat16, device=x.device)
@@ -111,6 +142,8 @@ def fp8_kahan_step(chunks, kahan, num_head, x, labels, lr, seeds=None, round_mod
                                 gf.data_ptr() if gf is not None else None, workspace.data_ptr(), workspace.numel(),
                                 _stream_ptr())
     _lib.check(st, "xmc_fp8_kahan_step")
+    if not kept:
+        _pass_on_error(workspace, step_error_offset())
     return (grad_out, gf) if want_f32 else grad_out
 
 
@@ -255,6 +288,9 @@ def alloc_tiled_workspace(num_chunks, rows_per_chunk, device, max_batch=MAX_BATC
     return ws
 
 
+TILED_ERROR_BYTES = 256      # the part of a tiled workspace, in front, that holds its error words
+
+
 def tiled_error_offset():
     """Byte offset of the tiled step's error word (int32) inside its workspace."""
     return int(_lib.load().xmc_tiled_error_offset())
@@ -283,7 +319,10 @@ def tiled_step(chunk_views, rows_per_chunk, weight_type, x, labels, lr, seeds=No
     the simulated one; `kahan` ([num_head, d] bf16 or float8_e5m2, updated in place) turns on the head-Kahan update of
     the first num_head rows of chunk 0 (chunked_head_kahan_fp8xmc_clf.py:127-131).  `loss_out` (a float32 device tensor
     with one element) receives the summed binary cross entropy of the step's logits (what chunked.py:57-72 is written
-    to compute).  weight_decay, dropout_p, dropout_seed: as in fp8_step."""
+    to compute).  weight_decay, dropout_p, dropout_seed: as in fp8_step.
+    The one-kernel form can fail, as the fused step can (xmc_tiled_error_offset), and does not raise: its error words are in
+    `workspace`, also where that is too small for the batch and the step runs in a temporary one.  Without a workspace
+    the next call without one, or check_steps, raises."""
     lib = _lib.load()
     assert x.is_cuda and x.dtype == torch.bfloat16 and x.is_contiguous() and x.dim() == 2
     feats = x.shape[1]
@@ -306,8 +345,10 @@ def tiled_step(chunk_views, rows_per_chunk, weight_type, x, labels, lr, seeds=No
     arr = (ctypes.c_void_p * nc)(*[c.data_ptr() for c in chunk_views])
     batch = x.shape[0]
     assert 0 < batch <= MAX_BATCH_TILED, "batch must be at most 512"
+    kept, temporary = workspace, None
     if workspace is None:
-        workspace = alloc_tiled_workspace(nc, rows_per_chunk, x.device, batch, feats)
+        _unkept_errors(x.device).check()
+        workspace = temporary = alloc_tiled_workspace(nc, rows_per_chunk, x.device, batch, feats)
     if grad_out is None:
         grad_out = torch.empty(batch, feats, dtype=torch.bfloat16, device=x.device)
     gf = torch.empty(batch, feats, dtype=torch.float32, device=x.device) if want_f32 else None
@@ -324,9 +365,14 @@ def tiled_step(chunk_views, rows_per_chunk, weight_type, x, labels, lr, seeds=No
             gf.data_ptr() if gf is not None else None, loss_out.data_ptr() if loss_out is not None else None)
     st = lib.xmc_tiled_step_ex(*args, workspace.data_ptr(), workspace.numel(), _stream_ptr())
     if st == _lib.XMC_ERR_WORKSPACE:     # nothing has been launched: the workspace is for smaller batches
-        workspace = alloc_tiled_workspace(nc, rows_per_chunk, x.device, batch, feats)
-        st = lib.xmc_tiled_step_ex(*args, workspace.data_ptr(), workspace.numel(), _stream_ptr())
+        if workspace.numel() < TILED_ERROR_BYTES:
+            kept = None
+            _unkept_errors(x.device).check()
+        temporary = alloc_tiled_workspace(nc, rows_per_chunk, x.device, batch, feats)
+        st = lib.xmc_tiled_step_ex(*args, temporary.data_ptr(), temporary.numel(), _stream_ptr())
     _lib.check(st, "xmc_tiled_step")
+    if temporary is not None:
+        _pass_on_error(temporary, tiled_error_offset(), kept)
     return (grad_out, gf) if want_f32 else grad_out
 
 

@@ -13,6 +13,46 @@ import torch
 from . import _lib
 
 
+def _failure_words(device):
+    """The host addresses of the device's two failure words, as ctypes integers."""
+    with torch.cuda.device(device):
+        address = _lib.load().xmc_failure_word()
+    if not address:
+        raise _lib.XmcError("no failure word: not a gfx950 device, or no pinned host memory")
+    return ctypes.c_int.from_address(address), ctypes.c_int.from_address(address + 4)
+
+
+def _failure(word):
+    return RuntimeError(
+        f"a classifier step failed (error word {word}): "
+        + ("a workgroup gave up waiting for its partners (another stream kept the device busy?); " if word & 1 else "")
+        + ("workgroups that exchange data were not placed on one XCD; " if word & 2 else "")
+        + "the weights and grad_input of that step are incomplete")
+
+
+class UnkeptStepErrors:
+    """Failures of the steps on a device that were given no workspace: the one they ran in went away with the call, and
+    its error word was passed on to the device's second failure word."""
+
+    def __init__(self, device):
+        self.device = torch.device(device)
+        self._word = _failure_words(self.device)[1]
+        self._seen = 0
+
+    def check(self):
+        """Raises if such a step has announced a failure.  Waits only if one has."""
+        if self._word.value != self._seen:
+            self.check_now()
+
+    def check_now(self):
+        """Waits for the steps enqueued so far and raises if such a step among them failed."""
+        torch.cuda.synchronize(self.device)
+        word = self._word.value      # (never cleared: a failure announced from here on changes it again)
+        if word != self._seen:
+            self._seen = word
+            raise _failure(word & 3)
+
+
 class StepErrors:
     """The sticky error words of a layer's workspaces.  `words`: int32 device tensors of one element each."""
 
@@ -22,11 +62,7 @@ class StepErrors:
         self._watch()
 
     def _watch(self):
-        with torch.cuda.device(self.device):
-            address = _lib.load().xmc_failure_word()
-        if not address:
-            raise _lib.XmcError("no failure word: not a gfx950 device, or no pinned host memory")
-        self._word = ctypes.c_int.from_address(address)
+        self._word = _failure_words(self.device)[0]
         self._seen = self._word.value
 
     def __getstate__(self):      # copies and pickles of a layer watch the word of the process they live in
@@ -57,8 +93,4 @@ class StepErrors:
             torch.cuda.synchronize(self.device)
         self._seen = self._word.value
         if word != 0:
-            raise RuntimeError(
-                f"a classifier step failed (error word {word}): "
-                + ("a workgroup gave up waiting for its partners (another stream kept the device busy?); " if word & 1 else "")
-                + ("workgroups that exchange data were not placed on one XCD; " if word & 2 else "")
-                + "the weights and grad_input of that step are incomplete")
+            raise _failure(word)

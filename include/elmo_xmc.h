@@ -284,11 +284,20 @@ size_t xmc_step_error_offset(void);
  * after handling a failure. */
 size_t xmc_step_sticky_error_offset(void);
 
-/* A word of host memory of the current device, there until the process ends (NULL without a usable device; no counterpart
- * in the reference): it changes whenever a step on the device (fused or tiled) ends while its workspace's sticky error
- * word is not zero.  Remember its value; when it has changed, wait for the device and look at the sticky word of your own
- * workspace: the failure may be another's. */
+/* Two words of host memory of the current device, there until the process ends (NULL without a usable device; no
+ * counterpart in the reference).  The first changes whenever a step on the device (fused or tiled) ends while its
+ * workspace's sticky error word is not zero.  Remember its value; when it has changed, wait for the device and look at the
+ * sticky word of your own workspace: the failure may be another's.  The second starts at zero and changes whenever
+ * xmc_pass_on_error finds a failure that has no workspace to go to; its two lowest bits are then the error bits. */
 int* xmc_failure_word(void);
+
+/* For a caller that ran a step in a workspace it is about to give back (no counterpart in the reference): enqueues, behind
+ * the step, the passing on of that workspace's error word.
+ *   error_word               device address of it: the workspace + xmc_step_error_offset() or xmc_tiled_error_offset()
+ *   into_error, into_sticky  device addresses of the words of a workspace that is kept: the first receives the error word,
+ *                            the second has it OR-ed in, as if the step had run there; or both null: a failure changes
+ *                            the second word of xmc_failure_word.  XMC_ERR_NULL if only one is given */
+int xmc_pass_on_error(const int32_t* error_word, int32_t* into_error, int32_t* into_sticky, void* stream);
 
 /* Diagnostics of the placement assumption of the fused kernel (no counterpart in the reference).  The kernel builds
  * quads out of workgroups g with equal g % 8 and expects them on one XCD; every workgroup records the XCC id it really

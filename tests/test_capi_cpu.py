@@ -172,3 +172,11 @@ def test_three_kernel_path_accepts_label_spaces_of_2_24_and_more():
     assert tiled(1, 1 << 24, 1 << 40) == -4       # one chunk must stay below 2^24 rows
     sarr = (ctypes.c_uint32 * nc)(*([0] * nc))
     assert lib.xmc_fp8_step(arr, nc, rows, P, 32, 768, P, 4, 0.05, sarr, 0, 1.0, 1.0, P, None, P, 1 << 40, None) == -4
+
+
+def test_pass_on_error_rejects_bad_arguments_before_touching_the_device():
+    lib = _lib.load()
+    P = 0x10000
+    assert lib.xmc_pass_on_error(None, P, P, None) == -1
+    assert lib.xmc_pass_on_error(P, P, None, None) == -1 and lib.xmc_pass_on_error(P, None, P, None) == -1
+    assert lib.xmc_pass_on_error(P + 2, P, P, None) == -3 and lib.xmc_pass_on_error(P, P, P + 1, None) == -3
