@@ -291,6 +291,11 @@ def alloc_tiled_workspace(num_chunks, rows_per_chunk, device, max_batch=MAX_BATC
 TILED_ERROR_BYTES = 256      # the part of a tiled workspace, in front, that holds its error words
 
 
+def alloc_tiled_error_words(device):
+    """A workspace that is too small for any batch and holds the error words of the tiled steps it is given to."""
+    return torch.zeros(TILED_ERROR_BYTES, dtype=torch.uint8, device=device)
+
+
 def tiled_error_offset():
     """Byte offset of the tiled step's error word (int32) inside its workspace."""
     return int(_lib.load().xmc_tiled_error_offset())

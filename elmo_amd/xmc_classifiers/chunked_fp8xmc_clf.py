@@ -94,7 +94,6 @@ class Fp8XMCBCEChunkedLayer(nn.Module):
         # all scratch memory of the step comes from the torch allocator (so that max_memory_allocated sees it)
         self._workspace = (None if self._other_width else
                            ops.alloc_workspace(self.num_chunks, self.num_labels_i, self.device))
-        self._tiled_workspace = None
         self._last = None            # workspace of the last step: its error word is defined from then on
         # batches of more than 128 rows (up to 512) also run on the tiled step, with the true-FP8 arithmetic
         self._max_batch = int(_opt(cfg.data, "batch_size", ops.MAX_BATCH))
@@ -109,6 +108,9 @@ class Fp8XMCBCEChunkedLayer(nn.Module):
             self._tiled_workspace = ops.alloc_tiled_workspace(self.num_chunks, self.num_labels_i, self.device,
                                                               min(max(self._max_batch, ops.MAX_BATCH), ops.MAX_BATCH_TILED),
                                                               features)
+        else:
+            # a batch larger than configured takes the tiled step in a temporary workspace; its error words are kept here
+            self._tiled_workspace = ops.alloc_tiled_error_words(self.device)
         self._errors = StepErrors(self.device, ops.sticky_error_words(self._workspace, self._tiled_workspace))
 
     def _chunks(self):

@@ -48,6 +48,7 @@ def layer(kind, configured):
 @pytest.mark.parametrize("kind,configured,batch", [
     ("bf16", 32, 256),       # the layer's workspace is for 128 rows
     ("fp8", 144, 512),       # ... for 144
+    ("fp8", 32, 256),        # the layer has no workspace for batches of this size
 ])
 def test_layer_reports_a_failed_step_of_a_larger_batch(gpu, kind, configured, batch):
     xfc = layer(kind, configured)
@@ -66,6 +67,17 @@ def test_layer_reports_a_failed_step_of_a_larger_batch(gpu, kind, configured, ba
     xfc.check_steps()
     if kind == "fp8":
         assert xfc.last_step_error() == 0
+
+
+def test_larger_batch_does_not_hide_an_earlier_failure(gpu):
+    xfc = layer("fp8", 32)
+    _, x, labels = inputs(256, gpu)
+    xfc.xfc_forward_backward(x[:32].contiguous(), labels, [0.05])
+    xfc._errors.words[0].fill_(1)                    # as the last kernel of a failed step of 32 rows would have left it
+    xfc.xfc_forward_backward(x, labels, [0.05])
+    with pytest.raises(RuntimeError, match="gave up waiting"):
+        xfc.check_steps()
+    xfc.check_steps()
 
 
 def test_step_in_a_workspace_that_is_too_small_leaves_its_error_word_in_it(gpu):
