@@ -81,7 +81,7 @@ class Fp8XMCBCEChunkedHeadKahanLayer(nn.Module):
         self._errors = StepErrors(self.device, ops.sticky_error_words(self._workspace, self._tiled_workspace))
 
     def _chunks(self):
-        return list(self.xfc_weight._parameters.values())
+        return ops.parameters_in_order(self.xfc_weight)
 
     @torch.no_grad()
     def xfc_forward(self, embed):

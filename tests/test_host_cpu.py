@@ -51,6 +51,20 @@ def make_cfg(device, num_labels=1000, num_chunks=2, simulated=False, **xmc_extra
                           precision=ns(mode="custom", purelp_dtype="bfloat16")))
 
 
+def test_private_torch_interfaces_have_a_fallback(monkeypatch):
+    import torch
+    from elmo_amd import ops
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: types.SimpleNamespace(cuda_stream=0x1230))
+    monkeypatch.setattr(ops, "_raw_device", lambda: 3, raising=False)
+    monkeypatch.setattr(ops, "_raw_stream", lambda device: 0x4560 + device, raising=False)
+    assert ops._stream_ptr().value == 0x4563
+    monkeypatch.setattr(ops, "_raw_stream", None)
+    assert ops._stream_ptr().value == 0x1230
+    entries = [torch.nn.Parameter(torch.zeros(i + 1)) for i in range(12)]      # (more than ten: "10" sorts before "2")
+    for plist in (torch.nn.ParameterList(entries), entries):                   # a plain list has no dict of parameters
+        assert [p.numel() for p in ops.parameters_in_order(plist)] == list(range(1, 13))
+
+
 def test_module_refuses_to_run_without_a_gpu():
     from xmc_classifiers.chunked_fp8xmc_clf import Fp8XMCBCEChunkedLayer
     with pytest.raises(AssertionError):
