@@ -225,7 +225,8 @@ class Fp8XMCBCEChunkedLayer(nn.Module):
 
     @property
     def _err_host(self):
-        """Non-zero if a step on the device has announced a failure that this layer has not looked into."""
+        """One element, non-zero if a step on the device has announced a failure that this layer has not looked into.  Read
+        by tests only (the step looks at StepErrors itself); a tensor, as the pinned copy was that it stands for."""
         return torch.tensor([int(self._errors.pending())])
 
     def _check_previous_steps(self):

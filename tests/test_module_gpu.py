@@ -196,12 +196,11 @@ def test_simulated_mode_forward_uses_the_unquantised_embedding(gpu):
 
 
 def test_module_reports_a_failed_step_without_synchronising(gpu):
-    """The last kernel of every fused step ORs the step's error word into a sticky word of the workspace, and the module
-    sends that word to pinned host memory behind every step; a later call raises once a non-zero copy has arrived.  The
-    failure is staged from the host (the step's error word is overwritten on the stream between the step kernel and
-    nothing else: here the sticky word itself, as the step's last kernel would have left it), every kernel runs
-    normally.  Further steps are enqueued behind the failed one without any synchronisation before the check: their
-    clean error words must not hide the failure."""
+    """The last kernel of every step ORs the step's error word into a sticky word of the workspace and, while that is not
+    zero, changes a word of pinned host memory; a later call that finds this word changed waits and raises.  The failure
+    is staged from the host (the sticky word is written as the last kernel of a failed step would have left it), every
+    kernel runs normally.  Further steps are enqueued behind the failed one without any synchronisation before the check:
+    their clean error words must not hide the failure."""
     import torch
     xfc = build(gpu, 1000, 2, rounding="rtn")
     x = torch.randn(16, 768, device=gpu).to(torch.bfloat16)
@@ -213,7 +212,7 @@ def test_module_reports_a_failed_step_without_synchronising(gpu):
     xfc._err_dev.fill_(2)                                # as if the placement check of a step had failed
     raised = 0
     for _ in range(8):                                   # clean steps behind it, no synchronisation: one of these calls
-        try:                                             # (whichever finds a copy of the word arrived) reports it
+        try:                                             # (whichever finds the host's word changed) reports it
             xfc.xfc_forward_backward(x, labels, [0.05])
         except RuntimeError as e:
             assert "XCD" in str(e)
