@@ -68,8 +68,7 @@ def test_fused_step_at_2m8_labels(gpu):
 
 
 def test_three_kernel_path_at_8m6_labels_and_a_batch_of_256(gpu):
-    """8,600,000 labels in 33 chunks, batch 256 in two halves, true-FP8 arithmetic on the three-kernel path: lr = 0 is
-    the identity, grad_X equals library GEMMs over all chunks, sampled rows equal the oracle after a real step."""
+    """8,600,000 labels in 33 chunks, batch 256, true-FP8 arithmetic on the tiled step (one kernel): lr = 0 is the identity, grad_X equals library GEMMs over all chunks, sampled rows equal the oracle after a real step."""
     import torch
     from elmo_amd import ops
     cfg, nc, rows, chunks, x, labels, x_np, labels_np = make_fp8_workload("cfg5_fp8_8m6", gpu)

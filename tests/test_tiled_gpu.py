@@ -1,4 +1,6 @@
-"""Parity of the three-kernel path (bf16 layer and simulated-FP8 mode, through the C ABI) against the CPU oracle.
+"""Parity of the tiled step (bf16 layer, simulated-FP8 mode, larger batches, through the C ABI) against the CPU oracle.  Plain
+steps run as one kernel (its edges: test_cluster_gpu.py); loss, weight decay and the compensated head as three (their other
+sizes and modes: test_three_kernel_gpu.py).
 
 Tolerances: round-to-nearest weights within 1 grid step (e4m3 step; bf16: one ulp of the operands of the update, see
 check_bf16_weights) of the oracle with all but a small fraction identical (the fp32 accumulators differ by summation order only); the reference's stochastic-rounding recipe
@@ -77,7 +79,7 @@ def test_bf16_layer_rtn_parity(gpu, L, nc, batch, seed):
 @pytest.mark.parametrize("wd,p", [(0.05, 0.0), (0.0, 0.3), (0.02, 0.1)])
 def test_weight_decay_and_fused_dropout_on_the_three_kernel_path(gpu, wd, p):
     """bf16 layer: T = W - lr (bf16(A) + wd W) and dropout of X in the preparation kernel; simulated-FP8 mode: the same
-    with the fp32 gradient.  Against the oracle, whose treatment of both is pinned by closed forms on the CPU."""
+    with the fp32 gradient.  (Dropout without decay runs as one kernel.)  Against the oracle, whose treatment of both is pinned by closed forms on the CPU."""
     import torch
     from elmo_amd import ops
     L, nc, batch, lr, dseed = 3000, 3, 40, 0.5, 0x1357_9BDF_2468
@@ -361,7 +363,7 @@ def test_head_kahan_parity(gpu, ktype, mode, path, shape):
 
 
 def test_true_fp8_on_the_tiled_path_matches_the_fused_oracle(gpu):
-    """quantize_x + saturate turn the three-kernel path into the arithmetic of the fused kernel (no buffer)."""
+    """quantize_x + saturate give the tiled step the arithmetic of the fused kernel (no buffer)."""
     from elmo_amd import ops
     case = H.make_case(2, 1024, 32, 82)
     chunks, x, labels = H.to_device_case(case, gpu)
@@ -375,7 +377,7 @@ def test_true_fp8_on_the_tiled_path_matches_the_fused_oracle(gpu):
 
 
 def test_true_fp8_with_a_batch_of_256(gpu):
-    """Batches above 128 rows run on the three-kernel path in two halves: logits and grad_X per half, grad_W over both."""
+    """Batches above 128 rows run on the tiled step: logits and grad_X per slice of the batch, grad_W over all of them."""
     import torch
     from elmo_amd import ops
     case = H.make_case(2, 1024, 256, 61, pos_mean=4.0, extra_labels=[[255, 2047], [128, 0], [127, 0], [200, 1000], [200, 1000]])
@@ -411,7 +413,7 @@ def test_true_fp8_with_a_batch_of_256(gpu):
 
 
 def test_true_fp8_fast_rounding_on_the_three_kernel_path(gpu):
-    """sr_fast with e4m3 weights: the same random words as the fused kernel (one hash per four weights of a global row),
+    """The tiled step's one-kernel form (the three-kernel form: test_three_kernel_gpu.py).  sr_fast with e4m3 weights: the same random words as the fused kernel (one hash per four weights of a global row),
     so the result equals the oracle's exact stochastic rounding fed with those words, and - with at most 128 batch rows -
     the fused kernel's own output except where the two paths' fp32 sums differ."""
     from elmo_amd import ops
@@ -490,9 +492,9 @@ def test_head_kahan_module(gpu):
 
 
 def test_tiled_step_replays_in_a_captured_graph(gpu):
-    """The three-kernel path launches kernels only (no memset, no allocation, no synchronisation), so a caller may record
-    it into a graph: three replays, with eager work and synchronisations between them, give bit for bit what three eager
-    steps give (bf16 layer, round-to-nearest, ragged chunks, batch in two halves)."""
+    """The tiled step launches kernels only (no memset, no allocation, no synchronisation), so a caller may record it into a
+    graph: three replays, with eager work and synchronisations between them, give bit for bit what three eager steps give
+    (bf16 layer, round-to-nearest, ragged chunks, a batch in four slices)."""
     import torch
     from elmo_amd import ops
     x, w, labels = bf16_case(3000, 200, 36)
@@ -561,8 +563,8 @@ def test_chunked_module_fp32_fp16_branch_with_weight_decay(gpu, dtype):
 
 @pytest.mark.gpu
 def test_true_fp8_arithmetic_at_batch_512(gpu):
-    """The FP8 layer at the batch its shipped 670K configuration uses twice over (512 rows, four halves on the three-kernel
-    path): logits from e4m3(X), saturating cast, round to nearest - against the true-FP8 oracle."""
+    """The FP8 layer at the batch its shipped 670K configuration uses twice over (512 rows, clusters of eight): logits from
+    e4m3(X), saturating cast, round to nearest - against the true-FP8 oracle."""
     from elmo_amd import ops
     case = H.make_case(2, 1024, 512, 64, pos_mean=4.0)
     chunks, x, labels = H.to_device_case(case, gpu)
@@ -576,16 +578,16 @@ def test_true_fp8_arithmetic_at_batch_512(gpu):
 
 
 @pytest.mark.parametrize("L,nc,batch,mode", [
-    (4096, 4, 32, "rtn"),             # four chunks of 1,024 rows in one launch
+    (4096, 4, 32, "rtn"),             # four chunks of 1,024 rows
     (4093, 4, 48, "rtn"),             # the last chunk three rows short
-    (10240, 10, 16, "sr_philox"),     # ten chunks: launches of eight and two; a seed per chunk
-    (2048, 2, 200, "sr_philox"),      # two batch halves
-    (64 * 1200, 2, 16, "rtn"),        # chunks above the row budget of a launch stay one per launch
+    (10240, 10, 16, "sr_philox"),     # ten chunks, a seed per chunk
+    (2048, 2, 200, "sr_philox"),      # clusters of four
+    (64 * 1200, 2, 16, "rtn"),        # large chunks
 ])
 def test_bf16_layer_with_several_chunks_per_launch(gpu, L, nc, batch, mode):
-    """Chunks that are a multiple of 64 rows long and lie one behind the other in memory (the bf16 layer's views) are taken
-    several per launch: same results as the oracle's chunk-by-chunk step - per-chunk seeds and random offsets, the
-    per-chunk bf16 rounding of grad_X."""
+    """Many chunks in one launch: same results as the oracle's chunk-by-chunk step - per-chunk seeds and random offsets, the
+    per-chunk bf16 rounding of grad_X.  (The row counts are those at which the three-kernel form shares launches or not;
+    test_three_kernel_gpu.py runs it at such.)"""
     x, w, labels = bf16_case(L, batch, 300 + nc)
     seeds = [1000 + 7 * c for c in range(nc)] if mode != "rtn" else None
     new, gf, gb = run_bf16(x, w, labels, nc, gpu, mode, seeds)
@@ -602,9 +604,8 @@ def test_bf16_layer_with_several_chunks_per_launch(gpu, L, nc, batch, mode):
 
 @pytest.mark.parametrize("mode,quant", [("sr_philox", False), ("sr_fast", True), ("rtn", False)])
 def test_e4m3_chunks_in_one_allocation_take_one_launch(gpu, mode, quant):
-    """e4m3 chunks that are views of one tensor (1,024 rows each) against the same chunks as separate tensors, which run one
-    per launch: bit-equal weights and grad_X bits (the partial sums keep their order within a chunk; across chunks the
-    fp32 totals are added in the same order)."""
+    """e4m3 chunks that are views of one tensor (1,024 rows each) against the same chunks as separate tensors: bit-equal
+    weights and grad_X bits, wherever the chunks lie in memory."""
     import torch
     from elmo_amd import ops
     nc, rows, batch = 3, 1024, 256 if quant else 64
