@@ -95,8 +95,8 @@ def device_settle(dev, want_ms, nc, rows, num_labels, batch, pos_mean, zipf_s):
 
 
 def bench_tiled(args, cfg):
-    """The secondary modes (bf16 layer, simulated FP8, true FP8 with a batch above 128): three kernels per chunk and
-    batch half; timed as a whole step with HIP events on the torch stream."""
+    """The secondary modes (bf16 layer, simulated FP8, true FP8 with a batch above 128) on the tiled step: one kernel over
+    all chunks with 768 features, three per chunk with 1,024; timed as a whole step with HIP events on the torch stream."""
     import numpy as np
     import torch
     from elmo_amd import ops, synth
@@ -149,6 +149,8 @@ def bench_tiled(args, cfg):
     elapsed = time.perf_counter() - t0
     dev_ms = e0.elapsed_time(e1) / args.steps
     assert bool(torch.isfinite(grad.float()).all())
+    (failed,) = ops.sticky_error_words(tiled_workspace=ws)
+    assert int(failed.item()) == 0, "a step gave up waiting: its time means nothing"
     peak_bytes = torch.cuda.max_memory_allocated() - base_alloc + weight_bytes
     algo_bytes = 2.0 * cfg.num_labels * cfg.dim * wbytes
     algo_flops = 6.0 * cfg.batch * cfg.num_labels * cfg.dim
@@ -161,14 +163,14 @@ def bench_tiled(args, cfg):
         roof = {"bound": "hbm", "achieved": algo_bytes / (dev_ms * 1e-3) / 1e9, "peak": HBM_PEAK_GBS, "unit": "GB/s"}
     roof["frac"] = roof["achieved"] / roof["peak"]
     out = {
-        "metric": "XMC classifier train steps/sec (%s)" % ("bf16 layer" if bf16 else "FP8, three-kernel path" if true_fp8 else "simulated FP8"),
+        "metric": "XMC classifier train steps/sec (%s)" % ("bf16 layer" if bf16 else "FP8, tiled step" if true_fp8 else "simulated FP8"),
         "value": args.steps / elapsed, "unit": "steps/s", "n_gpus": 1, "steps": args.steps, "warmup": args.warmup,
         "ms_per_step": elapsed / args.steps * 1e3, "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
-        "dtype": "bf16 MFMA, fp32 accumulate" + ("" if bf16 else ", e4m3 weights widened on load"), "data": "synthetic",
+        "dtype": "bf16 MFMA, fp32 accumulate" + ("" if bf16 else ", e4m3 weights widened on load" + (" but in the logits (FP8 MFMA)" if true_fp8 else "")), "data": "synthetic",
         "config": {"workload": cfg.name, "labels": cfg.num_labels, "features": cfg.dim, "batch": cfg.batch,
                    "chunks": len(views), "rows_per_chunk": rows, "positives": int(labels.shape[0]), "lr": cfg.lr,
                    "rounding": mode, "seed": cfg.seed},
-        "roofline": dict(roof, traffic=None, kernel="whole step of the tiled path (three kernels per chunk), HIP events",
+        "roofline": dict(roof, traffic=None, kernel="whole tiled step, HIP events",
                          kernel_ms=dev_ms, algorithmic_bytes_per_launch=algo_bytes, algorithmic_flops_per_launch=algo_flops),
         "roofline_step_frac": t_roof / (elapsed / args.steps),
         "peak_hbm_gb": peak_bytes / 1e9, "peak_hbm_over_weights": peak_bytes / weight_bytes,
@@ -401,8 +403,8 @@ def main():
     settle = device_settle(dev, args.settle_ms, nc, rows, cfg.num_labels, cfg.batch, cfg.pos_mean, cfg.zipf_s)
     torch.cuda.reset_peak_memory_stats()
     elapsed = timed_run()
-    err = ops.step_error_word(workspace, nc, rows)
-    assert err == 0, "a workgroup timed out waiting for its partner"
+    (failed,) = ops.sticky_error_words(workspace)      # of every step so far
+    assert int(failed.item()) == 0, "a step gave up waiting: its time means nothing"
     assert bool(torch.isfinite(grad.float()).all())
     kms = kernel_times(events)
     kernel_ms = float(np.mean(kms))
