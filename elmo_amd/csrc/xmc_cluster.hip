@@ -18,10 +18,13 @@
 // cores and the memory system are idle.  Here the four overlap.  The batch slice bounds the registers, not the label
 // rows, so one geometry serves every batch size.
 //
-// What bounds it: bf16 with a small batch the HBM stream (131 K labels, batch 32, round to nearest: 214 us before, 113 now,
-// 3.6 TB/s of weights); the Philox modes the vector units (143 clocks of the SIMD per 64 weights; 501 K labels, batch 128,
-// bf16: 1142 us before, 780 now; 500 K, e4m3: 1086 / 784; 131 K, batch 512: 882 / 600); true FP8 with batch 256 the length
-// of an iteration's dependent phases, about 40 % of whose cycles issue something (8.6 M labels: 11.07 ms before, 10.00 now).
+// What bounds it: bf16 with a small batch the HBM stream (131 K labels, batch 32, round to nearest: 212 us a step in three
+// kernels, 108 now, 74 of them here at 5.4 TB/s of weights).  The Philox modes with batch 128 the issue of vector and matrix
+// instructions, which add up more than they overlap: the words alone are 145 clocks of a SIMD per 64 weights, 0.35-0.37 ms
+// of the step (501 K labels, bf16: 1142 us in three kernels, 780 now, 548 with sr_fast; 500 K, e4m3: 1086 / 779, 447 to
+// nearest).  Clusters of four and eight the length of an iteration's dependent phases - three barriers, the exchange, a full
+// drain of the loads - about 40 % of whose cycles issue something (true FP8, batch 256, 8.6 M labels: 11.07 ms before, 10.0
+// now; bf16, batch 512, 131 K: 882 us before, 592 now, 506 of them left without Philox).
 #include "xmc_common.h"
 
 namespace xmc {
@@ -358,16 +361,22 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
   unsigned wold[C > 1 ? G::NBLK : 1][C > 1 ? RB : 1][WDW];   // clusters of several: the weights the lagging update starts from
 
   // ---- The words of the Philox recipe, the larger part of the update's vector work, depend on nothing but the element's
-  //      place: up to three blocks' words per half of the update are computed between the matrix instructions of the logits
-  //      (first half) and of grad_X (second half), whose operand reads and pipeline leave the vector units idle.  Only where
-  //      the words' registers do not make the loop spill.  With the falling priorities: 501 K labels, bf16, batch 128 812 us
-  //      without, 780 with; 500 K, e4m3 824 / 784.
+  //      place: up to three blocks' words per half of the update can be computed between the matrix instructions of the
+  //      logits (first half, EARLY) and of grad_X (second half, EARLY2).  Their place is worth little (a matrix instruction
+  //      hides only two vector instructions); what the long stretches of vector work need is the falling priority below.
+  //      us a step, us a step without early words / without the priorities / without either:
+  //        bf16, 501 K labels, batch 128 (C = 2)  781, 780 / 1001 / 808     bf16, 131 K, batch 32 (C = 1)  168, 170 / 173 / 174
+  //        e4m3, 500 K, batch 128 (C = 2)         779, 786 / 812 / 820      bf16, 131 K, batch 512 (C = 8) 592 all ways
+  //      So the words are early where their registers do not make the loop spill.  Where they do (131 K labels): EARLY with
+  //      e4m3 at C = 4 +5 %, with FP8 logits at C = 2 +3 % (C = 4: -1, C = 8: -2), at C = 8 with bf16 products 3 to 30 times the
+  //      time (one block, taken by some wavefronts only: the branches fill the registers); EARLY2 with bf16 at C = 2 +6 %.
   constexpr bool EARLY = MODE == ROUND_SR_PHILOX && !QX && (C == 2 || (C == 1 && (WT == CLU_BF16 || NBK == 2))), EARLY2 = EARLY && (NBK == 2 || (WT == CLU_E4M3 && C == 2));
   constexpr int NBE = G::NBLK < 3 ? G::NBLK : 3, EP = 8 * NBE;   // blocks; pieces (half an evaluation each)
   constexpr int RWN = WT == CLU_BF16 ? 2 : 4;                    // registers of four words (bf16 weights take 16 bits of each)
   unsigned rw[C == 1 ? 2 : 1][EARLY ? NBE : 1][RWN];
   // In long stretches of vector work the priority falls with the progress, so that the wavefront of a SIMD that is behind
   // goes first: otherwise the older one finishes early and waits, and one wavefront alone issues at half the rate of two.
+  // Measured with the early words above; FP8 logits, 670 K labels, batch 256, sr_fast 833 us with, 844 without.
   auto priority = [](int level) {
     if (level == 3) __builtin_amdgcn_s_setprio(3);
     else if (level == 2) __builtin_amdgcn_s_setprio(2);
@@ -712,9 +721,18 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __syncthreads();   // own G of tile i is visible
     // ---- Two jobs are left: grad_X of tile i (matrix instructions) and (the second half of) grad_W and update of this tile
-    //      (cluster of one) or of the one before (vector instructions).  The two wavefronts of a SIMD take them in opposite
-    //      order, so that each runs in the gaps of the other - except with the Philox recipe, where the vector work is several
-    //      times the matrix work and keeping in step measured 2-6 % faster.
+    //      (cluster of one) or of the one before (vector instructions).  The two wavefronts of a SIMD can take them in opposite
+    //      order, each in the gaps of the other, or in step.  Measured in step against opposite, us a step, 131 K labels,
+    //      batches of 32 / 64 / 128 / 256 / 512:
+    //        Philox   bf16  184/188 183/185 230/239 347/374 604/633   e4m3 159/161 180/179 235/243 364/372 610/626
+    //                 FP8 logits  -  -  213/218 337/336 536/556
+    //        sr_fast  bf16  92/93 103/106 152/158 269/289 516/535     FP8 logits  -  -  125/128 226/231 443/461
+    //        nearest  bf16  79/79 94/93 143/147 258/278 508/519       e4m3 62/64 82/81 142/145 274/276 503/518
+    //                 FP8 logits  -  -  119/120 218/223 435/452
+    //      and over larger label spaces, where the clock falls: bf16, 501 K, batch 128, sr_fast 553/548; e4m3, 500 K, nearest
+    //      447/447; FP8 logits, 670 K, batch 256, sr_fast 830/833.  In step is the faster order with Philox at every size; without
+    //      it the two are within 1 % of each other at the large sizes the line was drawn at, and in step is up to 7 % faster at
+    //      the small ones.
     constexpr bool OPPOSITE = MODE != ROUND_SR_PHILOX;
     auto update_part = [&] {
       if constexpr (C == 1) {
@@ -816,6 +834,10 @@ ClusterVariant cluster_variant_fp8(int c, int nbk, int round_mode);
 void cluster_set_lds_bf16();
 void cluster_set_lds_sim();
 void cluster_set_lds_fp8();
+
+// Registers spilled, as the compiler reports them: none but with e4m3 weights, FP8 logits, c = 4, Philox (24, 36 bytes of scratch
+// a lane) and with bf16 weights, c = 4, nearest and sr_fast (6, 12 bytes).  A scratch access inside the tile loop makes the waits
+// counted by hand stricter, never laxer: it is younger than the loads they wait for.
 
 #ifdef CLU_VARIANT   // a translation unit of variants: CLU_VARIANT(function suffix) with CLU_WT, CLU_QX
 #define CLU_PICK(C, NBK)                                                                                                         \

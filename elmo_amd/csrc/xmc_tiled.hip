@@ -1,12 +1,12 @@
-// Three-kernel ("tiled") classifier step for gfx950, for the two modes of the reference that keep bf16 temporaries:
+// Three-kernel form of the tiled classifier step for gfx950.  It takes what the one-pass form (xmc_cluster.hip) does not: 1,024
+// features, a loss, weight decay, a compensated head.  For the two modes of the reference that keep bf16 temporaries:
 //   * bf16 weights          src/xmc_classifiers/chunked.py:85-131 with src/triton_kernels/stochastic_rounding_kernel.py:65-99
 //   * simulated FP8 weights src/xmc_classifiers/chunked_fp8xmc_clf.py:98-99,110,115-116 with
 //                           src/triton_kernels/fuse_kernel.py:134-199
 // Per chunk, as the reference does: logits -> G (sigmoid minus targets, bf16, kept in HBM in both orientations),
 // grad_X partial (split over label ranges, summed in a fixed order), grad_W + SGD update in place.  All three GEMMs
-// are bf16 v_mfma_f32_16x16x32_bf16 with fp32 accumulation; e4m3 weights are widened exactly on load.  These modes are
-// not the headline path: the kernels take their operands straight from global memory (L2) in MFMA operand order and
-// stage only the one operand that needs a transposition (W in grad_X) through LDS.
+// are bf16 v_mfma_f32_16x16x32_bf16 with fp32 accumulation (the logits of true FP8 with more than 128 batch rows: FP8);
+// e4m3 weights are widened exactly on load.
 #include "xmc_common.h"
 #include <type_traits>
 

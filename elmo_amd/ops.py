@@ -338,14 +338,15 @@ def tiled_step(chunk_views, rows_per_chunk, weight_type, x, labels, lr, seeds=No
     the simulated one; `kahan` ([num_head, d] bf16 or float8_e5m2, updated in place) turns on the head-Kahan update of
     the first num_head rows of chunk 0 (chunked_head_kahan_fp8xmc_clf.py:127-131).  `loss_out` (a float32 device tensor
     with one element) receives the summed binary cross entropy of the step's logits (what chunked.py:57-72 is written
-    to compute).  weight_decay, dropout_p, dropout_seed: as in fp8_step.
+    to compute); the three-kernel form it takes sums in another order than the one-kernel form, so some weights round
+    differently than without it.  weight_decay, dropout_p, dropout_seed: as in fp8_step.
     The one-kernel form can fail, as the fused step can (xmc_tiled_error_offset), and does not raise: its error words are in
     `workspace`, also where that is too small for the batch and the step runs in a temporary one.  Without a workspace
     the next call without one, or check_steps, raises."""
     lib = _lib.load()
     assert x.is_cuda and x.dtype == torch.bfloat16 and x.is_contiguous() and x.dim() == 2
     feats = x.shape[1]
-    assert feats in TILED_FEATURES, "the three-kernel path is built for 768 and 1024 input features"
+    assert feats in TILED_FEATURES, "the tiled step is built for 768 and 1024 input features"
     ktype = 0
     if kahan is not None:
         assert weight_type == "e4m3" and kahan.is_cuda and kahan.is_contiguous() and kahan.shape == (num_head, feats)
@@ -396,7 +397,7 @@ def tiled_step(chunk_views, rows_per_chunk, weight_type, x, labels, lr, seeds=No
 
 
 def debug_spin_limit(limit):
-    """Test aid: polls of a partner's counter before a workgroup of the fused step gives up (negative: the default);
+    """Test aid: polls of a partner's counter before a workgroup of the fused or the tiled step gives up (negative: the default);
     returns the previous value."""
     return int(_lib.load().xmc_debug_spin_limit(int(limit)))
 

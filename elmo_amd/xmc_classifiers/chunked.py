@@ -18,7 +18,7 @@ here operation by operation, on the GPU, for any batch size; momentum stays unus
 
 Optional, not in the reference: training.xmc.rounding = "sr_philox" (default: the reference's Philox recipe) | "rtn" |
 "sr_fast" (the hardware's stochastic conversion to bf16 with a counter hash: unbiased, not the reference's random stream,
-and not bound by the 48 vector instructions per weight of the Philox recipe).
+and not bound by the Philox recipe, 17 wide products and 16 exclusive ors per weight).
 """
 import torch
 from torch import nn
@@ -116,7 +116,9 @@ class XMCBCECHUNKEDLayer(nn.Module):
             skip_loss: Whether to skip the loss calculation.  When False the summed binary cross entropy of the step's
                        logits is computed inside the logits kernel and returned (one host synchronisation).  This is
                        the value the reference's _compute_loss is written to return (chunked.py:57-72); the reference
-                       itself passes the weight chunk where the logits belong (chunked.py:109).
+                       itself passes the weight chunk where the logits belong (chunked.py:109).  Such a step runs as three
+                       kernels per chunk: 1.4 to 2.5 times as long, and because its sums are taken in another order some
+                       weights (up to 15 in a million, measured) round differently than with skip_loss=True.
         '''
         assert embed.is_cuda and embed.dim() == 2 and embed.shape[1] == self.features
         assert labels.is_cuda and labels.dim() == 2 and labels.shape[1] == 2

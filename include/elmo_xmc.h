@@ -187,8 +187,8 @@ int xmc_fp8_forward_topk_fused_rows(void* const* chunk_ptrs, int num_chunks, int
 int xmc_dropout_quantize(const void* x, int x_type, int rows, int cols, float p, unsigned long long seed, void* out_e4m3,
                          void* stream);
 
-/* Test aid (no counterpart in the reference): sets how often a workgroup of the fused step polls a partner's counter
- * before it gives up (see xmc_fp8_step), for all later calls of the process, and returns the previous value; a negative
+/* Test aid (no counterpart in the reference): sets how often a workgroup of the fused or the tiled step polls a partner's
+ * counter before it gives up (see xmc_fp8_step), for all later calls of the process, and returns the previous value; a negative
  * `limit` restores the default (2^18 polls).  With a limit of 0 every wait that is not satisfied at once expires: the
  * step then ends early with bit 0 of its error word set, every kernel still exits normally, and the tiles it did not
  * reach keep their old weights.  The tests use it to exercise the give-up path. */
@@ -205,13 +205,21 @@ enum {
   XMC_WEIGHT_BF16 = 1       /* bf16 layer (chunked.py:85-131) */
 };
 
-/* Bytes of workspace xmc_tiled_step needs for batches of up to max_batch rows (1..512). */
+/* Bytes of workspace xmc_tiled_step needs for batches of up to max_batch rows (1..512): the larger of what its two forms
+ * take, so that any option may be used with it.  One kernel: 5 MB, and 192 KiB of grad_X partials for each of its up to 256
+ * workgroups and for each workgroup of a cluster and chunk (500 K labels in eight chunks, batch 128: 59 MB).  Three kernels:
+ * 512 bytes of G per label row of a launch and 128 batch rows (two orientations), and 25 MB of partials per 128 batch rows
+ * (670 K labels in two chunks, batch 256: 395 MB). */
 size_t xmc_tiled_workspace_bytes(int num_chunks, int rows_per_chunk, int max_batch);
 /* The same for a layer of `features` inputs (768 or 1024; the function above is this one at 768).  0 for any other
  * width. */
 size_t xmc_tiled_workspace_bytes_ex(int num_chunks, int rows_per_chunk, int max_batch, int features);
 
-/* One training step of the modes in which the reference keeps bf16 temporaries, three kernels per chunk as there:
+/* One training step of the modes in which the reference keeps bf16 temporaries: one persistent kernel over all chunks where
+ * 768 features meet no compensated head, no loss and no weight decay (it can fail as xmc_fp8_step can: see
+ * xmc_tiled_error_offset), three kernels per chunk otherwise.  The two forms take their fp32 sums in different orders: a step
+ * with loss_out rounds some weights differently from the same step without (up to 15 in a million, measured) and takes
+ * 1.4 to 2.5 times as long.
  *   XMC_WEIGHT_BF16  XMCBCECHUNKEDLayer.xfc_forward_backward (chunked.py:76-133) with sgd_update
  *                    (stochastic_rounding_kernel.py:91-99): bf16 logits, grad_X partial rounded to bf16 per chunk,
  *                    grad_W rounded to bf16, W = SR16(W - lr*A) (XMC_ROUND_SR_PHILOX) or bf16(W - lr*A) (XMC_ROUND_RTN)
