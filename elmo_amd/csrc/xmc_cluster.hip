@@ -21,10 +21,9 @@
 // What bounds it: bf16 with a small batch the HBM stream (131 K labels, batch 32, round to nearest: 212 us a step in three
 // kernels, 108 now, 74 of them here at 5.4 TB/s of weights).  The Philox modes with batch 128 the issue of vector and matrix
 // instructions, which add up more than they overlap: the words alone are 145 clocks of a SIMD per 64 weights, 0.35-0.37 ms
-// of the step (501 K labels, bf16: 1142 us in three kernels, 780 now, 548 with sr_fast; 500 K, e4m3: 1086 / 779, 447 to
-// nearest).  Clusters of four and eight the length of an iteration's dependent phases - three barriers, the exchange, a full
-// drain of the loads - about 40 % of whose cycles issue something (true FP8, batch 256, 8.6 M labels: 11.07 ms before, 10.0
-// now; bf16, batch 512, 131 K: 882 us before, 592 now, 506 of them left without Philox).
+// of the step (501 K labels, bf16: 1142 us in three kernels, 765 now, 510 with sr_fast; 500 K, e4m3: 1086 / 750, 380 to
+// nearest).  The others the issue of vector, scalar and matrix instructions by two wavefronts per SIMD, and with bf16 weights
+// the memory path beside it (48 KiB of a tile through every member's; without loads and stores 430 of the 510 us).
 #include "xmc_common.h"
 
 namespace xmc {
@@ -77,24 +76,30 @@ template <int WT, int QX, int C, int NBK> struct CluGeom {
   static constexpr int ONC = ORS / 16;
   static constexpr int OSW = (ONC & -ONC) < 16 ? (ONC & -ONC) - 1 : 15;   // chunk swizzle of that image
   static constexpr int NBLK = C == 1 ? 6 : C == 2 ? 3 : C == 4 ? 2 : 1;   // feature blocks whose X^T operand a wavefront keeps
+  static constexpr int NIMG = C > 1 && WT == CLU_E4M3 && T == 32 ? 3 : 2;   // tiles in LDS
   static constexpr int L_W = 0;
   static constexpr int NOWN = C > 1 ? 2 : 1;
-  static constexpr int L_OWN = L_W + 2 * IMG;                  // own G of this tile (and of the one before: it is updated one tile behind)
+  static constexpr int L_OWN = L_W + NIMG * IMG;               // own G of this tile (and of the one before: it is updated one tile behind)
   static constexpr int L_PART = L_OWN + NOWN * GSL;            // the partners' G of one tile
   static constexpr int L_OUT = L_PART + (C - 1) * GSL;         // updated weights
   static constexpr int L_PS = L_OUT + OIMG;                    // partial logits (the K range is split between two wavefronts)
   static constexpr int L_MISC = L_PS + (QX ? 0 : 8192);        // see below
-  static constexpr int LDS = L_MISC + 64 + 256;                // abort word; at + 16 the range of positives of two tiles; at + 64 a
-                                                               // copy of the cluster's counters
+  static constexpr int LDS = L_MISC + 64;                      // abort word; at + 16 the range of positives of two tiles
   static constexpr int WPIECES = T * WB / 8;                   // direct-to-LDS loads of a wavefront per tile: 768 bytes each
   static constexpr int GPIECES = (C - 1) * GSL / 1024;         // ... of all wavefronts for the partners' G
-  static constexpr int OPIECES = OIMG / 1024;                  // wave-wide stores of updated weights
+  // stores of updated weights by clusters of several: 48 lanes x 16 bytes each, one row segment or several
+  static constexpr int RPI = 48 / ONC;                         // rows of a store
+  static constexpr int OPIECES = OIMG / 768, OPW = OPIECES / 8;   // stores of all wavefronts, of one
   static constexpr int PSLOT = NBK * 6 * 8 * 64;               // floatx4 values of a member's grad_X sum
   static_assert(LDS <= 160 * 1024, "LDS budget");
 };
 
 typedef __attribute__((address_space(3))) unsigned char clds_u8;
 template <int N> struct CluInt { static constexpr int value = N; };
+template <int A, int B, class F> __device__ __forceinline__ void clu_static_for(F&& f) {
+  if constexpr (A < B) { f(CluInt<A>{}); clu_static_for<A + 1, B>(f); }
+}
+constexpr int CLU_MID = 3072;   // loads of a wavefront reach from 3 KiB before to 3 KiB behind their base
 typedef unsigned cux2 __attribute__((ext_vector_type(2)));
 typedef short cshortx4 __attribute__((ext_vector_type(4)));
 typedef short cshortx8 __attribute__((ext_vector_type(8)));
@@ -109,14 +114,23 @@ __host__ __device__ constexpr int clu_slot(int r) { return (r & ~12) | ((r & 4) 
 // chunk swizzle of the 64-byte rows of G (four chunks; q = row / 4 % 4) for the same reads
 __device__ __forceinline__ int clu_gswz(int q) { return -q & 3; }
 
+// The memory instructions below are written out so that the waits can be counted by hand.  Their wait states: an SGPR written by
+// a vector instruction (v_readlane of a spilled scalar) may not be the address of a memory instruction within the next five, and
+// the compiler, which keeps that distance elsewhere, does not look into inline assembly.
 __device__ __forceinline__ void clu_lds_load16(const unsigned char* base, unsigned off, unsigned ldsoff_) {
   const unsigned ldsoff = __builtin_amdgcn_readfirstlane(ldsoff_);
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(ldsoff), "v"(off), "s"(base) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(ldsoff), "v"(off), "s"(base) : "memory", "m0");
+}
+// A load of 48 lanes, 16 bytes each, at base + off + MEM to LDS at l0 + AT + MEM + 16 lane (the immediate offset counts on both
+// sides).  All lanes are active in front of it.
+template <int AT, int MEM> __device__ __forceinline__ void clu_lds_load48(const unsigned char* base, unsigned off, unsigned l0) {
+  asm volatile("s_add_u32 m0, %0, %3\n\ts_bfm_b64 exec, 48, 0\n\ts_nop 2\n\tglobal_load_lds_dwordx4 %1, %2 offset:%4\n\ts_mov_b64 exec, -1"
+               : : "s"(l0), "v"(off), "s"(base), "n"(AT), "n"(MEM) : "memory", "m0", "scc");
 }
 // at device scope: never served by this compute unit's L1, which may hold an exchange slot's previous contents
 __device__ __forceinline__ void clu_lds_load16_l2(const unsigned char* base, unsigned off, unsigned ldsoff_) {
   const unsigned ldsoff = __builtin_amdgcn_readfirstlane(ldsoff_);
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2 sc1" : : "s"(ldsoff), "v"(off), "s"(base) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, %2 sc1" : : "s"(ldsoff), "v"(off), "s"(base) : "memory", "m0");
 }
 
 // 4 bytes per lane at device scope into LDS at ldsoff + 4 * lane
@@ -226,7 +240,6 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
     p.xcc[g] = (int)(__builtin_amdgcn_s_getreg((3 << 11) | 20) & 15);   // XCC_ID
     *(__attribute__((address_space(3))) int*)(lds + G::L_MISC) = 0;
   }
-  if (C > 1 && tid < 64) *(__attribute__((address_space(3))) int*)(lds + G::L_MISC + 64 + 4 * tid) = 0;
   const int v0 = (int)((long long)j * p.ntiles / p.nclusters), v1 = (int)((long long)(j + 1) * p.ntiles / p.nclusters);
   const int n_it = v1 - v0;
 
@@ -267,23 +280,41 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
     return q;
   };
 
+  // the lane number; `opaque` makes a new value of it, so that what is computed from it is computed where it is used instead of
+  // being kept in registers over the loop
+  int lid = clu_lane();
   // ---- loads of a tile: 48 lanes x 16 bytes = a row of e4m3 or half a row of bf16 weights each, so that no lane computes an
   //      address (a reload of an offset from scratch memory would make the compiler wait for every load issued before)
-  auto load_pieces = [&](const CluTile& q, int slot, int s0, int s1) {
-    const int ln = clu_lane();
-    // (the range of positives travels with the tile: as a scalar load it would make the next wait for an LDS read wait for it)
-    if (s0 == 0 && v == 7 && ln < 2) clu_lds_load4_l2(ctptr + (q.c * tpc64 + (q.row0 >> 6)) + ln, (unsigned)(G::L_MISC + 16 + slot * 8));
+  auto load_pieces = [&](const CluTile& q, unsigned wimg, int s0, int s1) {
+    const int ln = lid;
     if (ln < 48) {
 #pragma unroll
       for (int s = s0; s < s1; s++) {
         const int row = v * (T / 8) + s / G::WB, src = min(row, q.rows_valid - 1);   // rows past the end re-read the last valid one
-        clu_lds_load16(q.base + src * RS + (s % G::WB) * 768, (unsigned)ln * 16u, (unsigned)(G::L_W + slot * G::IMG + clu_slot(row) * G::LS + (s % G::WB) * 768));
+        clu_lds_load16(q.base + src * RS + (s % G::WB) * 768, (unsigned)ln * 16u, wimg + (unsigned)(G::L_W + clu_slot(row) * G::LS + (s % G::WB) * 768));
       }
     }
   };
-  auto load_tile = [&](const CluTile& q, int slot) { load_pieces(q, slot, 0, G::WPIECES); };
+  // the range of positives of a tile (as a scalar load it would make the next wait for an LDS read wait for it)
+  auto load_range = [&](const CluTile& q, int slot) {
+    const int ln = lid;
+    if (v == 7 && ln < 2) clu_lds_load4_l2(ctptr + (q.c * tpc64 + (q.row0 >> 6)) + ln, (unsigned)(G::L_MISC + 16 + slot * 8));
+  };
+  // the same for a full tile, pieces S0 .. S1-1: the rows of a wavefront lie a fixed distance apart in memory and in LDS, so
+  // that a load is one scalar addition (M0) and an immediate offset from the middle of its rows
+  const int wrow = v * (T / 8) * RS + CLU_MID;
+  auto load_full = [&](const CluTile& q, unsigned wimg, auto s0_c, auto s1_c) {
+    constexpr int S0 = decltype(s0_c)::value, S1 = decltype(s1_c)::value;
+    const unsigned char* base = q.base + wrow;
+    const unsigned off = (unsigned)lid * 16u, l0 = wimg + (unsigned)(G::L_W + clu_slot(v * (T / 8)) * G::LS);
+    clu_static_for<S0, S1>([&](auto s_c) {
+      constexpr int sv = decltype(s_c)::value, r = sv / G::WB, mem = r * RS + (sv % G::WB) * 768 - CLU_MID, at = clu_slot(r) * G::LS + (sv % G::WB) * 768 - mem;
+      clu_lds_load48<at, mem>(base, off, l0);
+    });
+  };
   CluTile cur = next_tile(), prev = cur, prev2 = cur, nxt = cur;
-  if (n_it > 0) load_tile(cur, 0);
+  load_range(cur, 0);
+  load_pieces(cur, 0u, 0, G::WPIECES);
 
   // ---- resident operands
   // Logits: with FP8 products wavefront v takes batch block v % 4 and half of the tile's row blocks; with bf16 products the
@@ -347,7 +378,6 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
     const unsigned ga = (unsigned)(l16 * 64 + (kg ^ clu_gswz(l16 >> 2)) * 16);
     pk_o = wold | (ga << 16);
   }
-  auto exch_slot = [&](int qm, int t) { return exq + (unsigned)((qm * CLU_SLOTS + (t & (CLU_SLOTS - 1))) * G::GSL); };
 
   auto read_old = [&](unsigned wimg, int k, int rb, unsigned (&wr)[WDW]) {
     const unsigned at = (pk_o & 0xFFFFu) + (wimg + (unsigned)(rb * 16 * LS + (m * G::FBN + block_of(k)) * 16 * G::WB));
@@ -361,22 +391,21 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
   unsigned wold[C > 1 ? G::NBLK : 1][C > 1 ? RB : 1][WDW];   // clusters of several: the weights the lagging update starts from
 
   // ---- The words of the Philox recipe, the larger part of the update's vector work, depend on nothing but the element's
-  //      place: up to three blocks' words per half of the update can be computed between the matrix instructions of the
-  //      logits (first half, EARLY) and of grad_X (second half, EARLY2).  Their place is worth little (a matrix instruction
-  //      hides only two vector instructions); what the long stretches of vector work need is the falling priority below.
+  //      place: up to three blocks' words can be computed between the matrix instructions of the logits (the first half of the
+  //      update, EARLY) and of grad_X (the second half, EARLY2).  Their place is worth little (a matrix instruction hides only two
+  //      vector instructions); what the long stretches of vector work need is the falling priority below.
   //      us a step, us a step without early words / without the priorities / without either:
-  //        bf16, 501 K labels, batch 128 (C = 2)  781, 780 / 1001 / 808     bf16, 131 K, batch 32 (C = 1)  168, 170 / 173 / 174
-  //        e4m3, 500 K, batch 128 (C = 2)         779, 786 / 812 / 820      bf16, 131 K, batch 512 (C = 8) 592 all ways
-  //      So the words are early where their registers do not make the loop spill.  Where they do (131 K labels): EARLY with
-  //      e4m3 at C = 4 +5 %, with FP8 logits at C = 2 +3 % (C = 4: -1, C = 8: -2), at C = 8 with bf16 products 3 to 30 times the
-  //      time (one block, taken by some wavefronts only: the branches fill the registers); EARLY2 with bf16 at C = 2 +6 %.
-  constexpr bool EARLY = MODE == ROUND_SR_PHILOX && !QX && (C == 2 || (C == 1 && (WT == CLU_BF16 || NBK == 2))), EARLY2 = EARLY && (NBK == 2 || (WT == CLU_E4M3 && C == 2));
+  //        bf16, 501 K labels, batch 128 (C = 2)  766, 779 / 784 / 788     bf16, 501 K, batch 32 (C = 1)  639, 641 / 662 / 661
+  //        e4m3, 500 K, batch 128 (C = 2)         755, 768 / 892 / 781     bf16, 501 K, batch 64 (C = 1)  680, 680 / 693 / 689
+  //      So the words are early where their registers do not make the loop spill (batch 32: both halves).  The words of one
+  //      wavefront of a SIMD beside the other's matrix instructions, in opposite order, are slower: 815 instead of 775 (C = 2).
+  constexpr bool EARLY = MODE == ROUND_SR_PHILOX && !QX && (C == 2 || (C == 1 && (WT == CLU_BF16 || NBK == 2))), EARLY2 = EARLY && NBK == 2;
   constexpr int NBE = G::NBLK < 3 ? G::NBLK : 3, EP = 8 * NBE;   // blocks; pieces (half an evaluation each)
   constexpr int RWN = WT == CLU_BF16 ? 2 : 4;                    // registers of four words (bf16 weights take 16 bits of each)
   unsigned rw[C == 1 ? 2 : 1][EARLY ? NBE : 1][RWN];
   // In long stretches of vector work the priority falls with the progress, so that the wavefront of a SIMD that is behind
   // goes first: otherwise the older one finishes early and waits, and one wavefront alone issues at half the rate of two.
-  // Measured with the early words above; FP8 logits, 670 K labels, batch 256, sr_fast 833 us with, 844 without.
+  // Measured with the early words above; FP8 logits, 670 K labels, batch 256, sr_fast 764 us with, 774 without.
   auto priority = [](int level) {
     if (level == 3) __builtin_amdgcn_s_setprio(3);
     else if (level == 2) __builtin_amdgcn_s_setprio(2);
@@ -384,7 +413,7 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
     else __builtin_amdgcn_s_setprio(0);
   };
   PhiloxState ps;
-  auto element_lanes = [&] { const int ln = clu_lane(); return (unsigned)((ln & 15) * D + 4 * (ln >> 4)); };   // a lane's part of the place
+  auto element_lanes = [&] { const int ln = lid; return (unsigned)((ln & 15) * D + 4 * (ln >> 4)); };   // a lane's part of the place
   auto words = [&](const CluTile& q, auto half_c, unsigned lanes, int p0, int p1) {
     constexpr int half = decltype(half_c)::value, n = half * (RB / 2);
     if constexpr (half == 0 ? EARLY : EARLY2) {
@@ -409,19 +438,19 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
   };
 
   // A^T and update of the tile q whose G is complete in LDS (own part at gown), the result to the image of updated weights
-  // (row blocks n0 .. n1-1 in this wavefront's order; `between` runs once, in the middle of the last one's vector work)
-  auto update_tile = [&](const CluTile& q, unsigned gown, unsigned wimg, auto n0_c, auto n1_c, auto&& between) {
-    constexpr int n0 = decltype(n0_c)::value, n1 = decltype(n1_c)::value;
+  auto update_tile = [&](const CluTile& q, unsigned gown, unsigned wimg) {
     const unsigned seed = q.seed;
     const unsigned grow0 = label0 + (unsigned)q.c * (unsigned)rpc + (unsigned)q.row0;
 #pragma unroll
-    for (int n = n0; n < n1; n++) {
+    for (int n = 0; n < RB; n++) {
       const int rb = row_block(n);
       if (C <= 4 || takes(0, n)) {
-        const int ln = clu_lane(), l16 = ln & 15, kg = ln >> 4;
+        const int ln = lid, l16 = ln & 15, kg = ln >> 4;
         const unsigned g_lane = ((pk_g & 0xFFFFu) ^ (unsigned)((rb & 1) * 32)) + (unsigned)((rb >> 1) * G::SL * 64);
-        // G operands one K step ahead of their products
-        bf16x8 bg[2];
+        // G operands GD - 1 K steps ahead of their products: as far as the registers go (a spilled register in this loop costs more
+        // than the depth gives: FP8 logits, c = 4, depth 3 spills five and takes 817 instead of 764 us at 670 K labels, batch 256)
+        constexpr int GD = C == 8 ? 4 : (C == 4 && !QX) || (C == 2 && MODE != ROUND_SR_PHILOX) ? 3 : 2;
+        bf16x8 bg[GD];
         auto rdg = [&](int ks) {
           const int d = ks * 32 / G::SL, kk = ks - d * (G::SL / 32);   // slice: own, next member's, ...; K step within it
           const unsigned a0 = g_lane + (d == 0 ? gown : (unsigned)(G::L_PART + (d - 1) * G::GSL));
@@ -430,13 +459,14 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
           return __builtin_bit_cast(bf16x8, cshortx8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]});
         };
         floatx4 aa[G::NBLK];
-        bg[0] = rdg(0);
+#pragma unroll
+        for (int ks = 0; ks < GD - 1 && ks < KS; ks++) bg[ks] = rdg(ks);
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) {
-          if (ks + 1 < KS) bg[(ks + 1) & 1] = rdg(ks + 1);
+          if (ks + GD - 1 < KS) bg[(ks + GD - 1) % GD] = rdg(ks + GD - 1);
 #pragma unroll
           for (int k = 0; k < G::NBLK; k++)
-            if (takes(k, n)) aa[k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xt[k][ks], bg[ks & 1], ks == 0 ? floatx4{0.f, 0.f, 0.f, 0.f} : aa[k], 0, 0, 0);
+            if (takes(k, n)) aa[k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xt[k][ks], bg[ks % GD], ks == 0 ? floatx4{0.f, 0.f, 0.f, 0.f} : aa[k], 0, 0, 0);
           CFENCE();
         }
         const unsigned row = (unsigned)(16 * rb + l16);
@@ -465,32 +495,40 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
             *(__attribute__((address_space(3))) unsigned*)(lds + G::L_OUT + row * G::ORS + (unsigned)((lb ^ (l16 & G::OSW)) * 16 + 4 * kg)) = wo[0];
           }
           CFENCE();
-          if (n == n1 - 1 && k == 0) between();
         }
       }
     }
   };
-  // the image of updated weights to memory, as whole 16-byte pieces of row segments; a full tile takes the same number of
-  // stores in every wavefront up to one (counted below), a partial one may take fewer
+  // the image of updated weights to memory; a full tile takes OPW stores (or one more) of every wavefront, a partial one may
+  // take fewer
   auto store_out = [&](const CluTile& q) {
-    int ln = clu_lane();
+    int ln = lid;
     COPAQUE(ln);
-    auto piece = [&](int pc, bool all) {
-      const int ch = pc * 64 + ln, row = ch / G::ONC, c = ch - row * G::ONC;
-      const intx4 ov = *(const __attribute__((address_space(3))) intx4*)(lds + G::L_OUT + row * G::ORS + ((c ^ (row & 15 & G::OSW)) * 16));
-      if (all || row < q.rows_valid) *(intx4*)(q.base + (unsigned)(row * RS + m * G::ORS + c * 16)) = ov;
-    };
-    if (q.rows_valid == T) {
+    if constexpr (C == 1) {   // whole rows: 1 KiB pieces of the image, 64 lanes x 16 bytes
 #pragma unroll
-      for (int s = 0; s < (G::OPIECES + 7) / 8; s++)
-        if (v + 8 * s < G::OPIECES) piece(v + 8 * s, true);
-    } else {
-      for (int s = v; s < G::OPIECES; s += 8) piece(s, false);
+      for (int s = 0; s < G::OIMG / 8192; s++) {
+        const int ch = (v + 8 * s) * 64 + ln, row = ch / G::ONC, c = ch - row * G::ONC;
+        const intx4 ov = *(const __attribute__((address_space(3))) intx4*)(lds + G::L_OUT + row * G::ORS + ((c ^ (row & 15 & G::OSW)) * 16));
+        if (q.rows_valid == T || row < q.rows_valid) *(intx4*)(q.base + (unsigned)(row * RS + c * 16)) = ov;
+      }
+    } else {   // 768 bytes of one or several row segments, 48 lanes x 16 bytes, whose places differ by constants between the stores
+      const int lr = G::ONC == 48 ? 0 : ln / G::ONC, lc = ln - lr * G::ONC;
+      if (ln < 48) {
+#pragma unroll
+        for (int s = 0; s < (G::OPIECES + 7) / 8; s++)
+          if (G::OPIECES % 8 == 0 || v + 8 * s < G::OPIECES) {
+            const int row = (v + 8 * s) * G::RPI + lr, sw = G::RPI > 1 ? (v * G::RPI + lr) & G::OSW : row & G::OSW;
+            if (row < q.rows_valid) {
+              const intx4 ov = *(const __attribute__((address_space(3))) intx4*)(lds + G::L_OUT + row * G::ORS + ((lc ^ sw) * 16));
+              *(intx4*)(q.base + (unsigned)(row * RS + m * G::ORS + lc * 16)) = ov;
+            }
+          }
+      }
     }
   };
   auto store_acc = [&](int slot) {
     unsigned char* dst = (unsigned char*)(p.partial + (size_t)(slot * C + m) * G::PSLOT + v * 64);   // (wave-uniform)
-    unsigned off = (unsigned)clu_lane() * 16u;
+    unsigned off = (unsigned)lid * 16u;
     COPAQUE(off);
 #pragma unroll
     for (int mb = 0; mb < NBK; mb++)
@@ -507,12 +545,11 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
   __builtin_amdgcn_s_waitcnt(0);   // (a wait the compiler knows of: nothing it loaded is outstanding in the loop)
 
   bool aborted = false;
-  const int last = C > 1 ? n_it + 1 : n_it;   // clusters of several update one tile behind
-#pragma unroll 1
-  for (int i = 0; i < last; i++) {
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __syncthreads();   // tile i has landed; the image of updated weights is complete
-    const bool do_a = C == 1 || i < n_it;
+  // ---- the parts of an iteration
+  constexpr int ZN = QX ? RB / 2 : NBK == 4 ? 2 : 1;   // row blocks of the products
+  constexpr int FN = QX ? RB / 2 : 1;                  // row blocks this wavefront finishes
+  floatx4 z[ZN];
+  auto opaque = [&] {
     asm volatile("" : "+s"(kp), "+s"(v), "+s"(m), "+s"(j), "+s"(b), "+s"(hi4));
     // (the operands count as used here, or the register allocator spills them in favour of short-lived values)
 #pragma unroll
@@ -526,131 +563,85 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
 #pragma unroll
       for (int k = 0; k < 12; k++) COPAQUE(xr[k]);
     }
-    COPAQUE(pk_w); COPAQUE(pk_g); COPAQUE(pk_o);
-    if (i + 1 < n_it) nxt = next_tile();
-    if (C == 1) {
-      if (i + 1 < n_it) load_tile(nxt, (i + 1) & 1);
-      if (i > 0) store_out(prev);
-    }
-    const int p0 = __builtin_amdgcn_readfirstlane(*(const __attribute__((address_space(3))) int*)(lds + G::L_MISC + 16 + (i & 1) * 8));
-    const int p1 = __builtin_amdgcn_readfirstlane(*(const __attribute__((address_space(3))) int*)(lds + G::L_MISC + 20 + (i & 1) * 8));
-    if (C > 1 && i > 0) {
-      // the partners' G of tile i-1: normally they had published it when the counters were read at the end of the
-      // iteration before
-      constexpr unsigned long long ALL = C == 8 ? ~0ull : (1ull << (8 * C & 63)) - 1ull;
-      const int seen = *(const __attribute__((address_space(3))) int*)(lds + G::L_MISC + 64 + 4 * (clu_lane() & (8 * C - 1)));
-      if ((__builtin_amdgcn_ballot_w64(seen >= i) & ALL) != ALL) {
-        for (int spin = 0;; spin++) {
-          const int fv = __hip_atomic_load(cflags + (clu_lane() & (8 * C - 1)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          if ((__builtin_amdgcn_ballot_w64(fv >= i) & ALL) == ALL) break;
-          if (spin >= p.spin_limit || ((spin & 1023) == 1023 && __hip_atomic_load(p.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
-            // give up: partners that wait for this workgroup see the error word and give up too
-            if (clu_lane() == 0) {
-              __hip_atomic_fetch_or(p.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-              *(__attribute__((address_space(3))) int*)(lds + G::L_MISC) = 1;
-            }
-            break;
-          }
-          __builtin_amdgcn_s_sleep(1);
-        }
+    COPAQUE(pk_w); COPAQUE(pk_g); COPAQUE(pk_o); COPAQUE(lid);
+  };
+  // logits of the tile in image wimg; the K halves' partial sums to LDS
+  auto logits_part = [&](unsigned wimg) {
+#pragma unroll
+    for (int n = 0; n < ZN; n++) z[n] = floatx4{0.f, 0.f, 0.f, 0.f};
+    const unsigned rb0 = QX ? (unsigned)(hi4 * (RB / 2) * 16 * LS) : NBK == 4 ? 0u : (unsigned)(((v >> 1) & 1) * 16 * LS);
+    const unsigned abase = wimg + (pk_w >> 16) + rb0 + (QX ? 0u : (unsigned)(hi4 * (WT == CLU_BF16 ? 768 : 64)));
+    unsigned lanes = EARLY ? element_lanes() : 0u;
+    if (EARLY) COPAQUE(lanes);
+    // operands are read LD - 1 steps (FP8 products: one) ahead of their products
+    constexpr int LD = C == 4 ? 3 : 4;
+    if constexpr (QX) {
+      constexpr int NS = 6 * ZN;
+      intx4 lo[2], hi[2];
+      auto rd = [&](int t) {
+        const int ks = t / ZN, n = t - ks * ZN;
+        lo[t & 1] = *(const __attribute__((address_space(3))) intx4*)(lds + abase + ks * 128 + n * 16 * LS);
+        hi[t & 1] = *(const __attribute__((address_space(3))) intx4*)(lds + abase + ks * 128 + 64 + n * 16 * LS);
+      };
+      rd(0);
+#pragma unroll
+      for (int t = 0; t < NS; t++) {
+        if (t + 1 < NS) rd(t + 1);
+        const intx4 l = lo[t & 1], h = hi[t & 1];
+        z[t % ZN] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(intx8{l[0], l[1], l[2], l[3], h[0], h[1], h[2], h[3]}, xq8[t / ZN], z[t % ZN], 0, 0, 0, 0, 0, 0);
+        if constexpr (EARLY) words(C == 1 ? cur : prev, CluInt<0>{}, lanes, t * EP / NS, (t + 1) * EP / NS);
+        CFENCE();
       }
+    } else if constexpr (WT == CLU_BF16) {
+      constexpr int NS = 12 * ZN;
+      bf16x8 wv[LD];
+      auto rd = [&](int t) {
+        const int k = t / ZN, n = t - k * ZN;
+        wv[t % LD] = *(const __attribute__((address_space(3))) bf16x8*)(lds + abase + k * 64 + n * 16 * LS);
+      };
+      
 #pragma unroll
-      for (int s = 0; s < (G::GPIECES + 7) / 8; s++) {
-        const int pc = v + 8 * s;
-        if (pc < G::GPIECES) {
-          const int d = pc / (G::GSL / 1024), part = pc - d * (G::GSL / 1024), qm = (m + 1 + d) & (C - 1);
-          clu_lds_load16_l2(exch_slot(qm, i - 1) + part * 1024, (unsigned)clu_lane() * 16u, (unsigned)(G::L_PART + pc * 1024));
-        }
-      }
-    }
-    const unsigned wimg = (unsigned)(G::L_W + (i & 1) * G::IMG), gown = (unsigned)(G::L_OWN + (C > 1 ? i & 1 : 0) * G::GSL);
-    constexpr int ZN = QX ? RB / 2 : NBK == 4 ? 2 : 1;   // row blocks of the products
-    constexpr int FN = QX ? RB / 2 : 1;                  // row blocks this wavefront finishes
-    floatx4 z[ZN];
-    if (do_a) {
+      for (int t = 0; t < LD - 1; t++) rd(t);
 #pragma unroll
-      for (int n = 0; n < ZN; n++) z[n] = floatx4{0.f, 0.f, 0.f, 0.f};
-      const unsigned rb0 = QX ? (unsigned)(hi4 * (RB / 2) * 16 * LS) : NBK == 4 ? 0u : (unsigned)(((v >> 1) & 1) * 16 * LS);
-      const unsigned abase = wimg + (pk_w >> 16) + rb0 + (QX ? 0u : (unsigned)(hi4 * (WT == CLU_BF16 ? 768 : 64)));
-      unsigned lanes = EARLY ? element_lanes() : 0u;
-      if (EARLY) COPAQUE(lanes);
-      // operands are read three steps ahead of their products
-      if constexpr (QX) {
-        constexpr int NS = 6 * ZN;
-        intx4 lo[2], hi[2];
-        auto rd = [&](int t) {
-          const int ks = t / ZN, n = t - ks * ZN;
-          lo[t & 1] = *(const __attribute__((address_space(3))) intx4*)(lds + abase + ks * 128 + n * 16 * LS);
-          hi[t & 1] = *(const __attribute__((address_space(3))) intx4*)(lds + abase + ks * 128 + 64 + n * 16 * LS);
-        };
-        rd(0);
-#pragma unroll
-        for (int t = 0; t < NS; t++) {
-          if (t + 1 < NS) rd(t + 1);
-          const intx4 l = lo[t & 1], h = hi[t & 1];
-          z[t % ZN] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(intx8{l[0], l[1], l[2], l[3], h[0], h[1], h[2], h[3]}, xq8[t / ZN], z[t % ZN], 0, 0, 0, 0, 0, 0);
-          if constexpr (EARLY) words(C == 1 ? cur : prev, CluInt<0>{}, lanes, t * EP / NS, (t + 1) * EP / NS);
-          CFENCE();
-        }
-      } else if constexpr (WT == CLU_BF16) {
-        constexpr int NS = 12 * ZN;
-        bf16x8 wv[4];
-        auto rd = [&](int t) {
-          const int k = t / ZN, n = t - k * ZN;
-          wv[t & 3] = *(const __attribute__((address_space(3))) bf16x8*)(lds + abase + k * 64 + n * 16 * LS);
-        };
-        rd(0); rd(1); rd(2);
-#pragma unroll
-        for (int t = 0; t < NS; t++) {
-          if (t + 3 < NS) rd(t + 3);
-          z[t % ZN] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[t & 3], xr[t / ZN], z[t % ZN], 0, 0, 0);
-          if constexpr (EARLY) words(C == 1 ? cur : prev, CluInt<0>{}, lanes, t * EP / NS, (t + 1) * EP / NS);
-          CFENCE();
-        }
-      } else {
-        constexpr int NS = 6 * ZN;
-        intx4 wv[4];
-        auto rd = [&](int t) {
-          const int k2 = t / ZN, n = t - k2 * ZN;
-          wv[t & 3] = *(const __attribute__((address_space(3))) intx4*)(lds + abase + k2 * 128 + n * 16 * LS);
-        };
-        rd(0); rd(1); rd(2);
-#pragma unroll
-        for (int t = 0; t < NS; t++) {
-          if (t + 3 < NS) rd(t + 3);
-          const intx4 w4 = wv[t & 3];
-          z[t % ZN] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(clu_widen8(intx2{w4.x, w4.y}), xr[2 * (t / ZN)], z[t % ZN], 0, 0, 0);
-          z[t % ZN] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(clu_widen8(intx2{w4.z, w4.w}), xr[2 * (t / ZN) + 1], z[t % ZN], 0, 0, 0);
-          if constexpr (EARLY) words(C == 1 ? cur : prev, CluInt<0>{}, lanes, t * EP / NS, (t + 1) * EP / NS);
-          CFENCE();
-        }
-      }
-      if constexpr (!QX) {
-        // the other K half's row block (64-row slices) or the upper half's sum (32-row slices) to the wavefront that finishes it
-        if (NBK == 4 || hi4 == 1)
-          *(__attribute__((address_space(3))) floatx4*)(lds + G::L_PS + v * 1024 + clu_lane() * 16) = NBK == 4 ? (hi4 ? z[0] : z[ZN - 1]) : z[0];
+      for (int t = 0; t < NS; t++) {
+        if (t + LD - 1 < NS) rd(t + LD - 1);
+        z[t % ZN] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[t % LD], xr[t / ZN], z[t % ZN], 0, 0, 0);
+        if constexpr (EARLY) words(C == 1 ? cur : prev, CluInt<0>{}, lanes, t * EP / NS, (t + 1) * EP / NS);
+        CFENCE();
       }
     } else {
-      if constexpr (EARLY) words(prev, CluInt<0>{}, element_lanes(), 0, EP);
+      constexpr int NS = 6 * ZN;
+      intx4 wv[LD];
+      auto rd = [&](int t) {
+        const int k2 = t / ZN, n = t - k2 * ZN;
+        wv[t % LD] = *(const __attribute__((address_space(3))) intx4*)(lds + abase + k2 * 128 + n * 16 * LS);
+      };
+      
+#pragma unroll
+      for (int t = 0; t < LD - 1; t++) rd(t);
+#pragma unroll
+      for (int t = 0; t < NS; t++) {
+        if (t + LD - 1 < NS) rd(t + LD - 1);
+        const intx4 w4 = wv[t % LD];
+        z[t % ZN] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(clu_widen8(intx2{w4.x, w4.y}), xr[2 * (t / ZN)], z[t % ZN], 0, 0, 0);
+        z[t % ZN] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(clu_widen8(intx2{w4.z, w4.w}), xr[2 * (t / ZN) + 1], z[t % ZN], 0, 0, 0);
+        if constexpr (EARLY) words(C == 1 ? cur : prev, CluInt<0>{}, lanes, t * EP / NS, (t + 1) * EP / NS);
+        CFENCE();
+      }
     }
-    if (C > 1) {
-      if (i > 1) store_out(prev2);   // the weights updated in the iteration before
-      // the partners' G has landed (younger than its loads: those stores)
-      if (i > 1 && prev2.rows_valid == T) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(G::OPIECES / 8) : "memory");
-      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if constexpr (!QX) {
+      // the other K half's row block (64-row slices) or the upper half's sum (32-row slices) to the wavefront that finishes it
+      if (NBK == 4 || hi4 == 1)
+        *(__attribute__((address_space(3))) floatx4*)(lds + G::L_PS + v * 1024 + lid * 16) = NBK == 4 ? (hi4 ? z[0] : z[ZN - 1]) : z[0];
+      if (NBK == 4 && hi4) z[0] = z[ZN - 1];   // ... and the one it finishes itself
     }
-    if (!QX || C > 1) {
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      __syncthreads();   // the partial logits and the partners' G of tile i-1 are visible; the image of updated weights has been read
-    }
-    if (C > 1) {
-      if (__builtin_amdgcn_readfirstlane(*(const __attribute__((address_space(3))) int*)(lds + G::L_MISC)) != 0) { aborted = true; break; }
-    }
-    if (do_a && (QX || NBK == 4 || hi4 == 0)) {
+  };
+  // G of the tile q (positives p0 .. p1-1) to LDS at gown and, in a cluster of several, to the exchange slot of position it
+  auto other_half = [&] { return QX ? floatx4{} : *(const __attribute__((address_space(3))) floatx4*)(lds + G::L_PS + (v ^ 4) * 1024 + lid * 16); };
+  auto sigmoid_part = [&](const CluTile& q, unsigned gown, int it, int p0, int p1, floatx4 o) {
+    if (QX || NBK == 4 || hi4 == 0) {
       if constexpr (!QX) {
-        const floatx4 o = *(const __attribute__((address_space(3))) floatx4*)(lds + G::L_PS + (v ^ 4) * 1024 + clu_lane() * 16);
-        const floatx4 own = NBK == 4 ? (hi4 ? z[ZN - 1] : z[0]) : z[0];
-        z[0] = NBK == 4 && hi4 ? o + own : own + o;   // lower K half first
+        z[0] = NBK == 4 && hi4 ? o + z[0] : z[0] + o;   // lower K half first
       }
       const float nlog2e = -1.44269504088896340736f;
 #pragma unroll
@@ -670,13 +661,13 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
           const __attribute__((address_space(4))) unsigned* ckeys = (const __attribute__((address_space(4))) unsigned*)p.keys[C == 8 ? m >> 2 : 0];
           typedef unsigned c_keysx8 __attribute__((ext_vector_type(8), aligned(4)));
           const unsigned brow0 = (unsigned)(((m * G::SL) & 255) + 16 * b);   // first batch row of this wavefront's block within the key's 256
-          const unsigned lbase = p.label0_seg + (unsigned)cur.c * (unsigned)p.rows_per_chunk + (unsigned)(cur.row0 + 16 * rb);
+          const unsigned lbase = p.label0_seg + (unsigned)q.c * (unsigned)p.rows_per_chunk + (unsigned)(q.row0 + 16 * rb);
           unsigned before = p0 > 0 ? ckeys[p0 - 1] : ~ckeys[p0];
           for (int e0 = p0; e0 < p1; e0 += 8) {
             const c_keysx8 kk = *(const __attribute__((address_space(4))) c_keysx8*)(ckeys + e0);
 #pragma unroll
             for (int jj = 0; jj < 8; jj++) {
-              const int ln = clu_lane();
+              const int ln = lid;
               const unsigned key = kk[jj];
               const unsigned lrel = (key >> 8) - lbase, br = (key & 255u) - brow0;
               if (e0 + jj < p1 && key != before && lrel < 16u && br < 16u) {
@@ -691,130 +682,223 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
           s01 = bf16_pack2(sg[0], sg[1]);
           s23 = bf16_pack2(sg[2], sg[3]);
         }
-        if (cur.rows_valid < T) {   // rows past the end of the chunk contribute nothing
-          const int r0 = 16 * rb + 4 * (clu_lane() >> 4);
-          if (r0 >= cur.rows_valid) s01 &= 0xFFFF0000u;
-          if (r0 + 1 >= cur.rows_valid) s01 &= 0x0000FFFFu;
-          if (r0 + 2 >= cur.rows_valid) s23 &= 0xFFFF0000u;
-          if (r0 + 3 >= cur.rows_valid) s23 &= 0x0000FFFFu;
+        if (q.rows_valid < T) {   // rows past the end of the chunk contribute nothing
+          const int r0 = 16 * rb + 4 * (lid >> 4);
+          if (r0 >= q.rows_valid) s01 &= 0xFFFF0000u;
+          if (r0 + 1 >= q.rows_valid) s01 &= 0x0000FFFFu;
+          if (r0 + 2 >= q.rows_valid) s23 &= 0xFFFF0000u;
+          if (r0 + 3 >= q.rows_valid) s23 &= 0x0000FFFFu;
         }
         const unsigned goff = ((pk_g >> 16) ^ (unsigned)(32 * (rb & 1))) + (unsigned)((rb >> 1) * G::SL * 64);
         const cux2 sv = cux2{s01, s23};
         *(__attribute__((address_space(3))) cux2*)(lds + gown + goff) = sv;
         if constexpr (C > 1) {
-          unsigned char* slot = exch_slot(m, i);
-          asm volatile("global_store_dwordx2 %0, %1, %2" : : "v"(goff), "v"(sv), "s"(slot) : "memory");
+          const unsigned at = goff + (unsigned)((m * CLU_SLOTS + (it & (CLU_SLOTS - 1))) * G::GSL);
+          asm volatile("s_nop 4\n\tglobal_store_dwordx2 %0, %1, %2" : : "v"(at), "v"(sv), "s"(exq) : "memory");
         }
       }
     }
-    // ---- first half of grad_W and update of the tile before (it only needs the partners' G): vector work beside the latencies
-    //      of the sigmoid
-    const unsigned gprev = (unsigned)(G::L_OWN + (C > 1 ? (i - 1) & 1 : 0) * G::GSL);
-    if constexpr (C > 1) {
-      if (i > 0) update_tile(prev, gprev, 0u, CluInt<0>{}, CluInt<RB / 2>{}, [] {});
-      if (do_a) {
-        // this wavefront's part of G(i) has reached the L2 by now: tell the partners
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        if (clu_lane() == 0) __hip_atomic_store(cflags + m * 8 + v, i + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  // grad_X += G^T W of the tile in image wimg
+  auto gradx_part = [&](unsigned wimg, unsigned gown, auto&& middle) {
+    unsigned lanes = EARLY ? element_lanes() : 0u;
+    if (EARLY2) COPAQUE(lanes);
+    const unsigned wtr_lane = (pk_w & 0xFFFFu) + wimg + (unsigned)(96 * G::WB * v), ga_lane = pk_o >> 16;
+#pragma unroll
+    for (int kt = 0; kt < KT; kt++) {
+      bf16x8 ga[NBK];
+#pragma unroll
+      for (int mb = 0; mb < NBK; mb++)
+        ga[mb] = *(const __attribute__((address_space(3))) bf16x8*)(lds + gown + ga_lane + kt * G::SL * 64 + mb * 1024);
+      // the W operand of a feature block is read one block ahead of its products
+      auto rdw = [&](int nn) {
+        if constexpr (WT == CLU_BF16) {
+          cshortx4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) cshortx4*)(lds + wtr_lane + kt * 32 * LS + nn * 32));
+          cshortx4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) cshortx4*)(lds + wtr_lane + kt * 32 * LS + 8 * LS + nn * 32));
+          return __builtin_bit_cast(bf16x8, cshortx8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]});
+        } else {
+          return __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) intx2*)(lds + wtr_lane + kt * 32 * LS + nn * 16));
+        }
+      };
+      decltype(rdw(0)) wraw[2];
+      wraw[0] = rdw(0);
+#pragma unroll
+      for (int nn = 0; nn < 6; nn++) {
+        if (nn + 1 < 6) wraw[(nn + 1) & 1] = rdw(nn + 1);
+        bf16x8 wb;
+        if constexpr (WT == CLU_BF16) wb = wraw[nn & 1];
+        else wb = clu_widen8(wraw[nn & 1]);
+#pragma unroll
+        for (int mb = 0; mb < NBK; mb++) acc[mb][nn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ga[mb], wb, acc[mb][nn], 0, 0, 0);
+        if (kt == KT - 1 && nn == 2) middle();
+        if constexpr (EARLY) words(C == 1 ? cur : prev, CluInt<1>{}, lanes, (6 * kt + nn) * EP / (6 * KT), (6 * kt + nn + 1) * EP / (6 * KT));
+        CFENCE();
       }
     }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __syncthreads();   // own G of tile i is visible
-    // ---- Two jobs are left: grad_X of tile i (matrix instructions) and (the second half of) grad_W and update of this tile
-    //      (cluster of one) or of the one before (vector instructions).  The two wavefronts of a SIMD can take them in opposite
-    //      order, each in the gaps of the other, or in step.  Measured in step against opposite, us a step, 131 K labels,
-    //      batches of 32 / 64 / 128 / 256 / 512:
-    //        Philox   bf16  184/188 183/185 230/239 347/374 604/633   e4m3 159/161 180/179 235/243 364/372 610/626
-    //                 FP8 logits  -  -  213/218 337/336 536/556
-    //        sr_fast  bf16  92/93 103/106 152/158 269/289 516/535     FP8 logits  -  -  125/128 226/231 443/461
-    //        nearest  bf16  79/79 94/93 143/147 258/278 508/519       e4m3 62/64 82/81 142/145 274/276 503/518
-    //                 FP8 logits  -  -  119/120 218/223 435/452
-    //      and over larger label spaces, where the clock falls: bf16, 501 K, batch 128, sr_fast 553/548; e4m3, 500 K, nearest
-    //      447/447; FP8 logits, 670 K, batch 256, sr_fast 830/833.  In step is the faster order with Philox at every size; without
-    //      it the two are within 1 % of each other at the large sizes the line was drawn at, and in step is up to 7 % faster at
-    //      the small ones.
-    constexpr bool OPPOSITE = MODE != ROUND_SR_PHILOX;
-    auto update_part = [&] {
-      if constexpr (C == 1) {
-        update_tile(cur, gown, wimg, CluInt<0>{}, CluInt<RB>{}, [] {});
-      } else {
-        auto snapshot = [&] {   // the counters as they are now go to LDS, looked at in the next iteration
-          const int ln = clu_lane();
-          if (v == 0 && ln < 8 * C) clu_lds_load4_l2(cflags + ln, (unsigned)(G::L_MISC + 64));
-        };
-        if (i > 0) update_tile(prev, gprev, 0u, CluInt<RB / 2>{}, CluInt<RB>{}, snapshot);
-        else snapshot();
-      }
-    };
-    auto gradx_part = [&](bool load) {   // load: request the next tile on the way
-      if (!do_a) {
-        if constexpr (EARLY) words(prev, CluInt<1>{}, element_lanes(), 0, EP);
-        return;
-      }
-      unsigned lanes = EARLY ? element_lanes() : 0u;
-      if (EARLY2) COPAQUE(lanes);
-      const unsigned wtr_lane = (pk_w & 0xFFFFu) + wimg + (unsigned)(96 * G::WB * v), ga_lane = pk_o >> 16;
-#pragma unroll
-      for (int kt = 0; kt < KT; kt++) {
-        bf16x8 ga[NBK];
-#pragma unroll
-        for (int mb = 0; mb < NBK; mb++)
-          ga[mb] = *(const __attribute__((address_space(3))) bf16x8*)(lds + gown + ga_lane + kt * G::SL * 64 + mb * 1024);
-        // the W operand of a feature block is read one block ahead of its products
-        auto rdw = [&](int nn) {
-          if constexpr (WT == CLU_BF16) {
-            cshortx4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) cshortx4*)(lds + wtr_lane + kt * 32 * LS + nn * 32));
-            cshortx4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) cshortx4*)(lds + wtr_lane + kt * 32 * LS + 8 * LS + nn * 32));
-            return __builtin_bit_cast(bf16x8, cshortx8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]});
-          } else {
-            return __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) intx2*)(lds + wtr_lane + kt * 32 * LS + nn * 16));
-          }
-        };
-        decltype(rdw(0)) wraw[2];
-        wraw[0] = rdw(0);
-#pragma unroll
-        for (int nn = 0; nn < 6; nn++) {
-          if (nn + 1 < 6) wraw[(nn + 1) & 1] = rdw(nn + 1);
-          bf16x8 wb;
-          if constexpr (WT == CLU_BF16) wb = wraw[nn & 1];
-          else wb = clu_widen8(wraw[nn & 1]);
-#pragma unroll
-          for (int mb = 0; mb < NBK; mb++) acc[mb][nn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ga[mb], wb, acc[mb][nn], 0, 0, 0);
-          if constexpr (EARLY) words(C == 1 ? cur : prev, CluInt<1>{}, lanes, (6 * kt + nn) * EP / (6 * KT), (6 * kt + nn + 1) * EP / (6 * KT));
-          // the next tile, spread over the products: issued together the loads of eight wavefronts fill the memory pipeline's
-          // queue and block them
-          if (C > 1 && kt == 0 && nn < 4 && load && i + 1 < n_it) load_pieces(nxt, (i + 1) & 1, nn * (G::WPIECES / 4), (nn + 1) * (G::WPIECES / 4));
-          CFENCE();
-        }
-      }
-      if (i + 1 == n_it || (p.flush && nxt.c != cur.c)) store_acc(p.flush ? j + cur.c : j);
-    };
-    if constexpr (OPPOSITE) {
-      if (C > 1 && hi4 && i + 1 < n_it) load_tile(nxt, (i + 1) & 1);
+  };
+
+  if constexpr (C == 1) {
 #pragma unroll 1
-      for (int ph = 0; ph < 2; ph++) {
-        asm volatile("" : "+s"(kp), "+s"(v), "+s"(m), "+s"(j), "+s"(b), "+s"(hi4));
-        COPAQUE(pk_w); COPAQUE(pk_g); COPAQUE(pk_o);
-        if (ph == hi4) gradx_part(hi4 == 0);
-        else update_part();
+    for (int i = 0; i < n_it; i++) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __syncthreads();   // tile i has landed; the image of updated weights is complete
+      opaque();
+      if (i + 1 < n_it) {
+        nxt = next_tile();
+        load_range(nxt, (i + 1) & 1);
+        load_pieces(nxt, (unsigned)(((i + 1) & 1) * G::IMG), 0, G::WPIECES);
       }
-    } else {
-      gradx_part(true);
-      update_part();
+      if (i > 0) store_out(prev);
+      const int p0 = __builtin_amdgcn_readfirstlane(*(const __attribute__((address_space(3))) int*)(lds + G::L_MISC + 16 + (i & 1) * 8));
+      const int p1 = __builtin_amdgcn_readfirstlane(*(const __attribute__((address_space(3))) int*)(lds + G::L_MISC + 20 + (i & 1) * 8));
+      const unsigned wimg = (unsigned)(G::L_W + (i & 1) * G::IMG), gown = (unsigned)G::L_OWN;
+      logits_part(wimg);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __syncthreads();   // the partial logits are visible; the image of updated weights has been read
+      sigmoid_part(cur, gown, i, p0, p1, other_half());
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __syncthreads();   // G of tile i is visible
+      // ---- Two jobs are left: grad_X (matrix instructions) and grad_W with the update (vector instructions).  The two wavefronts
+      //      of a SIMD can take them in opposite order, each in the gaps of the other, or in step.  Measured in step against
+      //      opposite, us a step, 131 K labels, batches of 32 / 64:
+      //        Philox   bf16  184/188 183/185   e4m3 159/161 180/179      sr_fast  bf16  92/93 103/106
+      //        nearest  bf16  79/79 94/93       e4m3 62/64 82/81
+      //      In step is the faster order with Philox; without it the two are within 1 % of each other at the large sizes the line was
+      //      drawn at, and in step is up to 3 % faster at the small ones.
+      constexpr bool OPPOSITE = MODE != ROUND_SR_PHILOX;
+      auto gx = [&] {
+        gradx_part(wimg, gown, [] {});
+        if (i + 1 == n_it || (WT == CLU_BF16 && nxt.c != cur.c)) store_acc(WT == CLU_BF16 ? j + cur.c : j);
+      };
+      auto upd = [&] { update_tile(cur, gown, wimg); };
+      if constexpr (OPPOSITE) {
+#pragma unroll 1
+        for (int ph = 0; ph < 2; ph++) {
+          asm volatile("" : "+s"(kp), "+s"(v), "+s"(m), "+s"(j), "+s"(b), "+s"(hi4));
+          COPAQUE(pk_w); COPAQUE(pk_g); COPAQUE(pk_o);
+          if (ph == hi4) gx();
+          else upd();
+        }
+      } else {
+        gx();
+        upd();
+      }
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // tile i+1 has landed
+      prev2 = prev;
+      prev = cur;
+      cur = nxt;
     }
-    if constexpr (C > 1) {
-      if (do_a) {
+  } else {
+    // A cluster of several.  An iteration is one tile in three intervals (two where three images fit):
+    //   grad_X of the tile before and its old weights to registers, the partners' counters and then their G requested;
+    //   the updated weights of the tile before that to memory, logits of this tile, half of the next one's loads (into the image
+    //   that grad_X has just read);
+    //   sigmoids and own G of this tile, the other half of the loads, A^T and update of the tile before.
+    // Everything an interval needs was started an interval or more before it, so that its latencies run beside the work of
+    // another tile, and its two kinds of work are independent.  (Before, each tile went through logits | sigmoids, first half of
+    // the update | grad_X, second half, loads, and the latencies of a tile's own chain - counters, gather, sigmoids, G to memory and
+    // published - stood in line: 10.5 K clocks a tile of 32 labels at C = 2 with sr_fast, 2.3 K of them matrix instructions.)
+    // A wavefront publishes its part of G(i) when all its memory operations are complete, at the end of the iteration, with a
+    // store that stays in the L2 (the next reader on the XCD waits 265 clocks for it; 590 behind an agent-scope store).
+    constexpr int GPW = (G::GPIECES + 7) / 8;   // gathering loads of a wavefront, at most
+    unsigned goff[GPW];                         // their places behind the cluster's exchange slots
+#pragma unroll
+    for (int s = 0; s < GPW; s++) {
+      const int pc = v + 8 * s, d = pc / (G::GSL / 1024), part = pc - d * (G::GSL / 1024), qm = (m + 1 + d) & (C - 1);
+      goff[s] = (unsigned)(qm * CLU_SLOTS * G::GSL + part * 1024);
+    }
+    unsigned w_prev = (G::NIMG - 1) * G::IMG, w_cur = 0, w_nxt = G::IMG;   // images of tiles i-1, i, i+1
+    // loads of the next tile that go out in front of the logits, the others behind the sigmoids.  us a step, none / half / all in
+    // front: two images (bf16, 501 K labels, batch 128, sr_fast) 550 / 510 / 548, three (e4m3, 500 K, nearest) 405 / 400 / 379
+    constexpr int LH = G::NIMG == 3 ? G::WPIECES : G::WPIECES / 2;
+#pragma unroll 1
+    for (int i = 0; i <= n_it; i++) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __syncthreads();   // tile i has landed; own G of tile i-1 and the image of updated weights of tile i-2 are complete
+      opaque();
+      const bool gathers = i > 0 && v < G::GPIECES, loads = i + 1 < n_it;
+      if (loads) {
+        nxt = next_tile();
+        load_range(nxt, (i + 1) & 1);
+      }
+      const bool lfull = loads && nxt.rows_valid == T, lpart = loads && nxt.rows_valid != T, sfull = i > 1 && prev2.rows_valid == T;
+      const unsigned gown = (unsigned)(G::L_OWN + (i & 1) * G::GSL), gprev = (unsigned)(G::L_OWN + ((i - 1) & 1) * G::GSL);
+      // ---- grad_X of the tile before, logits of this one
+      if (i > 0) {
+        int seen = 0;
+        gradx_part(w_prev, gprev, [&] {
+          if (gathers) seen = __hip_atomic_load(cflags + (lid & (8 * C - 1)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        });
 #pragma unroll
         for (int k = 0; k < G::NBLK; k++)
 #pragma unroll
           for (int n = 0; n < RB; n++)
-            if (takes(k, n)) read_old(wimg, k, row_block(n), wold[k][n]);
+            if (takes(k, n)) read_old(w_prev, k, row_block(n), wold[k][n]);
+        if (gathers) {
+          // the partners' G of the tile before
+          constexpr unsigned long long ALL = C == 8 ? ~0ull : (1ull << (8 * C & 63)) - 1ull;
+          if ((__builtin_amdgcn_ballot_w64(seen >= i) & ALL) != ALL) {
+            for (int spin = 0;; spin++) {
+              const int fv = __hip_atomic_load(cflags + (lid & (8 * C - 1)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+              if ((__builtin_amdgcn_ballot_w64(fv >= i) & ALL) == ALL) break;
+              if (spin >= p.spin_limit || ((spin & 1023) == 1023 && __hip_atomic_load(p.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
+                // give up: partners that wait for this workgroup see the error word and give up too
+                if (lid == 0) {
+                  __hip_atomic_fetch_or(p.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                  *(__attribute__((address_space(3))) int*)(lds + G::L_MISC) = 1;
+                }
+                break;
+              }
+              __builtin_amdgcn_s_sleep(1);
+            }
+          }
+          const unsigned voff = (unsigned)lid * 16u + (unsigned)(((i - 1) & 1) * G::GSL);
+#pragma unroll
+          for (int s = 0; s < GPW; s++)
+            if (v + 8 * s < G::GPIECES) clu_lds_load16_l2(exq, voff + goff[s], (unsigned)(G::L_PART + (v + 8 * s) * 1024));
+        }
+        if (i == n_it || (WT == CLU_BF16 && cur.c != prev.c)) store_acc(WT == CLU_BF16 ? j + prev.c : j);
       }
+      if (G::NIMG == 2) {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __syncthreads();   // image i-1 has been read
+      }
+      COPAQUE(lid);
+      if (i > 1) store_out(prev2);
+      const int p0 = __builtin_amdgcn_readfirstlane(*(const __attribute__((address_space(3))) int*)(lds + G::L_MISC + 16 + (i & 1) * 8));
+      const int p1 = __builtin_amdgcn_readfirstlane(*(const __attribute__((address_space(3))) int*)(lds + G::L_MISC + 20 + (i & 1) * 8));
+      if (lfull) load_full(nxt, w_nxt, CluInt<0>{}, CluInt<LH>{});
+      else if (lpart) load_pieces(nxt, w_nxt, 0, LH);
+      if (i < n_it) logits_part(w_cur);
+      else if constexpr (EARLY) words(prev, CluInt<0>{}, element_lanes(), 0, EP);
+      // the partners' G has landed (younger than its loads: those stores and loads)
+      if (sfull) {
+        if (loads) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(G::OPW + LH) : "memory");
+        else asm volatile("s_waitcnt vmcnt(%0)" : : "n"(G::OPW) : "memory");
+      } else {
+        if (loads) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(LH) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __syncthreads();   // the partial logits and the partners' G of tile i-1 are visible; the image of updated weights has been read
+      const floatx4 o = other_half();
+      if (__builtin_amdgcn_readfirstlane(*(const __attribute__((address_space(3))) int*)(lds + G::L_MISC)) != 0) { aborted = true; break; }
+      COPAQUE(lid);
+      // ---- G of this tile, grad_W and update of the tile before; the rest of the next tile is requested on the way
+      if (i < n_it) sigmoid_part(cur, gown, i, p0, p1, o);
+      if (lfull) load_full(nxt, w_nxt, CluInt<LH>{}, CluInt<G::WPIECES>{});
+      else if (lpart) load_pieces(nxt, w_nxt, LH, G::WPIECES);
+      if (i > 0) update_tile(prev, gprev, 0u);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // tile i+1 has landed, this wavefront's part of G(i) has reached the L2: tell the partners
+      if (i < n_it && lid == 0) __hip_atomic_store(cflags + m * 8 + v, i + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      prev2 = prev;
+      prev = cur;
+      cur = nxt;
+      const unsigned w = w_prev;
+      w_prev = w_cur;
+      w_cur = w_nxt;
+      w_nxt = G::NIMG == 2 ? w_prev : w;
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // tile i+1 has landed
-    prev2 = prev;
-    prev = cur;
-    cur = nxt;
   }
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
   __syncthreads();
@@ -835,9 +919,9 @@ void cluster_set_lds_bf16();
 void cluster_set_lds_sim();
 void cluster_set_lds_fp8();
 
-// Registers spilled, as the compiler reports them: none but with e4m3 weights, FP8 logits, c = 4, Philox (24, 36 bytes of scratch
-// a lane) and with bf16 weights, c = 4, nearest and sr_fast (6, 12 bytes).  A scratch access inside the tile loop makes the waits
-// counted by hand stricter, never laxer: it is younger than the loads they wait for.
+// Registers spilled, as the compiler reports them: none but with e4m3 weights, FP8 logits, c = 4, Philox (3, 12 bytes of scratch a
+// lane).  A scratch access inside the tile loop makes the waits counted by hand stricter, never laxer: it is younger than the loads
+// they wait for.  It also makes the compiler wait for every memory operation where the value is read back.
 
 #ifdef CLU_VARIANT   // a translation unit of variants: CLU_VARIANT(function suffix) with CLU_WT, CLU_QX
 #define CLU_PICK(C, NBK)                                                                                                         \
