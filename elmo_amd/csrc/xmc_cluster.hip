@@ -21,9 +21,9 @@
 // What bounds it: bf16 with a small batch the HBM stream (131 K labels, batch 32, round to nearest: 212 us a step in three
 // kernels, 108 now, 74 of them here at 5.4 TB/s of weights).  The Philox modes with batch 128 the issue of vector and matrix
 // instructions, which add up more than they overlap: the words alone are 145 clocks of a SIMD per 64 weights, 0.35-0.37 ms
-// of the step (501 K labels, bf16: 1142 us in three kernels, 765 now, 510 with sr_fast; 500 K, e4m3: 1086 / 750, 380 to
+// of the step (501 K labels, bf16: 1142 us in three kernels, 764 now, 505 with sr_fast; 500 K, e4m3: 1086 / 740, 368 to
 // nearest).  The others the issue of vector, scalar and matrix instructions by two wavefronts per SIMD, and with bf16 weights
-// the memory path beside it (48 KiB of a tile through every member's; without loads and stores 430 of the 510 us).
+// the memory path beside it (48 KiB of a tile through every member's; without loads and stores 408 of the 505 us).
 #include "xmc_common.h"
 
 namespace xmc {
@@ -146,9 +146,10 @@ __device__ __forceinline__ bf16x8 clu_widen8(intx2 raw) {   // eight e4m3 codes 
 }
 
 // Four consecutive features of one row: t = w - lr a, rounded (definitions: the comment in front of tiled_update_kernel).
-// a is rounded to bf16 first with bf16 weights.  rw: the Philox words, if they have been computed before (PRE).
+// a is rounded to bf16 first with bf16 weights.  at: the first weight's Philox counter, or index * FAST_MUL + seed of the fast hash.
+// rw: the Philox words, if they have been computed before (PRE).
 template <int WT, int MODE, bool PRE>
-__device__ __forceinline__ void clu_update4(floatx4 a, const unsigned (&wr)[WT == CLU_BF16 ? 2 : 1], float lr, unsigned off0, unsigned fidx,
+__device__ __forceinline__ void clu_update4(floatx4 a, const unsigned (&wr)[WT == CLU_BF16 ? 2 : 1], float lr, unsigned at,
                                             unsigned seed, const unsigned (&rw)[WT == CLU_BF16 ? 2 : 4], unsigned (&wo)[WT == CLU_BF16 ? 2 : 1]) {
   float w[4], t[4];
   if constexpr (WT == CLU_BF16) {
@@ -165,11 +166,11 @@ __device__ __forceinline__ void clu_update4(floatx4 a, const unsigned (&wr)[WT =
   for (int e = 0; e < 4; e++) {
     t[e] = __builtin_fmaf(-lr, a[e], w[e]);
     if (MODE == ROUND_SR_PHILOX) {
-      const unsigned r = !PRE ? philox_word0(off0 + (unsigned)e, seed, 0u) : WT == CLU_E4M3 ? rw[e & (WT == CLU_BF16 ? 1 : 3)] : e & 1 ? rw[e >> 1] >> 16 : rw[e >> 1];
+      const unsigned r = !PRE ? philox_word0(at + (unsigned)e, seed, 0u) : WT == CLU_E4M3 ? rw[e & (WT == CLU_BF16 ? 1 : 3)] : e & 1 ? rw[e >> 1] >> 16 : rw[e >> 1];
       const unsigned mask = WT == CLU_BF16 ? 0xFFFFu : 0xFFFFFu;
       unsigned tb = __float_as_uint(t[e]) + (r & mask);
       if (WT == CLU_E4M3) tb &= ~mask;   // (bf16: the lower half is dropped by the pack below)
-      if (!PRE) asm volatile("" : "+v"(off0), "+v"(tb));   // one chain of ten rounds at a time: no registers for four
+      if (!PRE) asm volatile("" : "+v"(at), "+v"(tb));   // one chain of ten rounds at a time: no registers for four
       t[e] = __uint_as_float(tb);
     }
   }
@@ -178,7 +179,7 @@ __device__ __forceinline__ void clu_update4(floatx4 a, const unsigned (&wr)[WT =
       wo[0] = __builtin_amdgcn_perm(__float_as_uint(t[1]), __float_as_uint(t[0]), 0x07060302u);
       wo[1] = __builtin_amdgcn_perm(__float_as_uint(t[3]), __float_as_uint(t[2]), 0x07060302u);
     } else if (MODE == ROUND_SR_FAST) {
-      const unsigned h = fast_mix(fidx, seed);
+      const unsigned h = fast_mix_tail(at);
       bf16x2 lo = {}, hi = {};
       lo = __builtin_amdgcn_cvt_sr_bf16_f32(lo, t[0], fast_word(h, 0), false);
       lo = __builtin_amdgcn_cvt_sr_bf16_f32(lo, t[1], fast_word(h, 1), true);
@@ -191,9 +192,10 @@ __device__ __forceinline__ void clu_update4(floatx4 a, const unsigned (&wr)[WT =
       wo[1] = bf16_pack2(t[2], t[3]);
     }
   } else {
-    int packed = 0;   // saturating or not: MODE.FP16_OVFL, set once per launch
+    int packed;   // saturating or not: MODE.FP16_OVFL, set once per launch
+    asm volatile("" : "=v"(packed));   // (every byte is written below)
     if (MODE == ROUND_SR_FAST) {
-      const unsigned h = fast_mix(fidx, seed);
+      const unsigned h = fast_mix_tail(at);
       packed = __builtin_amdgcn_cvt_sr_fp8_f32(t[0], fast_word(h, 0), packed, 0);
       packed = __builtin_amdgcn_cvt_sr_fp8_f32(t[1], fast_word(h, 1), packed, 1);
       packed = __builtin_amdgcn_cvt_sr_fp8_f32(t[2], fast_word(h, 2), packed, 2);
@@ -226,8 +228,9 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
   constexpr int T = G::T, RB = G::RB, KT = G::KT, RS = G::RS, KS = G::KS, WDW = WT == CLU_BF16 ? 2 : 1;
   clu_cparams kp = (clu_cparams)__builtin_amdgcn_kernarg_segment_ptr();
 #define p (*kp)
-  extern __shared__ __attribute__((aligned(16))) unsigned char clu_lds[];
-  clds_u8* lds = (clds_u8*)clu_lds;
+  // (the kernel has no other LDS; as a symbol the base would be added to every address and keep constants out of the offsets)
+  size_t lds0 = 0;   // (a variable: the constant 0 would be the null pointer, which is not address 0 here)
+  clds_u8* lds = (clds_u8*)lds0;
   const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, kg = lane >> 4;
   int v = __builtin_amdgcn_readfirstlane(tid >> 6);
   // members of cluster j: workgroups ((j / 8) C + m) 8 + j % 8, which share an XCD (workgroup g runs on XCD g % 8) and are
@@ -441,21 +444,32 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
   auto update_tile = [&](const CluTile& q, unsigned gown, unsigned wimg) {
     const unsigned seed = q.seed;
     const unsigned grow0 = label0 + (unsigned)q.c * (unsigned)rpc + (unsigned)q.row0;
+    const int ln = lid, l16 = ln & 15, kg = ln >> 4;
+    // a lane's part of a weight's place (the other part is scalar): Philox counter, product of the fast hash, image of updated weights.
+    // Computed per block of weights, these places were 13 of the 30 vector instructions of four weights with sr_fast; with the G
+    // operands' addresses (four per row block here, the rest in the instructions' offsets) the step took 767 instead of 739 us at
+    // FP8 670 K labels, batch 256, 511 instead of 494 at bf16, 131 K, batch 512, Philox.
+    const unsigned lane_at = MODE == ROUND_SR_PHILOX ? (unsigned)(l16 * D + 4 * kg) : MODE == ROUND_SR_FAST ? (unsigned)(l16 * (D / 4) + kg) * FAST_MUL : 0u;
+    unsigned out_lane = (unsigned)(G::L_OUT + l16 * G::ORS) + (WT == CLU_BF16 ? 8u * (kg & 1) : 4u * kg);
+    COPAQUE(out_lane);
+    const unsigned out_swz = WT == CLU_BF16 ? (unsigned)((kg >> 1) ^ (l16 & G::OSW)) : (unsigned)(l16 & G::OSW);
 #pragma unroll
     for (int n = 0; n < RB; n++) {
       const int rb = row_block(n);
       if (C <= 4 || takes(0, n)) {
-        const int ln = lid, l16 = ln & 15, kg = ln >> 4;
         const unsigned g_lane = ((pk_g & 0xFFFFu) ^ (unsigned)((rb & 1) * 32)) + (unsigned)((rb >> 1) * G::SL * 64);
-        // G operands GD - 1 K steps ahead of their products: as far as the registers go (a spilled register in this loop costs more
-        // than the depth gives: FP8 logits, c = 4, depth 3 spills five and takes 817 instead of 764 us at 670 K labels, batch 256)
+        unsigned own_lo = g_lane + gown, own_hi = (g_lane ^ 48u) + gown, part_lo = g_lane + (unsigned)G::L_PART, part_hi = (g_lane ^ 48u) + (unsigned)G::L_PART;
+        COPAQUE(own_lo); COPAQUE(own_hi);   // (what is added to them below goes into the instructions' offsets)
+        if constexpr (C > 1) { COPAQUE(part_lo); COPAQUE(part_hi); }
+        // G operands GD - 1 K steps ahead of their products: as far as the registers go (five spilled registers in this loop cost more
+        // than the depth gave: FP8 logits, c = 4, depth 3, 670 K labels, batch 256 817 us instead of 764)
         constexpr int GD = C == 8 ? 4 : (C == 4 && !QX) || (C == 2 && MODE != ROUND_SR_PHILOX) ? 3 : 2;
         bf16x8 bg[GD];
         auto rdg = [&](int ks) {
           const int d = ks * 32 / G::SL, kk = ks - d * (G::SL / 32);   // slice: own, next member's, ...; K step within it
-          const unsigned a0 = g_lane + (d == 0 ? gown : (unsigned)(G::L_PART + (d - 1) * G::GSL));
-          cshortx4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) cshortx4*)(lds + a0 + kk * 32 * 64));
-          cshortx4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) cshortx4*)(lds + (a0 ^ 48u) + (kk * 32 + 4) * 64));
+          const int at = kk * 32 * 64 + (d == 0 ? 0 : (d - 1) * G::GSL);
+          cshortx4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) cshortx4*)(lds + (d == 0 ? own_lo : part_lo) + at));
+          cshortx4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) cshortx4*)(lds + (d == 0 ? own_hi : part_hi) + at + 256));
           return __builtin_bit_cast(bf16x8, cshortx8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]});
         };
         floatx4 aa[G::NBLK];
@@ -469,8 +483,6 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
             if (takes(k, n)) aa[k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xt[k][ks], bg[ks % GD], ks == 0 ? floatx4{0.f, 0.f, 0.f, 0.f} : aa[k], 0, 0, 0);
           CFENCE();
         }
-        const unsigned row = (unsigned)(16 * rb + l16);
-        const unsigned orow = (unsigned)q.row0 + row;
 #pragma unroll
         for (int k = 0; k < G::NBLK; k++) {
           if (!takes(k, n)) continue;
@@ -484,16 +496,16 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
             for (int d = 0; d < WDW; d++) wr[d] = wold[k][n][d];
           }
           const int lb = block_of(k);
-          const unsigned col = (unsigned)((m * G::FBN + lb) * 16 + 4 * kg);
+          const unsigned fb = (unsigned)(m * G::FBN + lb);   // feature block (wave-uniform, as are the scalar parts below)
+          const unsigned at = MODE == ROUND_SR_PHILOX ? lane_at + ((unsigned)(q.row0 + 16 * rb) * (unsigned)D + fb * 16u)
+                                                      : lane_at + (((grow0 + (unsigned)(16 * rb)) * (unsigned)(D / 4) + fb * 4u) * FAST_MUL + seed);
           if (EARLY && k < NBE && (n == 0 || (EARLY2 && n == RB / 2)))
-            clu_update4<WT, MODE, true>(a, wr, lr, 0u, 0u, seed, rw[C == 1 ? n / (RB / 2) : 0][k < NBE ? k : 0], wo);
+            clu_update4<WT, MODE, true>(a, wr, lr, 0u, seed, rw[C == 1 ? n / (RB / 2) : 0][k < NBE ? k : 0], wo);
           else
-            clu_update4<WT, MODE, false>(a, wr, lr, orow * (unsigned)D + col, (grow0 + row) * (unsigned)(D / 4) + (col >> 2), seed, {}, wo);
-          if constexpr (WT == CLU_BF16) {
-            *(__attribute__((address_space(3))) cux2*)(lds + G::L_OUT + row * G::ORS + (unsigned)(((2 * lb + (kg >> 1)) ^ (l16 & G::OSW)) * 16 + 8 * (kg & 1))) = cux2{wo[0], wo[1]};
-          } else {
-            *(__attribute__((address_space(3))) unsigned*)(lds + G::L_OUT + row * G::ORS + (unsigned)((lb ^ (l16 & G::OSW)) * 16 + 4 * kg)) = wo[0];
-          }
+            clu_update4<WT, MODE, false>(a, wr, lr, at, seed, {}, wo);
+          const unsigned oat = out_lane + (((unsigned)((WT == CLU_BF16 ? 2 : 1) * lb) ^ out_swz) << 4) + (unsigned)(rb * 16 * G::ORS);
+          if constexpr (WT == CLU_BF16) *(__attribute__((address_space(3))) cux2*)(lds + oat) = cux2{wo[0], wo[1]};
+          else *(__attribute__((address_space(3))) unsigned*)(lds + oat) = wo[0];
           CFENCE();
         }
       }
@@ -793,7 +805,7 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
     //   grad_X of the tile before and its old weights to registers, the partners' counters and then their G requested;
     //   the updated weights of the tile before that to memory, logits of this tile, half of the next one's loads (into the image
     //   that grad_X has just read);
-    //   sigmoids and own G of this tile, the other half of the loads, A^T and update of the tile before.
+    //   the other half of the loads, sigmoids and own G of this tile, A^T and update of the tile before.
     // Everything an interval needs was started an interval or more before it, so that its latencies run beside the work of
     // another tile, and its two kinds of work are independent.  (Before, each tile went through logits | sigmoids, first half of
     // the update | grad_X, second half, loads, and the latencies of a tile's own chain - counters, gather, sigmoids, G to memory and
@@ -808,7 +820,7 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
       goff[s] = (unsigned)(qm * CLU_SLOTS * G::GSL + part * 1024);
     }
     unsigned w_prev = (G::NIMG - 1) * G::IMG, w_cur = 0, w_nxt = G::IMG;   // images of tiles i-1, i, i+1
-    // loads of the next tile that go out in front of the logits, the others behind the sigmoids.  us a step, none / half / all in
+    // loads of the next tile that go out in front of the logits, the others in front of the sigmoids.  us a step, none / half / all in
     // front: two images (bf16, 501 K labels, batch 128, sr_fast) 550 / 510 / 548, three (e4m3, 500 K, nearest) 405 / 400 / 379
     constexpr int LH = G::NIMG == 3 ? G::WPIECES : G::WPIECES / 2;
 #pragma unroll 1
@@ -885,9 +897,9 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
       if (__builtin_amdgcn_readfirstlane(*(const __attribute__((address_space(3))) int*)(lds + G::L_MISC)) != 0) { aborted = true; break; }
       COPAQUE(lid);
       // ---- G of this tile, grad_W and update of the tile before; the rest of the next tile is requested on the way
-      if (i < n_it) sigmoid_part(cur, gown, i, p0, p1, o);
       if (lfull) load_full(nxt, w_nxt, CluInt<LH>{}, CluInt<G::WPIECES>{});
       else if (lpart) load_pieces(nxt, w_nxt, LH, G::WPIECES);
+      if (i < n_it) sigmoid_part(cur, gown, i, p0, p1, o);
       if (i > 0) update_tile(prev, gprev, 0u);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // tile i+1 has landed, this wavefront's part of G(i) has reached the L2: tell the partners
       if (i < n_it && lid == 0) __hip_atomic_store(cflags + m * 8 + v, i + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -919,9 +931,8 @@ void cluster_set_lds_bf16();
 void cluster_set_lds_sim();
 void cluster_set_lds_fp8();
 
-// Registers spilled, as the compiler reports them: none but with e4m3 weights, FP8 logits, c = 4, Philox (3, 12 bytes of scratch a
-// lane).  A scratch access inside the tile loop makes the waits counted by hand stricter, never laxer: it is younger than the loads
-// they wait for.  It also makes the compiler wait for every memory operation where the value is read back.
+// No variant spills a vector register.  A scratch access inside the tile loop would make the waits counted by hand stricter, never
+// laxer (it is younger than the loads they wait for), and the compiler wait for every memory operation where the value is read back.
 
 #ifdef CLU_VARIANT   // a translation unit of variants: CLU_VARIANT(function suffix) with CLU_WT, CLU_QX
 #define CLU_PICK(C, NBK)                                                                                                         \

@@ -122,11 +122,12 @@ __host__ __device__ inline unsigned fast_seed(unsigned s) {
   s ^= s >> 16; s *= 0x7FEB352Du; s ^= s >> 15; s *= 0x846CA68Bu; s ^= s >> 16;
   return s;
 }
-__device__ __forceinline__ unsigned fast_mix(unsigned idx, unsigned seed) {
-  unsigned h = idx * 0x9E3779B1u + seed;
+constexpr unsigned FAST_MUL = 0x9E3779B1u;
+__device__ __forceinline__ unsigned fast_mix_tail(unsigned h) {   // h = idx * FAST_MUL + seed
   h ^= h >> 16; h *= 0x85EBCA77u; h ^= h >> 15;
   return h;
 }
+__device__ __forceinline__ unsigned fast_mix(unsigned idx, unsigned seed) { return fast_mix_tail(idx * FAST_MUL + seed); }
 __device__ __forceinline__ unsigned fast_word(unsigned h, int i) {
   const unsigned k[4] = {1u, 0x27D4EB2Fu, 0x165667B1u, 0x9E3779B1u};
   return h * k[i];
