@@ -241,6 +241,78 @@ int xmc_fp8_step(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, co
 
 }  // extern "C"
 
+// The one-pass form of the step (xmc_cluster.hip): 768 features, no compensated head, no loss, no weight decay (options
+// that would have to stay in its main loop, whose registers are full).  Within these it was the faster form at every size
+// tried, from 2 K to 8.6 M labels and 1 to 512 batch rows.  The arguments have been checked by the caller.
+static int cluster_step(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, int rows_last_chunk, int weight_type,
+                        const void* x_bf16, int batch, const int32_t* labels_coo, int nnz, float lr, const uint32_t* seeds,
+                        int round_mode, int quantize_x, int saturate, const DropoutParams& dp, void* grad_x_bf16, float* grad_x_f32,
+                        const ClusterPlace& at, bool profiled, int cus, int* failure_word, hipStream_t stream) {
+  const bool bf16 = weight_type == W_BF16, fp8 = !bf16 && quantize_x;
+  const int c = cluster_size(batch), nbk = cluster_blocks(batch), bp = c * 16 * nbk, pairs = (bp + 255) / 256;
+  const int tile_rows = fp8 && c < 8 ? 64 : 32;
+  const int tpc64 = (rows_per_chunk + TL - 1) / TL;
+  const int n_pad = (nnz + 63) / 64 * 64;   // whole blocks of the sort
+  // a sort key keeps 24 bits for the label: larger label spaces are taken in segments of whole chunks
+  int seg_chunks = ((1 << 24) - 2) / rows_per_chunk;
+  if (seg_chunks > num_chunks) seg_chunks = num_chunks;
+  if (seg_chunks < 1) return XMC_ERR_RANGE;
+  const ClusterVariant var = bf16 ? cluster_variant_bf16(c, nbk, round_mode) : fp8 ? cluster_variant_fp8(c, nbk, round_mode) : cluster_variant_sim(c, nbk, round_mode);
+  for (int c0 = 0; c0 < num_chunks; c0 += seg_chunks) {
+    const int nch = c0 + seg_chunks <= num_chunks ? seg_chunks : num_chunks - c0;
+    const bool last = c0 + nch == num_chunks;
+    const int sort_blocks = n_pad / 64, ptr_blocks = (nch * tpc64 + 1 + 255) / 256, prep_blocks = (bp * (D / 4) + 255) / 256;
+    const ClusterPrep pp = {labels_coo, nnz, n_pad, batch, c0 * rows_per_chunk, nch * rows_per_chunk, pairs, rows_per_chunk, tpc64, nch * tpc64,
+                            sort_blocks, ptr_blocks, at.keys, at.tile_ptr, at.tp_stride, (const unsigned short*)x_bf16, bp, bf16 ? 0 : fp8 ? 2 : 1,
+                            at.xq, at.xt, at.flags, c0 == 0 ? at.err : nullptr};   // (a failure in one segment stays visible behind the others)
+    cluster_prep_kernel<<<(sort_blocks + ptr_blocks) * pairs + prep_blocks, 256, (size_t)(n_pad + 256) * 4, stream>>>(pp, dp);
+    ClusterParams p;
+    for (int k = 0; k < MAX_CHUNKS; k++) {
+      p.chunk[k] = k < nch ? (unsigned char*)chunk_ptrs[c0 + k] : nullptr;
+      p.seed[k] = k < nch && seeds ? (round_mode == XMC_ROUND_SR_FAST ? fast_seed(seeds[c0 + k]) : seeds[c0 + k]) : 0u;
+    }
+    p.nchunks = nch;
+    p.rows_per_chunk = rows_per_chunk;
+    p.rows_last = last ? rows_last_chunk : rows_per_chunk;
+    p.tpc = (rows_per_chunk + tile_rows - 1) / tile_rows;
+    p.tpc_last = (p.rows_last + tile_rows - 1) / tile_rows;
+    p.perm = tile_stride(p.tpc);
+    p.perm_last = tile_stride(p.tpc_last);
+    p.tpc64 = tpc64;
+    p.ntiles = (nch - 1) * p.tpc + p.tpc_last;
+    const int most = (cus < CLU_MAXWG ? cus : CLU_MAXWG) / 8 / c * 8;   // whole clusters on every XCD
+    p.nclusters = p.ntiles < most ? p.ntiles : most;
+    p.label0_seg = 0u;
+    p.label0 = (unsigned)c0 * (unsigned)rows_per_chunk;
+    p.xq = at.xq;
+    p.xt = (const bf16x8*)at.xt;
+    for (int q = 0; q < 2; q++) {
+      const int pr = q < pairs ? q : 0;
+      p.keys[q] = at.keys + (size_t)pr * MAX_POS;
+      p.tile_ptr[q] = at.tile_ptr + pr * at.tp_stride;
+    }
+    p.partial = at.partial;
+    p.exch = at.exch;
+    p.flags = at.flags;
+    p.xcc = at.xcc;
+    p.err = at.err;
+    p.lr = lr;
+    p.flush = bf16 ? 1 : 0;   // the reference rounds each chunk's sum where the weights are bf16
+    p.saturate = saturate;
+    p.spin_limit = g_spin_limit.load(std::memory_order_relaxed);
+    if (profiled && g_prof_start) (void)hipEventRecord(g_prof_start, stream);
+    var.fn<<<(p.nclusters + 7) / 8 * 8 * c, CLU_NT, var.lds, stream>>>(p);
+    if (profiled) {
+      if (g_prof_stop) (void)hipEventRecord(g_prof_stop, stream);
+      g_prof_start = g_prof_stop = nullptr;
+    }
+    const ClusterReduce rd = {p.partial, c, nbk, p.nclusters, p.ntiles, p.tpc, nch, p.flush, at.xcc, at.err, at.sticky, failure_word, at.gx, c0 > 0 ? 1 : 0, last ? 1 : 0, batch,
+                              (unsigned short*)grad_x_bf16, grad_x_f32};
+    cluster_reduce_kernel<<<c * nbk * 6 * 8, CLU_RW * 64, 0, stream>>>(rd, dp);
+  }
+  return launch_status();
+}
+
 // The fused step behind xmc_fp8_step, xmc_fp8_step_ex and xmc_fp8_kahan_step.  kahan_type 0: no compensated head.
 static int fused_step(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, const void* x_bf16, int batch,
                       int features, const int32_t* labels_coo, int nnz, float lr, const uint32_t* seeds, int round_mode,
@@ -651,79 +723,6 @@ int xmc_tiled_step(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, 
 
 }  // extern "C"
 
-// The one-pass form of the step (xmc_cluster.hip): 768 features, no compensated head, no loss, no weight decay (options
-// that would have to stay in its main loop, whose registers are full).  Within these it was the faster form at every size
-// tried, from 2 K to 8.6 M labels and 1 to 512 batch rows.  The arguments have been checked by the caller.
-static int cluster_step(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, int rows_last_chunk, int weight_type,
-                        const void* x_bf16, int batch, const int32_t* labels_coo, int nnz, float lr, const uint32_t* seeds,
-                        int round_mode, int quantize_x, int saturate, const DropoutParams& dp, void* grad_x_bf16, float* grad_x_f32,
-                        unsigned char* ws, int cus, int* failure_word, hipStream_t stream) {
-  const bool bf16 = weight_type == W_BF16, fp8 = !bf16 && quantize_x;
-  const int c = cluster_size(batch, fp8), nbk = cluster_blocks(batch, fp8), bp = c * 16 * nbk, pairs = (bp + 255) / 256;
-  const ClusterLayout lay = cluster_layout(num_chunks, rows_per_chunk, bp);
-  const int tile_rows = fp8 && c < 8 ? 64 : 32;
-  const int tpc64 = (rows_per_chunk + TL - 1) / TL;
-  const int n_pad = (nnz + 63) / 64 * 64;   // whole blocks of the sort
-  // a sort key keeps 24 bits for the label: larger label spaces are taken in segments of whole chunks
-  int seg_chunks = ((1 << 24) - 2) / rows_per_chunk;
-  if (seg_chunks > num_chunks) seg_chunks = num_chunks;
-  if (seg_chunks < 1) return XMC_ERR_RANGE;
-  int* err = (int*)(ws + TW_ERR);
-  unsigned* keys = (unsigned*)(ws + lay.keys);
-  int* tile_ptr = (int*)(ws + lay.tile_ptr);
-  float* gx_total = (float*)(ws + lay.gx);
-  const ClusterVariant var = bf16 ? cluster_variant_bf16(c, nbk, round_mode) : fp8 ? cluster_variant_fp8(c, nbk, round_mode) : cluster_variant_sim(c, nbk, round_mode);
-  for (int c0 = 0; c0 < num_chunks; c0 += seg_chunks) {
-    const int nch = c0 + seg_chunks <= num_chunks ? seg_chunks : num_chunks - c0;
-    const bool last = c0 + nch == num_chunks;
-    const int sort_blocks = n_pad / 64, ptr_blocks = (nch * tpc64 + 1 + 255) / 256, prep_blocks = (bp * (D / 4) + 255) / 256;
-    const ClusterPrep pp = {labels_coo, nnz, n_pad, batch, c0 * rows_per_chunk, nch * rows_per_chunk, pairs, rows_per_chunk, tpc64, nch * tpc64,
-                            sort_blocks, ptr_blocks, keys, tile_ptr, lay.tp_stride, (const unsigned short*)x_bf16, bp, bf16 ? 0 : fp8 ? 2 : 1,
-                            ws + lay.xq, (unsigned short*)(ws + lay.xt), (int*)(ws + lay.flags),
-                            c0 == 0 ? err : nullptr};   // (a failure in one segment stays visible behind the others)
-    cluster_prep_kernel<<<(sort_blocks + ptr_blocks) * pairs + prep_blocks, 256, (size_t)(n_pad + 256) * 4, stream>>>(pp, dp);
-    ClusterParams p;
-    for (int k = 0; k < MAX_CHUNKS; k++) {
-      p.chunk[k] = k < nch ? (unsigned char*)chunk_ptrs[c0 + k] : nullptr;
-      p.seed[k] = k < nch && seeds ? (round_mode == XMC_ROUND_SR_FAST ? fast_seed(seeds[c0 + k]) : seeds[c0 + k]) : 0u;
-    }
-    p.nchunks = nch;
-    p.rows_per_chunk = rows_per_chunk;
-    p.rows_last = last ? rows_last_chunk : rows_per_chunk;
-    p.tpc = (rows_per_chunk + tile_rows - 1) / tile_rows;
-    p.tpc_last = (p.rows_last + tile_rows - 1) / tile_rows;
-    p.perm = tile_stride(p.tpc);
-    p.perm_last = tile_stride(p.tpc_last);
-    p.tpc64 = tpc64;
-    p.ntiles = (nch - 1) * p.tpc + p.tpc_last;
-    const int most = (cus < CLU_MAXWG ? cus : CLU_MAXWG) / 8 / c * 8;   // whole clusters on every XCD
-    p.nclusters = p.ntiles < most ? p.ntiles : most;
-    p.label0_seg = 0u;
-    p.label0 = (unsigned)c0 * (unsigned)rows_per_chunk;
-    p.xq = ws + lay.xq;
-    p.xt = (const bf16x8*)(ws + lay.xt);
-    for (int q = 0; q < 2; q++) {
-      const int pr = q < pairs ? q : 0;
-      p.keys[q] = keys + (size_t)pr * MAX_POS;
-      p.tile_ptr[q] = tile_ptr + pr * lay.tp_stride;
-    }
-    p.partial = (floatx4*)(ws + lay.partial);
-    p.exch = ws + lay.exch;
-    p.flags = (int*)(ws + lay.flags);
-    p.xcc = (int*)(ws + lay.xcc);
-    p.err = err;
-    p.lr = lr;
-    p.flush = bf16 ? 1 : 0;   // the reference rounds each chunk's sum where the weights are bf16
-    p.saturate = saturate;
-    p.spin_limit = g_spin_limit.load(std::memory_order_relaxed);
-    var.fn<<<(p.nclusters + 7) / 8 * 8 * c, CLU_NT, var.lds, stream>>>(p);
-    const ClusterReduce rd = {p.partial, c, nbk, p.nclusters, p.ntiles, p.tpc, nch, p.flush, p.xcc, err, failure_word, gx_total, c0 > 0 ? 1 : 0, last ? 1 : 0, batch,
-                              (unsigned short*)grad_x_bf16, grad_x_f32};
-    cluster_reduce_kernel<<<c * nbk * 6 * 8, CLU_RW * 64, 0, stream>>>(rd, dp);
-  }
-  return launch_status();
-}
-
 // xmc_tiled_step_ex for DD features (768 or 1024)
 template <int DD>
 static int tiled_step_t(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, int rows_last_chunk, int weight_type,
@@ -759,10 +758,17 @@ static int tiled_step_t(void* const* chunk_ptrs, int num_chunks, int rows_per_ch
   if (di.ok != 1) return XMC_ERR_DEVICE;
   hipStream_t stream = (hipStream_t)stream_;
   // (a cluster needs its members on one XCD at the same time: a partition of the GPU too small for one keeps the three kernels)
-  const int cluster = cluster_size(batch, weight_type != W_BF16 && quantize_x);
+  const int cluster = cluster_size(batch);
   if (DD == D && kahan_type == 0 && !loss_out && weight_decay == 0.f && di.cus / 8 / cluster >= 1)
+  {
+    unsigned char* w0 = (unsigned char*)workspace;
+    const ClusterLayout lay = cluster_layout(num_chunks, rows_per_chunk, batch);
+    const ClusterPlace at = {w0 + lay.xq, (unsigned short*)(w0 + lay.xt), (unsigned*)(w0 + lay.keys), (int*)(w0 + lay.flags), (int*)(w0 + lay.xcc),
+                             (float*)(w0 + lay.gx), (int*)(w0 + lay.tile_ptr), lay.tp_stride, w0 + lay.exch, (floatx4*)(w0 + lay.partial),
+                             (int*)(w0 + TW_ERR), (int*)(w0 + TW_ERR) + 1};
     return cluster_step(chunk_ptrs, num_chunks, rows_per_chunk, rows_last_chunk, weight_type, x_bf16, batch, labels_coo, nnz, lr, seeds,
-                        round_mode, quantize_x, saturate, dp, grad_x_bf16, grad_x_f32, (unsigned char*)workspace, di.cus, di.failure_word, stream);
+                        round_mode, quantize_x, saturate, dp, grad_x_bf16, grad_x_f32, at, false, di.cus, di.failure_word, stream);
+  }
   unsigned char* ws = (unsigned char*)workspace + TW_HEAD;
 
   const int rows_pad = (rows_per_chunk + TL - 1) / TL * TL;

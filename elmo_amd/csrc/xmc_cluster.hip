@@ -19,7 +19,7 @@
 // rows, so one geometry serves every batch size.
 //
 // What bounds it: bf16 with a small batch the HBM stream (131 K labels, batch 32, round to nearest: 212 us a step in three
-// kernels, 108 now, 74 of them here at 5.4 TB/s of weights).  The Philox modes with batch 128 the issue of vector and matrix
+// kernels, 105 now, 71 of them here at 5.6 TB/s of weights).  The Philox modes with batch 128 the issue of vector and matrix
 // instructions, which add up more than they overlap: the words alone are 145 clocks of a SIMD per 64 weights, 0.35-0.37 ms
 // of the step (501 K labels, bf16: 1142 us in three kernels, 764 now, 505 with sr_fast; 500 K, e4m3: 1086 / 740, 368 to
 // nearest).  The others the issue of vector, scalar and matrix instructions by two wavefronts per SIMD, and with bf16 weights
@@ -320,7 +320,8 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
   load_pieces(cur, 0u, 0, G::WPIECES);
 
   // ---- resident operands
-  // Logits: with FP8 products wavefront v takes batch block v % 4 and half of the tile's row blocks; with bf16 products the
+  // Logits: with FP8 products wavefront v takes batch block v % 4 and half of the tile's row blocks (32-row slices: batch block
+  // v % 2 and a quarter of the row blocks); with bf16 products the
   // K range is split in two instead (a wavefront's share of X is then half as large) and the partial sums go through LDS.
   // 64-row slices: batch block v % 4, K half v / 4, both row blocks, of which it finishes one; 32-row slices: batch block
   // v % 2, row block (v / 2) % 2, K half v / 4, finished by the lower half.
@@ -402,7 +403,7 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
   //        e4m3, 500 K, batch 128 (C = 2)         755, 768 / 892 / 781     bf16, 501 K, batch 64 (C = 1)  680, 680 / 693 / 689
   //      So the words are early where their registers do not make the loop spill (batch 32: both halves).  The words of one
   //      wavefront of a SIMD beside the other's matrix instructions, in opposite order, are slower: 815 instead of 775 (C = 2).
-  constexpr bool EARLY = MODE == ROUND_SR_PHILOX && !QX && (C == 2 || (C == 1 && (WT == CLU_BF16 || NBK == 2))), EARLY2 = EARLY && NBK == 2;
+  constexpr bool EARLY = MODE == ROUND_SR_PHILOX && (C == 1 ? QX || WT == CLU_BF16 || NBK == 2 : C == 2 && !QX), EARLY2 = EARLY && NBK == 2;
   constexpr int NBE = G::NBLK < 3 ? G::NBLK : 3, EP = 8 * NBE;   // blocks; pieces (half an evaluation each)
   constexpr int RWN = WT == CLU_BF16 ? 2 : 4;                    // registers of four words (bf16 weights take 16 bits of each)
   unsigned rw[C == 1 ? 2 : 1][EARLY ? NBE : 1][RWN];
@@ -558,8 +559,8 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
 
   bool aborted = false;
   // ---- the parts of an iteration
-  constexpr int ZN = QX ? RB / 2 : NBK == 4 ? 2 : 1;   // row blocks of the products
-  constexpr int FN = QX ? RB / 2 : 1;                  // row blocks this wavefront finishes
+  constexpr int ZN = QX ? RB * NBK / 8 : NBK == 4 ? 2 : 1;   // row blocks of the products
+  constexpr int FN = QX ? ZN : 1;                            // row blocks this wavefront finishes
   floatx4 z[ZN];
   auto opaque = [&] {
     asm volatile("" : "+s"(kp), "+s"(v), "+s"(m), "+s"(j), "+s"(b), "+s"(hi4));
@@ -581,7 +582,7 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
   auto logits_part = [&](unsigned wimg) {
 #pragma unroll
     for (int n = 0; n < ZN; n++) z[n] = floatx4{0.f, 0.f, 0.f, 0.f};
-    const unsigned rb0 = QX ? (unsigned)(hi4 * (RB / 2) * 16 * LS) : NBK == 4 ? 0u : (unsigned)(((v >> 1) & 1) * 16 * LS);
+    const unsigned rb0 = QX ? (unsigned)((NBK == 4 ? hi4 : v >> 1) * ZN * 16 * LS) : NBK == 4 ? 0u : (unsigned)(((v >> 1) & 1) * 16 * LS);
     const unsigned abase = wimg + (pk_w >> 16) + rb0 + (QX ? 0u : (unsigned)(hi4 * (WT == CLU_BF16 ? 768 : 64)));
     unsigned lanes = EARLY ? element_lanes() : 0u;
     if (EARLY) COPAQUE(lanes);
@@ -658,7 +659,7 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
       const float nlog2e = -1.44269504088896340736f;
 #pragma unroll
       for (int n = 0; n < FN; n++) {
-        const int rb = QX ? hi4 * (RB / 2) + n : NBK == 4 ? hi4 : (v >> 1) & 1;   // row block (wave-uniform)
+        const int rb = QX ? (NBK == 4 ? hi4 : v >> 1) * ZN + n : NBK == 4 ? hi4 : (v >> 1) & 1;   // row block (wave-uniform)
         const unsigned z01 = bf16_pack2(z[n][0], z[n][1]), z23 = bf16_pack2(z[n][2], z[n][3]);
         const float zf[4] = {__uint_as_float(z01 << 16), __uint_as_float(z01 & 0xFFFF0000u), __uint_as_float(z23 << 16), __uint_as_float(z23 & 0xFFFF0000u)};
         float s[4];
@@ -758,18 +759,28 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
       if (i + 1 < n_it) {
         nxt = next_tile();
         load_range(nxt, (i + 1) & 1);
-        load_pieces(nxt, (unsigned)(((i + 1) & 1) * G::IMG), 0, G::WPIECES);
       }
       if (i > 0) store_out(prev);
       const int p0 = __builtin_amdgcn_readfirstlane(*(const __attribute__((address_space(3))) int*)(lds + G::L_MISC + 16 + (i & 1) * 8));
       const int p1 = __builtin_amdgcn_readfirstlane(*(const __attribute__((address_space(3))) int*)(lds + G::L_MISC + 20 + (i & 1) * 8));
       const unsigned wimg = (unsigned)(G::L_W + (i & 1) * G::IMG), gown = (unsigned)G::L_OWN;
       logits_part(wimg);
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      __syncthreads();   // the partial logits are visible; the image of updated weights has been read
+      // The next tile is requested behind the last one's stores and behind the logits.  In front of them, where the loads have longer,
+      // they made the logits and the stores wait: us a step, 501 K labels, batches of 32 / 64, in front against here
+      //   e4m3, FP8 logits: nearest 193/175 222/199, sr_fast 215/194 243/224, Philox 558/530 584/550
+      //   e4m3, bf16 logits: nearest 209/184 249/226, Philox 576/553 609/583;  bf16: nearest 341/339 361/342, Philox 636/593 670/638
+      // (131 K labels, bf16, batch 32, nearest: 78.9/75.5).  Loads first and then the stores, both here: no gain.
+      if (i + 1 < n_it) {
+        if (nxt.rows_valid == T) load_full(nxt, (unsigned)(((i + 1) & 1) * G::IMG), CluInt<0>{}, CluInt<G::WPIECES>{});
+        else load_pieces(nxt, (unsigned)(((i + 1) & 1) * G::IMG), 0, G::WPIECES);
+      }
+      if constexpr (!QX) {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __syncthreads();   // the partial logits are visible
+      }
       sigmoid_part(cur, gown, i, p0, p1, other_half());
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      __syncthreads();   // G of tile i is visible
+      __syncthreads();   // G of tile i is visible; the image of updated weights has been read
       // ---- Two jobs are left: grad_X (matrix instructions) and grad_W with the update (vector instructions).  The two wavefronts
       //      of a SIMD can take them in opposite order, each in the gaps of the other, or in step.  Measured in step against
       //      opposite, us a step, 131 K labels, batches of 32 / 64:
@@ -917,11 +928,12 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
   // the last tile's image; prev is the tile of the last iteration (cluster of one) or a repetition of it (the iteration
   // behind the last tile)
   if (!aborted && n_it > 0) store_out(C > 1 ? prev2 : prev);
+  if (C == 1 && v == 0 && lid == 0) p.xcc[blockIdx.x] = (int)(__builtin_amdgcn_s_getreg((3 << 11) | 20) & 15);   // (at the start it costs spills)
 #undef p
 }
 
 // The variants, one translation unit per arithmetic (bf16 weights; e4m3 weights with bf16 products; e4m3 with FP8 logits).
-// c: workgroups of a cluster (1, 2, 4, 8; FP8 logits: 2, 4, 8), nbk: 16-row batch blocks of a member (4, or 2 with c = 1).
+// c: workgroups of a cluster (1, 2, 4, 8), nbk: 16-row batch blocks of a member (4, or 2 with c = 1).
 typedef void (*clu_kernel_t)(const ClusterParams);
 struct ClusterVariant { clu_kernel_t fn; int lds; };
 ClusterVariant cluster_variant_bf16(int c, int nbk, int round_mode);
@@ -944,16 +956,14 @@ void cluster_set_lds_fp8();
 #define CLU_CAT2(a, b) a##b
 #define CLU_CAT(a, b) CLU_CAT2(a, b)
 ClusterVariant CLU_CAT(cluster_variant_, CLU_VARIANT)(int c, int nbk, int round_mode) {
-#if !CLU_QX
   if (c == 1 && nbk == 2) CLU_PICK(1, 2);
   if (c == 1) CLU_PICK(1, 4);
-#endif
   if (c == 2) CLU_PICK(2, 4);
   if (c == 4) CLU_PICK(4, 4);
   CLU_PICK(8, 4);
 }
 void CLU_CAT(cluster_set_lds_, CLU_VARIANT)() {   // opt in to the LDS size, once per device
-  for (int c = CLU_QX ? 2 : 1; c <= 8; c *= 2)
+  for (int c = 1; c <= 8; c *= 2)
     for (int nbk = c == 1 ? 2 : 4; nbk <= 4; nbk += 2)
       for (int mode = 0; mode < 3; mode++) {
         const ClusterVariant v = CLU_CAT(cluster_variant_, CLU_VARIANT)(c, nbk, mode);

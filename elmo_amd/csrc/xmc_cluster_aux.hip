@@ -6,11 +6,18 @@ namespace xmc {
 
 // members of a cluster for a batch, and 16-row batch blocks of a member.  64 rows per member fill the registers; a batch
 // of up to 32 rows takes half of them.
-inline int cluster_size(int batch, bool fp8_logits) {
-  const int c = batch <= 64 ? 1 : batch <= 128 ? 2 : batch <= 256 ? 4 : 8;
-  return fp8_logits && c < 2 ? 2 : c;
-}
-inline int cluster_blocks(int batch, bool fp8_logits) { return !fp8_logits && batch <= 32 ? 2 : 4; }
+inline int cluster_size(int batch) { return batch <= 64 ? 1 : batch <= 128 ? 2 : batch <= 256 ? 4 : 8; }
+inline int cluster_blocks(int batch) { return batch <= 32 ? 2 : 4; }
+
+// Where the launches of a step keep what they pass on to one another.
+struct ClusterPlace {
+  unsigned char* xq; unsigned short* xt;   // operand images of X
+  unsigned* keys; int* flags; int* xcc;    // sorted positives (MAX_POS per 256 batch rows); CLU_FLAG_INTS counters; XCC ids
+  float* gx;                               // grad_X of the segments before (label spaces of several segments)
+  int* tile_ptr; size_t tp_stride;
+  unsigned char* exch; floatx4* partial;
+  int* err; int* sticky;
+};
 
 // workspace of the cluster path (byte offsets, 256-byte aligned); the first 256 bytes hold the error words
 constexpr size_t TW_ERR = 0;        // int: error word of the last step; next int: the error words of all steps, OR-ed
@@ -18,7 +25,7 @@ constexpr size_t TW_HEAD = 256;
 struct ClusterLayout { size_t xq, xt, keys, flags, xcc, gx, tile_ptr, tp_stride, exch, partial, bytes; int slots; };
 inline ClusterLayout cluster_layout(int num_chunks, int rows_per_chunk, int batch) {
   ClusterLayout l;
-  const int c = cluster_size(batch, true);   // (what a cluster of one would need fits as well)
+  const int c = batch <= 64 ? 2 : cluster_size(batch);   // (what a cluster of one needs fits as well)
   const size_t bp = (size_t)c * 64, pairs = (bp + 255) / 256;
   auto up = [](size_t b) { return (b + 255) / 256 * 256; };
   l.xq = TW_HEAD;
@@ -112,7 +119,7 @@ __global__ __launch_bounds__(256) void cluster_prep_kernel(const ClusterPrep p, 
 //   add: continue from gx_total;  final: write grad_X (with the dropout's backward) instead of gx_total
 struct ClusterReduce {
   const floatx4* partial; int c, nbk, nclusters, ntiles, tpc, nchunks, flush;
-  const int* xcc; int* err; int* failure_word;
+  const int* xcc; int* err; int* sticky; int* failure_word;
   float* gx_total; int add, final_out, batch;
   unsigned short* gx_bf16; float* gx_f32;
 };
@@ -125,7 +132,7 @@ __global__ __launch_bounds__(CLU_RW * 64) void cluster_reduce_kernel(const Clust
         if (r.xcc[((tid >> 3) * r.c + m) * 8 + (tid & 7)] != r.xcc[(tid >> 3) * r.c * 8 + (tid & 7)])
           __hip_atomic_fetch_or(r.err, 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
-    if (tid == 0) report_step_error(r.err, r.err + 1, r.failure_word);
+    if (tid == 0) report_step_error(r.err, r.sticky, r.failure_word);
   }
   __shared__ floatx4 sh[CLU_RW][64];
   const int pslot = r.nbk * 6 * 8 * 64;

@@ -63,6 +63,17 @@ def test_one_pass_step_matches_the_oracle(gpu, kind, nc, rows, batch, mode):
     check_gx(gf.cpu().numpy(), g.float().cpu().numpy(), ref_gx)
 
 
+@pytest.mark.parametrize("nc,rows,batch,mode", [
+    (1, 16, 16, "sr_fast"),                  # one partial tile, 32-row slices
+    (3, 80, 32, "sr_philox"),                # a tile and a quarter to a chunk
+    (5, 4112, 33, "rtn"),                    # 64-row slices, more tiles than clusters
+    (2, 9232, 64, "sr_philox"),              # one to three tiles to a cluster
+    (2, 16400, 24, "sr_fast"),
+])
+def test_one_pass_step_with_fp8_logits_in_clusters_of_one(gpu, nc, rows, batch, mode):
+    test_one_pass_step_matches_the_oracle(gpu, "fp8", nc, rows, batch, mode)
+
+
 def test_one_pass_step_gives_up_cleanly(gpu):
     """A polling limit of 0, set from the host: a wait that is not satisfied at once ends the workgroup's walk.  Every kernel
     ends, the error words say so, no weight is updated from missing data, the layer raises, and the next step is clean."""
