@@ -45,6 +45,8 @@ def load():
     lib.xmc_error_string.argtypes = [i32]
     lib.xmc_workspace_bytes.restype = sz
     lib.xmc_workspace_bytes.argtypes = [i32, i32]
+    lib.xmc_workspace_bytes_ex.restype = sz
+    lib.xmc_workspace_bytes_ex.argtypes = [i32, i32, i32]
     lib.xmc_fp8_step.restype = i32
     lib.xmc_fp8_step.argtypes = [ctypes.POINTER(vp), i32, i32, vp, i32, i32, vp, i32, f32,
                                  ctypes.POINTER(ctypes.c_uint32), i32, f32, f32, vp, vp, vp, sz, vp]

@@ -197,6 +197,29 @@ int forward_launch(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, 
   return launch_status();
 }
 
+// Whether a true-FP8 step of at most 64 batch rows takes the one-pass form in clusters of one (xmc_cluster.hip) rather than the
+// fused kernel (xmc_fp8_role.hip).  The fused kernel computes 128 batch rows whatever the batch, and the four workgroups of a quad
+// wait for one another; a cluster of one computes 32 or 64 rows and waits for nobody, but walks whole tiles of 64 labels, one per
+// compute unit at a time, and stores a grad_X sum per workgroup.  So it needs tiles enough: few of them leave compute units idle (a
+// quad takes a tile in a quarter of the time), and the sums of 64 rows are as much memory traffic as 4 tiles.  With Philox both are
+// bound by the same vector work, and the uneven last round counts for more.  us a step, fused / one pass, at 16 K, 28 K, 65 K, 131 K,
+// 300 K, 1 M labels:
+//   32 rows, nearest  28/33  35/28  50/38   81/56  174/107   597/327     Philox  40/40  54/52  95/86  171/163  361/327  1156/1032
+//            sr_fast  29/33  35/30  52/41   84/63  172/118   585/362
+//   64 rows, nearest  32/39  36/36  52/47   81/68  177/125   593/375     Philox  44/47  56/61  97/94  172/176  365/345  1164/1068
+//            sr_fast  33/39  38/38  54/51   86/75  173/139   558/423
+// (weights and grad_X are the same to the bit.)  In tiles per compute unit the lines lie at 1.5 and 4 for 32 and 64 rows, with Philox
+// at 4 and 12.
+bool small_batch_one_pass(int batch, long long tiles, int round_mode, int cus) {
+  const bool philox = round_mode == XMC_ROUND_SR_PHILOX;
+  return batch <= 32 ? 2 * tiles >= (philox ? 8 : 3) * (long long)cus : batch <= 64 && tiles >= (philox ? 12 : 4) * (long long)cus;
+}
+// Its places in the fused step's workspace: the grad_X sums from WS_PARTIAL on (32 rows: as many bytes as the fused kernel's; 64 rows:
+// twice that, which only workspaces of xmc_workspace_bytes_ex hold), then the first key of every tile.
+constexpr size_t one_pass_partial(int batch) { return (size_t)CLU_MAXWG * CluGeom<CLU_E4M3, 1, 1, 2>::PSLOT * 16 * (batch <= 32 ? 1 : 2); }
+size_t one_pass_end(int batch, size_t tiles) { return (WS_PARTIAL + one_pass_partial(batch) + (tiles + 1) * 4 + 255) / 256 * 256; }
+static_assert(QF_WORDS - QF_CNT2 >= CLU_FLAG_INTS && WS_PARTIAL + one_pass_partial(32) <= WS_EXCH, "one-pass step in the fused step's workspace");
+
 }  // namespace
 
 extern "C" {
@@ -229,6 +252,14 @@ size_t xmc_workspace_bytes(int num_chunks, int rows_per_chunk) {
   // 32-byte tile descriptors, one run per quad (up to MAX_WG / 4 runs, each rounded up to whole entries; two tables with a
   // compensated head)
   return WS_DESC + (tiles + MAX_WG / 2) * 32;
+}
+
+size_t xmc_workspace_bytes_ex(int num_chunks, int rows_per_chunk, int batch) {
+  const size_t base = xmc_workspace_bytes(num_chunks, rows_per_chunk);
+  if (base == 0) return 0;
+  const size_t tiles = (size_t)num_chunks * ((rows_per_chunk + TL - 1) / TL);
+  const size_t one = one_pass_end(batch, tiles);
+  return small_batch_one_pass(batch, (long long)tiles, XMC_ROUND_RTN, MAX_WG) && one > base ? one : base;
 }
 
 int xmc_fp8_step(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, const void* x_bf16, int batch,
@@ -349,6 +380,15 @@ static int fused_step(void* const* chunk_ptrs, int num_chunks, int rows_per_chun
   const int num_tiles = num_chunks * tiles_per_chunk;
   const int n_pad = (nnz + 63) / 64 * 64;   // whole blocks of the sort
 
+  // (the one-pass form has neither scales nor decay; a workspace that does not hold its sums keeps the fused kernel)
+  if (kahan_type == 0 && weight_decay == 0.f && scale_w == 1.f && scale_x == 1.f && small_batch_one_pass(batch, num_tiles, round_mode, di.cus) &&
+      workspace_bytes >= one_pass_end(batch, (size_t)num_tiles)) {
+    int* flags = (int*)(ws + WS_FLAGS);
+    const ClusterPlace at = {ws + WS_XQ, (unsigned short*)(ws + WS_XT), (unsigned*)(ws + WS_KEYS), flags + QF_CNT2, flags + QF_XCC, nullptr,
+                             (int*)(ws + WS_PARTIAL + one_pass_partial(batch)), 0, nullptr, (floatx4*)(ws + WS_PARTIAL), flags + QF_ERR, flags + QF_STICKY};
+    return cluster_step(chunk_ptrs, num_chunks, rows_per_chunk, rows_per_chunk, W_E4M3, x_bf16, batch, labels_coo, nnz, lr, seeds, round_mode, 1, 1,
+                        dp, grad_x_bf16, grad_x_f32, at, true, di.cus, di.failure_word, stream);
+  }
   {
     QuadParams p;
     for (int c = 0; c < MAX_CHUNKS; c++) {

@@ -47,15 +47,16 @@ def _chunk_array(chunks):
     return (ctypes.c_void_p * len(chunks))(*[c.data_ptr() for c in chunks]), rows
 
 
-def workspace_bytes(num_chunks, rows_per_chunk):
-    n = _lib.load().xmc_workspace_bytes(num_chunks, rows_per_chunk)
+def workspace_bytes(num_chunks, rows_per_chunk, batch=MAX_BATCH // 2):
+    """Bytes for steps of `batch` rows (the default: of any batch); they also serve every other batch, if perhaps by a slower form."""
+    n = _lib.load().xmc_workspace_bytes_ex(num_chunks, rows_per_chunk, batch)
     if n == 0:
         raise _lib.XmcError("unsupported chunk geometry")
     return n
 
 
-def alloc_workspace(num_chunks, rows_per_chunk, device):
-    ws = torch.empty(workspace_bytes(num_chunks, rows_per_chunk), dtype=torch.uint8, device=device)
+def alloc_workspace(num_chunks, rows_per_chunk, device, batch=MAX_BATCH // 2):
+    ws = torch.empty(workspace_bytes(num_chunks, rows_per_chunk, batch), dtype=torch.uint8, device=device)
     # the sticky error word is only ever OR-ed into by the kernels: it starts at zero
     off = step_sticky_error_offset()
     ws[off:off + 4].zero_()
@@ -102,7 +103,7 @@ def fp8_step(chunks, x, labels, lr, seeds=None, round_mode="rtn", scale_w=1.0, s
     kept = workspace is not None
     if not kept:
         _unkept_errors(x.device).check()
-        workspace = alloc_workspace(nc, rows, x.device)
+        workspace = alloc_workspace(nc, rows, x.device, batch)
     if grad_out is None:
         grad_out = torch.empty(batch, feat, dtype=torch.bfloat16, device=x.device)
     gf = torch.empty(batch, feat, dtype=torch.float32, device=x.device) if want_f32 else None
@@ -143,7 +144,7 @@ def fp8_kahan_step(chunks, kahan, num_head, x, labels, lr, seeds=None, round_mod
     kept = workspace is not None
     if not kept:
         _unkept_errors(x.device).check()
-        workspace = alloc_workspace(nc, rows, x.device)
+        workspace = alloc_workspace(nc, rows, x.device, MAX_BATCH)
     if grad_out is None:
         grad_out = torch.empty(batch, feat, dtype=torch.bfloat16, device=x.device)
     gf = torch.empty(batch, feat, dtype=torch.float32, device=x.device) if want_f32 else None
@@ -176,7 +177,7 @@ def fp8_forward(chunks, x, num_labels, scale_w=1.0, scale_x=1.0, workspace=None)
     arr, rows = _chunk_array(chunks)
     nc = len(chunks)
     if workspace is None:
-        workspace = alloc_workspace(nc, rows, x.device)
+        workspace = alloc_workspace(nc, rows, x.device, MAX_BATCH)
     total = xb.shape[0]
     # like the reference, which returns outlogit[:, :num_labels] of the concatenated chunk outputs, the result is a
     # view of a [B, num_chunks * rows] buffer: rows start on 32-byte boundaries, which the kernel's stores want
@@ -224,7 +225,7 @@ def fp8_forward_topk(chunks, x, num_labels, k, scale_w=1.0, scale_x=1.0, workspa
     arr, rows = _chunk_array(chunks)
     nc = len(chunks)
     if workspace is None:
-        workspace = alloc_workspace(nc, rows, x.device)
+        workspace = alloc_workspace(nc, rows, x.device, MAX_BATCH)
     total = xb.shape[0]
     vals = torch.empty(total, k, dtype=torch.bfloat16, device=x.device)
     idx = torch.empty(total, k, dtype=torch.int64, device=x.device)

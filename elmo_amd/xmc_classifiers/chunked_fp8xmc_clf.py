@@ -92,8 +92,9 @@ class Fp8XMCBCEChunkedLayer(nn.Module):
         self.iteration = 0
         self.grad_input = None
         # all scratch memory of the step comes from the torch allocator (so that max_memory_allocated sees it)
+        batch = int(_opt(cfg.data, "batch_size", ops.MAX_BATCH // 2))
         self._workspace = (None if self._other_width else
-                           ops.alloc_workspace(self.num_chunks, self.num_labels_i, self.device))
+                           ops.alloc_workspace(self.num_chunks, self.num_labels_i, self.device, batch))
         self._last = None            # workspace of the last step: its error word is defined from then on
         # batches of more than 128 rows (up to 512) also run on the tiled step, with the true-FP8 arithmetic
         self._max_batch = int(_opt(cfg.data, "batch_size", ops.MAX_BATCH))

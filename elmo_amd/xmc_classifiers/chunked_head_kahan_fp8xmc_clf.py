@@ -75,7 +75,7 @@ class Fp8XMCBCEChunkedHeadKahanLayer(nn.Module):
         self.loss = torch.tensor(0.0, device=self.device)
         self.iteration = 0
         self.grad_input = None
-        self._workspace = None if self._other_width else ops.alloc_workspace(self.num_chunks, self.num_labels_i, self.device)
+        self._workspace = None if self._other_width else ops.alloc_workspace(self.num_chunks, self.num_labels_i, self.device, ops.MAX_BATCH)
         self._tiled_workspace = (ops.alloc_tiled_workspace(self.num_chunks, self.num_labels_i, self.device, ops.MAX_BATCH,
                                                            features) if self._tiled else None)
         self._errors = StepErrors(self.device, ops.sticky_error_words(self._workspace, self._tiled_workspace))

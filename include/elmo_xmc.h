@@ -52,6 +52,11 @@ const char* xmc_error_string(int status);
  * Returns 0 for an unsupported shape. */
 size_t xmc_workspace_bytes(int num_chunks, int rows_per_chunk);
 
+/* The same, with room for the form that is the fastest at steps of `batch` rows (no counterpart in the
+ * reference): 24 MiB more for 33 to 64 rows of a large label space.  In a workspace of xmc_workspace_bytes these take the
+ * other form; the results are the same. */
+size_t xmc_workspace_bytes_ex(int num_chunks, int rows_per_chunk, int batch);
+
 /* One training step over all chunks: logits, sigmoid minus sparse targets, grad_X, grad_W and the in-place
  * SGD update (chunked_fp8xmc_clf.py:91-123).
  *   chunk_ptrs      host array of num_chunks device pointers, each [rows_per_chunk, 768] e4m3fn, updated in place

@@ -74,6 +74,44 @@ def test_one_pass_step_with_fp8_logits_in_clusters_of_one(gpu, nc, rows, batch, 
     test_one_pass_step_matches_the_oracle(gpu, "fp8", nc, rows, batch, mode)
 
 
+@pytest.mark.parametrize("nc,tiles,batch,mode,dropout", [
+    (1, 384, 16, "sr_fast", 0.0),            # the first size that takes the one-pass form (256 compute units), 32-row slices
+    (3, 128, 32, "rtn", 0.3),                # the same, a partial tile at the end of every chunk
+    (2, 512, 32, "sr_philox", 0.0),
+    (4, 256, 48, "sr_fast", 0.3),            # 64-row slices
+    (4, 256, 64, "rtn", 0.0),
+    (3, 1024, 64, "sr_philox", 0.0),
+])
+def test_small_batches_take_the_one_pass_form_with_the_same_results(gpu, nc, tiles, batch, mode, dropout):
+    """xmc_fp8_step on both of its forms: a batch of at most 64 rows, and the same batch with rows of zeros up to 80, which
+    takes the fused kernel.  The added rows contribute exact zeros, so the weights
+    agree to the bit."""
+    import torch
+    from elmo_amd import ops
+    rows = 64 * tiles - 48
+    seeds = None if mode == "rtn" else [5 + 3 * c for c in range(nc)]
+    g = torch.Generator(device=gpu).manual_seed(900 + batch)
+    chunks = [torch.randn(rows, 768, generator=g, device=gpu).mul_(0.05).to(torch.float8_e4m3fn) for _ in range(nc)]
+    padded = [c.clone() for c in chunks]
+    x = torch.randn(batch, 768, generator=g, device=gpu).to(torch.bfloat16)
+    x80 = torch.cat([x, torch.zeros(80 - batch, 768, dtype=torch.bfloat16, device=gpu)])
+    n = 9 * batch
+    labels = torch.stack([torch.arange(n, device=gpu) % batch, torch.randint(0, nc * rows, (n,), generator=g, device=gpu)], 1)
+    edges = [[batch - 1, nc * rows - 1], [0, 0], [0, 0], [0, rows - 1], [-1, 3], [0, nc * rows]]        # (the last two are ignored)
+    labels = torch.cat([labels, torch.tensor(edges, device=gpu)]).to(torch.int32).contiguous()
+    ws = ops.alloc_workspace(nc, rows, gpu)
+    off = ops.step_sticky_error_offset()
+    for _ in range(2):                       # (the second step on what the first left in the workspace)
+        g1, f1 = ops.fp8_step(chunks, x, labels, 0.05, seeds=seeds, round_mode=mode, workspace=ws, want_f32=True, dropout_p=dropout, dropout_seed=7)
+        g2, f2 = ops.fp8_step(padded, x80, labels, 0.05, seeds=seeds, round_mode=mode, workspace=ws, want_f32=True, dropout_p=dropout, dropout_seed=7)
+        for a, b in zip(chunks, padded):
+            assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+        # two groupings of one fp32 sum (of at most 256 partial sums behind one another): 2^8 roundings of 2^-24 at most
+        tol = 2 ** -16 * f2[:batch].abs().max().item()
+        assert (f1 - f2[:batch]).abs().max().item() <= tol and torch.allclose(g1.float(), g2[:batch].float(), rtol=2 ** -7, atol=tol)
+        assert ops.step_error_word(ws, nc, rows) == 0 and int(ws[off:off + 4].view(torch.int32).item()) == 0
+
+
 def test_one_pass_step_gives_up_cleanly(gpu):
     """A polling limit of 0, set from the host: a wait that is not satisfied at once ends the workgroup's walk.  Every kernel
     ends, the error words say so, no weight is updated from missing data, the layer raises, and the next step is clean."""
