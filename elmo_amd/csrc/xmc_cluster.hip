@@ -136,7 +136,7 @@ __device__ __forceinline__ void clu_lds_load16_l2(const unsigned char* base, uns
 // 4 bytes per lane at device scope into LDS at ldsoff + 4 * lane
 __device__ __forceinline__ void clu_lds_load4_l2(const void* g, unsigned ldsoff_) {
   const unsigned ldsoff = __builtin_amdgcn_readfirstlane(ldsoff_);
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, off sc1" : : "s"(ldsoff), "v"(g) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off sc1" : : "s"(ldsoff), "v"(g) : "memory", "m0");
 }
 
 __device__ __forceinline__ bf16x8 clu_widen8(intx2 raw) {   // eight e4m3 codes as bf16, exact

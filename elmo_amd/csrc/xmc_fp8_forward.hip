@@ -83,7 +83,7 @@ __device__ __forceinline__ void fwd_issue_tile(const unsigned char* gtile, int r
     for (int j = 0; j < FT / WAVES; j++) {
       const int row = FT / WAVES * v + j, src = min(row, rows_valid - 1);   // rows past the end re-read the last valid one
       const unsigned ldsoff = __builtin_amdgcn_readfirstlane(lds_off + (unsigned)(row * WS));
-      asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(ldsoff), "v"(lane * 16), "s"(gtile + src * D) : "memory", "m0");
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(ldsoff), "v"(lane * 16), "s"(gtile + src * D) : "memory", "m0");
     }
   }
 }

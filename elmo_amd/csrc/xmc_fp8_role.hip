@@ -544,12 +544,16 @@ __global__ __launch_bounds__(QNT, 1) void fp8_step_role_kernel(const QuadParams 
             // written through (system scope): the updated weights are not read again by this launch, and as ordinary
             // stores they push the exchanged G tiles and the weight tiles between their two fetches out of the XCD's
             // L2 (reads from memory 1.34 instead of 1.12 times the weights); same speed either way
-            asm volatile("global_store_dwordx4 %0, %1, %2 sc0 sc1" : : "v"(off), "v"(ov), "s"(qp_base) : "memory");
+            // (the registers of a store of more than 8 bytes may not be written by the next vector instruction: it is the
+            // address of the next read here, and with the other wavefront at a higher priority a few addresses in a hundred
+            // thousand were stored for weights.  The compiler keeps that distance only from stores it knows, and a
+            // waiting instruction in between is none.)
+            asm volatile("global_store_dwordx4 %0, %1, %2 sc0 sc1\n\ts_nop 1" : : "v"(off), "v"(ov), "s"(qp_base) : "memory");
           } else {
             // rows past the end of the chunk go to a place nobody reads (the padding behind an exchange slot), so that
             // the wavefront issues the same number of memory operations for every tile
             unsigned char* dst = row < qp_base_valid ? qp_base + off : exq + (size_t)(m * 2) * QG_BYTES + RG_BYTES + a * 1024 + lane * 16;
-            asm volatile("global_store_dwordx4 %0, %1, off ; clamped rows" : : "v"(dst), "v"(ov) : "memory");
+            asm volatile("global_store_dwordx4 %0, %1, off\n\ts_nop 1" : : "v"(dst), "v"(ov) : "memory");
           }
         }
       }

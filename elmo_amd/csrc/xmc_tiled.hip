@@ -149,7 +149,7 @@ template <int WT, int DD> struct TlgGeom {
 // assembly: the compiler neither orders later LDS accesses behind it nor waits for it; completion is enforced by hand.
 __device__ __forceinline__ void t_lds_load16(const unsigned char* g, unsigned ldsoff_) {
   const unsigned ldsoff = __builtin_amdgcn_readfirstlane(ldsoff_);
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(ldsoff), "v"(g) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(ldsoff), "v"(g) : "memory", "m0");
 }
 
 // Vector memory operations retire in order.  Per sub-tile a wavefront issues its loads of the sub-tile two steps ahead
