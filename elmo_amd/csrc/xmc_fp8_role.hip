@@ -58,6 +58,7 @@ constexpr int RLDS_O = RLDS_C + RC_RING * QWC_BYTES;
 constexpr int RLDS_G = RLDS_O + RO_RING * RO_BYTES;
 constexpr int RLDS_R = RLDS_G + RG_BUF * RG_BYTES;
 constexpr int RLDS_M = RLDS_R + RR_RING * RROW_BYTES;   // per A wavefront two snapshots of four counters (32 bytes); at +128 two abort words
+constexpr int RLDS_T = RLDS_M + 160;                    // what the B wavefronts need to know of a tile: two entries of 16 bytes
 constexpr int RLDS_BYTES = RLDS_M + 256;
 // tiles-published counters: flags[p.cnt_base + quad*16 + member*4 + A wavefront]
 
@@ -265,6 +266,12 @@ __global__ __launch_bounds__(QNT, 1) void fp8_step_role_kernel(const QuadParams 
     return __builtin_bit_cast(bf16x8, shortx8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]});
   };
 
+  // hash part, seed and first row of the tile of an iteration, for the B wavefronts (slot: iteration & 1)
+  typedef __attribute__((address_space(3))) intx4 lds_intx4;
+  auto pass_on = [&](int slot, const QTile& q) {
+    if (lane == 0) *(lds_intx4*)(lds + RLDS_T + slot * 16) = intx4{(int)(q.label0 * (unsigned)(D / 4) * 0x9E3779B1u + q.seed), (int)q.seed, q.row0, 0};
+  };
+
   if (v < 4) {
     // =========================================================================================== A wavefronts
     const int a = v;
@@ -468,7 +475,10 @@ __global__ __launch_bounds__(QNT, 1) void fp8_step_role_kernel(const QuadParams 
       }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the stores of G included
-    if (lane == 0 && n_it > 0) __hip_atomic_store(myflag, min(RQ, n_it), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // (a store that stays in the XCD's L2, where the quad's members look for it, as the G tiles do.  At agent scope it is written
+    // through to memory, and the loop's waits, which count in order, wait for that: 670 K labels, batch 128, nearest 398 us a step
+    // instead of 353; with a compensated head, nearest 527 instead of 478, sr_fast 525 instead of 496; 131 K, batch 96, 86.3 / 85.3)
+    if (lane == 0 && n_it > 0) __hip_atomic_store(myflag, min(RQ, n_it), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     if (n_it > 0) {
       wait_published(1, 0, 1);   // an expiry here is seen behind the first barrier of the loop (slot 1 = "iteration -1")
       gather(0, 0);
@@ -478,6 +488,7 @@ __global__ __launch_bounds__(QNT, 1) void fp8_step_role_kernel(const QuadParams 
 
     // descriptors of the next iteration: the tile of its stage A (whose columns it also fetches), the tile whose rows it
     // fetches and the tile of its share of stage B; loaded one iteration ahead through the scalar path
+    if (a == 0) pass_on(0, q_desc_full(cdesc, tile_at(0)));
     QTile qa_n = q_desc_full(cdesc, tile_at(RQ)), qr_n = q_desc_head(cdesc, tile_at(RQ + RR_RING - 1)), qb_n = q_desc_full(cdesc, tile_at(0));
     unsigned char* qp_base = nullptr;   // the tile of the iteration before: base pointer and valid rows
     int qp_base_valid = 0;
@@ -487,9 +498,10 @@ __global__ __launch_bounds__(QNT, 1) void fp8_step_role_kernel(const QuadParams 
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       __syncthreads();
       const QTile qa = qa_n, qr = qr_n, qb = qb_n;
-      const int abort_word = *(const lds_int*)(lds + abort_base + ((i + 1) & 1) * 4);
+      int abort_word = *(const lds_int*)(lds + abort_base + ((i + 1) & 1) * 4);
       // the counters as they were in the middle of the iteration before
-      const intx4 fl = *(const __attribute__((address_space(3))) intx4*)(lds + RLDS_M + a * 32 + ((i + 1) & 1) * 16);
+      intx4 fl = *(const __attribute__((address_space(3))) intx4*)(lds + RLDS_M + a * 32 + ((i + 1) & 1) * 16);
+      asm volatile("" : "+v"(abort_word), "+v"(fl));   // (one wait for both)
       if (__builtin_amdgcn_readfirstlane(abort_word) != 0) break;
       if (i + 1 < n_it) {
         const int fmin = min(min((int)__builtin_amdgcn_readfirstlane(fl.x), (int)__builtin_amdgcn_readfirstlane(fl.y)),
@@ -558,6 +570,7 @@ __global__ __launch_bounds__(QNT, 1) void fp8_step_role_kernel(const QuadParams 
         }
       }
       qp_base = qb.base; qp_base_valid = qb.rows_valid;
+      if (a == 0) pass_on((i + 1) & 1, qb_n);
       // ---- the update of those blocks, with the rows of position i + RQ + 2 (the only loads that miss the L2) requested
       //      between its pieces
       {
@@ -592,7 +605,7 @@ __global__ __launch_bounds__(QNT, 1) void fp8_step_role_kernel(const QuadParams 
           default: asm volatile("s_waitcnt vmcnt(9)" ::: "memory"); break;
         }
       }
-      if (lane == 0) __hip_atomic_store(myflag, min(i + RQ, n_it), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (lane == 0) __hip_atomic_store(myflag, min(i + RQ, n_it), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
       sa = sa == RR_RING - 1 ? 0 : sa + 1;
       w0 = w0 == RC_RING - 1 ? 0 : w0 + 1;
     }
@@ -626,19 +639,16 @@ __global__ __launch_bounds__(QNT, 1) void fp8_step_role_kernel(const QuadParams 
     if (k + 1 < RQ && k + 1 >= RR_RING) __syncthreads();
   }
 
-  QTile q_n = q_desc_full(cdesc, tile_at(0)), q_p = q_n;
   int w0 = 0;   // i % RC_RING
   int n_done = 0;
   for (int i = 0; i < n_it; i++) {
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __syncthreads();
-    const QTile q = q_n;
     const unsigned oimg = (unsigned)(RLDS_O + (i & 1) * RO_BYTES);
     const unsigned wc = (unsigned)(RLDS_C + w0 * QWC_BYTES);
     const unsigned gb = (unsigned)(RLDS_G + (i & 1) * RG_BYTES);
     const unsigned gxa = gb + ga_lane, gwl = gb + bl.bg_lane, gwh = gb + (bl.bg_lane ^ 128u);
     const unsigned wtr = wc + wtr_lane, wrow = wc + bl.wrow_lane;
-    const unsigned hash_tile = q.label0 * (unsigned)(D / 4) * 0x9E3779B1u + q.seed;
 
     // The tile is a sequence of 16 + 4 NBB steps of one LDS operand and three matrix instructions each.  The first
     // 8 NBB alternate:
@@ -662,6 +672,9 @@ __global__ __launch_bounds__(QNT, 1) void fp8_step_role_kernel(const QuadParams 
       }
     };
     const int abort_word = *(const lds_int*)(lds + abort_base + ((i + 1) & 1) * 4);
+    // (the tile's descriptor comes through LDS: a scalar load in this wavefront, whose every wait is for LDS reads, stood in front of
+    // the barrier with its whole latency; 131 K labels, batch 96, 88.1 us a step with it, 86.4 without)
+    const intx4 qd = *(const lds_intx4*)(lds + RLDS_T + (i & 1) * 16);
 #pragma unroll
     for (int k = 0; k < PD; k++) request(k);
     intx2 wraw[2][3];
@@ -671,6 +684,10 @@ __global__ __launch_bounds__(QNT, 1) void fp8_step_role_kernel(const QuadParams 
       for (int nn = 0; nn < 3; nn++)
         wraw[ks2][nn] = __builtin_amdgcn_ds_read_tr8_b64_v2i32((__attribute__((address_space(3))) intx2*)(lds + wtr + ks2 * 32 * QWS + nn * 16));
     if (__builtin_amdgcn_readfirstlane(abort_word) != 0) break;
+    QTile q = {};
+    const unsigned hash_tile = MODE == ROUND_SR_FAST ? (unsigned)__builtin_amdgcn_readfirstlane(qd.x) : 0u;
+    if (MODE == ROUND_SR_PHILOX) q.seed = (unsigned)__builtin_amdgcn_readfirstlane(qd.y);
+    if (MODE == ROUND_SR_PHILOX || KT != 0) q.row0 = __builtin_amdgcn_readfirstlane(qd.z);
     n_done = i + 1;
     bf16x8 wb[2][3];
 
@@ -747,8 +764,6 @@ __global__ __launch_bounds__(QNT, 1) void fp8_step_role_kernel(const QuadParams 
 #pragma unroll
       for (int c = 0; c < 8; c++) r_update_piece<MODE, WD, KT>(c, 3, aa[1], wq[1], t, hs, outw, knew, bl, q, hash_tile, p.lr_eff, p.wd_eff, l16, lds, oimg, kb[1], p.kahan, p.num_head);
     }
-    q_p = q;
-    q_n = q_desc_full(cdesc, tile_at(i + 1));
     w0 = w0 == RC_RING - 1 ? 0 : w0 + 1;
   }
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -757,6 +772,7 @@ __global__ __launch_bounds__(QNT, 1) void fp8_step_role_kernel(const QuadParams 
   // per lane, three per B wavefront (the A wavefronts, which store the other tiles' images one iteration later, have
   // left): chunk ch = (3s + jj) * 64 + lane is bytes 16 (ch % 12).. of row ch / 12.
   if (n_done > 0) {
+    const QTile q_p = q_desc_head(cdesc, tile_at(n_done - 1));
 #pragma unroll
     for (int jj = 0; jj < 3; jj++) {
       const int ch = (3 * s + jj) * 64 + lane, row = ch / 12;
