@@ -91,6 +91,13 @@ __device__ __forceinline__ void q_lds_load4_l2(const void* g, unsigned ldsoff) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off sc1" : : "s"(ldsoff), "v"(g) : "memory", "m0");
 }
 
+// a wave-uniform pointer as the scalar operand of inline assembly (under register pressure the compiler may hold it in vector registers)
+__device__ __forceinline__ unsigned char* q_uniform(unsigned char* p) {
+  const unsigned long long u = (unsigned long long)p;
+  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)u), hi = __builtin_amdgcn_readfirstlane((unsigned)(u >> 32));
+  return (unsigned char*)(((unsigned long long)hi << 32) | lo);
+}
+
 // eight e4m3 codes -> eight bf16 values (exact), two per instruction
 __device__ __forceinline__ bf16x8 q_fp8x8_to_bf16x8(intx2 raw) {
   bf16x2 c0 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(raw.x, 1.0f, false), c1 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(raw.x, 1.0f, true);

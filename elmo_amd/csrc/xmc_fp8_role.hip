@@ -445,46 +445,63 @@ __global__ __launch_bounds__(QNT, 1) void fp8_step_role_kernel(const QuadParams 
       *(uint2*)(dst + 512) = uint2{sb[1][0], sb[1][1]};
     };
 
-    // ---- prologue: rows and columns of the first RQ positions, their stage A, rows of the next two, G of position 0
+    // ---- prologue: rows and columns of the first RQ positions, their stage A, rows of the next two, G of position 0; all that
+    //      only as far as the sequence goes.  A launch spends 6 - 10 us here, most of them waiting for memory, so that nothing
+    //      waits for more than it needs: stage A for the rows (the columns, which come from the L2 behind them, land under it),
+    //      stage A of position 3 for its rows, and the gather of G(0) for no load at all.
 #pragma unroll
-    for (int k = 0; k < RR_RING; k++) rows_pieces(k, q_desc_head(cdesc, tile_at(k)));
-#pragma unroll
-    for (int k = 0; k < RQ; k++) {
-      const QTile t = q_desc_head(cdesc, tile_at(k));
-#pragma unroll
-      for (int s = 0; s < 4; s++) wcol_piece(k, t, s);
-    }
+    for (int k = 0; k < RR_RING; k++)
+      if (k < n_it) rows_pieces(k, q_desc_head(cdesc, tile_at(k)));
     // a wait the compiler knows of: without it, it takes the loads of xq above for outstanding wherever the loop below
     // uses them (it cannot see the waits written as inline assembly) and waits for all memory operations there
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();   // P1
-    // stage A of positions 0..RQ-1; the rows image of position k + RR_RING replaces that of position k behind a barrier
 #pragma unroll
-    for (int k = 0; k < RQ; k++) {
-      floatx4 z[2];
+    for (int k = 0; k < RQ; k++)
       if (k < n_it) {
-        stage_a_logits(k % RR_RING, z, [](int) {});
-        stage_a_finish(k, q_desc_full(cdesc, tile_at(k)), z);
+        const QTile t = q_desc_head(cdesc, tile_at(k));
+#pragma unroll
+        for (int s = 0; s < 4; s++) wcol_piece(k, t, s);
       }
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      __syncthreads();   // P2.k: every A wavefront has read the rows image
-      if (k + RR_RING < RQ + RR_RING - 1) rows_pieces(k % RR_RING, q_desc_head(cdesc, tile_at(k + RR_RING)));
-      if (k + 1 < RQ && k + 1 >= RR_RING) {   // the next stage A reads an image that was just requested
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-      }
-    }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the stores of G included
-    // (a store that stays in the XCD's L2, where the quad's members look for it, as the G tiles do.  At agent scope it is written
+    // (stays in the XCD's L2, where the quad's members look for it, as the G tiles do.  At agent scope it is written
     // through to memory, and the loop's waits, which count in order, wait for that: 670 K labels, batch 128, nearest 398 us a step
     // instead of 353; with a compensated head, nearest 527 instead of 478, sr_fast 525 instead of 496; 131 K, batch 96, 86.3 / 85.3)
-    if (lane == 0 && n_it > 0) __hip_atomic_store(myflag, min(RQ, n_it), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    auto publish = [&](int tiles) {
+      if (lane == 0) __hip_atomic_store(myflag, tiles, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    };
+    // stage A of positions 0..RQ-1; the rows image of position k + RR_RING replaces that of position k behind a barrier
+    static_assert(RQ == 4 && RR_RING == 3, "the waits below");
+#pragma unroll
+    for (int k = 0; k < RQ; k++) {
+      if (k >= n_it) continue;
+      if (k == RR_RING) {   // this stage A reads an image that was requested behind position 0
+        // (younger than its loads: two stores of G and the loads of a tile, twice)
+        if (n_it <= RR_RING + 2) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        else if (ra == 0) asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(10)" ::: "memory");
+        publish(1);
+        __syncthreads();   // P3
+      }
+      floatx4 z[2];
+      stage_a_logits(k % RR_RING, z, [](int) {});
+      stage_a_finish(k, q_desc_full(cdesc, tile_at(k)), z);
+      if (k < RR_RING && k + RR_RING < n_it) {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __syncthreads();   // P2.k: every A wavefront has read the rows image
+        rows_pieces(k, q_desc_head(cdesc, tile_at(k + RR_RING)));
+      }
+    }
     if (n_it > 0) {
+      if (n_it <= RR_RING) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the stores of G included
+        publish(n_it);
+      }
       wait_published(1, 0, 1);   // an expiry here is seen behind the first barrier of the loop (slot 1 = "iteration -1")
       gather(0, 0);
     }
     issue_snapshot(1);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (n_it > RR_RING) publish(min(RQ, n_it));
 
     // descriptors of the next iteration: the tile of its stage A (whose columns it also fetches), the tile whose rows it
     // fetches and the tile of its share of stage B; loaded one iteration ahead through the scalar path
@@ -510,10 +527,10 @@ __global__ __launch_bounds__(QNT, 1) void fp8_step_role_kernel(const QuadParams 
         gather(i + 1, (i + 1) & 1);
       }
       // ---- stage A of position i + RQ, the columns of the same tile requested between its matrix instructions
-      const bool do_a = i + RQ < n_it;
+      const bool do_a = i + RQ < n_it, do_r = i + RQ + RR_RING - 1 < n_it;   // (the sequence's end)
       const int wslot = w0 == 0 ? RC_RING - 1 : w0 - 1;   // (i + RQ) % RC_RING
       floatx4 z[2];
-      stage_a_logits(sa, z, [&](int ks) { if (ks < 4) wcol_piece(wslot, qa, ks); });
+      if (do_a) stage_a_logits(sa, z, [&](int ks) { if (ks < 4) wcol_piece(wslot, qa, ks); });
       // the counters as they are now, for the next iteration; everything behind this point may stay in flight over the
       // barrier
       issue_snapshot(i);
@@ -560,7 +577,7 @@ __global__ __launch_bounds__(QNT, 1) void fp8_step_role_kernel(const QuadParams 
             // address of the next read here, and with the other wavefront at a higher priority a few addresses in a hundred
             // thousand were stored for weights.  The compiler keeps that distance only from stores it knows, and a
             // waiting instruction in between is none.)
-            asm volatile("global_store_dwordx4 %0, %1, %2 sc0 sc1\n\ts_nop 1" : : "v"(off), "v"(ov), "s"(qp_base) : "memory");
+            asm volatile("s_nop 4\n\tglobal_store_dwordx4 %0, %1, %2 sc0 sc1\n\ts_nop 1" : : "v"(off), "v"(ov), "s"(q_uniform(qp_base)) : "memory");
           } else {
             // rows past the end of the chunk go to a place nobody reads (the padding behind an exchange slot), so that
             // the wavefront issues the same number of memory operations for every tile
@@ -585,32 +602,33 @@ __global__ __launch_bounds__(QNT, 1) void fp8_step_role_kernel(const QuadParams 
           for (int c = 0; c < 8; c++) {
             constexpr int every = 2 * NBA;
             const int pc = (nb - NBB) * 8 + c;
-            if (pc % every == 0) rows_piece(rslot, qr, pc / every);
+            if (pc % every == 0 && do_r) rows_piece(rslot, qr, pc / every);
             r_update_piece<MODE, WD, 0>(c, nb, aa[nb - NBB], wq[nb - NBB], t, hs, outw, knew, bl, qb, hash_tile, p.lr_eff, p.wd_eff, l16, lds, oimg, nok, nullptr, 0);
           }
-        if (NBB == 4) rows_pieces(rslot, qr);
+        if (NBB == 4 && do_r) rows_pieces(rslot, qr);
       }
       // Loads and stores complete in order.  Waiting for all but the stores of G and the rows covers the gather, the
       // columns and the snapshot, all issued long before, and everything of the iteration before, whose stores of G can
       // now be published.
       {
-        const int cnt = (do_a ? 2 : 0) + (i > 0 ? 3 : 0) + (ra == 0 ? 4 : 3);
+        const int cnt = (do_a ? 2 : 0) + (i > 0 ? 3 : 0) + (do_r ? (ra == 0 ? 4 : 3) : 0);
         switch (cnt) {
-          case 3: asm volatile("s_waitcnt vmcnt(3)" ::: "memory"); break;
-          case 4: asm volatile("s_waitcnt vmcnt(4)" ::: "memory"); break;
-          case 5: asm volatile("s_waitcnt vmcnt(5)" ::: "memory"); break;
-          case 6: asm volatile("s_waitcnt vmcnt(6)" ::: "memory"); break;
-          case 7: asm volatile("s_waitcnt vmcnt(7)" ::: "memory"); break;
+          case 9: asm volatile("s_waitcnt vmcnt(9)" ::: "memory"); break;
           case 8: asm volatile("s_waitcnt vmcnt(8)" ::: "memory"); break;
-          default: asm volatile("s_waitcnt vmcnt(9)" ::: "memory"); break;
+          case 6: asm volatile("s_waitcnt vmcnt(6)" ::: "memory"); break;
+          case 5: asm volatile("s_waitcnt vmcnt(5)" ::: "memory"); break;
+          case 3: asm volatile("s_waitcnt vmcnt(3)" ::: "memory"); break;
+          case 2: asm volatile("s_waitcnt vmcnt(2)" ::: "memory"); break;
+          default: asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); break;
         }
       }
-      if (lane == 0) __hip_atomic_store(myflag, min(i + RQ, n_it), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      publish(min(i + RQ, n_it));
       sa = sa == RR_RING - 1 ? 0 : sa + 1;
       w0 = w0 == RC_RING - 1 ? 0 : w0 + 1;
     }
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");   // the last loads still target LDS
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __syncthreads();   // the last tile's updated weights are in LDS: the B wavefronts store them
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the last loads still target LDS
     return;
   }
 
@@ -634,10 +652,9 @@ __global__ __launch_bounds__(QNT, 1) void fp8_step_role_kernel(const QuadParams 
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();   // P1
 #pragma unroll
-  for (int k = 0; k < RQ; k++) {
-    __syncthreads();   // P2.k
-    if (k + 1 < RQ && k + 1 >= RR_RING) __syncthreads();
-  }
+  for (int k = 0; k < RR_RING; k++)
+    if (k + RR_RING < n_it) __syncthreads();   // P2.k
+  if (RR_RING < n_it) __syncthreads();         // P3
 
   int w0 = 0;   // i % RC_RING
   int n_done = 0;
