@@ -834,6 +834,10 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
     // loads of the next tile that go out in front of the logits, the others in front of the sigmoids.  us a step, none / half / all in
     // front: two images (bf16, 501 K labels, batch 128, sr_fast) 550 / 510 / 548, three (e4m3, 500 K, nearest) 405 / 400 / 379
     constexpr int LH = G::NIMG == 3 ? G::WPIECES : G::WPIECES / 2;
+    // ... or behind the logits.  us a step, in front / behind: bf16, 131 K labels, batch 512, nearest 424 / 419, Philox 498 / 494; e4m3
+    // (bf16 logits), 500 K, batch 250, Philox 1077 / 1067; but bf16, 501 K, batch 256 1094 / 1100, batch 128 522 / 530, and FP8 logits,
+    // 670 K, batch 256, sr_fast 764 / 771, batch 512 1614 / 1626
+    constexpr bool BEHIND = !QX && (C == 8 || (C == 4 && WT == CLU_E4M3));
 #pragma unroll 1
     for (int i = 0; i <= n_it; i++) {
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -890,10 +894,14 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
       if (i > 1) store_out(prev2);
       const int p0 = __builtin_amdgcn_readfirstlane(*(const __attribute__((address_space(3))) int*)(lds + G::L_MISC + 16 + (i & 1) * 8));
       const int p1 = __builtin_amdgcn_readfirstlane(*(const __attribute__((address_space(3))) int*)(lds + G::L_MISC + 20 + (i & 1) * 8));
-      if (lfull) load_full(nxt, w_nxt, CluInt<0>{}, CluInt<LH>{});
-      else if (lpart) load_pieces(nxt, w_nxt, 0, LH);
+      auto first_loads = [&] {
+        if (lfull) load_full(nxt, w_nxt, CluInt<0>{}, CluInt<LH>{});
+        else if (lpart) load_pieces(nxt, w_nxt, 0, LH);
+      };
+      if (!BEHIND) first_loads();
       if (i < n_it) logits_part(w_cur);
       else if constexpr (EARLY) words(prev, CluInt<0>{}, element_lanes(), 0, EP);
+      if (BEHIND) first_loads();
       // the partners' G has landed (younger than its loads: those stores and loads)
       if (sfull) {
         if (loads) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(G::OPW + LH) : "memory");
