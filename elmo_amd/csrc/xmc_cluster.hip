@@ -1,7 +1,8 @@
 // One-pass training step of the extreme-classifier layers for gfx950 (MI355X): logits, G = sigmoid - targets, grad_X,
 // grad_W and the in-place update of one tile of label rows after the other, every weight read from HBM once and written
 // once.  It covers the modes that keep bf16 temporaries (bf16 weights, src/xmc_classifiers/chunked.py:85-131; simulated FP8,
-// chunked_fp8xmc_clf.py:98-99,110,115-116) and the true-FP8 arithmetic for batches of more than 128 rows (:81-123).
+// chunked_fp8xmc_clf.py:98-99,110,115-116) and the true-FP8 arithmetic (:81-123) for batches of more than 128 rows or of up to
+// 64 of a large label space.
 //
 // A cluster of C workgroups (one per compute unit, all on one XCD) walks a sequence of tiles of T label rows.  Every
 // member loads the whole tile into LDS (from HBM once, then from the XCD's L2) and
@@ -19,7 +20,7 @@
 // rows, so one geometry serves every batch size.
 //
 // What bounds it: bf16 with a small batch the HBM stream (131 K labels, batch 32, round to nearest: 212 us a step in three
-// kernels, 105 now, 71 of them here at 5.6 TB/s of weights).  The Philox modes with batch 128 the issue of vector and matrix
+// kernels, 105 now, 69 of them here at 5.8 TB/s of weights).  The Philox modes with batch 128 the issue of vector and matrix
 // instructions, which add up more than they overlap: the words alone are 145 clocks of a SIMD per 64 weights, 0.35-0.37 ms
 // of the step (501 K labels, bf16: 1142 us in three kernels, 764 now, 505 with sr_fast; 500 K, e4m3: 1086 / 740, 368 to
 // nearest).  The others the issue of vector, scalar and matrix instructions by two wavefronts per SIMD, and with bf16 weights

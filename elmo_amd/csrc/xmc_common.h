@@ -38,7 +38,8 @@ constexpr size_t WS_DESC = WS_EXCH + (size_t)(MAX_WG / 4) * 8 * 20480;      // t
 //   [QF_CNT2, +1024)      the same for the step's second launch (the head-Kahan layer runs the compensated tiles first)
 //   [QF_XCC, QF_XCC+256)  XCC id every workgroup of the step kernel found itself on
 //   [QF_ERR]              error word: bit 0 = a bounded wait expired, bit 1 = the workgroups of a quad were not placed on
-//                         one XCD (their exchange of G through that XCD's L2 is then not coherent)
+//                         one XCD (their exchange of G through that XCD's L2 is then not coherent, and
+//                         their counters do not reach one another: bit 0 comes with it)
 //   [QF_STICKY]           the error words of all steps since the caller last cleared it, OR-ed together by the step's
 //                         last kernel; no kernel ever clears it
 constexpr int QF_WORDS = 4096;
