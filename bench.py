@@ -78,7 +78,7 @@ def device_settle(dev, want_ms, nc, rows, num_labels, batch, pos_mean, zipf_s):
     chunks = [(torch.randn(rows, 768, generator=gen, device=dev) * 0.02).to(torch.float8_e4m3fn) for _ in range(nc)]
     x = torch.from_numpy(synth.make_x(batch, 768, 99)).to(dev).to(torch.bfloat16)
     labels = torch.from_numpy(synth.make_labels(batch, num_labels, pos_mean, zipf_s, 99)).to(dev)
-    ws = ops.alloc_workspace(nc, rows, dev)
+    ws = ops.alloc_workspace(nc, rows, dev, batch)
     torch.cuda.synchronize()
     t0 = time.perf_counter()
     n = 0
@@ -192,7 +192,7 @@ def bench_inference(args, cfg):
               for _ in range(nc)]
     batch = min(cfg.batch, ops.MAX_BATCH)
     x = torch.from_numpy(synth.make_x(batch, cfg.dim, cfg.seed)).to(dev).to(torch.bfloat16)
-    ws = ops.alloc_workspace(nc, rows, dev)
+    ws = ops.alloc_workspace(nc, rows, dev, batch)
     k = 100
     topk = args.mode == "forward_topk"
     # forward_topk: the two-pass selection (under 1 MB of scratch); --topk-path chunkwise times the general path instead
@@ -339,7 +339,7 @@ def main():
     torch.cuda.reset_peak_memory_stats()
     base_alloc = torch.cuda.memory_allocated()
 
-    workspace = ops.alloc_workspace(nc, rows, dev)
+    workspace = ops.alloc_workspace(nc, rows, dev, cfg.batch)
     grad = torch.empty(cfg.batch, cfg.dim, dtype=torch.bfloat16, device=dev)
     seed_rng = np.random.default_rng(cfg.seed)
 
