@@ -783,13 +783,14 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       __syncthreads();   // G of tile i is visible; the image of updated weights has been read
       // ---- Two jobs are left: grad_X (matrix instructions) and grad_W with the update (vector instructions).  The two wavefronts
-      //      of a SIMD can take them in opposite order, each in the gaps of the other, or in step.  Measured in step against
-      //      opposite, us a step, 131 K labels, batches of 32 / 64:
-      //        Philox   bf16  184/188 183/185   e4m3 159/161 180/179      sr_fast  bf16  92/93 103/106
-      //        nearest  bf16  79/79 94/93       e4m3 62/64 82/81
-      //      In step is the faster order with Philox; without it the two are within 1 % of each other at the large sizes the line was
-      //      drawn at, and in step is up to 3 % faster at the small ones.
-      constexpr bool OPPOSITE = MODE != ROUND_SR_PHILOX;
+      //      of a SIMD can take them in opposite order, each in the gaps of the other, or in step.  Measured in opposite order against
+      //      in step, us a step, batches of 32 / 64:
+      //        e4m3, FP8 logits   131 K labels, nearest 55.4/53.7 66.9/67.2, sr_fast 62.1/60.9 74.0/74.5;  501 K 172.7/168.8 197/196, 192/187 219/221
+      //        e4m3, bf16 logits  131 K, nearest 59.7/58.4 76.2/76.4, sr_fast 69.3/66.7 84.2/83.5;  501 K 183/179 224/221, 215/204 253/248
+      //        bf16               131 K, nearest 74.9/75.8 85.8/85.2, sr_fast 82.8/81.7 96.1/96.0;  501 K 337/336 342/343, 333/333 350/347
+      //        Philox             bf16, 131 K 188/184 185/183;  e4m3 161/159 179/180
+      //      So opposite order is left where the stream of bf16 weights is what bounds a step.
+      constexpr bool OPPOSITE = MODE != ROUND_SR_PHILOX && WT == CLU_BF16;
       auto gx = [&] {
         gradx_part(wimg, gown, [] {});
         if (i + 1 == n_it || (WT == CLU_BF16 && nxt.c != cur.c)) store_acc(WT == CLU_BF16 ? j + cur.c : j);
