@@ -534,7 +534,11 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
             const int row = (v + 8 * s) * G::RPI + lr, sw = G::RPI > 1 ? (v * G::RPI + lr) & G::OSW : row & G::OSW;
             if (row < q.rows_valid) {
               const intx4 ov = *(const __attribute__((address_space(3))) intx4*)(lds + G::L_OUT + row * G::ORS + ((lc ^ sw) * 16));
-              *(intx4*)(q.base + (unsigned)(row * RS + m * G::ORS + lc * 16)) = ov;
+              intx4* dst = (intx4*)(q.base + (unsigned)(row * RS + m * G::ORS + lc * 16));
+              // (past the L2's other contents where it serves four members' loads of FP8-logits tiles: 670 K labels, batch 256, sr_fast 750 us a
+              // step as ordinary stores, 741 so; 2 M labels, C = 2 and e4m3 with bf16 products the same; C = 8 1 % slower, C = 1 8 %)
+              if constexpr (QX && C == 4) __builtin_nontemporal_store(ov, dst);
+              else *dst = ov;
             }
           }
       }
@@ -587,8 +591,9 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
     const unsigned abase = wimg + (pk_w >> 16) + rb0 + (QX ? 0u : (unsigned)(hi4 * (WT == CLU_BF16 ? 768 : 64)));
     unsigned lanes = EARLY ? element_lanes() : 0u;
     if (EARLY) COPAQUE(lanes);
-    // operands are read LD - 1 steps (FP8 products: one) ahead of their products
-    constexpr int LD = C == 4 ? 3 : 4;
+    // operands are read LD - 1 steps (FP8 products: one) ahead of their products (bf16, C = 4, 501 K labels, Philox: depth 3 1101 us a
+    // step, 5 1090, 6 1092; with e4m3 weights and at C = 1, 2 no depth differs by more than 0.3 %)
+    constexpr int LD = WT == CLU_BF16 && C >= 4 ? 5 : C == 4 ? 3 : 4;
     if constexpr (QX) {
       constexpr int NS = 6 * ZN;
       intx4 lo[2], hi[2];
