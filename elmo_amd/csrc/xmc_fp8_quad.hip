@@ -65,24 +65,18 @@ typedef __attribute__((address_space(3))) unsigned char qlds_u8;
 typedef short shortx4 __attribute__((ext_vector_type(4)));
 typedef short shortx8 __attribute__((ext_vector_type(8)));
 
-// 16 bytes per lane from global memory straight into LDS at byte offset ldsoff + 16*lane (wave-uniform offset).
+// 16 bytes per lane from global memory (wave-uniform base pointer, 32-bit per-lane byte offset) straight into LDS at byte
+// offset ldsoff + 16*lane (wave-uniform).
 // Issued through inline assembly on purpose: the compiler orders every later LDS access behind a direct-to-LDS
 // load it knows about, which would serialise the prefetch.  Completion is enforced by hand (s_waitcnt vmcnt +
 // barrier) before the data is read.  The compiler does not look into inline assembly for wait states either: one behind the
 // write of M0, five between a vector instruction that wrote the scalar base (v_readlane of a spilled one) and the load.  (ldsoff is wave-uniform as
 // it comes: read with v_readfirstlane, its arithmetic was done in vector registers.)
-__device__ __forceinline__ void q_lds_load16(const unsigned char* g, unsigned ldsoff) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(ldsoff), "v"(g) : "memory", "m0");
-}
-// same with a wave-uniform base pointer and a 32-bit per-lane byte offset
 __device__ __forceinline__ void q_lds_load16_sbase(const unsigned char* base, unsigned off, unsigned ldsoff) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(ldsoff), "v"(off), "s"(base) : "memory", "m0");
 }
 // same, at device scope (sc1): never served by this compute unit's L1, which may still hold the previous contents
 // of an exchange slot
-__device__ __forceinline__ void q_lds_load16_l2(const unsigned char* g, unsigned ldsoff) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off sc1" : : "s"(ldsoff), "v"(g) : "memory", "m0");
-}
 __device__ __forceinline__ void q_lds_load16_l2_sbase(const unsigned char* base, unsigned off, unsigned ldsoff) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, %2 sc1" : : "s"(ldsoff), "v"(off), "s"(base) : "memory", "m0");
 }
