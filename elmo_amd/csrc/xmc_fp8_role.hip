@@ -594,10 +594,10 @@ __global__ __launch_bounds__(QNT, 1) void fp8_step_role_kernel(const QuadParams 
             // written through (system scope): the updated weights are not read again by this launch, and as ordinary
             // stores they push the exchanged G tiles and the weight tiles between their two fetches out of the XCD's
             // L2 (reads from memory 1.34 instead of 1.12 times the weights); same speed either way
-            // (the registers of a store of more than 8 bytes may not be written by the next vector instruction: it is the
-            // address of the next read here, and with the other wavefront at a higher priority a few addresses in a hundred
-            // thousand were stored for weights.  The compiler keeps that distance only from stores it knows, and a
-            // waiting instruction in between is none.)
+            // (the registers of a store of more than 8 bytes may not be written by a vector instruction within the next two wait
+            // states: it is the address of the next read here, and with the other wavefront at a higher priority a few
+            // addresses in a hundred thousand were stored for weights.  The compiler keeps that distance only from stores it
+            // knows, and waiting instructions in between do not count.)
             asm volatile("s_nop 4\n\tglobal_store_dwordx4 %0, %1, %2 sc0 sc1\n\ts_nop 1" : : "v"(off), "v"(ov), "s"(q_uniform(qp_base)) : "memory");
           } else {
             // rows past the end of the chunk go to a place nobody reads (the padding behind an exchange slot), so that
