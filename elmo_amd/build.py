@@ -16,8 +16,9 @@ HIPCC_FLAGS = [
 ]
 # The second translation unit holds the variants of the step kernel whose tile loop is too large for the compiler's
 # default "#pragma unroll" size limit (see the head of that file); everything else keeps the default.  The scheduler
-# settings are those of the third unit: with them the Philox variant spills 7 registers instead of 39 (0.92 against
-# 1.11 ms per launch) and the head-Kahan ones 15 instead of 26.
+# settings are those of the third unit: when they were chosen, the Philox variant spilled 7 registers with them instead of 39
+# (0.92 against 1.11 ms per launch) and the head-Kahan ones 15 instead of 26.  Now they spill 4 and 5 to 8, the variants of the
+# other units none (tests/test_registers_cpu.py).
 HEAVY_FLAGS = ["-mllvm", "-pragma-unroll-threshold=1000000", "-mllvm", "-misched-cluster=0", "-mllvm", "-amdgpu-use-amdgpu-trackers=1"]
 # The third one holds the headline variants of the step kernel, with the instruction scheduler settings that measured
 # best for them (see the head of that file).

@@ -292,11 +292,11 @@ __global__ __launch_bounds__(QNT, 1) void fp8_step_role_kernel(const QuadParams 
     const int ra = (a + 3) & 3;
     auto wcol_offset = [&](int s, int last_row) {
       const int ch = (a + 4 * s) * 64 + lane, wr = ch / 13;
-      return (unsigned)(min(wr, last_row) * D + QCOLS * m + min(ch - wr * 13, 11) * 16);
+      return __umul24(min(wr, last_row), D) + (unsigned)(QCOLS * m + min(ch - wr * 13, 11) * 16);
     };
     auto rows_offset = [&](int s, int last_row) {
       const int ch = (ra + 4 * s) * 64 + lane, rr = ch / (QRS / 16);
-      return (unsigned)(min(16 * m + min(rr, 15), last_row) * D + min(ch - rr * (QRS / 16), 47) * 16);
+      return __umul24(min(16 * m + min(rr, 15), last_row), D) + (unsigned)(min(ch - rr * (QRS / 16), 47) * 16);
     };
     unsigned woff[4], roff[4];
 #pragma unroll
@@ -307,6 +307,11 @@ __global__ __launch_bounds__(QNT, 1) void fp8_step_role_kernel(const QuadParams 
     // The offsets belong to tiles of w_valid and r_valid rows; a change (the end of a chunk) computes them anew.  (A choice between
     // a full tile's and the others in front of every load: 670 K labels, batch 128, Philox 774 us a step instead of 764, nearest
     // 344 / 336, with a compensated head 477 / 471; sr_fast the same.)
+    // (24-bit products: as plain ones they became 64-bit multiply-adds with register pairs for their lane parts, which are kept over
+    // the loop; the sr_fast variant spilled two registers and the Philox one nine, one of them read back in front of every tile's
+    // logits.  Now none and four, which are read back where the height changes only; the times are the same.  Without any - offsets
+    // two to a register, or their lane parts computed anew - Philox took 781 - 787 us instead of 779, at 131 K labels, batch 96,
+    // 170 - 171 instead of 168.)
     int w_valid = TL, r_valid = TL;
     auto w_rows = [&](const QTile& q) {
       if (q.rows_valid == w_valid) return;
