@@ -814,7 +814,6 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
         upd();
       }
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // tile i+1 has landed
-      prev2 = prev;
       prev = cur;
       cur = nxt;
     }
@@ -943,7 +942,9 @@ __global__ __launch_bounds__(CLU_NT, 1) void cluster_step_kernel(const ClusterPa
   // the last tile's image; prev is the tile of the last iteration (cluster of one) or a repetition of it (the iteration
   // behind the last tile)
   if (!aborted && n_it > 0) store_out(C > 1 ? prev2 : prev);
-  if (C == 1 && v == 0 && lid == 0) p.xcc[blockIdx.x] = (int)(__builtin_amdgcn_s_getreg((3 << 11) | 20) & 15);   // (at the start it costs spills)
+  // for xmc_step_xcc_ids, which reads the ids of the fused step's workspace whichever form the step took (the sum of the partials looks
+  // at them in clusters of several only); at the start it costs spills
+  if (C == 1 && v == 0 && lid == 0) p.xcc[blockIdx.x] = (int)(__builtin_amdgcn_s_getreg((3 << 11) | 20) & 15);
 #undef p
 }
 

@@ -112,6 +112,27 @@ def test_small_batches_take_the_one_pass_form_with_the_same_results(gpu, nc, til
         assert ops.step_error_word(ws, nc, rows) == 0 and int(ws[off:off + 4].view(torch.int32).item()) == 0
 
 
+def test_fp8_step_in_the_one_pass_form_records_the_xcds_too(gpu):
+    """xmc_step_xcc_ids reads the ids of the last step, whichever form it took: here one in clusters of one, in a workspace whose
+    previous ids are no XCDs."""
+    import ctypes
+    import torch
+    from elmo_amd import _lib, ops
+    lib = _lib.load()
+    nc, rows = 1, 64 * 512
+    ws = ops.alloc_workspace(nc, rows, gpu)
+    ws.fill_(0x55)
+    off = ops.step_sticky_error_offset()
+    ws[off:off + 4].zero_()
+    w = torch.zeros(rows, 768, device=gpu).to(torch.float8_e4m3fn)
+    ops.fp8_step([w], torch.zeros(16, 768, dtype=torch.bfloat16, device=gpu), torch.zeros(0, 2, dtype=torch.int32, device=gpu), 0.05,
+                 workspace=ws)
+    n = lib.xmc_step_workgroups()
+    ids = (ctypes.c_int32 * n)()
+    _lib.check(lib.xmc_step_xcc_ids(ws.data_ptr(), ids, n, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)), "xmc_step_xcc_ids")
+    assert len(set(ids)) == 8 and all(0 <= v < 8 for v in ids), list(ids)
+
+
 def test_one_pass_step_gives_up_cleanly(gpu):
     """A polling limit of 0, set from the host: a wait that is not satisfied at once ends the workgroup's walk.  Every kernel
     ends, the error words say so, no weight is updated from missing data, the layer raises, and the next step is clean."""
