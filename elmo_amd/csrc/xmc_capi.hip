@@ -208,14 +208,15 @@ int forward_launch(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, 
 //            sr_fast  29/33  35/30  52/41   84/63  172/118   585/362
 //   64 rows, nearest  32/39  36/36  52/47   81/68  177/125   593/375     Philox  44/47  56/61  97/94  172/176  365/345  1164/1068
 //            sr_fast  33/39  38/38  54/51   86/75  173/139   558/423
-// (weights and grad_X are the same to the bit.)  In tiles per compute unit the lines lie at 1.5 and 4 for 32 and 64 rows, with Philox
+// (The weights are the same to the bit; grad_X's fp32 sum is grouped by 256 workgroups instead of 64 quads.)  In tiles per compute unit the lines lie at 1.5 and 4 for 32 and 64 rows, with Philox
 // at 4 and 12.
 bool small_batch_one_pass(int batch, long long tiles, int round_mode, int cus) {
   const bool philox = round_mode == XMC_ROUND_SR_PHILOX;
   return batch <= 32 ? 2 * tiles >= (philox ? 8 : 3) * (long long)cus : batch <= 64 && tiles >= (philox ? 12 : 4) * (long long)cus;
 }
 // Its places in the fused step's workspace: the grad_X sums from WS_PARTIAL on (32 rows: as many bytes as the fused kernel's; 64 rows:
-// twice that, which only workspaces of xmc_workspace_bytes_ex hold), then the first key of every tile.
+// twice that, over the exchange ring and the descriptors, which this form does not use, and up to 14 MiB beyond: only workspaces of
+// xmc_workspace_bytes_ex hold them), then the first key of every tile.
 constexpr size_t one_pass_partial(int batch) { return (size_t)CLU_MAXWG * CluGeom<CLU_E4M3, 1, 1, 2>::PSLOT * 16 * (batch <= 32 ? 1 : 2); }
 size_t one_pass_end(int batch, size_t tiles) { return (WS_PARTIAL + one_pass_partial(batch) + (tiles + 1) * 4 + 255) / 256 * 256; }
 static_assert(QF_WORDS - QF_CNT2 >= CLU_FLAG_INTS && WS_PARTIAL + one_pass_partial(32) <= WS_EXCH, "one-pass step in the fused step's workspace");

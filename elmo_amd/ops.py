@@ -48,7 +48,9 @@ def _chunk_array(chunks):
 
 
 def workspace_bytes(num_chunks, rows_per_chunk, batch=MAX_BATCH // 2):
-    """Bytes for steps of `batch` rows (the default: of any batch); they also serve every other batch, if perhaps by a slower form."""
+    """Bytes for the fastest form at steps of `batch` rows; they serve every other batch too, if perhaps by a slower form (the same
+    weights, grad_X up to the order of its sum).  The default is the largest: 33 to 64 rows of a large label space take up to
+    14 MiB more than any other batch, so a program that knows its batch gives it."""
     n = _lib.load().xmc_workspace_bytes_ex(num_chunks, rows_per_chunk, batch)
     if n == 0:
         raise _lib.XmcError("unsupported chunk geometry")

@@ -53,8 +53,9 @@ const char* xmc_error_string(int status);
 size_t xmc_workspace_bytes(int num_chunks, int rows_per_chunk);
 
 /* The same, with room for the form that is the fastest at steps of `batch` rows (no counterpart in the
- * reference): 24 MiB more for 33 to 64 rows of a large label space.  In a workspace of xmc_workspace_bytes these take the
- * other form; the results are the same. */
+ * reference): up to 14 MiB more for 33 to 64 rows of a large label space, nothing more otherwise.  In a workspace of
+ * xmc_workspace_bytes these take the other form: the same weights to the bit, and grad_x up to the order of its fp32 sum.
+ * (A workspace of either size gives the same results on every call.) */
 size_t xmc_workspace_bytes_ex(int num_chunks, int rows_per_chunk, int batch);
 
 /* One training step over all chunks: logits, sigmoid minus sparse targets, grad_X, grad_W and the in-place

@@ -52,6 +52,20 @@ def test_workspace_bytes():
     assert lib.xmc_workspace_bytes(0, 64) == 0 and lib.xmc_workspace_bytes(65, 64) == 0 and lib.xmc_workspace_bytes(2, 0) == 0
 
 
+@pytest.mark.parametrize("nc,rows,large", [(1, 64, False), (1, 65472, False), (1, 65536, True), (11, 60928, True), (33, 260608, True), (64, 262128, True)])
+def test_workspace_bytes_for_a_batch(nc, rows, large):
+    """Only steps of 33 to 64 rows of a large label space (1,024 tiles of 64 labels) need more than the plain size, and at most 14 MiB; without
+    a batch the tensor-level call allows for them."""
+    from elmo_amd import ops
+    lib = _lib.load()
+    plain = lib.xmc_workspace_bytes(nc, rows)
+    for batch in (1, 16, 32, 48, 64, 80, 128):
+        more = lib.xmc_workspace_bytes_ex(nc, rows, batch) - plain
+        assert (0 < more <= 14 * 2 ** 20) if large and 32 < batch <= 64 else more == 0
+        assert ops.workspace_bytes(nc, rows, batch) <= ops.workspace_bytes(nc, rows)
+    assert ops.workspace_bytes(nc, rows) == lib.xmc_workspace_bytes_ex(nc, rows, 64)
+
+
 def _call_step(lib, chunk_ptrs, nc, rows, x, batch, feat, labels, nnz, seeds, mode, sw, sx, gout, ws, wsb):
     arr = (ctypes.c_void_p * max(nc, 1))(*chunk_ptrs) if chunk_ptrs is not None else None
     sarr = (ctypes.c_uint32 * max(nc, 1))(*seeds) if seeds is not None else None
