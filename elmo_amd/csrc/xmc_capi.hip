@@ -343,6 +343,7 @@ static int cluster_step(void* const* chunk_ptrs, int num_chunks, int rows_per_ch
     p.flush = bf16 ? 1 : 0;   // the reference rounds each chunk's sum where the weights are bf16
     p.saturate = saturate;
     p.spin_limit = g_spin_limit.load(std::memory_order_relaxed);
+    p.loads_behind = clu_loads_behind((long long)p.ntiles * tile_rows * (D * 2));
     if (profiled && g_prof_start) (void)hipEventRecord(g_prof_start, stream);
     var.fn<<<(p.nclusters + 7) / 8 * 8 * c, CLU_NT, var.lds, stream>>>(p);
     if (profiled) {
