@@ -91,8 +91,6 @@ def load():
                                                vp, i32, vp, sz, vp, sz, vp, vp]
     lib.xmc_fp8_forward_topk_fused_rows.restype = i32
     lib.xmc_fp8_forward_topk_fused_rows.argtypes = lib.xmc_fp8_forward_topk_fused.argtypes
-    lib.xmc_fp8_forward_topk_complete_rows.restype = i32
-    lib.xmc_fp8_forward_topk_complete_rows.argtypes = lib.xmc_fp8_forward_topk_fused.argtypes
     lib.xmc_fp8_forward_topk_wide.restype = i32
     lib.xmc_fp8_forward_topk_wide.argtypes = lib.xmc_fp8_forward_topk_fused.argtypes
     lib.xmc_dropout_quantize.restype = i32

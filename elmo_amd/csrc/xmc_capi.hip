@@ -730,14 +730,6 @@ int xmc_fp8_forward_topk_fused_rows(void* const* chunk_ptrs, int num_chunks, int
                     out_idx, idx_int64, workspace, workspace_bytes, scratch, scratch_bytes, status, stream_, 1, false);
 }
 
-int xmc_fp8_forward_topk_complete_rows(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, const void* x_bf16, int batch,
-                               int features, float scale_w, float scale_x, long long num_labels, int k, void* out_val_bf16,
-                               void* out_idx, int idx_int64, void* workspace, size_t workspace_bytes, void* scratch,
-                               size_t scratch_bytes, int32_t* status, void* stream_) {
-  return topk_fused(chunk_ptrs, num_chunks, rows_per_chunk, x_bf16, batch, features, scale_w, scale_x, num_labels, k, out_val_bf16,
-                    out_idx, idx_int64, workspace, workspace_bytes, scratch, scratch_bytes, status, stream_, 1, true);
-}
-
 int xmc_fp8_forward_topk_wide(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, const void* x_bf16, int batch,
                               int features, float scale_w, float scale_x, long long num_labels, int k, void* out_val_bf16,
                               void* out_idx, int idx_int64, void* workspace, size_t workspace_bytes, void* scratch,

@@ -188,15 +188,9 @@ int xmc_fp8_forward_topk_fused_rows(void* const* chunk_ptrs, int num_chunks, int
                                     void* out_idx, int idx_int64, void* workspace, size_t workspace_bytes, void* scratch,
                                     size_t scratch_bytes, int32_t* status, void* stream);
 
-/* xmc_fp8_forward_topk_fused_rows, and rows that overflow are done over by the call's last launch: the outputs are valid whatever
- * status says, and nobody has to wait for it. */
-int xmc_fp8_forward_topk_complete_rows(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, const void* x_bf16, int batch,
-                                       int features, float scale_w, float scale_x, long long num_labels, int k, void* out_val_bf16,
-                                       void* out_idx, int idx_int64, void* workspace, size_t workspace_bytes, void* scratch,
-                                       size_t scratch_bytes, int32_t* status, void* stream);
-
-/* xmc_fp8_forward_topk_complete_rows for any batch of 1..256 rows: one pass over the weights (and one over a sample of them), where
- * slices of 128 rows take two. */
+/* xmc_fp8_forward_topk_fused for any batch of 1..256 rows: one pass over the weights (and one over a sample of them), where slices
+ * of 128 rows take two; and rows that overflow are done over by the call's last launch: the outputs are valid whatever status says,
+ * and nobody has to wait for it. */
 int xmc_fp8_forward_topk_wide(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, const void* x_bf16, int batch,
                               int features, float scale_w, float scale_x, long long num_labels, int k, void* out_val_bf16,
                               void* out_idx, int idx_int64, void* workspace, size_t workspace_bytes, void* scratch,
