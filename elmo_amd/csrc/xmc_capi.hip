@@ -247,7 +247,7 @@ const char* xmc_error_string(int status) {
   switch (status) {
     case XMC_OK: return "ok";
     case XMC_ERR_NULL: return "null pointer";
-    case XMC_ERR_SHAPE: return "unsupported shape (features must be 768, batch a multiple of 16 and <= 128, rows per chunk a multiple of 16)";
+    case XMC_ERR_SHAPE: return "unsupported shape (features, batch, rows per chunk, labels or k: see the limits of the function that was called)";
     case XMC_ERR_ALIGN: return "device pointer not sufficiently aligned";
     case XMC_ERR_RANGE: return "too many chunks, labels or positives";
     case XMC_ERR_WORKSPACE: return "workspace too small";

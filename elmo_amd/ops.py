@@ -243,12 +243,13 @@ def fp8_forward_topk(chunks, x, num_labels, k, scale_w=1.0, scale_x=1.0, workspa
             need = lib.xmc_topk_fused_scratch_bytes()
             if fused_scratch is None or fused_scratch.numel() < need:
                 fused_scratch = torch.empty(need, dtype=torch.uint8, device=x.device)
-            entry = lib.xmc_fp8_forward_topk_fused_rows if defer_check else lib.xmc_fp8_forward_topk_wide
-            st = entry(arr, nc, rows, xs.data_ptr(), n, FEATURES, float(scale_w), float(scale_x), int(num_labels), int(k),
-                       vals[lo:hi].data_ptr(), idx[lo:hi].data_ptr(), 1, workspace.data_ptr(), workspace.numel(),
-                       fused_scratch.data_ptr(), fused_scratch.numel(), status[si:].data_ptr(), _stream_ptr())
+            entry = "xmc_fp8_forward_topk_fused_rows" if defer_check else "xmc_fp8_forward_topk_wide"
+            st = getattr(lib, entry)(
+                arr, nc, rows, xs.data_ptr(), n, FEATURES, float(scale_w), float(scale_x), int(num_labels), int(k),
+                vals[lo:hi].data_ptr(), idx[lo:hi].data_ptr(), 1, workspace.data_ptr(), workspace.numel(),
+                fused_scratch.data_ptr(), fused_scratch.numel(), status[si:].data_ptr(), _stream_ptr())
             if st != _lib.XMC_ERR_RANGE:
-                _lib.check(st, "xmc_fp8_forward_topk_fused_rows")
+                _lib.check(st, entry)
                 done = True
             else:                # too few labels, for every slice: the general path, which takes 128 rows
                 fused = False

@@ -57,3 +57,12 @@ def test_logits_of_many_labels(gpu, nc, rows, labels):
     for batch in (17, 40, 128):
         got = ops.fp8_forward(chunks, x[:batch].contiguous(), labels)
         assert torch.equal(got.contiguous().view(torch.int16), want[:batch].contiguous().view(torch.int16))
+
+
+@pytest.mark.parametrize("defer,entry", [(False, "xmc_fp8_forward_topk_wide"), (True, "xmc_fp8_forward_topk_fused_rows")])
+def test_a_refused_call_names_its_function(gpu, defer, entry):
+    from elmo_amd import _lib, ops
+    chunks, x = layer(gpu, 2, 16400, 20, 5)
+    workspace = ops.alloc_workspace(2, 16400, gpu)[:1024]        # too small: refused before anything is launched
+    with pytest.raises(_lib.XmcError, match="^%s failed: workspace too small" % entry):
+        ops.fp8_forward_topk(chunks, x, 32800, 5, workspace=workspace, defer_check=defer)
