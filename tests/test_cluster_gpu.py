@@ -134,7 +134,7 @@ def test_fp8_step_in_the_one_pass_form_records_the_xcds_too(gpu):
 
 
 def test_one_pass_step_gives_up_cleanly(gpu):
-    """A polling limit of 0, set from the host: a wait that is not satisfied at once ends the workgroup's walk.  Every kernel
+    """A polling limit of 0, set from the host: the second member leaves after three tiles, and its partners' waits expire.  Every kernel
     ends, the error words say so, no weight is updated from missing data, the layer raises, and the next step is clean."""
     import torch
     from elmo_amd import ops
@@ -145,32 +145,23 @@ def test_one_pass_step_gives_up_cleanly(gpu):
     cfg.data.batch_size = batch
     xfc = Fp8XMCBCEChunkedLayer(cfg)
     assert xfc.xfc_weight[0].shape[0] == rows
-    # every label of six tiles positive for the batch rows of the first member: its partners have to wait for it there
-    dense = [[b, 1024 * t + l] for t in range(6) for l in range(64) for b in range(64)]
-    case = H.make_case(nc, rows, batch, 611, extra_labels=dense)
+    case = H.make_case(nc, rows, batch, 611)
     chunks, x, labels = H.to_device_case(case, gpu)
     ref_codes, _, _ = O.fp8_step(case["chunks"], case["x"], case["labels"], 0.05, sr_mode="rtn")
     prev = ops.debug_spin_limit(0)
     try:
-        raised = False
-        for attempt in range(8):              # whether a wait finds its counter at once depends on timing
-            for wt, c in zip(xfc.xfc_weight, chunks):
-                wt.data.copy_(c.view(torch.float8_e4m3fn))
-            try:
-                xfc.xfc_forward_backward(x, labels, [0.05])
-                xfc.check_steps()
-            except RuntimeError as e:
-                raised = "gave up waiting" in str(e)
-            assert xfc.last_step_error() == int(raised)
-            for wt, old, ref in zip(xfc.xfc_weight, case["chunks"], ref_codes):
-                new = wt.data.view(torch.uint8).cpu().numpy()
-                # the unit of the update is a member's quarter of the features of a row
-                same_old = (new == old).reshape(-1, 4, 192).all(axis=2)
-                good = (H.e4m3_ulp_distance(new, ref) <= 1).reshape(-1, 4, 192).all(axis=2)
-                assert np.all(same_old | good), "weights were updated from incomplete data"
-            if raised:
-                break
-        assert raised, "no wait expired in eight steps with a polling limit of 0"
+        for wt, c in zip(xfc.xfc_weight, chunks):
+            wt.data.copy_(c.view(torch.float8_e4m3fn))
+        with pytest.raises(RuntimeError, match="gave up waiting"):
+            xfc.xfc_forward_backward(x, labels, [0.05])
+            xfc.check_steps()
+        assert xfc.last_step_error() == 1
+        for wt, old, ref in zip(xfc.xfc_weight, case["chunks"], ref_codes):
+            new = wt.data.view(torch.uint8).cpu().numpy()
+            # the unit of the update is a member's quarter of the features of a row
+            same_old = (new == old).reshape(-1, 4, 192).all(axis=2)
+            good = (H.e4m3_ulp_distance(new, ref) <= 1).reshape(-1, 4, 192).all(axis=2)
+            assert np.all(same_old | good), "weights were updated from incomplete data"
     finally:
         ops.debug_spin_limit(prev)
     xfc.xfc_forward_backward(x, labels, [0.05])

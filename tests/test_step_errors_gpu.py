@@ -1,7 +1,7 @@
 """Failed steps that ran in a workspace of their own (a batch larger than the layer's workspace, a call without one) are
-reported like every other.  The failure is forced from the host: with a polling limit of 0 a wait that is not satisfied
-at once ends the workgroup's walk, every kernel ends normally and the step's error word says so.  Whether a wait finds its
-counter at once depends on timing, so a step is tried a few times."""
+reported like every other.  The failure is forced from the host: with a polling limit of 0 the second member of every
+group that exchanges G leaves after three tiles, its partners' waits expire, every kernel ends normally and the step's
+error word says so.  A call without a workspace reports the failure of the one before it."""
 import pytest
 
 import helpers as H
@@ -13,17 +13,17 @@ NC, ROWS = 2, 8192
 
 
 def inputs(batch, gpu):
-    # every label of six tiles is positive for the rows of a cluster's first member: its partners have to wait for it there
+    # (every label of six tiles is positive for the rows of a cluster's first member)
     dense = [[b, 1024 * t + l] for t in range(6) for l in range(64) for b in range(64)]
     return H.to_device_case(H.make_case(NC, ROWS, batch, 611, extra_labels=dense), gpu)
 
 
 def failing(step):
-    """Runs `step` with a polling limit of 0 until it raises the report of a failed step; returns whether it did."""
+    """Runs `step` with a polling limit of 0, twice if need be, until it raises the report of a failed step; returns whether it did."""
     from elmo_amd import ops
     prev = ops.debug_spin_limit(0)
     try:
-        for _ in range(8):
+        for _ in range(2):
             try:
                 step()
             except RuntimeError as e:
