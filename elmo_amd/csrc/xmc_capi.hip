@@ -286,8 +286,9 @@ int xmc_fp8_step(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, co
 }  // extern "C"
 
 // The one-pass form of the step (xmc_cluster.hip): 768 features, no compensated head, no loss, no weight decay (options
-// that would have to stay in its main loop, whose registers are full).  Within these it was the faster form at every size
-// tried, from 2 K to 8.6 M labels and 1 to 512 batch rows.  The arguments have been checked by the caller.
+// that would have to stay in its main loop, whose registers are full).  Within these it was faster than the three kernels at every size
+// tried, from 2 K to 8.6 M labels and 1 to 512 batch rows; true FP8 of up to 128 rows has the fused kernel besides, and
+// small_batch_one_pass decides.  The arguments have been checked by the caller.
 static int cluster_step(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, int rows_last_chunk, int weight_type,
                         const void* x_bf16, int batch, const int32_t* labels_coo, int nnz, float lr, const uint32_t* seeds,
                         int round_mode, int quantize_x, int saturate, const DropoutParams& dp, void* grad_x_bf16, float* grad_x_f32,
@@ -820,8 +821,8 @@ static int tiled_step_t(void* const* chunk_ptrs, int num_chunks, int rows_per_ch
   if (batch <= 0 || batch > T_HALVES * BP) return XMC_ERR_SHAPE;
   if (rows_per_chunk <= 0 || rows_last_chunk <= 0 || rows_last_chunk > rows_per_chunk) return XMC_ERR_SHAPE;
   if (num_chunks <= 0 || num_chunks > MAX_CHUNKS) return XMC_ERR_RANGE;
-  // a sort key keeps 24 bits for the label: larger label spaces are taken in segments of whole chunks, each with its own
-  // sorted list of the positives that fall into it and labels counted from the segment's first
+  // a key keeps 24 bits for the label: larger label spaces are taken in segments of whole chunks, each with its own
+  // list of the positives that fall into it and labels counted from the segment's first
   if (rows_per_chunk >= (1 << 24) - 1 || (long long)num_chunks * rows_per_chunk > 0x7FFFFFFFLL) return XMC_ERR_RANGE;
   if (nnz < 0 || nnz > MAX_POS) return XMC_ERR_RANGE;
   if (weight_type != W_E4M3 && weight_type != W_BF16) return XMC_ERR_MODE;

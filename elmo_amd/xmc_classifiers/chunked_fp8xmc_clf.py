@@ -100,7 +100,7 @@ class Fp8XMCBCEChunkedLayer(nn.Module):
         self._max_batch = int(_opt(cfg.data, "batch_size", ops.MAX_BATCH))
         if self.fake_fp8_matmul:
             assert self.scale_w == 1.0 and self.scale_x == 1.0, "simulated FP8 has no per-tensor scales"
-        # the fused kernel's sort keys hold 24 bits of label: larger label spaces run on the tiled step, which sorts
+        # the fused step's keys of positives hold 24 bits of label: larger label spaces run on the tiled step, which takes
         # the positives per segment of the label space
         self._wide = self.num_labels >= (1 << 24) - 1
         if self._other_width:

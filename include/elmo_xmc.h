@@ -167,7 +167,7 @@ size_t xmc_topk_fused_scratch_bytes(void);
 
 /* The same result as xmc_fp8_forward_topk (evaluate.py:158-159,235-236 on chunked_fp8xmc_clf.py:45-60) with the
  * selection inside the logits kernel: no logits reach memory.  Two passes over the weights: the first visits one tile
- * in 8 or 16 and yields, per batch row, a lower bound of the k-th largest logit; the second visits every tile and keeps
+ * in 1 to 16 (by k and the number of labels: 8 or 16 of a large label space) and yields, per batch row, a lower bound of the k-th largest logit; the second visits every tile and keeps
  * the logits at or above the bound (a few hundred per row), which a last kernel ranks.
  *   out_idx  device [batch, k] label ids, int32, or int64 (what torch.topk returns) with idx_int64 != 0
  *   status   device int32, written by the call's kernels: 0 = outputs valid; bit 0 = a row had more than 2,048 logits
@@ -251,8 +251,8 @@ size_t xmc_tiled_workspace_bytes_ex(int num_chunks, int rows_per_chunk, int max_
  *   chunk_ptrs       host array of device pointers to the chunks' first rows; [rows, d] row-major each; all chunks
  *                    have rows_per_chunk rows except the last (rows_last_chunk <= rows_per_chunk); any row count
  *   labels_coo       as xmc_fp8_step; label id = chunk * rows_per_chunk + row.  The label space may exceed the 2^24 labels
- *                    the sort keys of xmc_fp8_step hold (up to 2^31 - 1 labels, a chunk below 2^24 - 1 rows): the
- *                    positives are then sorted once per segment of whole chunks with fewer than 2^24 - 1 labels
+ *                    the keys of xmc_fp8_step hold (up to 2^31 - 1 labels, a chunk below 2^24 - 1 rows): the
+ *                    positives are then taken once per segment of whole chunks with fewer than 2^24 - 1 labels
  *   round_mode       XMC_ROUND_RTN, XMC_ROUND_SR_PHILOX, or XMC_ROUND_SR_FAST with the random words of xmc_fp8_step's
  *                    mode of that name (bf16 weights: the hardware converter to bf16, which adds the upper 16 bits of the
  *                    word to the fp32 pattern); batch: 1..512, any value (processed in one, two or four halves of 128 rows)
