@@ -647,14 +647,24 @@ static_assert(SELW_COUNT + (size_t)(SEL_ROWS + SEL_ROWS / 32) * SEL_COUNT_STRIDE
 
 size_t xmc_topk_fused_scratch_bytes(void) { return SELS_BYTES; }
 
-// tiles pass 1 skips between two it visits: the k-th largest of the group maxima of a 1/step sample leaves about
-// k * step candidates per row, which have to stay well below the list size; at least four groups per wanted entry.  (670 K labels, batch
-// 128, k = 100, us a call: every fourth tile 140, with lists of 1,024; every eighth, of 2,048, 131; every sixteenth, of 4,096, 135 - what
-// the shorter pass 1 gains, pass 2 loses on candidates.)
-static int topk_fused_step(int tiles, int k) {
+// Pass 1 visits one tile in `step`: the k-th largest of the group maxima of such a sample leaves about k * step candidates per row, which
+// have to stay well below the list size; at least four groups per wanted entry.  What a shorter pass 1 gains, pass 2 loses on candidates:
+// more than 512 of them pay from about 3/2 k step^2 tiles on (the time is as c tiles / step + d k step), or in the form for more than
+// 128 rows, whose pass 2 has twice the rows behind every tile.  us a call, at most 512 / at most 1,024 candidates:
+//   128 rows  k = 40 (step 8 / 16)  90 K labels 38.5/43.8  131 K 42.6/47.9  262 K 58.5/59.8  400 K 77.0/79.1  670 K 119/116  1 M 173/163
+//             k = 64 (step 8 / 16)            -            131 K 45.6/56.3  262 K 60.5/68.6  400 K 78.9/84.4  670 K 118/121  1 M 172/169
+//             k = 100 (step 4 / 8)            -            131 K 45.8/52.9  262 K 64.2/67.1  400 K 83.7/86.4  670 K 126/122  1 M 189/173
+//   8 rows    k = 100                                      131 K 40.7/44.0  262 K 58.7/60.8  400 K 78.7/75.3  670 K 123/117  1 M 182/168
+//   256 rows  k = 40                 90 K 55.4/54.5        131 K 65.2/64.2  262 K 94.7/92.1  400 K 129/128    670 K 191/191  1 M 263/266
+//             k = 100                                      131 K 71.1/73.0  262 K 104/102    400 K 141/138    670 K 211/204  1 M 295/282
+// (2,048 candidates, lists of 4,096: 670 K labels, 128 rows, k = 100 135 us, 131 with 1,024.)
+static int topk_fused_step(int tiles, int k, bool wide) {
+  auto fits = [&](int step) {
+    return tiles / step >= 4 * k && (k * step <= SEL_CAP / 4 || (k * step <= SEL_CAP / 2 && (wide || 2 * tiles >= 3 * k * step * step)));
+  };
   int step = 16;
-  while (step > 1 && (k * step > SEL_CAP / 2 || tiles / step < 4 * k)) step >>= 1;
-  return tiles / step >= 4 * k ? step : 0;
+  while (step > 1 && !fits(step)) step >>= 1;
+  return fits(step) ? step : 0;
 }
 
 static int topk_fused(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, const void* x_bf16, int batch, int features,
@@ -674,7 +684,8 @@ static int topk_fused(void* const* chunk_ptrs, int num_chunks, int rows_per_chun
   sp.tiles_per_chunk = (rows_per_chunk + FT - 1) / FT;
   const int last_chunk = (int)((num_labels - 1) / rows_per_chunk);
   const int tiles = last_chunk * sp.tiles_per_chunk + (int)((num_labels - (long long)last_chunk * rows_per_chunk + FT - 1) / FT);
-  const int step = topk_fused_step(tiles, k);
+  const bool wide = batch > BP;
+  const int step = topk_fused_step(tiles, k, wide);
   if (step == 0) return XMC_ERR_RANGE;   // too few labels for a useful bound: xmc_fp8_forward_topk takes these
   DeviceInfo di = device_info();
   if (di.ok != 1) return XMC_ERR_DEVICE;
@@ -697,7 +708,6 @@ static int topk_fused(void* const* chunk_ptrs, int num_chunks, int rows_per_chun
   sp.tile_step = step;
   sp.n_visit = (tiles + step - 1) / step;
   // (a workgroup to a compute unit, or two: with more, the last ones would start when the first ones are done)
-  const bool wide = batch > BP;
   const int most = wide && di.cus < SEL_GROUPS && di.cus >= 2 * k ? di.cus : SEL_GROUPS;
   const int groups = sp.n_visit < most ? sp.n_visit : most;
   if (wide) fp8_forward_select_kernel<0, 8><<<groups, 512, SelGeom<8>::LDS, stream>>>(sp);
