@@ -447,7 +447,8 @@ def main():
     tpath = os.path.join(ROOT, "profiles", "hbm_traffic.json")
     if os.path.exists(tpath):
         with open(tpath) as f:
-            traffic = json.load(f).get(f"{kernel_name}:{cfg.name}:{args.round}")
+            head = "" if args.head_kahan == "none" else f":{args.head_kahan}_head_{num_head}"
+            traffic = json.load(f).get(f"{kernel_name}:{cfg.name}:{args.round}{head}")
 
     out = {
         "metric": "XMC classifier train steps/sec at 670K labels FP8" if cfg.name == "cfg2_fp8_670k" else
