@@ -247,7 +247,8 @@ const char* xmc_error_string(int status) {
   switch (status) {
     case XMC_OK: return "ok";
     case XMC_ERR_NULL: return "null pointer";
-    case XMC_ERR_SHAPE: return "unsupported shape (features, batch, rows per chunk, labels or k: see the limits of the function that was called)";
+    case XMC_ERR_SHAPE: return "unsupported shape: features (768, the tiled step also 1024), batch (up to 128, wide inference 256, the tiled step 512; a multiple of 16 "
+                                "where the function says so), rows per chunk, labels or k";
     case XMC_ERR_ALIGN: return "device pointer not sufficiently aligned";
     case XMC_ERR_RANGE: return "too many chunks, labels or positives";
     case XMC_ERR_WORKSPACE: return "workspace too small";
