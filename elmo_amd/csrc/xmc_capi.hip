@@ -719,7 +719,7 @@ static int topk_fused(void* const* chunk_ptrs, int num_chunks, int rows_per_chun
   sp.n_visit = tiles;
   if (wide) fp8_forward_select_kernel<1, 8><<<tiles < di.cus ? tiles : di.cus, 512, SelGeom<8>::LDS, stream>>>(sp);
   else fp8_forward_select_kernel<1, 4><<<tiles < 2 * di.cus ? tiles : 2 * di.cus, 256, SelGeom<4>::LDS, stream>>>(sp);
-  const int repairers = repair ? (batch + 31) / 32 * REP_SLICES : 0;
+  const int repairers = repair ? rep_blocks(batch) : 0;
   topk_pick_kernel<<<batch + repairers, REP_NT, repair ? REP_LDS : PICK_LDS, stream>>>(
       sp, k, (unsigned short*)out_val_bf16, out_idx, idx_int64 ? 1 : 0, status,
       repair ? (unsigned long long*)((unsigned char*)workspace + SELW_LISTS) : nullptr);

@@ -358,6 +358,7 @@ __global__ __launch_bounds__(TOPK_GROUPS) void topk_bound_kernel(const unsigned 
   const int b = blockIdx.x, g = threadIdx.x;
   if (g == 0) {
     count[b * SEL_COUNT_STRIDE] = 0u;
+    count[b * SEL_COUNT_STRIDE + 1] = 0u;                                   // (entries of the row's lists in topk_repair)
     if (b < SEL_ROWS / 32) count[(SEL_ROWS + b) * SEL_COUNT_STRIDE] = 0u;   // (workgroups of topk_repair that are done)
     if (b == 0) *status = 0;
     if (b >= batch) bound[b] = 0xFFFFu;
@@ -369,52 +370,77 @@ __global__ __launch_bounds__(TOPK_GROUPS) void topk_bound_kernel(const unsigned 
 }
 
 // ---- Rows whose list is of no use - more logits at or above the bound than it holds (massive ties, say), or fewer than k - are done
-// over by topk_repair, in the launch that ranks the other rows' lists: 64 workgroups for every 32 batch rows, each with a 64th of the
-// labels, which look at the rows' counts and are usually done with that.  (Before, the host waited for a status word after every call,
-// to launch the general path if need be: 27 - 32 us of a call of 158 in which the GPU had nothing to do.)  A workgroup computes its
-// logits anew, 128 labels a round, and keeps the best k of every row in LDS; the last one of the 64 merges their lists.  Nobody waits
-// for anybody.
-// (670 K labels, batch 128, k = 100: 131 us a call, 160 before; with every logit of every row alike, where pass 2 takes 7.8 ms and this
-// 0.8, 8.8 ms, 9.2 before.)
+// over by topk_repair, in the launch that ranks the other rows' lists: up to 256 workgroups, which look at the rows' counts and are
+// usually done with that.  (Before, the host waited for a status word after every call, to launch the general path if need be: 27 - 32 us
+// of a call of 158 in which the GPU had nothing to do.)  The workgroups share the groups of 32 batch rows that have such a row, and
+// those of a group the labels.  A workgroup computes its logits anew, 256 labels a round, and keeps the best k of every row in LDS; the
+// last one of a group merges their lists.  Nobody waits for anybody.
+// Bound by memory: every group reads all weights, each wavefront its sixteen labels of the next round into the registers that this
+// round's products have just read.  The row's bound, which k logits at least reach, keeps nearly everything else off the lists.
+// us a call, k = 100, 6,000 equal labels the best of one row / of all rows: with the host's wait and the general path / with 64
+// workgroups for every group, which loaded nothing ahead and ranked lists against one another / now:
+//   128 rows  131 K labels 349/285/179  339/547/328   670 K 667/772/328  627/1121/579   2 M 1370/1944/737  1340/2399/1255
+//   256 rows  131 K 692/360/256  668/961/421          670 K 810/864/412  1239/2103/904   2 M 1753/2178/933  2664/4503/2087
+// With no such row 131 K 74/48/48, 670 K 160/131/122; with every logit of one row alike, where pass 2 takes nearly all, 670 K 8744/8214/7840.
 constexpr int REP_NT = 1024;              // threads: as many as topk_pick's, which shares the launch
-constexpr int REP_SLICES = 64;            // workgroups per 32 batch rows
+constexpr int REP_BLOCKS = 64;            // workgroups for every 32 rows of a batch of up to 128, all of a larger one's: 256
+constexpr int REP_SLICES = 128;           // most workgroups of a group: the last one reads as many lists
 constexpr int REP_CAP = 256;              // entries of a row's list in LDS; cut to the best k <= TOPK_MAX before it overflows
-constexpr int REP_STEP = 128;             // labels a round
-constexpr int REP_LDS = 32 * REP_CAP * 8 + 32 * REP_STEP * 2 + 64;
-constexpr size_t REP_BYTES = (size_t)(SEL_ROWS / 32) * REP_SLICES * 32 * TOPK_MAX * 8;   // lists of the workgroups
+constexpr int REP_STEP = 256;             // labels a round, sixteen a wavefront
+constexpr int REP_KS = REP_STEP + 8;      // stride of a row of keys
+constexpr int REP_X = 32 * REP_CAP * 8;                // LDS: lists | operand image of the group's X | keys of two rounds | a word
+constexpr int REP_KEYS = REP_X + 12 * 2048;
+constexpr int REP_WORD = REP_KEYS + 2 * 32 * REP_KS * 2;
+constexpr int REP_LDS = REP_WORD + 64;
+constexpr int rep_blocks(int batch) { return (batch < BP ? (batch + 31) / 32 : BP / 32) * REP_BLOCKS; }
+constexpr size_t REP_BYTES = (size_t)rep_blocks(SEL_ROWS) * 32 * TOPK_MAX * 8;   // lists of the workgroups
 static_assert(REP_CAP >= TOPK_MAX + 64, "a wavefront's worth of new entries behind a cut list");
+static_assert(REP_STEP == REP_NT / 64 * 16 && REP_BLOCKS % 8 == 0 && SEL_ROWS == 256, "shares of the wavefronts and the workgroups");
 
 // An entry: order key << 32 | ~label, larger = better value, then smaller label; 0 = none.
 struct RepList { unsigned long long* ent; int n; unsigned long long above; };   // entries above `above` are still wanted
-// cuts the list of a wavefront's row to its best k, best first
-__device__ __forceinline__ void rep_cut(RepList& l, int k) {
+// Cuts the list of a wavefront's row to its best k, in no order: the k-th entry bit by bit, as all entries are different (ranked against
+// one another instead, 128 rows of 6,000 equal labels: 131 K labels 402 us a call, now 328, 670 K 711, now 579).  label_bits: bits that
+// labels differ in.
+__device__ __forceinline__ void rep_cut(RepList& l, int k, int label_bits) {
+  if (l.n <= k) return;
   const int lane = threadIdx.x & 63;
   unsigned long long e[REP_CAP / 64];
-  int r[REP_CAP / 64];
+#pragma unroll
+  for (int u = 0; u < REP_CAP / 64; u++) e[u] = lane + 64 * u < l.n ? l.ent[lane + 64 * u] : 0ull;
+  auto at_least = [&](unsigned long long t) {
+    int c = 0;
+#pragma unroll
+    for (int u = 0; u < REP_CAP / 64; u++) c += __popcll(__ballot(e[u] >= t));
+    return c;
+  };
+  unsigned long long T = 0ull;   // at least k entries at or above it
+  int have = l.n;
+  for (int bit = 47; bit >= 0 && have > k; bit--) {
+    if (bit == 31) {   // (the upper bits of an inverted label are ones)
+      T |= 0xFFFFFFFFull >> label_bits << label_bits;
+      bit = label_bits - 1;
+    }
+    const int c = at_least(T | 1ull << bit);
+    if (c >= k) { T |= 1ull << bit; have = c; }
+  }
+  int n = 0;
 #pragma unroll
   for (int u = 0; u < REP_CAP / 64; u++) {
-    e[u] = lane + 64 * u < l.n ? l.ent[lane + 64 * u] : 0ull;
-    r[u] = 0;
-  }
-  for (int j = 0; j < l.n; j++) {
-    const unsigned long long o = l.ent[j];
-#pragma unroll
-    for (int u = 0; u < REP_CAP / 64; u++) r[u] += o > e[u] ? 1 : 0;
+    const unsigned long long who = __ballot(e[u] >= T);
+    if (e[u] >= T) l.ent[n + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(who >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)who, 0u))] = e[u];
+    n += __popcll(who);
   }
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-#pragma unroll
-  for (int u = 0; u < REP_CAP / 64; u++)
-    if (e[u] != 0ull && r[u] < k) l.ent[r[u]] = e[u];
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  l.n = l.n < k ? l.n : k;
-  l.above = l.n == k ? l.ent[k - 1] : 0ull;
+  l.n = n;
+  l.above = T - 1ull;
 }
 // a wavefront's worth of entries, one per lane
-__device__ __forceinline__ void rep_add(RepList& l, unsigned long long e, int k) {
+__device__ __forceinline__ void rep_add(RepList& l, unsigned long long e, int k, int label_bits) {
   unsigned long long who = __ballot(e > l.above);
   if (who == 0) return;
   if (l.n + __popcll(who) > REP_CAP) {
-    rep_cut(l, k);
+    rep_cut(l, k, label_bits);
     who = __ballot(e > l.above);
   }
   if (e > l.above) l.ent[l.n + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(who >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)who, 0u))] = e;
@@ -428,80 +454,156 @@ __device__ __forceinline__ void topk_write(unsigned short* out_val, void* out_id
   else ((int*)out_idx)[at] = lab;
 }
 
-__device__ __forceinline__ void topk_repair(const SelectParams& p, int blk, int k, unsigned long long* lists, unsigned short* out_val, void* out_idx,
-                                            int idx64, unsigned char* lds) {
-  const int group = blk / REP_SLICES, slice = blk - group * REP_SLICES;
+// blk of nblk workgroups
+__device__ __forceinline__ void topk_repair(const SelectParams& p, int blk, int nblk, int k, unsigned long long* lists, unsigned short* out_val,
+                                            void* out_idx, int idx64, unsigned char* lds) {
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l16 = lane & 15, kg = lane >> 4;
-  // rows of this group to be done over (the same in every wavefront)
-  const int row = 32 * group + (lane & 31);
-  const unsigned have = row < p.batch ? p.count[row * SEL_COUNT_STRIDE] : (unsigned)k;
-  const unsigned rows = (unsigned)__ballot(have > (unsigned)SEL_CAP || have < (unsigned)k);
-  if (rows == 0u) return;
-  unsigned short* keys = (unsigned short*)(lds + 32 * REP_CAP * 8);   // [32 rows][REP_STEP]
+  // rows to be done over, a bit each.  (Four wavefronts look at 64 counts each, which are a cache line apart.)
+  unsigned* word = (unsigned*)(lds + REP_WORD);
+  if (w < SEL_ROWS / 64) {
+    const int row = 64 * w + lane;
+    const unsigned have = row < p.batch ? p.count[row * SEL_COUNT_STRIDE] : (unsigned)k;
+    const unsigned long long m = __ballot(have > (unsigned)SEL_CAP || have < (unsigned)k);
+    if (lane < 2) word[2 * w + lane] = (unsigned)(m >> (32 * lane));
+  }
+  __syncthreads();
+  unsigned need[SEL_ROWS / 32];
+  int ngroups = 0;
+#pragma unroll
+  for (int g = 0; g < SEL_ROWS / 32; g++) {
+    need[g] = __builtin_amdgcn_readfirstlane(word[g]);
+    ngroups += need[g] != 0u ? 1 : 0;
+  }
+  if (ngroups == 0) return;
+  // eight workgroups side by side take neighbouring slices of one group's labels, the eight behind them those of the next group
+  const int q8 = (blk >> 3) / ngroups, which = (blk >> 3) - q8 * ngroups, slice = q8 * 8 + (blk & 7);
+  const int most = (nblk >> 3) / ngroups * 8, slices = most < REP_SLICES ? most : REP_SLICES;
+  if (slice >= slices) return;
+  int group = 0;
+  unsigned rows = 0u;
+  {
+    int at = 0;
+#pragma unroll
+    for (int g = 0; g < SEL_ROWS / 32; g++) {
+      if (need[g] == 0u) continue;
+      if (at == which) { group = g; rows = need[g]; }
+      at++;
+    }
+  }
   RepList l[2];                                                       // rows 2w, 2w + 1 of the group
+  unsigned long long floor[2];   // what their bounds leave out (a row with fewer than k logits at its bound has none)
 #pragma unroll
-  for (int q = 0; q < 2; q++) l[q] = RepList{(unsigned long long*)lds + (2 * w + q) * REP_CAP, 0, 0ull};
-  // logits: wavefront w takes sixteen batch rows (w & 1) and every eighth sixteen labels (w >> 1); sixteen labels are rows of one chunk
-  const int rb = w & 1, sub = w >> 1;
-  intx8 xq[6];
-#pragma unroll
-  for (int ks = 0; ks < 6; ks++) xq[ks] = *(const intx8*)(p.xq + ((size_t)((group * 2 + rb) * 6 + ks) * 64 + lane) * 32);
+  for (int q = 0; q < 2; q++) {
+    const int row = 32 * group + 2 * w + q;
+    floor[q] = 0ull;
+    if (rows >> (2 * w + q) & 1u) {
+      const unsigned bound = p.bound[row];
+      if (p.count[row * SEL_COUNT_STRIDE] >= (unsigned)k && bound != 0u) floor[q] = ((unsigned long long)bound << 32) - 1ull;
+    }
+    l[q] = RepList{(unsigned long long*)lds + (2 * w + q) * REP_CAP, 0, floor[q]};
+  }
+  // the operand image of X, the two halves of a lane's 32 bytes apart
+  for (int i = tid; i < 12 * 128; i += REP_NT)
+    *(intx4*)(lds + REP_X + (i >> 7) * 2048 + (i & 1) * 1024 + ((i & 127) >> 1) * 16) = *(const intx4*)(p.xq + (size_t)group * 12 * 2048 + (size_t)i * 16);
+  __syncthreads();
+  // logits: wavefront w takes sixteen labels of a round, which are rows of one chunk, and all 32 batch rows
   const long long n16 = (p.num_labels + 15) / 16;
-  const int s_end = (int)(n16 * (slice + 1) / REP_SLICES);
-  for (int s0 = (int)(n16 * slice / REP_SLICES); s0 < s_end; s0 += REP_STEP / 16) {
-    const int s = s0 + sub;
-    unsigned short key4[4] = {0, 0, 0, 0};
-    if (s < s_end) {
-      const unsigned label = 16u * (unsigned)s, c = label / (unsigned)p.rows_per_chunk, r0 = label - c * (unsigned)p.rows_per_chunk;
-      const unsigned char* src = p.chunk[__builtin_amdgcn_readfirstlane(c)] + (size_t)(r0 + l16) * D + kg * 32;
-      intx8 a[6];
+  const int label_bits = 32 - __builtin_clz((unsigned)(n16 * 16));   // (fewer than 2^31 labels)
+  const int s_begin = (int)(n16 * slice / slices), s_end = (int)(n16 * (slice + 1) / slices);
+  if (s_begin < s_end) {
+    intx8 a[6];
+    auto place = [&](int s) {   // behind the last one: the last one again
+      const unsigned label = 16u * (unsigned)(s < s_end ? s : s_end - 1), c = label / (unsigned)p.rows_per_chunk, r0 = label - c * (unsigned)p.rows_per_chunk;
+      return p.chunk[__builtin_amdgcn_readfirstlane(c)] + (size_t)(r0 + l16) * D + kg * 32;
+    };
+    auto load = [&](const unsigned char* src, int ks) {
+      const intx4 lo = *(const intx4*)(src + ks * 128), hi = *(const intx4*)(src + ks * 128 + 16);
+      a[ks] = intx8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    };
+    {
+      const unsigned char* src = place(s_begin + w);
+#pragma unroll
+      for (int ks = 0; ks < 6; ks++) load(src, ks);
+    }
+    int par = 0;
+    for (int s0 = s_begin; s0 < s_end; s0 += REP_STEP / 16, par ^= 1) {
+      const int s = s0 + w;
+      const unsigned char* next = place(s + REP_STEP / 16);
+      unsigned char* keys = lds + REP_KEYS + par * (32 * REP_KS * 2);   // [32 rows][REP_KS]
+      floatx4 z[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
       for (int ks = 0; ks < 6; ks++) {
-        const intx4 lo = *(const intx4*)(src + ks * 128), hi = *(const intx4*)(src + ks * 128 + 16);
-        a[ks] = intx8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-      }
-      floatx4 z = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int ks = 0; ks < 6; ks++) z = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a[ks], xq[ks], z, 0, 0, 0, 0, 0, 0);
-#pragma unroll
-      for (int e = 0; e < 4; e++)
-        if ((long long)label + 4 * kg + e < p.num_labels) key4[e] = (unsigned short)topk_key(bf16_bits(z[e] * p.zscale));
-    }
-    *(uint2*)(keys + (16 * rb + l16) * REP_STEP + sub * 16 + 4 * kg) =
-        uint2{(unsigned)key4[0] | ((unsigned)key4[1] << 16), (unsigned)key4[2] | ((unsigned)key4[3] << 16)};
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < 2; q++)
-      if (rows >> (2 * w + q) & 1u)
-        for (int h = 0; h < REP_STEP; h += 64) {
-          const unsigned key = keys[(2 * w + q) * REP_STEP + h + lane];
-          rep_add(l[q], key ? ((unsigned long long)key << 32) | (0xFFFFFFFFu - (16u * (unsigned)s0 + (unsigned)(h + lane))) : 0ull, k);
+        for (int rb = 0; rb < 2; rb++) {
+          const unsigned char* x = lds + REP_X + (rb * 6 + ks) * 2048 + lane * 16;
+          const intx4 lo = *(const intx4*)x, hi = *(const intx4*)(x + 1024);
+          z[rb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a[ks], intx8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]}, z[rb], 0, 0, 0, 0, 0, 0);
         }
-    __syncthreads();
+        load(next, ks);
+      }
+      const long long left = s < s_end ? p.num_labels - 16ll * s - 4 * kg : 0;   // labels from this lane's first on
+#pragma unroll
+      for (int rb = 0; rb < 2; rb++) {
+        unsigned short key4[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) key4[e] = e < left ? (unsigned short)topk_key(bf16_bits(z[rb][e] * p.zscale)) : (unsigned short)0;
+        *(uint2*)(keys + (16 * rb + l16) * (REP_KS * 2) + (16 * w + 4 * kg) * 2) =
+            uint2{(unsigned)key4[0] | ((unsigned)key4[1] << 16), (unsigned)key4[2] | ((unsigned)key4[3] << 16)};
+      }
+      __syncthreads();   // (the keys of the round before are read by all: its barrier lies behind this round's)
+#pragma unroll
+      for (int q = 0; q < 2; q++)
+        if (rows >> (2 * w + q) & 1u)
+          for (int h = 0; h < REP_STEP; h += 64) {
+            const unsigned key = *(const unsigned short*)(keys + (2 * w + q) * (REP_KS * 2) + (h + lane) * 2);
+            rep_add(l[q], key ? ((unsigned long long)key << 32) | (0xFFFFFFFFu - (16u * (unsigned)s0 + (unsigned)(h + lane))) : 0ull, k, label_bits);
+          }
+    }
   }
-  unsigned long long* out = lists + (size_t)(group * REP_SLICES + slice) * 32 * TOPK_MAX;
+  // the lists of a row, one behind the other in the order of their arrival (the second word of the row's counter line counts)
+  lists += (size_t)which * slices * 32 * TOPK_MAX;   // the group's, [row][slices * TOPK_MAX]
 #pragma unroll
   for (int q = 0; q < 2; q++)
     if (rows >> (2 * w + q) & 1u) {
-      rep_cut(l[q], k);
-      for (int h = lane; h < TOPK_MAX; h += 64) out[(2 * w + q) * TOPK_MAX + h] = h < l[q].n ? l[q].ent[h] : 0ull;
+      rep_cut(l[q], k, label_bits);
+      unsigned at = 0;
+      if (lane == 0) at = atomicAdd(p.count + (32 * group + 2 * w + q) * SEL_COUNT_STRIDE + 1, (unsigned)l[q].n);
+      at = __builtin_amdgcn_readfirstlane(at);
+      for (int h = lane; h < l[q].n; h += 64) lists[(size_t)(2 * w + q) * slices * TOPK_MAX + at + h] = l[q].ent[h];
     }
   __threadfence();
   __syncthreads();
-  unsigned* arrived = (unsigned*)(lds + REP_LDS - 64);
+  unsigned* arrived = word + SEL_ROWS / 32;
   if (tid == 0) *arrived = atomicAdd(p.count + (SEL_ROWS + group) * SEL_COUNT_STRIDE, 1u);
   __syncthreads();
-  if (*arrived != REP_SLICES - 1) return;
+  if (*arrived != (unsigned)slices - 1u) return;
   __threadfence();   // the last one: everybody's lists are in memory
 #pragma unroll
   for (int q = 0; q < 2; q++) {
     if (!(rows >> (2 * w + q) & 1u)) continue;
     l[q].n = 0;
-    l[q].above = 0ull;
-    for (int sl = 0; sl < REP_SLICES; sl++)
-      for (int h = 0; h < TOPK_MAX; h += 64) rep_add(l[q], lists[((size_t)(group * REP_SLICES + sl) * 32 + 2 * w + q) * TOPK_MAX + h + lane], k);
-    rep_cut(l[q], k);
-    for (int h = lane; h < k; h += 64) topk_write(out_val, out_idx, idx64, (size_t)(32 * group + 2 * w + q) * k + h, l[q].ent[h]);
+    l[q].above = floor[q];
+    const unsigned long long* src = lists + (size_t)(2 * w + q) * slices * TOPK_MAX;
+    const int total = (int)__hip_atomic_load(p.count + (32 * group + 2 * w + q) * SEL_COUNT_STRIDE + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int h = lane; h - lane < total; h += 512) {   // (512 at once, or every 64 would be a memory latency)
+      unsigned long long e[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) e[u] = h + 64 * u < total ? src[h + 64 * u] : 0ull;
+#pragma unroll
+      for (int u = 0; u < 8; u++) rep_add(l[q], e[u], k, label_bits);
+    }
+    rep_cut(l[q], k, label_bits);
+    // best first
+    const unsigned long long e0 = lane < l[q].n ? l[q].ent[lane] : 0ull, e1 = lane + 64 < l[q].n ? l[q].ent[lane + 64] : 0ull;
+    int r0 = 0, r1 = 0;
+    for (int j = 0; j < l[q].n; j++) {
+      const unsigned long long o = l[q].ent[j];
+      r0 += o > e0 ? 1 : 0;
+      r1 += o > e1 ? 1 : 0;
+    }
+    const size_t at = (size_t)(32 * group + 2 * w + q) * k;
+    if (e0 != 0ull) topk_write(out_val, out_idx, idx64, at + r0, e0);
+    if (e1 != 0ull) topk_write(out_val, out_idx, idx64, at + r1, e1);
   }
 }
 
@@ -518,7 +620,7 @@ __global__ __launch_bounds__(REP_NT) void topk_pick_kernel(const SelectParams p,
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
   const int b = blockIdx.x, tid = threadIdx.x;
   if (b >= p.batch) {
-    topk_repair(p, b - p.batch, k, lists, out_val, out_idx, idx64, lds_raw);
+    topk_repair(p, b - p.batch, (int)gridDim.x - p.batch, k, lists, out_val, out_idx, idx64, lds_raw);
     return;
   }
   unsigned long long* ent = (unsigned long long*)lds_raw;
