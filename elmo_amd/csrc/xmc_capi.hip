@@ -65,9 +65,9 @@ void fill_device_info(int dev) {
   (void)hipFuncSetAttribute((const void*)fp8_forward_select_kernel<0, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, SelGeom<8>::LDS);
   (void)hipFuncSetAttribute((const void*)fp8_forward_select_kernel<1, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, SelGeom<8>::LDS);
   (void)hipFuncSetAttribute((const void*)topk_pick_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, REP_LDS > PICK_LDS ? REP_LDS : PICK_LDS);
-  (void)hipFuncSetAttribute((const void*)quad_sort_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (MAX_POS + 256) * 4);
   (void)hipFuncSetAttribute((const void*)quad_prep_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, MAX_POS * 4);
 #define XMC_TILED_ATTR(DD)                                                                                                                        \
+  (void)hipFuncSetAttribute((const void*)tiled_prep_kernel<DD>, hipFuncAttributeMaxDynamicSharedMemorySize, MAX_POS * 4);                          \
   (void)hipFuncSetAttribute((const void*)tiled_gradx_kernel<W_BF16, 1, DD>, hipFuncAttributeMaxDynamicSharedMemorySize, TgxGeom<W_BF16, 1, DD>::LDS); \
   (void)hipFuncSetAttribute((const void*)tiled_gradx_kernel<W_E4M3, 1, DD>, hipFuncAttributeMaxDynamicSharedMemorySize, TgxGeom<W_E4M3, 1, DD>::LDS); \
   (void)hipFuncSetAttribute((const void*)tiled_gradx_kernel<W_BF16, 2, DD>, hipFuncAttributeMaxDynamicSharedMemorySize, TgxGeom<W_BF16, 2, DD>::LDS); \
@@ -890,7 +890,6 @@ static int tiled_step_t(void* const* chunk_ptrs, int num_chunks, int rows_per_ch
   int* tile_ptr = (int*)(glb + halves * g_half);
   const size_t tp_stride = (size_t)(num_tiles + 1 + 63) / 64 * 64;   // entries of one pair's tile_ptr
   float* loss_part = (float*)(tile_ptr + pairs * tp_stride);         // one share per sub-tile of 32 rows
-  const int n_pad = (nnz + 63) / 64 * 64;   // whole blocks of the sort
 
   // chunks per segment of the label space: a multiple of the launch group, fewer than 2^24 - 1 labels
   int seg_chunks = ((1 << 24) - 2) / rows_per_chunk / group * group;
@@ -899,24 +898,17 @@ static int tiled_step_t(void* const* chunk_ptrs, int num_chunks, int rows_per_ch
   const bool fp8_logits = weight_type == W_E4M3 && quantize_x && halves >= 2 && !loss_out;
   // e4m3 weights, two batch halves, no compensated head: the feature-split update kernel (X^T in registers)
   const bool split_update = weight_type == W_E4M3 && halves == 2 && kahan_type == 0 && DD == D;
-  tiled_prep_x_kernel<DD><<<(halves * BP * DD + 255) / 256, 256, 0, stream>>>((const unsigned short*)x_bf16, batch, halves, quantize_x,
-                                                                        fp8_logits ? 1 : 0, split_update ? 1 : 0, xb, xT, gx_total,
-                                                                        loss_part, loss_out ? 2 * num_tiles : 0, (int*)((unsigned char*)workspace + TW_ERR), dp);
   for (int c = 0; c < num_chunks; c += group) {
     const int seg0 = c / seg_chunks * seg_chunks;   // first chunk of the segment
     if (c == seg0) {
-      // the segment's positives of every 256 batch rows as their own sorted list (the key keeps eight bits for the row),
-      // and the first key of each of its tiles
-      const int seg_n = seg0 + seg_chunks <= num_chunks ? seg_chunks : num_chunks - seg0;
-      for (int pr = 0; pr < pairs; pr++) {
-        if (n_pad > 0)
-          quad_sort_kernel<<<n_pad / 64, 256, (size_t)(n_pad + 256) * 4, stream>>>(labels_coo, nnz, n_pad, batch, 256 * pr,
-                                                                                seg0 * rows_per_chunk, seg_n * rows_per_chunk,
-                                                                                keys + (size_t)pr * MAX_POS);
-        tile_ptr_kernel<<<(seg_n * tiles_per_chunk + 1 + 255) / 256, 256, 0, stream>>>(
-            keys + (size_t)pr * MAX_POS, n_pad, rows_per_chunk, tiles_per_chunk, seg_n * tiles_per_chunk,
-            tile_ptr + pr * tp_stride + seg0 * tiles_per_chunk);
-      }
+      // the segment's positives of every 256 batch rows as a list of their own (the key keeps eight bits for the row), grouped by
+      // tile, and the first key of each of its tiles; in front of the first segment the images of X besides
+      const int seg_n = seg0 + seg_chunks <= num_chunks ? seg_chunks : num_chunks - seg0, seg_tiles = seg_n * tiles_per_chunk;
+      const int ptr_blocks = (seg_tiles + PREP_NT) / PREP_NT, x_blocks = c == 0 ? (halves * BP * DD + PREP_NT - 1) / PREP_NT : 0;
+      const TiledPrep pp = {labels_coo, nnz, batch, seg0 * rows_per_chunk, seg_n * rows_per_chunk, rows_per_chunk, tiles_per_chunk, seg_tiles, ptr_blocks, pairs,
+                            keys, tile_ptr + seg0 * tiles_per_chunk, tp_stride, (const unsigned short*)x_bf16, halves, quantize_x, fp8_logits ? 1 : 0,
+                            split_update ? 1 : 0, xb, xT, gx_total, loss_part, loss_out ? 2 * num_tiles : 0, (int*)((unsigned char*)workspace + TW_ERR)};
+      tiled_prep_kernel<DD><<<ptr_blocks * pairs + x_blocks, PREP_NT, (size_t)nnz * 4, stream>>>(pp, dp);
     }
     void* w = chunk_ptrs[c];
     const int nch = c + group <= num_chunks ? group : num_chunks - c;                       // chunks of this launch
@@ -924,7 +916,7 @@ static int tiled_step_t(void* const* chunk_ptrs, int num_chunks, int rows_per_ch
     const int rp = (rows + TL - 1) / TL * TL;           // padded rows of this launch (the G buffers use the stride rows_buf)
     const int tiles = rp / TL;
     const unsigned label0 = (unsigned)c * (unsigned)rows_per_chunk;                  // global: the fast rounding's random words
-    const unsigned label0_seg = (unsigned)(c - seg0) * (unsigned)rows_per_chunk;     // within the segment: the sorted keys
+    const unsigned label0_seg = (unsigned)(c - seg0) * (unsigned)rows_per_chunk;     // within the segment: the keys
     TiledSeeds sd;
     for (int k = 0; k < T_GROUP; k++)
       sd.s[k] = seeds && k < nch ? (round_mode == XMC_ROUND_SR_FAST ? fast_seed(seeds[c + k]) : seeds[c + k]) : 0u;

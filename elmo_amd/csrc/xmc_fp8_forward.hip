@@ -1,5 +1,4 @@
-// Inference logits of the FP8 extreme-classifier layer for gfx950 (MI355X), top-k of them without storing them, and a small
-// kernel of the training paths: the first positive of every tile (tile_ptr_kernel).
+// Inference logits of the FP8 extreme-classifier layer for gfx950 (MI355X), and top-k of them without storing them.
 //
 // Reference semantics: src/xmc_classifiers/chunked_fp8xmc_clf.py:45-60 (xfc_forward).
 #include "xmc_common.h"
@@ -28,27 +27,6 @@ __global__ void prep_x_kernel(const unsigned short* x, int batch, int n, float i
   packed = __builtin_amdgcn_cvt_pk_fp8_f32(val(raw.y << 16), val(raw.y & 0xFFFF0000u), packed, true);
   const int w = b >> 5, nb = (b >> 4) & 1, ks = k >> 7, kgq = (k >> 5) & 3, jq = k & 31;
   *(int*)(xq + ((size_t)((w * 2 + nb) * 6 + ks) * 64 + ((b & 15) + 16 * kgq)) * 32 + jq) = packed;
-}
-
-// tile_ptr[t] = first key whose label >= first label of tile t; tile_ptr[num_tiles] = first key past the last tile
-__global__ void tile_ptr_kernel(const unsigned* keys, int n_pad, int rows_per_chunk, int tiles_per_chunk, int num_tiles,
-                                int* tile_ptr) {
-  int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t > num_tiles) return;
-  unsigned long long label0;
-  if (t == num_tiles) {
-    label0 = (unsigned long long)(num_tiles / tiles_per_chunk) * rows_per_chunk;
-  } else {
-    int c = t / tiles_per_chunk, tj = t - c * tiles_per_chunk;
-    label0 = (unsigned long long)c * rows_per_chunk + (unsigned long long)tj * TL;
-  }
-  unsigned long long bound = label0 << 8;
-  int lo = 0, hi = n_pad;
-  while (lo < hi) {
-    int mid = (lo + hi) >> 1;
-    if ((unsigned long long)keys[mid] < bound) lo = mid + 1; else hi = mid;
-  }
-  tile_ptr[t] = lo;
 }
 
 // Inference logits: out[b, label - col0] = bf16(zscale * sum_k Xq[b,k] W[label,k]) for the 32-label tiles

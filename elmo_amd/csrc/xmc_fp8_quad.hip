@@ -138,67 +138,6 @@ __device__ __forceinline__ unsigned positive_key(int2 e, int batch, int row0, in
   return (r >= 0 && r < 256 && r + row0 < batch && e.y >= 0 && lab >= 0 && lab < label_count && lab < (1 << 24) - 1) ? (((unsigned)lab << 8) | (unsigned)r) : 0xFFFFFFFFu;
 }
 
-// Sorts the positives by rank (the three-kernel form, whose kernels tell repeated keys by their neighbours).  Block b ranks keys 64b..64b+63 of the n_pad (a multiple of 64): every block
-// builds all keys in LDS ((n_pad + 256) * 4 bytes), its four wavefronts each count the keys that precede the block's own
-// over a quarter of the set (equal keys: the one that comes first in the input precedes), and the sum of the four counts
-// is the key's position in the output.  256 threads.  (Padded to whole blocks only: up to the next power of two, the
-// preparation of a step with 4,608 positives took 28 us; 17 now.)
-__global__ __launch_bounds__(256) void quad_sort_kernel(const int* coo, int nnz, int n_pad, int batch, int row0, int label_base,
-                                                        int label_count, unsigned* keys) {
-  const int block = (int)blockIdx.x;
-  // (aligned for the 16-byte reads below: behind a kernel's static LDS it would start at any word, and the sort of 4,608
-  // positives took 62 us instead of 28)
-  extern __shared__ __attribute__((aligned(16))) unsigned sk[];
-  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63;
-  // eight (row, label) pairs per thread in flight at a time: the loads miss every cache
-  const int2* coo2 = (const int2*)coo;
-  for (int i0 = tid; i0 < n_pad; i0 += 8 * 256) {
-    int2 e[8];
-#pragma unroll
-    for (int u = 0; u < 8; u++) {
-      const int i = i0 + u * 256;
-      e[u] = i < nnz ? coo2[i] : int2{-1, -1};
-    }
-#pragma unroll
-    for (int u = 0; u < 8; u++) {
-      const int i = i0 + u * 256;
-      if (i < n_pad) sk[i] = positive_key(e[u], batch, row0, label_base, label_count);
-    }
-  }
-  __syncthreads();
-  const int i0 = block * 64;
-  const unsigned mine = sk[i0 + l];
-  const int quarter = n_pad >> 2;
-  // keys in front of the workgroup's own 64 precede on <=, keys behind them on <, the own 64 by position; each part
-  // is a branch-free loop over groups of four so that several LDS reads are in flight
-  const int jb = w * quarter, je = (w + 1) * quarter;
-  const int e0 = min(je, max(jb, i0)), b2 = max(jb, min(je, i0 + 64));
-  const uint4* sk4 = (const uint4*)sk;
-  int rank = 0;
-#pragma unroll 4
-  for (int j = jb >> 2; j < e0 >> 2; j++) {
-    const uint4 o = sk4[j];
-    rank += (o.x <= mine) + (o.y <= mine) + (o.z <= mine) + (o.w <= mine);
-  }
-#pragma unroll 4
-  for (int j = b2 >> 2; j < je >> 2; j++) {
-    const uint4 o = sk4[j];
-    rank += (o.x < mine) + (o.y < mine) + (o.z < mine) + (o.w < mine);
-  }
-  if (e0 < b2) {   // the part of the own 64 keys that lies in this wavefront's quarter
-    const int me = i0 + l;
-    for (int j = e0; j < b2; j += 4) {
-      const uint4 o = sk4[j >> 2];
-      rank += (o.x < mine || (o.x == mine && j < me)) + (o.y < mine || (o.y == mine && j + 1 < me)) +
-              (o.z < mine || (o.z == mine && j + 2 < me)) + (o.w < mine || (o.w == mine && j + 3 < me));
-    }
-  }
-  unsigned* part = sk + n_pad;
-  part[tid] = (unsigned)rank;
-  __syncthreads();
-  if (w == 0) keys[part[l] + part[64 + l] + part[128 + l] + part[192 + l]] = mine;
-}
-
 // The positives of PREP_NT consecutive tiles, grouped by tile (the step kernels take a tile's in any order, repeated or not): keys
 // p0 .. p1-1 are those of tile t0 + tid.  The block reads all positives, counts those in front of its tiles and those in each of them,
 // and puts the latter behind one another.  Bound by latency: two passes over the positives, the second in LDS.  Until now they were

@@ -39,7 +39,7 @@ __host__ __device__ inline int tiled_halves(int batch) { return batch <= BP ? 1 
 struct TiledLayout {
   size_t xb;     // X   [halves][128][768] bf16 in operand order, rows beyond the batch zero
   size_t xt;     // X^T [halves][768][128] bf16 in operand order
-  size_t keys;   // sorted positive keys, one list of MAX_POS entries per pair of halves (key = label*256 + row in the pair)
+  size_t keys;   // positive keys grouped by tile, one list of MAX_POS entries per pair of halves (key = label*256 + row in the pair)
   size_t gx;     // grad_X total, fp32 [halves*128][768]
   size_t part;   // grad_X partials [halves][T_SPLITS][128*768] fp32
   size_t g;      // per half: G then G^T, rows_pad x 128 bf16 each, in operand order; then tile_ptr per pair, loss shares
@@ -83,10 +83,9 @@ __device__ __forceinline__ bf16x8 t_load_w8(const void* w, size_t idx) {
 // of 32 batch rows, 8 over both halves][lane][8], row 4kq + e of block cg being feature 12kq + 4cg + e of the wavefront's 48.
 // DD: features of the layer (768, or 1024 = 4 x 4 x 64; every kernel of this path takes it as its last template argument).
 template <int DD>
-__global__ void tiled_prep_x_kernel(const unsigned short* x, int batch, int halves, int quantize, int fp8_image, int xt_split,
-                                    unsigned short* xb, unsigned short* xT, float* gx_total, float* loss_part, int n_loss,
-                                    int* err, const DropoutParams dp) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void tiled_prep_x_thread(int i, const unsigned short* x, int batch, int halves, int quantize, int fp8_image,
+                                                    int xt_split, unsigned short* xb, unsigned short* xT, float* gx_total, float* loss_part,
+                                                    int n_loss, int* err, const DropoutParams& dp) {
   if (i == 0) *err = 0;   // these kernels do not wait for one another: their steps cannot fail
   if (i >= halves * BP * DD) return;
   gx_total[i] = 0.f;
@@ -117,6 +116,33 @@ __global__ void tiled_prep_x_kernel(const unsigned short* x, int batch, int halv
   } else {
     xT[(size_t)half * BP * DD + ((size_t)(blk * (BP / 32) + (bh >> 5)) * 64 + (4 * kgk + e) + 16 * ((bh >> 3) & 3)) * 8 + (bh & 7)] = v;
   }
+}
+
+// The launch in front of a segment's chunks, PREP_NT threads a block: ptr_blocks per pair of batch halves group the segment's positives by
+// 64-row tile and write the first key of each, the others (in front of the first segment only) prepare X.  Bound by latency.  Before,
+// the images of X and, for every pair, a rank sort and a search for each tile's first key were launches one behind the other, and the
+// logits kernels went through a tile's keys one by one for every wavefront (a third of all positives lies in the first tile).  us a
+// step, 1,024 features, then / now: FP8 sr_fast, 19,655 labels, batch 448, 9.6 positives a row 419 / 154, 46 K, 208, 5.2 195 / 131,
+// 300 K, 96, 5 416 / 402; e4m3 with bf16 products, nearest, 8 K, 200, 36 451 / 74; bf16, nearest, 300 K, 256, 5 915 / 873.
+struct TiledPrep {
+  const int* coo; int nnz, batch, label_base, label_count, rows_per_chunk, tiles_per_chunk, num_tiles, ptr_blocks, pairs;
+  unsigned* keys; int* tile_ptr; size_t tp_stride;
+  const unsigned short* x; int halves, quantize, fp8_image, xt_split;
+  unsigned short* xb; unsigned short* xT; float* gx_total; float* loss_part; int n_loss; int* err;
+};
+template <int DD>
+__global__ __launch_bounds__(PREP_NT) void tiled_prep_kernel(const TiledPrep p, const DropoutParams dp) {
+  const int blk = blockIdx.x;
+  if (blk < p.ptr_blocks * p.pairs) {
+    const int pr = blk / p.ptr_blocks, t0 = (blk - pr * p.ptr_blocks) * PREP_NT, t = t0 + (int)threadIdx.x;
+    int p0, p1;
+    group_positives_block(t0, p.coo, p.nnz, p.batch, 256 * pr, p.label_base, p.label_count, p.rows_per_chunk, 1.0f / (float)p.rows_per_chunk,
+                          p.tiles_per_chunk, p.keys + (size_t)pr * MAX_POS, &p0, &p1);
+    if (t <= p.num_tiles) p.tile_ptr[pr * p.tp_stride + t] = p0;
+    return;
+  }
+  tiled_prep_x_thread<DD>((blk - p.ptr_blocks * p.pairs) * PREP_NT + (int)threadIdx.x, p.x, p.batch, p.halves, p.quantize, p.fp8_image, p.xt_split, p.xb,
+                          p.xT, p.gx_total, p.loss_part, p.n_loss, p.err, dp);
 }
 
 // ---- logits, sigmoid minus targets.  Persistent workgroups of 8 wavefronts; wavefront v keeps the X operand of batch
@@ -152,6 +178,26 @@ __device__ __forceinline__ void t_lds_load16(const unsigned char* g, unsigned ld
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(ldsoff), "v"(g) : "memory", "m0");
 }
 
+__device__ __forceinline__ float t_bf16_half(unsigned pair, int upper) { return __uint_as_float(upper ? pair & 0xFFFF0000u : pair << 16); }
+
+// G of a lane's four consecutive labels r0.. of one batch row (bf16, two to a word; zero for labels past the last): to `gt` in operand
+// order for grad_X (block (label / 32, batch block) of 16 batch rows x 32 labels), and, label-major (32 bytes a label), to the wavefront's
+// KiB of LDS, through which its 32 labels x 16 batch rows are transposed for the update kernel.
+__device__ __forceinline__ void t_store_g(const unsigned (&sg)[2], int r0, int rows, unsigned short* gt, __attribute__((address_space(3))) unsigned char* stg) {
+  unsigned s01 = sg[0], s23 = sg[1];
+  if (r0 + 3 >= rows) {
+    if (r0 >= rows) s01 &= 0xFFFF0000u;
+    if (r0 + 1 >= rows) s01 &= 0x0000FFFFu;
+    if (r0 + 2 >= rows) s23 &= 0xFFFF0000u;
+    s23 &= 0x0000FFFFu;
+  }
+  *(uint2*)gt = uint2{s01, s23};
+  *(__attribute__((address_space(3))) unsigned short*)stg = (unsigned short)s01;
+  *(__attribute__((address_space(3))) unsigned short*)(stg + 32) = (unsigned short)(s01 >> 16);
+  *(__attribute__((address_space(3))) unsigned short*)(stg + 64) = (unsigned short)s23;
+  *(__attribute__((address_space(3))) unsigned short*)(stg + 96) = (unsigned short)(s23 >> 16);
+}
+
 // Vector memory operations retire in order.  Per sub-tile a wavefront issues its loads of the sub-tile two steps ahead
 // (always, past the end they fetch the last sub-tile again into a buffer nobody reads, so that the count is the same in
 // every step) and then ten stores of G.  The wait at the top of a step leaves in flight what was issued after the
@@ -168,9 +214,9 @@ __global__ __launch_bounds__(512, 1) void tiled_logits_kernel(const void* w, int
   // no static LDS in this kernel: the direct-to-LDS loads address LDS from byte 0
   __attribute__((address_space(3))) float* wsum = (__attribute__((address_space(3))) float*)(lds + NB * G::BUF);
   const int tid = threadIdx.x, v = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l16 = lane & 15, kg = lane >> 4;
-  // the sorted keys and the tile ranges were written by earlier launches: read them through the scalar (constant) path,
-  // so that no vector-memory wait of this loop covers them
-  const __attribute__((address_space(4))) unsigned* ckeys = (const __attribute__((address_space(4))) unsigned*)keys;
+  // the tile ranges were written by an earlier launch: read them through the scalar (constant) path, so that no vector-memory
+  // wait of this loop covers them.  (So are a tile's keys, up to eight.  More are vector loads that are waited for where they
+  // are used: whatever was issued before them is then complete too, and the waits counted by hand become stricter only.)
   const __attribute__((address_space(4))) int* ctile_ptr = (const __attribute__((address_space(4))) int*)tile_ptr;
   // source row and byte offset within the row of this lane's slot in pieces v, v+8, ..
   int prow[G::PER_WAVE], pcol[G::PER_WAVE];
@@ -242,64 +288,40 @@ __global__ __launch_bounds__(512, 1) void tiled_logits_kernel(const void* w, int
     }
     // acc[lb][e] = Z[label 32 st + 16 lb + 4kg + e][batch 16v + l16]
     float lsum = 0.f;
-    float sg[2][4], zf[2][4];
+    unsigned sg[2][2], zp[2][2];   // sigmoids and logits, four bf16 values each
 #pragma unroll
     for (int lb = 0; lb < 2; lb++) {
       const int r0 = st * TLG_ROWS + 16 * lb;
+      zp[lb][0] = bf16_pack2(acc[lb][0], acc[lb][1]);
+      zp[lb][1] = bf16_pack2(acc[lb][2], acc[lb][3]);
+      float s[4];
 #pragma unroll
       for (int e = 0; e < 4; e++) {
-        zf[lb][e] = bf16_rt(acc[lb][e]);
-        sg[lb][e] = bf16_rt(__builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(zf[lb][e] * nlog2e)));
+        const float z = t_bf16_half(zp[lb][e >> 1], e & 1);
+        s[e] = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(z * nlog2e));
         if (LOSS && r0 + 4 * kg + e < rows && (int)brow0 + 16 * v + l16 < batch)
-          lsum += __builtin_fmaxf(zf[lb][e], 0.f) + 0.69314718055994530942f * __builtin_amdgcn_logf(1.0f + __builtin_amdgcn_exp2f(-__builtin_fabsf(zf[lb][e]) * 1.44269504088896340736f));
+          lsum += __builtin_fmaxf(z, 0.f) + 0.69314718055994530942f * __builtin_amdgcn_logf(1.0f + __builtin_amdgcn_exp2f(-__builtin_fabsf(z) * 1.44269504088896340736f));
       }
+      sg[lb][0] = bf16_pack2(s[0], s[1]);
+      sg[lb][1] = bf16_pack2(s[2], s[3]);
     }
-    // Positives of the enclosing 64-row tile (set semantics: a repeated key counts once).  The keys come eight at a time
-    // through the scalar path (the first tiles of a chunk sorted by label frequency hold hundreds), and a key costs vector
-    // instructions only if it lies in this wavefront's block (the sub-tile's 32 labels, batch rows 16v.. of this half).
-    // Up to seven keys behind the tile's last are read and ignored; the buffer behind the keys belongs to the workspace.
-    if (p1 > p0) {
-      typedef unsigned t_keysx8 __attribute__((ext_vector_type(8), aligned(4)));
-      const unsigned lbase = label0_chunk + (unsigned)(st * TLG_ROWS);
-      unsigned prev = p0 > 0 ? ckeys[p0 - 1] : ~ckeys[p0];
-      for (int e0 = p0; e0 < p1; e0 += 8) {
-        const t_keysx8 kk = *(const __attribute__((address_space(4))) t_keysx8*)(ckeys + e0);
+    if (p1 > p0) {   // positives of the enclosing 64-row tile; the bits of many go through the wavefront's staging, which is free here
+      const unsigned hit = positive_hits<32, 16>(keys, p0, p1, label0_chunk + (unsigned)(st * TLG_ROWS), brow0 + (unsigned)(16 * v), (unsigned)lane, stg);
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-          const unsigned key = kk[j];
-          const unsigned lrel = (key >> 8) - lbase;      // label within the sub-tile
-          const unsigned b = (key & 255u) - brow0;       // batch row within this half
-          if (e0 + j < p1 && key != prev && lrel < (unsigned)TLG_ROWS && (b >> 4) == (unsigned)v) {
-            const bool mine = (unsigned)kg == ((lrel >> 2) & 3u) && (unsigned)l16 == (b & 15u);
-            const unsigned sel = ((lrel >> 4) << 2) | (lrel & 3u);   // wave-uniform: label block and one of the lane's four labels
+      for (int lb = 0; lb < 2; lb++) {
+        sg[lb][0] = minus_hits(sg[lb][0], hit, 4 * lb);
+        sg[lb][1] = minus_hits(sg[lb][1], hit, 4 * lb + 2);
+        if (LOSS) {
 #pragma unroll
-            for (int c = 0; c < 8; c++)
-              if (sel == (unsigned)c) {
-                if (LOSS && st * TLG_ROWS + 16 * (c >> 2) + 4 * kg + (c & 3) < rows) lsum -= mine ? zf[c >> 2][c & 3] : 0.f;
-                sg[c >> 2][c & 3] = mine ? bf16_rt(sg[c >> 2][c & 3] - 1.0f) : sg[c >> 2][c & 3];
-              }
-          }
-          prev = key;
+          for (int e = 0; e < 4; e++)
+            if (((hit >> (4 * lb + e)) & 1u) && st * TLG_ROWS + 16 * lb + 4 * kg + e < rows) lsum -= t_bf16_half(zp[lb][e >> 1], e & 1);
         }
       }
     }
 #pragma unroll
-    for (int lb = 0; lb < 2; lb++) {
-      const int r0 = st * TLG_ROWS + 16 * lb;
-      unsigned short sb[4];
-#pragma unroll
-      for (int e = 0; e < 4; e++) sb[e] = (r0 + 4 * kg + e < rows) ? bf16_bits(sg[lb][e]) : (unsigned short)0;
-      uint2 o;
-      o.x = (unsigned)sb[0] | ((unsigned)sb[1] << 16);
-      o.y = (unsigned)sb[2] | ((unsigned)sb[3] << 16);
-      // G^T in operand order for grad_X: block (label / 32, batch block) of 16 batch rows x 32 labels
-      *(uint2*)(gbl + ((size_t)(st * 8 + v) * 64 + l16 + 16 * (2 * lb + (kg >> 1))) * 8 + 4 * (kg & 1)) = o;
-      // G for the update kernel: this wavefront's 32 labels x 16 batch rows, transposed through its own KiB of LDS
-      // (label-major, 32 bytes per label)
-#pragma unroll
-      for (int e = 0; e < 4; e++)
-        *(__attribute__((address_space(3))) unsigned short*)(stg + (16 * lb + 4 * kg + e) * 32 + 2 * l16) = sb[e];
-    }
+    for (int lb = 0; lb < 2; lb++)
+      t_store_g(sg[lb], st * TLG_ROWS + 16 * lb + 4 * kg, rows, gbl + ((size_t)(st * 8 + v) * 64 + l16 + 16 * (2 * lb + (kg >> 1))) * 8 + 4 * (kg & 1),
+                stg + (16 * lb + 4 * kg) * 32 + 2 * l16);
     {
       // ... and stored in the operand order of A = G X: block (16 labels, 32 batch rows) = 64 lanes x 8 batch rows,
       // lane = label + 16 * (batch row / 8).  This wavefront's batch rows are half of K step v / 2: lanes 0..31 store
@@ -326,7 +348,7 @@ __global__ __launch_bounds__(512, 1) void tiled_logits_kernel(const void* w, int
 //      e4m3 operand of batch rows 16v.. of BOTH halves (96 registers, as the bf16 operand of one half took): one pass over
 //      the weights yields the G of 256 batch rows.  Tile loop, positives, rounding and both layouts of G as above; the
 //      products are exact in fp32 either way, only the order of the fp32 sums differs from the bf16 form.
-//      xq: e4m3 image of the pair's X in B-operand order, [half][(16-row block)*6 + ks][lane][32 bytes] (tiled_prep_x_kernel)
+//      xq: e4m3 image of the pair's X in B-operand order, [half][(16-row block)*6 + ks][lane][32 bytes] (tiled_prep_x_thread)
 template <int DD>
 __global__ __launch_bounds__(512, 1) void tiled_logits_fp8_kernel(const void* w, int rows, int nsub, const unsigned char* xq,
                                                                   const unsigned* keys, const int* tile_ptr, unsigned label0_chunk,
@@ -337,7 +359,6 @@ __global__ __launch_bounds__(512, 1) void tiled_logits_fp8_kernel(const void* w,
   extern __shared__ __attribute__((aligned(16))) unsigned char tlg_lds[];
   __attribute__((address_space(3))) unsigned char* lds = (__attribute__((address_space(3))) unsigned char*)tlg_lds;
   const int tid = threadIdx.x, v = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l16 = lane & 15, kg = lane >> 4;
-  const __attribute__((address_space(4))) unsigned* ckeys = (const __attribute__((address_space(4))) unsigned*)keys;
   const __attribute__((address_space(4))) int* ctile_ptr = (const __attribute__((address_space(4))) int*)tile_ptr;
   int prow[G::PER_WAVE], pcol[G::PER_WAVE];
 #pragma unroll
@@ -406,51 +427,30 @@ __global__ __launch_bounds__(512, 1) void tiled_logits_fp8_kernel(const void* w,
     // acc[lb][hf][e] = Z[label 32 st + 16 lb + 4kg + e][batch 128 hf + 16v + l16]
 #pragma unroll
     for (int hf = 0; hf < 2; hf++) {
-      float sg[2][4];
+      unsigned sg[2][2];   // sigmoids, four bf16 values each
 #pragma unroll
-      for (int lb = 0; lb < 2; lb++)
+      for (int lb = 0; lb < 2; lb++) {
+        float s[4];
 #pragma unroll
-        for (int e = 0; e < 4; e++)
-          sg[lb][e] = bf16_rt(__builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(bf16_rt(acc[lb][hf][e]) * nlog2e)));
+        for (int e = 0; e < 4; e++) s[e] = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(bf16_rt(acc[lb][hf][e]) * nlog2e));
+        sg[lb][0] = bf16_pack2(s[0], s[1]);
+        sg[lb][1] = bf16_pack2(s[2], s[3]);
+      }
       // positives of the enclosing 64-row tile, as in tiled_logits_kernel; the keys hold the row within the pair of halves
       if (p1 > p0) {
-        typedef unsigned t_keysx8 __attribute__((ext_vector_type(8), aligned(4)));
-        const unsigned lbase = label0_chunk + (unsigned)(st * TLG_ROWS);
-        unsigned prev = p0 > 0 ? ckeys[p0 - 1] : ~ckeys[p0];
-        for (int e0 = p0; e0 < p1; e0 += 8) {
-          const t_keysx8 kk = *(const __attribute__((address_space(4))) t_keysx8*)(ckeys + e0);
+        const unsigned hit = positive_hits<32, 16>(keys, p0, p1, label0_chunk + (unsigned)(st * TLG_ROWS), (unsigned)(BP * hf + 16 * v), (unsigned)lane, stg);
 #pragma unroll
-          for (int j = 0; j < 8; j++) {
-            const unsigned key = kk[j];
-            const unsigned lrel = (key >> 8) - lbase;                  // label within the sub-tile
-            const unsigned b = (key & 255u) - (unsigned)(BP * hf);     // batch row within this half
-            if (e0 + j < p1 && key != prev && lrel < (unsigned)TLG_ROWS && (b >> 4) == (unsigned)v) {
-              const bool mine = (unsigned)kg == ((lrel >> 2) & 3u) && (unsigned)l16 == (b & 15u);
-              const unsigned sel = ((lrel >> 4) << 2) | (lrel & 3u);
-#pragma unroll
-              for (int c = 0; c < 8; c++)
-                if (sel == (unsigned)c) sg[c >> 2][c & 3] = mine ? bf16_rt(sg[c >> 2][c & 3] - 1.0f) : sg[c >> 2][c & 3];
-            }
-            prev = key;
-          }
+        for (int lb = 0; lb < 2; lb++) {
+          sg[lb][0] = minus_hits(sg[lb][0], hit, 4 * lb);
+          sg[lb][1] = minus_hits(sg[lb][1], hit, 4 * lb + 2);
         }
       }
       unsigned short* gl = glb + (size_t)hf * g_half;
       unsigned short* gb = gbl + (size_t)hf * g_half;
 #pragma unroll
-      for (int lb = 0; lb < 2; lb++) {
-        const int r0 = st * TLG_ROWS + 16 * lb;
-        unsigned short sb[4];
-#pragma unroll
-        for (int e = 0; e < 4; e++) sb[e] = (r0 + 4 * kg + e < rows) ? bf16_bits(sg[lb][e]) : (unsigned short)0;
-        uint2 o;
-        o.x = (unsigned)sb[0] | ((unsigned)sb[1] << 16);
-        o.y = (unsigned)sb[2] | ((unsigned)sb[3] << 16);
-        *(uint2*)(gb + ((size_t)(st * 8 + v) * 64 + l16 + 16 * (2 * lb + (kg >> 1))) * 8 + 4 * (kg & 1)) = o;
-#pragma unroll
-        for (int e = 0; e < 4; e++)
-          *(__attribute__((address_space(3))) unsigned short*)(stg + (16 * lb + 4 * kg + e) * 32 + 2 * l16) = sb[e];
-      }
+      for (int lb = 0; lb < 2; lb++)
+        t_store_g(sg[lb], st * TLG_ROWS + 16 * lb + 4 * kg, rows, gb + ((size_t)(st * 8 + v) * 64 + l16 + 16 * (2 * lb + (kg >> 1))) * 8 + 4 * (kg & 1),
+                  stg + (16 * lb + 4 * kg) * 32 + 2 * l16);
       {
         const int lbo = lane >> 5, half = (lane >> 4) & 1;
         const intx4 gq = *(const __attribute__((address_space(3))) intx4*)(stg + (lane & 15) * 32 + 512 * lbo + 16 * half);
@@ -641,7 +641,7 @@ __global__ void tiled_finalize_kernel(const float* gx_total, int batch, unsigned
 
 // ---- grad_W and the SGD update of one chunk, in place.  blockIdx = tile*4 + fb; wavefront w owns label rows 16w..16w+15
 //      of the tile and features 192fb.. (12 blocks of 16).  A^T[f][l] = sum_b X^T[f][b] G[l][b].  The rows of a feature
-//      block are permuted (row 4kg+e of block nn = 4c+q is feature 192fb + 64c + 16kg + 4q + e, see tiled_prep_x_kernel)
+//      block are permuted (row 4kg+e of block nn = 4c+q is feature 192fb + 64c + 16kg + 4q + e, see tiled_prep_x_thread)
 //      so that a lane ends up with 16 consecutive features of one label row per step c, and the four lanes of a row
 //      with 64 consecutive bytes.
 //        bf16 weights : a = bf16(A); t = w - lr*a; RTN: bf16(t);  SR: bits(t) + (philox(seed, l*768+f) & 0xFFFF), clear 16 bits
@@ -912,7 +912,7 @@ __global__ __launch_bounds__(HALVES == 1 ? 256 : 512, HALVES == 1 ? 3 : HALVES =
 //      the tile's G - 32 KiB, already in operand order in memory - goes straight to LDS once per workgroup, two buffers,
 //      and every wavefront reads its 32 blocks from there: a third of the LDS traffic.  A^T[48 features x 16 rows] per
 //      row block, the features of a block permuted (row 4kg + e of block cg is feature 12kg + 4cg + e of the 48, see
-//      tiled_prep_x_kernel) so that a lane ends up with 12 consecutive bytes of one weight row.  Persistent: stream s of
+//      tiled_prep_x_thread) so that a lane ends up with 12 consecutive bytes of one weight row.  Persistent: stream s of
 //      the launch walks tiles s, s + streams, ...; its four workgroups (one per feature quarter) sit on one XCD, eight
 //      apart in launch order, and share the tile's G through that XCD's L2.  The first workgroups sum the grad_X
 //      partials, as in tiled_update_kernel.  Same arithmetic, rounding modes and random words as there.

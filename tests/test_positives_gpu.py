@@ -5,6 +5,7 @@ import pytest
 
 import helpers as H
 import test_cluster_gpu as T
+import test_three_kernel_gpu as K
 from test_fp8_step_gpu import check_rtn
 
 pytestmark = pytest.mark.gpu
@@ -39,3 +40,20 @@ def test_one_pass_step(gpu, kind, batch, n, monkeypatch):
     monkeypatch.setattr(H, "make_case", lambda *a, **k: dict(make_case(*a, **k), labels=labels))
     monkeypatch.setattr(T, "bf16_case", lambda *a, **k: bf16_case(*a, **k)[:2] + (labels,))
     T.test_one_pass_step_matches_the_oracle(gpu, kind, 3, ROWS, batch, "rtn")
+
+
+@pytest.mark.parametrize("kind,batch", [("bf16", 20), ("bf16", 300), ("sim", 128), ("fp8", 64), ("fp8", 300)])
+@pytest.mark.parametrize("n", [8, 9, 257, 5000])
+def test_three_kernel_step(gpu, kind, batch, n, monkeypatch):
+    labels = crowded(n, batch, ROWS)
+    make_case, bf16_case = H.make_case, K.bf16_case
+    monkeypatch.setattr(H, "make_case", lambda *a, **k: dict(make_case(*a, **k), labels=labels))
+    monkeypatch.setattr(K, "bf16_case", lambda *a, **k: bf16_case(*a, **k)[:2] + (labels,))
+    K.test_step_with_weight_decay_matches_the_oracle(gpu, kind, 3, ROWS, batch, "rtn")
+
+
+@pytest.mark.parametrize("n", [9, 5000])
+def test_loss(gpu, n, monkeypatch):
+    labels, bf16_case = crowded(n, 300, ROWS), K.bf16_case
+    monkeypatch.setattr(K, "bf16_case", lambda *a, **k: bf16_case(*a, **k)[:2] + (labels,))
+    K.test_loss_over_four_halves(gpu)
