@@ -84,7 +84,7 @@ void fill_device_info(int dev) {
   (void)hipFuncSetAttribute((const void*)tiled_update2_kernel<ROUND_SR_PHILOX>, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * TU2_GBUF);
   (void)hipFuncSetAttribute((const void*)tiled_update2_kernel<ROUND_SR_FAST>, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * TU2_GBUF);
   // the update kernels with two batch halves keep 96 KiB of operands in LDS, more than the default limit
-#define XMC_UPD_ATTR_D(WTYPE, RMODE, KH, DD) (void)hipFuncSetAttribute((const void*)tiled_update_kernel<WTYPE, RMODE, 2, KH, DD>, hipFuncAttributeMaxDynamicSharedMemorySize, tup_lds_bytes(2, DD))
+#define XMC_UPD_ATTR_D(WTYPE, RMODE, KH, DD) (void)hipFuncSetAttribute((const void*)tiled_update_kernel<WTYPE, RMODE, 2, KH, DD, BP / 32>, hipFuncAttributeMaxDynamicSharedMemorySize, tup_lds_bytes(2, DD))
 #define XMC_UPD_ATTR(WTYPE, RMODE, KH) XMC_UPD_ATTR_D(WTYPE, RMODE, KH, D); XMC_UPD_ATTR_D(WTYPE, RMODE, KH, 1024)
   XMC_UPD_ATTR(W_BF16, ROUND_RTN, false); XMC_UPD_ATTR(W_BF16, ROUND_SR_PHILOX, false); XMC_UPD_ATTR(W_BF16, ROUND_SR_FAST, false);
   XMC_UPD_ATTR(W_E4M3, ROUND_RTN, false); XMC_UPD_ATTR(W_E4M3, ROUND_SR_PHILOX, false); XMC_UPD_ATTR(W_E4M3, ROUND_SR_FAST, false);
@@ -898,6 +898,8 @@ static int tiled_step_t(void* const* chunk_ptrs, int num_chunks, int rows_per_ch
   const bool fp8_logits = weight_type == W_E4M3 && quantize_x && halves >= 2 && !loss_out;
   // e4m3 weights, two batch halves, no compensated head: the feature-split update kernel (X^T in registers)
   const bool split_update = weight_type == W_E4M3 && halves == 2 && kahan_type == 0 && DD == D;
+  // batch rows whose G is written and read; the feature-split update reads the G of both halves whole
+  const int live = split_update ? halves * BP : batch;
   for (int c = 0; c < num_chunks; c += group) {
     const int seg0 = c / seg_chunks * seg_chunks;   // first chunk of the segment
     if (c == seg0) {
@@ -933,9 +935,10 @@ static int tiled_step_t(void* const* chunk_ptrs, int num_chunks, int rows_per_ch
       const int nsub = 2 * tiles, lgrid = nsub < di.cus ? nsub : di.cus;
       tiled_logits_fp8_kernel<DD><<<lgrid, 512, TlgGeom<W_E4M3, DD>::LDS, stream>>>(
           w, rows, nsub, (const unsigned char*)xb + (size_t)hh * BP * DD, keys + (size_t)(hh >> 1) * MAX_POS,
-          tile_ptr + (hh >> 1) * tp_stride + c * tiles_per_chunk, label0_seg, glb + hh * g_half, gbl + hh * g_half, g_half);
+          tile_ptr + (hh >> 1) * tp_stride + c * tiles_per_chunk, label0_seg, glb + hh * g_half, gbl + hh * g_half, g_half, live - hh * BP);
     }
     for (int hh = 0; !fp8_logits && hh < halves; hh++) {
+      if (hh * BP >= live && !loss_out) break;   // (a loss is summed over every launch's tiles)
       unsigned short* gl = glb + hh * g_half;
       unsigned short* gb = gbl + hh * g_half;
       const unsigned short* xh = xb + (size_t)hh * BP * DD;
@@ -946,11 +949,11 @@ static int tiled_step_t(void* const* chunk_ptrs, int num_chunks, int rows_per_ch
       const int nsub = 2 * tiles;                                   // sub-tiles of 32 label rows
       const int lgrid = nsub < di.cus ? nsub : di.cus;              // persistent: one workgroup per compute unit
       if (weight_type == W_BF16) {
-        if (loss_out) tiled_logits_kernel<W_BF16, true, DD><<<lgrid, 512, TlgGeom<W_BF16, DD>::LDS, stream>>>(w, rows, nsub, xh, kh, tp, label0_seg, gl, gb, pbatch, brow0, lp);
-        else tiled_logits_kernel<W_BF16, false, DD><<<lgrid, 512, TlgGeom<W_BF16, DD>::LDS, stream>>>(w, rows, nsub, xh, kh, tp, label0_seg, gl, gb, pbatch, brow0, lp);
+        if (loss_out) tiled_logits_kernel<W_BF16, true, DD><<<lgrid, 512, TlgGeom<W_BF16, DD>::LDS, stream>>>(w, rows, nsub, xh, kh, tp, label0_seg, gl, gb, pbatch, brow0, live - hh * BP, lp);
+        else tiled_logits_kernel<W_BF16, false, DD><<<lgrid, 512, TlgGeom<W_BF16, DD>::LDS, stream>>>(w, rows, nsub, xh, kh, tp, label0_seg, gl, gb, pbatch, brow0, live - hh * BP, lp);
       } else {
-        if (loss_out) tiled_logits_kernel<W_E4M3, true, DD><<<lgrid, 512, TlgGeom<W_E4M3, DD>::LDS, stream>>>(w, rows, nsub, xh, kh, tp, label0_seg, gl, gb, pbatch, brow0, lp);
-        else tiled_logits_kernel<W_E4M3, false, DD><<<lgrid, 512, TlgGeom<W_E4M3, DD>::LDS, stream>>>(w, rows, nsub, xh, kh, tp, label0_seg, gl, gb, pbatch, brow0, lp);
+        if (loss_out) tiled_logits_kernel<W_E4M3, true, DD><<<lgrid, 512, TlgGeom<W_E4M3, DD>::LDS, stream>>>(w, rows, nsub, xh, kh, tp, label0_seg, gl, gb, pbatch, brow0, live - hh * BP, lp);
+        else tiled_logits_kernel<W_E4M3, false, DD><<<lgrid, 512, TlgGeom<W_E4M3, DD>::LDS, stream>>>(w, rows, nsub, xh, kh, tp, label0_seg, gl, gb, pbatch, brow0, live - hh * BP, lp);
       }
     }
     // grad_X of the launch's chunks: one pass over W per pair of batch halves, then the fixed-order sums per half
@@ -960,25 +963,29 @@ static int tiled_step_t(void* const* chunk_ptrs, int num_chunks, int rows_per_ch
       const unsigned short* gsrc = gbl + h0 * g_half;
       floatx4* pdst = partial + h0 * part_half;
       if (weight_type == W_BF16) {
-        if (halves == 1) tiled_gradx_kernel<W_BF16, 1, DD><<<ggrid, 512, TgxGeom<W_BF16, 1, DD>::LDS, stream>>>(w, rows, (int)rows_buf, rp, range, cs, spc, gsrc, g_half, pdst, part_half);
-        else tiled_gradx_kernel<W_BF16, 2, DD><<<ggrid, 512, TgxGeom<W_BF16, 2, DD>::LDS, stream>>>(w, rows, (int)rows_buf, rp, range, cs, spc, gsrc, g_half, pdst, part_half);
+        if (halves == 1) tiled_gradx_kernel<W_BF16, 1, DD><<<ggrid, 512, TgxGeom<W_BF16, 1, DD>::LDS, stream>>>(w, rows, (int)rows_buf, rp, range, cs, spc, gsrc, g_half, live - h0 * BP, pdst, part_half);
+        else tiled_gradx_kernel<W_BF16, 2, DD><<<ggrid, 512, TgxGeom<W_BF16, 2, DD>::LDS, stream>>>(w, rows, (int)rows_buf, rp, range, cs, spc, gsrc, g_half, live - h0 * BP, pdst, part_half);
       } else {
-        if (halves == 1) tiled_gradx_kernel<W_E4M3, 1, DD><<<ggrid, 512, TgxGeom<W_E4M3, 1, DD>::LDS, stream>>>(w, rows, (int)rows_buf, rp, range, cs, spc, gsrc, g_half, pdst, part_half);
-        else tiled_gradx_kernel<W_E4M3, 2, DD><<<ggrid, 512, TgxGeom<W_E4M3, 2, DD>::LDS, stream>>>(w, rows, (int)rows_buf, rp, range, cs, spc, gsrc, g_half, pdst, part_half);
+        if (halves == 1) tiled_gradx_kernel<W_E4M3, 1, DD><<<ggrid, 512, TgxGeom<W_E4M3, 1, DD>::LDS, stream>>>(w, rows, (int)rows_buf, rp, range, cs, spc, gsrc, g_half, live - h0 * BP, pdst, part_half);
+        else tiled_gradx_kernel<W_E4M3, 2, DD><<<ggrid, 512, TgxGeom<W_E4M3, 2, DD>::LDS, stream>>>(w, rows, (int)rows_buf, rp, range, cs, spc, gsrc, g_half, live - h0 * BP, pdst, part_half);
       }
     }
     const int nsub_u = tup_threads(halves) / 256;    // tiles a workgroup of the update kernel works on at a time
     const int ugroups = (tiles + TUP_TILES * nsub_u - 1) / (TUP_TILES * nsub_u);   // rounded up to eight: see the kernel's index map
     const int ugrid = tred_waves(DD) * halves / (tup_threads(halves) / 64) + ((DD / 64) / tup_csteps(halves, DD)) * ((ugroups + 7) / 8 * 8);
-#define XMC_LAUNCH_UPDATE_K(WTYPE, RMODE, HV, KH)                                                                               \
-  tiled_update_kernel<WTYPE, RMODE, HV, KH, DD><<<ugrid, tup_threads(HV), (size_t)tup_lds_bytes(HV, DD), stream>>>(                           \
-      w, rows, tiles, glb, g_half, xT, lr, wd, sd, cs, saturate, kahan, kahan_type, nh, label0, partial, part_half, nch, spc, range, rp,  \
-      weight_type == W_BF16 ? 1 : 0, gx_total)
+    const bool final_sum = c + nch == num_chunks;
+    const TiledSum sum = {partial, part_half, nch, spc, range, rp, weight_type == W_BF16 ? 1 : 0, gx_total, batch,
+                          final_sum ? (unsigned short*)grad_x_bf16 : nullptr, final_sum ? grad_x_f32 : nullptr};
+#define XMC_LAUNCH_UPDATE_K(WTYPE, RMODE, HV, KH, NKS)                                                                          \
+  tiled_update_kernel<WTYPE, RMODE, HV, KH, DD, NKS><<<ugrid, tup_threads(HV), (size_t)tup_lds_bytes(HV, DD, NKS), stream>>>(   \
+      w, rows, tiles, glb, g_half, xT, lr, wd, sd, cs, saturate, kahan, kahan_type, nh, label0, live, sum, dp)
 #define XMC_LAUNCH_UPDATE_H(WTYPE, RMODE, KH)                                                                                  \
   do {                                                                                                                         \
-    if (halves == 1) XMC_LAUNCH_UPDATE_K(WTYPE, RMODE, 1, KH);                                                                 \
-    else if (halves == 2) XMC_LAUNCH_UPDATE_K(WTYPE, RMODE, 2, KH);                                                            \
-    else XMC_LAUNCH_UPDATE_K(WTYPE, RMODE, 4, KH);                                                                             \
+    if (halves == 1 && batch <= 32) XMC_LAUNCH_UPDATE_K(WTYPE, RMODE, 1, KH, 1);                                               \
+    else if (halves == 1 && batch <= 64) XMC_LAUNCH_UPDATE_K(WTYPE, RMODE, 1, KH, 2);                                          \
+    else if (halves == 1) XMC_LAUNCH_UPDATE_K(WTYPE, RMODE, 1, KH, 4);                                                         \
+    else if (halves == 2) XMC_LAUNCH_UPDATE_K(WTYPE, RMODE, 2, KH, 4);                                                         \
+    else XMC_LAUNCH_UPDATE_K(WTYPE, RMODE, 4, KH, 4);                                                                          \
   } while (0)
     const bool with_head = kahan_type != 0 && nh > 0;   // only chunk 0 of the head-Kahan layer
     if (split_update) {
@@ -987,7 +994,7 @@ static int tiled_step_t(void* const* chunk_ptrs, int num_chunks, int rows_per_ch
       const int grid2 = tred_waves(D) * 2 / 4 + 4 * streams;
 #define XMC_LAUNCH_UPDATE2(RMODE)                                                                                              \
   tiled_update2_kernel<RMODE><<<grid2, 256, 2 * TU2_GBUF, stream>>>(w, rows, tiles, glb, g_half, (const bf16x8*)xT, lr, wd, sd, cs, saturate, \
-                                                                    label0, partial, part_half, nch, spc, range, rp, gx_total)
+                                                                    label0, sum, dp)
       if (round_mode == XMC_ROUND_RTN) XMC_LAUNCH_UPDATE2(ROUND_RTN);
       else if (round_mode == XMC_ROUND_SR_FAST) XMC_LAUNCH_UPDATE2(ROUND_SR_FAST);
       else XMC_LAUNCH_UPDATE2(ROUND_SR_PHILOX);
@@ -1008,7 +1015,6 @@ static int tiled_step_t(void* const* chunk_ptrs, int num_chunks, int rows_per_ch
 #undef XMC_LAUNCH_UPDATE_H
 #undef XMC_LAUNCH_UPDATE_K
   }
-  tiled_finalize_kernel<DD><<<(batch * DD + 255) / 256, 256, 0, stream>>>(gx_total, batch, (unsigned short*)grad_x_bf16, grad_x_f32, dp);
   if (loss_out) tiled_loss_kernel<<<1, 256, 0, stream>>>(loss_part, 2 * num_tiles, loss_out);
   return launch_status();
 }

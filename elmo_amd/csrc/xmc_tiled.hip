@@ -198,6 +198,11 @@ __device__ __forceinline__ void t_store_g(const unsigned (&sg)[2], int r0, int r
   *(__attribute__((address_space(3))) unsigned short*)(stg + 96) = (unsigned short)(s23 >> 16);
 }
 
+// Batch rows come in K steps of 32 (of the update's products).  Wavefronts of the logits kernels and of the grad_X kernel whose rows lie in
+// none that has any only take part in the loads, and the update takes zeros in place of their G, which is not written: a batch of 8
+// to 32 rows used to pay for 128.  us a step, 1,024 features, before / now: bf16, Philox, 16 K labels, batch 13 75 / 61, 245 K, 12
+// 664 / 590; FP8, nearest, 120 K, 32 161 / 120; e4m3 with bf16 products, Philox, 92 K, 44 226 / 196.
+
 // Vector memory operations retire in order.  Per sub-tile a wavefront issues its loads of the sub-tile two steps ahead
 // (always, past the end they fetch the last sub-tile again into a buffer nobody reads, so that the count is the same in
 // every step) and then ten stores of G.  The wait at the top of a step leaves in flight what was issued after the
@@ -206,7 +211,7 @@ template <int WT, bool LOSS, int DD>
 __global__ __launch_bounds__(512, 1) void tiled_logits_kernel(const void* w, int rows, int nsub, const unsigned short* xb,
                                                               const unsigned* keys, const int* tile_ptr, unsigned label0_chunk,
                                                               unsigned short* glb, unsigned short* gbl, int batch, unsigned brow0,
-                                                              float* loss_part) {
+                                                              int live_rows, float* loss_part) {
   typedef TlgGeom<WT, DD> G;
   constexpr int NB = G::NBUF;
   extern __shared__ __attribute__((aligned(16))) unsigned char tlg_lds[];
@@ -246,13 +251,15 @@ __global__ __launch_bounds__(512, 1) void tiled_logits_kernel(const void* w, int
 #pragma unroll
   for (int ks = 0; ks < DD / 32; ks++) xr[ks] = *(const bf16x8*)(xb + ((size_t)(v * (DD / 32) + ks) * 64 + lane) * 8);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // from here on the loop counts its own operations: nothing is in flight
+  const bool active = LOSS || 32 * (v >> 1) < live_rows;   // its K step of 32 batch rows has any
   int it = 0, b0 = 0, b2 = NB - 1;   // it % NB, (it + NB - 1) % NB
   for (int st = blockIdx.x; st < nsub; st += gs, it++) {
     // younger than the loads of this sub-tile: the loads of the next one and the stores of up to two steps
     // (three stores per wavefront and step: two of G^T, one of G); with two buffers only the stores of the step before
     if (NB == 2) {
-      if (it > 0) asm volatile("s_waitcnt vmcnt(3)" ::: "memory");
-    } else if (it == 0) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(G::PER_WAVE_MIN) : "memory");
+      if (!active) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      else if (it > 0) asm volatile("s_waitcnt vmcnt(3)" ::: "memory");
+    } else if (it == 0 || !active) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(G::PER_WAVE_MIN) : "memory");
     else if (it == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(G::PER_WAVE_MIN + 3) : "memory");
     else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(G::PER_WAVE_MIN + 6) : "memory");
     // range of positives of the enclosing 64-row tile: asked for here, needed after the MFMAs
@@ -262,6 +269,7 @@ __global__ __launch_bounds__(512, 1) void tiled_logits_kernel(const void* w, int
     const int buf = b0;
     b0 = b0 == NB - 1 ? 0 : b0 + 1;
     b2 = b2 == NB - 1 ? 0 : b2 + 1;
+    if (!active) continue;
     floatx4 acc[2] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
     const unsigned abase = (unsigned)(buf * G::BUF + l16 * G::STRIDE + kg * (WT == W_BF16 ? 16 : 8));
     // the LDS reads run three K steps ahead of the MFMAs (everything unrolled: xr must stay in registers)
@@ -352,7 +360,7 @@ __global__ __launch_bounds__(512, 1) void tiled_logits_kernel(const void* w, int
 template <int DD>
 __global__ __launch_bounds__(512, 1) void tiled_logits_fp8_kernel(const void* w, int rows, int nsub, const unsigned char* xq,
                                                                   const unsigned* keys, const int* tile_ptr, unsigned label0_chunk,
-                                                                  unsigned short* glb, unsigned short* gbl, size_t g_half) {
+                                                                  unsigned short* glb, unsigned short* gbl, size_t g_half, int live_rows) {
   typedef TlgGeom<W_E4M3, DD> G;
   static_assert(G::NBUF == 3, "three buffers");
   constexpr int KS = DD / 128;   // K steps of the FP8 matrix instruction
@@ -388,12 +396,14 @@ __global__ __launch_bounds__(512, 1) void tiled_logits_fp8_kernel(const void* w,
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) xr[hf][ks] = *(const intx8*)(xq + (size_t)hf * BP * DD + ((size_t)(v * KS + ks) * 64 + lane) * 32);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // from here on the loop counts its own operations: nothing is in flight
+  const int nhf = 32 * (v >> 1) >= live_rows ? 0 : BP + 32 * (v >> 1) >= live_rows ? 1 : 2;   // halves in which this wavefront has batch rows
   int it = 0, b0 = 0, b2 = 2;   // it % 3, (it + 2) % 3
   for (int st = blockIdx.x; st < nsub; st += gs, it++) {
     // younger than the loads of this sub-tile: the loads of the next one and the stores of up to two steps (six per
     // wavefront and step: per half two of G^T and one of G)
-    if (it == 0) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(G::PER_WAVE_MIN) : "memory");
-    else if (it == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(G::PER_WAVE_MIN + 6) : "memory");
+    if (it == 0 || nhf == 0) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(G::PER_WAVE_MIN) : "memory");
+    else if (nhf == 1 && it == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(G::PER_WAVE_MIN + 3) : "memory");
+    else if (nhf == 1 || it == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(G::PER_WAVE_MIN + 6) : "memory");
     else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(G::PER_WAVE_MIN + 12) : "memory");
     const int p0 = ctile_ptr[st >> 1], p1 = ctile_ptr[(st >> 1) + 1];
     __syncthreads();
@@ -401,6 +411,7 @@ __global__ __launch_bounds__(512, 1) void tiled_logits_fp8_kernel(const void* w,
     const int buf = b0;
     b0 = b0 == 2 ? 0 : b0 + 1;
     b2 = b2 == 2 ? 0 : b2 + 1;
+    if (nhf == 0) continue;
     floatx4 acc[2][2];   // [label block][half]
 #pragma unroll
     for (int lb = 0; lb < 2; lb++) { acc[lb][0] = floatx4{0.f, 0.f, 0.f, 0.f}; acc[lb][1] = floatx4{0.f, 0.f, 0.f, 0.f}; }
@@ -427,6 +438,7 @@ __global__ __launch_bounds__(512, 1) void tiled_logits_fp8_kernel(const void* w,
     // acc[lb][hf][e] = Z[label 32 st + 16 lb + 4kg + e][batch 128 hf + 16v + l16]
 #pragma unroll
     for (int hf = 0; hf < 2; hf++) {
+      if (hf >= nhf) break;
       unsigned sg[2][2];   // sigmoids, four bf16 values each
 #pragma unroll
       for (int lb = 0; lb < 2; lb++) {
@@ -507,7 +519,8 @@ template <int WT, int HV, int DD> struct TgxGeom {
 //      a chunk boundary, so that each chunk's sum can be rounded by itself.
 template <int WT, int HV, int DD>
 __global__ __launch_bounds__(512) void tiled_gradx_kernel(const void* w, int rows, int rows_pad, int bound, int range, int cs, int spc,
-                                                          const unsigned short* gbl, size_t g_half, floatx4* partial, size_t part_half) {
+                                                          const unsigned short* gbl, size_t g_half, int live_rows, floatx4* partial,
+                                                          size_t part_half) {
   typedef TgxGeom<WT, HV, DD> G;
   constexpr int NN = G::NN;
   extern __shared__ __attribute__((aligned(16))) unsigned char tgx_lds[];
@@ -542,8 +555,9 @@ __global__ __launch_bounds__(512) void tiled_gradx_kernel(const void* w, int row
         t_lds_load16((const unsigned char*)w + ((size_t)lr * DD + G::FB * fb) * (WT == W_BF16 ? 2 : 1) + 16 * c16,
                      lds0 + (unsigned)(stage * G::STAGE + piece * 1024));
       } else {
-        const int gp = piece - G::WPIECES;   // piece gp & 7 of batch half gp >> 3
-        t_lds_load16((const unsigned char*)(gbl + (size_t)(gp >> 3) * g_half + ((size_t)((l0 >> 5) * 8 + (gp & 7)) * 64 + lane) * 8),
+        const int gp = piece - G::WPIECES;   // piece gp & 7 of batch half gp >> 3 (in place of one without batch rows the first)
+        const bool rows_in = 32 * ((gp & 7) >> 1) + BP * (gp >> 3) < live_rows;
+        t_lds_load16((const unsigned char*)(gbl + (rows_in ? (size_t)(gp >> 3) * g_half : 0) + ((size_t)((l0 >> 5) * 8 + (rows_in ? gp & 7 : 0)) * 64 + lane) * 8),
                      lds0 + (unsigned)(stage * G::STAGE + G::WBYTES + gp * 1024));
       }
     }
@@ -553,11 +567,14 @@ __global__ __launch_bounds__(512) void tiled_gradx_kernel(const void* w, int row
     issue_step(1, 1);
   }
   int stage = 0;
+  const bool active = BP * hw + 16 * mb0 < live_rows;
   for (int st = 0; st < nsteps; st++) {
     asm volatile("s_waitcnt vmcnt(%0)" : : "n"(G::PER_WAVE) : "memory");
     __syncthreads();   // step st has landed for every wavefront; the stage of step st-1 is free
     issue_step(st + 2, stage == 0 ? 2 : stage - 1);
     const __attribute__((address_space(3))) unsigned char* wt = lds + stage * G::STAGE;
+    stage = stage == 2 ? 0 : stage + 1;
+    if (!active) continue;
     const __attribute__((address_space(3))) unsigned char* gt = wt + G::WBYTES;
     bf16x8 ga[G::NMB];
 #pragma unroll
@@ -581,9 +598,9 @@ __global__ __launch_bounds__(512) void tiled_gradx_kernel(const void* w, int row
     for (int mb = 0; mb < G::NMB; mb++)
 #pragma unroll
       for (int nn = 0; nn < NN; nn++) acc[mb][nn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ga[mb], wb[nn], acc[mb][nn], 0, 0, 0);
-    stage = stage == 2 ? 0 : stage + 1;
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the loads past the end still target LDS
+  if (!active) return;
   // acc[mb][nn][e] = C[batch 128hw + 16(mb0 + mb) + 4kg + e][feature FB fb + FW fw + 16nn + l16]
   floatx4* dst = partial + (size_t)hw * part_half + ((size_t)split * 4 + fb) * (8 * NN) * 256;
 #pragma unroll
@@ -597,9 +614,19 @@ __global__ __launch_bounds__(512) void tiled_gradx_kernel(const void* w, int row
 // in the first workgroups of the chunk's update launch (the two do not depend on each other), so the sum costs no
 // launch of its own and hides behind the update.
 constexpr int tred_waves(int dd) { return 8 * (dd / 256) * 16; }   // (slot, feature quarter, wavefront): 384 or 512
+// The sum of a step's last launch is grad_X itself: it goes out (behind the dropout's backward) instead of to the total.  (A launch of its
+// own before, 4.7 us a step and the gap in front of it.)
+struct TiledSum {
+  const floatx4* partial; size_t part_half;   // of a batch half
+  int nchunks, spc, range, bound, round_bf16;
+  float* total;
+  int batch;
+  unsigned short* gx_bf16; float* gx_f32;     // the step's last launch only, else null
+};
 template <int DD>
-__device__ __forceinline__ void tiled_reduce_wave(int widx, int lane, const floatx4* partial, int nchunks, int spc, int cs, int range,
-                                                  int bound, int round_bf16, float* gx_total) {
+__device__ __forceinline__ void tiled_reduce_wave(int widx, int half, int lane, const TiledSum& r, int cs, const DropoutParams& dp) {
+  const floatx4* partial = r.partial + (size_t)half * r.part_half;
+  const int spc = r.spc, range = r.range, bound = r.bound;
   // (slot, fb, wavefront of the grad_X kernel's layout); eight loads in flight
   const int slot = widx >> 4, fb = (widx >> 2) & 3, wv = widx & 3;
   const int tid = wv * 64 + lane, l16 = lane & 15, kg = lane >> 4;
@@ -607,7 +634,9 @@ __device__ __forceinline__ void tiled_reduce_wave(int widx, int lane, const floa
   const int mb = slot / NN, nn = slot - mb * NN;
   const int col = (DD / 4) * fb + (DD / 16) * wv + 16 * nn + l16;
   floatx4 tot = {0.f, 0.f, 0.f, 0.f};
-  for (int ck = 0; ck < nchunks; ck++) {   // the chunks of the launch, each summed (and rounded) by itself
+  const int row0 = BP * half + 16 * mb;
+  if (row0 >= r.batch) return;
+  for (int ck = 0; ck < r.nchunks; ck++) {   // the chunks of the launch, each summed (and rounded) by itself
     const int crows = min((ck + 1) * cs, bound) - ck * cs, splits = (crows + range - 1) / range;
     const floatx4* pc = partial + (size_t)ck * spc * 4 * SL * 256;
     floatx4 s = {0.f, 0.f, 0.f, 0.f};
@@ -621,22 +650,21 @@ __device__ __forceinline__ void tiled_reduce_wave(int widx, int lane, const floa
     }
     for (; sp < splits; sp++) s += pc[(((size_t)sp * 4 + fb) * SL + slot) * 256 + tid];
 #pragma unroll
-    for (int i = 0; i < 4; i++) tot[i] += round_bf16 ? bf16_rt(s[i]) : s[i];
+    for (int i = 0; i < 4; i++) tot[i] += r.round_bf16 ? bf16_rt(s[i]) : s[i];
   }
 #pragma unroll
   for (int i = 0; i < 4; i++) {
-    const int b = 16 * mb + 4 * kg + i;
-    gx_total[(size_t)b * DD + col] += tot[i];
+    const int b = row0 + 4 * kg + i;
+    const size_t at = (size_t)b * DD + col;
+    const float sum = r.total[at] + tot[i];
+    if (!r.gx_bf16) {
+      r.total[at] = sum;
+    } else if (b < r.batch) {
+      const float g = dropout_backward(sum, (unsigned)at, dp);
+      if (r.gx_f32) r.gx_f32[at] = g;
+      r.gx_bf16[at] = bf16_bits(g);
+    }
   }
-}
-
-template <int DD>
-__global__ void tiled_finalize_kernel(const float* gx_total, int batch, unsigned short* gx_bf16, float* gx_f32, const DropoutParams dp) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= batch * DD) return;
-  const float v = dropout_backward(gx_total[i], (unsigned)i, dp);
-  if (gx_f32) gx_f32[i] = v;
-  gx_bf16[i] = bf16_bits(v);
 }
 
 // ---- grad_W and the SGD update of one chunk, in place.  blockIdx = tile*4 + fb; wavefront w owns label rows 16w..16w+15
@@ -747,28 +775,28 @@ constexpr int TUP_TILES = 4;                       // tiles of 64 label rows tha
 // features: CS = 2; CS = 1: 64 features, with four halves) and keeps their X^T operand blocks of every batch half in LDS:
 // 16 KiB per step and half.
 constexpr int tup_csteps(int halves, int dd = D) { return halves > 2 ? 1 : dd % 192 == 0 ? 3 : 2; }
-constexpr int tup_xbytes(int halves, int dd = D) { return tup_csteps(halves, dd) * 4 * (BP / 32) * 1024; }
+constexpr int tup_xbytes(int halves, int dd = D, int nks = BP / 32) { return tup_csteps(halves, dd) * 4 * nks * 1024; }
 constexpr int tup_threads(int halves) { return halves == 1 ? 256 : 512; }
-constexpr int tup_lds_bytes(int halves, int dd = D) { return halves * tup_xbytes(halves, dd); }
+constexpr int tup_lds_bytes(int halves, int dd = D, int nks = BP / 32) { return halves * tup_xbytes(halves, dd, nks); }
 
 // Launched with tup_threads(HALVES) threads and tup_lds(HALVES) bytes of LDS: four wavefronts per tile, so that a
 // compute unit runs at least eight wavefronts with one batch half (three workgroups) as with more (one workgroup of
 // eight wavefronts, two tiles at a time).
 // HALVES (batch halves: 1, 2 or 4) and KAHAN (a compensated head may be present) are template parameters: with run-time
 // branches around the products the compiler issued every LDS operand read right in front of its matrix instruction.
-template <int WT, int MODE, int HALVES, bool KAHAN, int DD>
+// NKS: K steps of 32 batch rows (of a half; 1, 2 or 4 with one half).
+template <int WT, int MODE, int HALVES, bool KAHAN, int DD, int NKS>
 __global__ __launch_bounds__(HALVES == 1 ? 256 : 512, HALVES == 1 ? 3 : HALVES == 2 ? 2 : 1) void tiled_update_kernel(
     void* w, int rows, int ntiles, const unsigned short* glb, size_t g_half_stride, const unsigned short* xT, float lr, float wd, TiledSeeds seeds,
-    int cs, int saturate, void* kahan, int kahan_type, int num_head, unsigned label0, const floatx4* red_partial, size_t red_part_half,
-    int red_nchunks, int red_spc, int red_range, int red_bound, int red_round_bf16, float* red_total) {
+    int cs, int saturate, void* kahan, int kahan_type, int num_head, unsigned label0, int live_rows, TiledSum red, DropoutParams dp) {
   static_assert(!KAHAN || WT == W_E4M3, "the compensated head belongs to the FP8 layer");
   // the first workgroups sum the chunk's grad_X partials (384 wavefronts per batch half), the others update the weights
-  constexpr int CS = tup_csteps(HALVES, DD), XB = tup_xbytes(HALVES, DD), NFB = (DD / 64) / CS, WAVES = tup_threads(HALVES) / 64;
+  static_assert(NKS == BP / 32 || HALVES == 1, "a K step of the first half only");
+  constexpr int CS = tup_csteps(HALVES, DD), XB = tup_xbytes(HALVES, DD, NKS), NFB = (DD / 64) / CS, WAVES = tup_threads(HALVES) / 64;
   constexpr int TRED_WAVES = tred_waves(DD), RED_BLOCKS = TRED_WAVES * HALVES / WAVES;
   if ((int)blockIdx.x < RED_BLOCKS) {
     const int widx = (int)blockIdx.x * WAVES + ((int)threadIdx.x >> 6), hh = widx / TRED_WAVES;
-    tiled_reduce_wave<DD>(widx - hh * TRED_WAVES, (int)threadIdx.x & 63, red_partial + (size_t)hh * red_part_half, red_nchunks, red_spc, cs,
-                      red_range, red_bound, red_round_bf16, red_total + (size_t)hh * BP * DD);
+    tiled_reduce_wave<DD>(widx - hh * TRED_WAVES, hh, (int)threadIdx.x & 63, red, cs, dp);
     return;
   }
   extern __shared__ __attribute__((aligned(16))) unsigned char tup_lds[];
@@ -783,15 +811,17 @@ __global__ __launch_bounds__(HALVES == 1 ? 256 : 512, HALVES == 1 ? 3 : HALVES =
   // wavefronts of the workgroup; from global memory every MFMA would fetch its operand through L1 again.
 #pragma unroll
   for (int hh = 0; hh < HALVES; hh++) {
-    const intx4* src = (const intx4*)(xT + (size_t)hh * DD * BP + (size_t)fb * (XB / 2));
-    for (int s = tid; s < XB / 16; s += (int)blockDim.x)
-      *(__attribute__((address_space(3))) intx4*)(lds + hh * XB + s * 16) = src[s];
+    const intx4* src = (const intx4*)(xT + (size_t)hh * DD * BP) + (size_t)fb * CS * 4 * (BP / 32) * 64;
+    for (int s = tid; s < XB / 16; s += (int)blockDim.x) {
+      const int blk = s / (NKS * 64);   // feature block; in memory it has all four K steps
+      *(__attribute__((address_space(3))) intx4*)(lds + hh * XB + s * 16) = src[s + blk * (BP / 32 - NKS) * 64];
+    }
   }
   __syncthreads();
   // The G rows and the weights of the next tile are loaded before the products of the current one: a wavefront waits
   // for memory once per launch, not four times per tile.
   constexpr int WDW = WT == W_BF16 ? 8 : 4;   // dwords of 16 weights
-  bf16x8 gf_n[HALVES][4];
+  bf16x8 gf_n[HALVES][NKS];
   intx4 wr_n[CS][WDW / 4];
   auto load_tile = [&](int tile) {
     const int row = tile * TL + 16 * wv + l16;
@@ -799,8 +829,8 @@ __global__ __launch_bounds__(HALVES == 1 ? 256 : 512, HALVES == 1 ? 3 : HALVES =
 #pragma unroll
     for (int hh = 0; hh < HALVES; hh++)
 #pragma unroll
-      for (int ks = 0; ks < 4; ks++)
-        gf_n[hh][ks] = tile < ntiles ? *(const bf16x8*)(glb + hh * g_half_stride + ((size_t)((tile * 4 + wv) * 4 + ks) * 64 + lane) * 8) : bf16x8{};
+      for (int ks = 0; ks < NKS; ks++)
+        gf_n[hh][ks] = tile < ntiles && BP * hh + 32 * ks < live_rows ? *(const bf16x8*)(glb + hh * g_half_stride + ((size_t)((tile * 4 + wv) * 4 + ks) * 64 + lane) * 8) : bf16x8{};
 #pragma unroll
     for (int c = 0; c < CS; c++) {
       const intx4* src = (const intx4*)((const unsigned char*)w + ((size_t)row * DD + 64 * (CS * fb + c) + 16 * kg) * (WT == W_BF16 ? 2 : 1));
@@ -822,12 +852,12 @@ __global__ __launch_bounds__(HALVES == 1 ? 256 : 512, HALVES == 1 ? 3 : HALVES =
   const unsigned seed = seeds.s[ck];
   const int crow = row - ck * cs;
   const int orow = (WT == W_E4M3 && !head) ? crow - num_head : crow;   // row of the random offset
-  bf16x8 gf[HALVES][4];
+  bf16x8 gf[HALVES][NKS];
   intx4 wr_t[CS][WDW / 4];
 #pragma unroll
   for (int hh = 0; hh < HALVES; hh++)
 #pragma unroll
-    for (int ks = 0; ks < 4; ks++) gf[hh][ks] = gf_n[hh][ks];
+    for (int ks = 0; ks < NKS; ks++) gf[hh][ks] = gf_n[hh][ks];
 #pragma unroll
   for (int c = 0; c < CS; c++)
 #pragma unroll
@@ -861,22 +891,22 @@ __global__ __launch_bounds__(HALVES == 1 ? 256 : 512, HALVES == 1 ? 3 : HALVES =
     constexpr int QB = HALVES == 1 ? 4 : HALVES == 2 ? 2 : 1;
 #pragma unroll
     for (int q0 = 0; q0 < 4; q0 += QB) {
-      bf16x8 xa[QB][HALVES][4];
+      bf16x8 xa[QB][HALVES][NKS];
 #pragma unroll
       for (int qq = 0; qq < QB; qq++)
 #pragma unroll
         for (int hh = 0; hh < HALVES; hh++)
 #pragma unroll
-          for (int ks = 0; ks < 4; ks++)
+          for (int ks = 0; ks < NKS; ks++)
             xa[qq][hh][ks] = *(const __attribute__((address_space(3))) bf16x8*)(lds + hh * XB +
-                                                                                (((4 * c + q0 + qq) * (BP / 32) + ks) * 64 + lane) * 16);
+                                                                                (((4 * c + q0 + qq) * NKS + ks) * 64 + lane) * 16);
 #pragma unroll
       for (int qq = 0; qq < QB; qq++) {
         floatx4 a = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int hh = 0; hh < HALVES; hh++)
 #pragma unroll
-          for (int ks = 0; ks < 4; ks++) a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[qq][hh][ks], gf[hh][ks], a, 0, 0, 0);
+          for (int ks = 0; ks < NKS; ks++) a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[qq][hh][ks], gf[hh][ks], a, 0, 0, 0);
         acc[q0 + qq] = a;
       }
     }
@@ -920,13 +950,11 @@ constexpr int TU2_GBUF = 32768;   // one tile's G: [half][row block][K step] blo
 template <int MODE>
 __global__ __launch_bounds__(256, 2) void tiled_update2_kernel(
     void* w, int rows, int ntiles, const unsigned short* glb, size_t g_half, const bf16x8* xt2, float lr, float wd, TiledSeeds seeds, int cs,
-    int saturate, unsigned label0, const floatx4* red_partial, size_t red_part_half, int red_nchunks, int red_spc, int red_range,
-    int red_bound, float* red_total) {
+    int saturate, unsigned label0, TiledSum red, DropoutParams dp) {
   constexpr int TRED_WAVES = tred_waves(D), RED_BLOCKS = TRED_WAVES * 2 / 4;   // (768 features only)
   if ((int)blockIdx.x < RED_BLOCKS) {
     const int widx = (int)blockIdx.x * 4 + ((int)threadIdx.x >> 6), hh = widx / TRED_WAVES;
-    tiled_reduce_wave<D>(widx - hh * TRED_WAVES, (int)threadIdx.x & 63, red_partial + (size_t)hh * red_part_half, red_nchunks, red_spc, cs,
-                      red_range, red_bound, 0, red_total + (size_t)hh * BP * D);
+    tiled_reduce_wave<D>(widx - hh * TRED_WAVES, hh, (int)threadIdx.x & 63, red, cs, dp);
     return;
   }
   extern __shared__ __attribute__((aligned(16))) unsigned char tu2_lds[];

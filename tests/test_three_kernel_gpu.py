@@ -40,6 +40,14 @@ def bf16_views(w, nc, device):
     ("fp8", 3, 3088, 256, "sr_philox"),
     ("fp8", 2, 1040, 272, "sr_fast"),
     ("fp8", 5, 848, 512, "rtn"),
+    # batches that end in front of, at and behind a K step of 32 rows, and whose last halves have no rows
+    ("bf16", 2, 300, 33, "sr_philox"),
+    ("bf16", 2, 300, 65, "rtn"),
+    ("bf16", 1, 300, 385, "rtn"),
+    ("sim", 1, 304, 64, "sr_philox"),
+    ("sim", 1, 304, 97, "rtn"),
+    ("fp8", 1, 304, 257, "rtn"),
+    ("fp8", 2, 304, 416, "sr_fast"),
 ])
 def test_step_with_weight_decay_matches_the_oracle(gpu, kind, nc, rows, batch, mode):
     import torch
@@ -72,6 +80,27 @@ def test_step_with_weight_decay_matches_the_oracle(gpu, kind, nc, rows, batch, m
     dist = np.concatenate([H.e4m3_ulp_distance(a, b).ravel() for a, b in zip(H.chunks_to_numpy(chunks), ref_codes)])
     assert dist.max() <= 1 and (dist != 0).mean() < 5e-3, (dist.max(), (dist != 0).mean())
     check_gx(gf.cpu().numpy(), g.float().cpu().numpy(), ref_gx)
+
+
+@pytest.mark.parametrize("kind", ["bf16", "sim", "fp8"])
+@pytest.mark.parametrize("batch", [1, 32, 33, 64, 65, 129, 161, 257, 300, 385])
+def test_nothing_is_read_of_rows_that_the_batch_does_not_have(gpu, kind, batch):
+    """G of K steps without batch rows is not written: a workspace full of NaN gives bit for bit what one of zeros gives."""
+    import torch
+    from elmo_amd import ops
+    rows, d = 400, 1024
+    gen = torch.Generator(device=gpu).manual_seed(batch)
+    w0 = torch.randn(rows, d, generator=gen, device=gpu) * 0.02
+    x = torch.randn(batch, d, generator=gen, device=gpu).to(torch.bfloat16)
+    labels = torch.tensor([[0, 0], [batch - 1, rows - 1]], dtype=torch.int32, device=gpu)
+    out = []
+    for fill in (0, 255):
+        w = w0.to(torch.bfloat16 if kind == "bf16" else torch.float8_e4m3fn)
+        ws = torch.full((ops.tiled_workspace_bytes(1, rows, batch, d),), fill, dtype=torch.uint8, device=gpu)
+        g = ops.tiled_step([w], rows, "bf16" if kind == "bf16" else "e4m3", x, labels, 0.1, workspace=ws, quantize_x=kind == "fp8", saturate=kind == "fp8")
+        out.append((w.view(torch.uint8), g))
+    assert torch.isfinite(out[1][1].float()).all()
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
 
 
 def test_loss_over_four_halves(gpu):
