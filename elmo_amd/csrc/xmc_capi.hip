@@ -971,8 +971,12 @@ static int tiled_step_t(void* const* chunk_ptrs, int num_chunks, int rows_per_ch
       }
     }
     const int nsub_u = tup_threads(halves) / 256;    // tiles a workgroup of the update kernel works on at a time
-    const int ugroups = (tiles + TUP_TILES * nsub_u - 1) / (TUP_TILES * nsub_u);   // rounded up to eight: see the kernel's index map
-    const int ugrid = tred_waves(DD) * halves / (tup_threads(halves) / 64) + ((DD / 64) / tup_csteps(halves, DD)) * ((ugroups + 7) / 8 * 8);
+    const int nfb = (DD / 64) / tup_csteps(halves, DD);
+    // streams of tiles: as many as the compute units hold at once, a multiple of eight (see the kernel's index map)
+    int ustreams = ((tiles + nsub_u - 1) / nsub_u + 7) / 8 * 8;
+    const int umost = di.cus * (halves == 1 ? 3 : 1) / nfb / 8 * 8;
+    if (ustreams > umost && umost > 0) ustreams = umost;
+    const int ugrid = tred_waves(DD) * halves / (tup_threads(halves) / 64) + nfb * ustreams;
     const bool final_sum = c + nch == num_chunks;
     const TiledSum sum = {partial, part_half, nch, spc, range, rp, weight_type == W_BF16 ? 1 : 0, gx_total, batch,
                           final_sum ? (unsigned short*)grad_x_bf16 : nullptr, final_sum ? grad_x_f32 : nullptr};

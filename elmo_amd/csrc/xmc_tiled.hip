@@ -770,7 +770,6 @@ __device__ __forceinline__ void t_update4(floatx4 a, const unsigned* wraw, const
   }
 }
 
-constexpr int TUP_TILES = 4;                       // tiles of 64 label rows that each group of four wavefronts processes
 // A workgroup owns CS steps of 64 features (768 features: CS = 3, a feature quarter, with one or two batch halves; 1024
 // features: CS = 2; CS = 1: 64 features, with four halves) and keeps their X^T operand blocks of every batch half in LDS:
 // 16 KiB per step and half.
@@ -779,6 +778,9 @@ constexpr int tup_xbytes(int halves, int dd = D, int nks = BP / 32) { return tup
 constexpr int tup_threads(int halves) { return halves == 1 ? 256 : 512; }
 constexpr int tup_lds_bytes(int halves, int dd = D, int nks = BP / 32) { return halves * tup_xbytes(halves, dd, nks); }
 
+// Streams of tiles, as many as the compute units hold workgroups for, so that none starts when others are half done (four tiles a workgroup
+// before: 1,024 features, FP8 sr_fast, 46 K labels, batch 208 55 us a launch, now 48, 20 K, 448 62 / 53; bf16, 150 K, 256 189 / 180; one
+// batch half the same).
 // Launched with tup_threads(HALVES) threads and tup_lds(HALVES) bytes of LDS: four wavefronts per tile, so that a
 // compute unit runs at least eight wavefronts with one batch half (three workgroups) as with more (one workgroup of
 // eight wavefronts, two tiles at a time).
@@ -803,10 +805,11 @@ __global__ __launch_bounds__(HALVES == 1 ? 256 : 512, HALVES == 1 ? 3 : HALVES =
   __attribute__((address_space(3))) unsigned char* lds = (__attribute__((address_space(3))) unsigned char*)tup_lds;
   const int tid = threadIdx.x, wv = (tid >> 6) & 3, sub = tid >> 8, nsub = (int)blockDim.x >> 8;
   const int lane = tid & 63, l16 = lane & 15, kg = lane >> 4;
-  // fb: CS steps of 64 features.  The NFB workgroups of a tile group read the same rows of G: they sit on one XCD
+  // fb: CS steps of 64 features.  The NFB workgroups of a stream of tiles read the same rows of G: they sit on one XCD
   // (workgroups go to the XCDs round robin), eight apart in launch order, and share that XCD's L2.
-  const int jb = (int)blockIdx.x - RED_BLOCKS, fb = (jb >> 3) % NFB, group = ((jb >> 3) / NFB) * 8 + (jb & 7);
-  if (group * TUP_TILES * nsub >= ntiles) return;   // the grid is rounded up to eight tile groups
+  const int jb = (int)blockIdx.x - RED_BLOCKS, fb = (jb >> 3) % NFB, stream = ((jb >> 3) / NFB) * 8 + (jb & 7);
+  const int step = ((int)gridDim.x - RED_BLOCKS) / NFB * nsub;   // tiles from one of a stream to the next
+  if (stream * nsub >= ntiles) return;   // the grid is rounded up to eight streams
   // The X^T operand of these features goes to LDS once (it is contiguous in the image) and serves all tiles and
   // wavefronts of the workgroup; from global memory every MFMA would fetch its operand through L1 again.
 #pragma unroll
@@ -838,11 +841,10 @@ __global__ __launch_bounds__(HALVES == 1 ? 256 : 512, HALVES == 1 ? 3 : HALVES =
       for (int q = 0; q < WDW / 4; q++) wr_n[c][q] = live ? src[q] : intx4{0, 0, 0, 0};
     }
   };
-  load_tile(group * TUP_TILES * nsub + sub);
+  load_tile(stream * nsub + sub);
 #pragma unroll 1
-  for (int tt = 0; tt < TUP_TILES; tt++) {
-  const int tile = (group * TUP_TILES + tt) * nsub + sub;
-  if (tile >= ntiles) break;
+  for (int tile = stream * nsub + sub; tile < ntiles; tile += step) {
+  asm volatile("" ::: "memory");   // (or the X^T operands are read in front of the loop, into registers that there are not)
   const int row = tile * TL + 16 * wv + l16;
   const bool live = row < rows;
   const bool head = KAHAN && kahan_type != 0 && row < num_head;
@@ -862,7 +864,7 @@ __global__ __launch_bounds__(HALVES == 1 ? 256 : 512, HALVES == 1 ? 3 : HALVES =
   for (int c = 0; c < CS; c++)
 #pragma unroll
     for (int q = 0; q < WDW / 4; q++) wr_t[c][q] = wr_n[c][q];
-  if (tt + 1 < TUP_TILES) load_tile(tile + nsub);
+  load_tile(tile + step);
 #pragma unroll
   for (int c = 0; c < CS; c++) {              // 16 consecutive features of this lane's row at a time
     const int col0 = 64 * (CS * fb + c) + 16 * kg;
