@@ -188,9 +188,9 @@ def fp8_forward(chunks, x, num_labels, scale_w=1.0, scale_x=1.0, workspace=None)
     out = torch.empty(total, stride, dtype=torch.bfloat16, device=x.device)
     for lo in range(0, total, MAX_BATCH_INFERENCE):
         hi = min(lo + MAX_BATCH_INFERENCE, total)
-        xs = _aligned_rows(xb[lo:hi])
+        xs = _aligned_rows(xb if hi - lo == total else xb[lo:hi])      # (a slice costs 1 us of a call that takes 15)
         st = lib.xmc_fp8_forward_wide(arr, nc, rows, xs.data_ptr(), hi - lo, FEATURES, float(scale_w), float(scale_x),
-                                      out[lo:hi].data_ptr(), stride, num_labels, workspace.data_ptr(), workspace.numel(),
+                                      out.data_ptr() + 2 * stride * lo, stride, num_labels, workspace.data_ptr(), workspace.numel(),
                                       _stream_ptr())
         _lib.check(st, "xmc_fp8_forward_wide")
     return out[:, :num_labels]
@@ -237,7 +237,7 @@ def fp8_forward_topk(chunks, x, num_labels, k, scale_w=1.0, scale_x=1.0, workspa
     while lo < total:
         hi = min(lo + (MAX_BATCH_INFERENCE if fused and not defer_check else MAX_BATCH), total)
         n, si = hi - lo, lo // MAX_BATCH
-        xs = _aligned_rows(xb[lo:hi])
+        xs = _aligned_rows(xb if n == total else xb[lo:hi])
         done = False
         if fused:
             need = lib.xmc_topk_fused_scratch_bytes()
@@ -246,8 +246,8 @@ def fp8_forward_topk(chunks, x, num_labels, k, scale_w=1.0, scale_x=1.0, workspa
             entry = "xmc_fp8_forward_topk_fused_rows" if defer_check else "xmc_fp8_forward_topk_wide"
             st = getattr(lib, entry)(
                 arr, nc, rows, xs.data_ptr(), n, FEATURES, float(scale_w), float(scale_x), int(num_labels), int(k),
-                vals[lo:hi].data_ptr(), idx[lo:hi].data_ptr(), 1, workspace.data_ptr(), workspace.numel(),
-                fused_scratch.data_ptr(), fused_scratch.numel(), status[si:].data_ptr(), _stream_ptr())
+                vals.data_ptr() + 2 * k * lo, idx.data_ptr() + 8 * k * lo, 1, workspace.data_ptr(), workspace.numel(),
+                fused_scratch.data_ptr(), fused_scratch.numel(), status.data_ptr() + 4 * si, _stream_ptr())
             if st != _lib.XMC_ERR_RANGE:
                 _lib.check(st, entry)
                 done = True
