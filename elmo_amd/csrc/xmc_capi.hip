@@ -924,9 +924,9 @@ static int tiled_step_t(void* const* chunk_ptrs, int num_chunks, int rows_per_ch
     for (int k = 0; k < T_GROUP; k++)
       sd.s[k] = seeds && k < nch ? (round_mode == XMC_ROUND_SR_FAST ? fast_seed(seeds[c + k]) : seeds[c + k]) : 0u;
     const int nh = c == 0 ? num_head : 0;   // the compensated head lives in chunk 0 (chunked_head_kahan_fp8xmc_clf.py:127)
-    // label ranges of the grad_X kernel: T_SPLITS slots shared by the launch's chunks, none across a chunk boundary
+    // label ranges of the grad_X kernel: slots shared by the launch's chunks, none across a chunk boundary
     const int cs = nch > 1 ? rows_per_chunk : rp;       // rows of a chunk as the kernels see them
-    const int spc_max = T_SPLITS / nch;
+    const int spc_max = tiled_splits(rp) / nch > 0 ? tiled_splits(rp) / nch : 1;   // (a launch has at most eight chunks)
     int range = (cs + spc_max - 1) / spc_max;
     range = (range + TL - 1) / TL * TL;
     const int spc = (cs + range - 1) / range;            // slots (and at most ranges) per chunk

@@ -13,7 +13,19 @@
 namespace xmc {
 
 enum WType { W_E4M3 = 0, W_BF16 = 1 };
-constexpr int T_SPLITS = 64;                       // label ranges of the grad_X kernel
+constexpr int T_SPLITS = 64;                       // most label ranges of the grad_X kernel
+// Label ranges (times four feature quarters: workgroups) of a grad_X launch over `rows` label rows.  A range writes the sums of all batch rows,
+// 512 KiB a batch half at 1,024 features, which the update's launch reads again; with few labels that costs more than the idle
+// compute units of fewer ranges.  s ranges take steps / s steps of 32 labels and s sums, least where s^2 is proportional to the steps:
+// 64 from 65 K labels on, 8 up to 1,024.  us a step, 64 ranges / with s^2 = 0.5, 1, 2 times the steps (1,024 features): FP8, batch 448,
+// 2,500 labels 72.7 / 72.9 68.9 69.0, 8 K 97.8 / 94.3 94.3 90.7, 20 K 141 / 149 139 137, 46 K 220 / 234 228 221;  batch 208, 8 K 52.6 / 53.0
+// 52.8 50.5;  bf16, batch 16, 8 K 39.0 / 35.1 37.3 37.8, 46 K 80.3 / 84.4 81.3 79.0;  batch 300, 8 K 95.5 / 94.5 95.7 92.0.
+inline int tiled_splits(int rows) {
+  const int steps = rows / 32;
+  int s = 8;
+  while (s < T_SPLITS && s * s < 2 * steps) s += 8;
+  return s;
+}
 constexpr int T_GROUP = 8;                         // most chunks one launch covers
 constexpr int T_GROUP_ROWS = 65536;                // ... and most rows (the G buffers hold the rows of one launch)
 struct TiledSeeds { unsigned s[T_GROUP]; };        // rounding seed of every chunk of a launch
