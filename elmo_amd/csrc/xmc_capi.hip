@@ -76,8 +76,7 @@ void fill_device_info(int dev) {
   (void)hipFuncSetAttribute((const void*)tiled_logits_kernel<W_BF16, false, DD>, hipFuncAttributeMaxDynamicSharedMemorySize, TlgGeom<W_BF16, DD>::LDS); \
   (void)hipFuncSetAttribute((const void*)tiled_logits_kernel<W_E4M3, true, DD>, hipFuncAttributeMaxDynamicSharedMemorySize, TlgGeom<W_E4M3, DD>::LDS); \
   (void)hipFuncSetAttribute((const void*)tiled_logits_kernel<W_E4M3, false, DD>, hipFuncAttributeMaxDynamicSharedMemorySize, TlgGeom<W_E4M3, DD>::LDS); \
-  (void)hipFuncSetAttribute((const void*)tiled_logits_fp8_kernel<DD, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, TlgGeom<W_E4M3, DD>::LDS); \
-  (void)hipFuncSetAttribute((const void*)tiled_logits_fp8_kernel<DD, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, TlgGeom<W_E4M3, DD>::LDS)
+  (void)hipFuncSetAttribute((const void*)tiled_logits_fp8_kernel<DD>, hipFuncAttributeMaxDynamicSharedMemorySize, TlgGeom<W_E4M3, DD>::LDS)
   XMC_TILED_ATTR(D);
   XMC_TILED_ATTR(1024);
 #undef XMC_TILED_ATTR
@@ -895,8 +894,8 @@ static int tiled_step_t(void* const* chunk_ptrs, int num_chunks, int rows_per_ch
   // chunks per segment of the label space: a multiple of the launch group, fewer than 2^24 - 1 labels
   int seg_chunks = ((1 << 24) - 2) / rows_per_chunk / group * group;
   if (seg_chunks < group) return XMC_ERR_RANGE;
-  // true-FP8 arithmetic: FP8 matrix products, the logits of a pair of halves in one pass
-  const bool fp8_logits = weight_type == W_E4M3 && quantize_x && !loss_out;
+  // true-FP8 arithmetic with two or four batch halves: FP8 matrix products, the logits of a pair of halves in one pass
+  const bool fp8_logits = weight_type == W_E4M3 && quantize_x && halves >= 2 && !loss_out;
   // e4m3 weights, two batch halves, no compensated head: the feature-split update kernel (X^T in registers)
   const bool split_update = weight_type == W_E4M3 && halves == 2 && kahan_type == 0 && DD == D;
   // batch rows whose G is written and read; the feature-split update reads the G of both halves whole
@@ -934,13 +933,9 @@ static int tiled_step_t(void* const* chunk_ptrs, int num_chunks, int rows_per_ch
     float* lp = loss_part + 2 * c * tiles_per_chunk;
     for (int hh = 0; fp8_logits && hh < halves; hh += 2) {
       const int nsub = 2 * tiles, lgrid = nsub < di.cus ? nsub : di.cus;
-#define XMC_LAUNCH_LOGITS_FP8(NHF)                                                                                              \
-  tiled_logits_fp8_kernel<DD, NHF><<<lgrid, 512, TlgGeom<W_E4M3, DD>::LDS, stream>>>(                                           \
-      w, rows, nsub, (const unsigned char*)xb + (size_t)hh * BP * DD, keys + (size_t)(hh >> 1) * MAX_POS,                       \
-      tile_ptr + (hh >> 1) * tp_stride + c * tiles_per_chunk, label0_seg, glb + hh * g_half, gbl + hh * g_half, g_half, live - hh * BP)
-      if (live - hh * BP <= BP) XMC_LAUNCH_LOGITS_FP8(1);
-      else XMC_LAUNCH_LOGITS_FP8(2);
-#undef XMC_LAUNCH_LOGITS_FP8
+      tiled_logits_fp8_kernel<DD><<<lgrid, 512, TlgGeom<W_E4M3, DD>::LDS, stream>>>(
+          w, rows, nsub, (const unsigned char*)xb + (size_t)hh * BP * DD, keys + (size_t)(hh >> 1) * MAX_POS,
+          tile_ptr + (hh >> 1) * tp_stride + c * tiles_per_chunk, label0_seg, glb + hh * g_half, gbl + hh * g_half, g_half, live - hh * BP);
     }
     for (int hh = 0; !fp8_logits && hh < halves; hh++) {
       if (hh * BP >= live && !loss_out) break;   // (a loss is summed over every launch's tiles)

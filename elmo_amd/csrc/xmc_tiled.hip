@@ -362,16 +362,14 @@ __global__ __launch_bounds__(512, 1) void tiled_logits_kernel(const void* w, int
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the last loads still target LDS
 }
 
-// ---- the same for the true-FP8 arithmetic with NHF batch halves per pass: the logits of e4m3 weights against e4m3(X)
+// ---- the same for the true-FP8 arithmetic with two batch halves per pass: the logits of e4m3 weights against e4m3(X)
 //      are FP8 matrix products (chunked_fp8xmc_clf.py:101-102), so the rows go from LDS into v_mfma_f32_16x16x128_f8f6f4
 //      as they are (no widening to bf16, a quarter of the matrix instructions per batch row) and wavefront v keeps the
 //      e4m3 operand of batch rows 16v.. of BOTH halves (96 registers, as the bf16 operand of one half took): one pass over
 //      the weights yields the G of 256 batch rows.  Tile loop, positives, rounding and both layouts of G as above; the
-//      products are exact in fp32 either way, only the order of the fp32 sums differs from the bf16 form.  One half took the bf16
-//      form before, whose eight wavefronts each widen every weight.  us a step, then / now: 1,024 features, 300 K labels, batch 96,
-//      sr_fast 384 / 357, 120 K, 32, nearest 120 / 112;  768, compensated head, 100 K, 120 166 / 154, 30 K, 72 72 / 60.
+//      products are exact in fp32 either way, only the order of the fp32 sums differs from the bf16 form.
 //      xq: e4m3 image of the pair's X in B-operand order, [half][(16-row block)*6 + ks][lane][32 bytes] (tiled_prep_x_thread)
-template <int DD, int NHF>
+template <int DD>
 __global__ __launch_bounds__(512, 1) void tiled_logits_fp8_kernel(const void* w, int rows, int nsub, const unsigned char* xq,
                                                                   const unsigned* keys, const int* tile_ptr, unsigned label0_chunk,
                                                                   unsigned short* glb, unsigned short* gbl, size_t g_half, int live_rows) {
@@ -404,13 +402,13 @@ __global__ __launch_bounds__(512, 1) void tiled_logits_fp8_kernel(const void* w,
   __attribute__((address_space(3))) unsigned char* stg = lds + G::STAGE0 + v * 1024;
   issue_sub(blockIdx.x, 0);
   issue_sub(blockIdx.x + gs, 1);
-  intx8 xr[NHF][KS];   // the e4m3 operands of this wavefront's batch rows in either half
+  intx8 xr[2][KS];   // the e4m3 operands of this wavefront's batch rows in either half
 #pragma unroll
-  for (int hf = 0; hf < NHF; hf++)
+  for (int hf = 0; hf < 2; hf++)
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) xr[hf][ks] = *(const intx8*)(xq + (size_t)hf * BP * DD + ((size_t)(v * KS + ks) * 64 + lane) * 32);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // from here on the loop counts its own operations: nothing is in flight
-  const int nhf = 32 * (v >> 1) >= live_rows ? 0 : NHF == 1 || BP + 32 * (v >> 1) >= live_rows ? 1 : 2;   // halves in which this wavefront has batch rows
+  const int nhf = 32 * (v >> 1) >= live_rows ? 0 : BP + 32 * (v >> 1) >= live_rows ? 1 : 2;   // halves in which this wavefront has batch rows
   int it = 0, b0 = 0, b2 = 2;   // it % 3, (it + 2) % 3
   for (int st = blockIdx.x; st < nsub; st += gs, it++) {
     // younger than the loads of this sub-tile: the loads of the next one and the stores of up to two steps (six per
@@ -426,11 +424,9 @@ __global__ __launch_bounds__(512, 1) void tiled_logits_fp8_kernel(const void* w,
     b0 = b0 == 2 ? 0 : b0 + 1;
     b2 = b2 == 2 ? 0 : b2 + 1;
     if (nhf == 0) continue;
-    floatx4 acc[2][NHF];   // [label block][half]
+    floatx4 acc[2][2];   // [label block][half]
 #pragma unroll
-    for (int lb = 0; lb < 2; lb++)
-#pragma unroll
-      for (int hf = 0; hf < NHF; hf++) acc[lb][hf] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int lb = 0; lb < 2; lb++) { acc[lb][0] = floatx4{0.f, 0.f, 0.f, 0.f}; acc[lb][1] = floatx4{0.f, 0.f, 0.f, 0.f}; }
     const unsigned abase = (unsigned)(buf * G::BUF + l16 * G::STRIDE + kg * 32);
     auto rd = [&](int ks, int lb) {
       const __attribute__((address_space(3))) intx4* q = (const __attribute__((address_space(3))) intx4*)(lds + abase + lb * 16 * G::STRIDE + ks * 128);
@@ -447,13 +443,13 @@ __global__ __launch_bounds__(512, 1) void tiled_logits_fp8_kernel(const void* w,
 #pragma unroll
       for (int lb = 0; lb < 2; lb++)
 #pragma unroll
-        for (int hf = 0; hf < NHF; hf++)
+        for (int hf = 0; hf < 2; hf++)
           acc[lb][hf] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(araw[ks % 3][lb], xr[hf][ks], acc[lb][hf], 0, 0, 0, 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
     }
     // acc[lb][hf][e] = Z[label 32 st + 16 lb + 4kg + e][batch 128 hf + 16v + l16]
 #pragma unroll
-    for (int hf = 0; hf < NHF; hf++) {
+    for (int hf = 0; hf < 2; hf++) {
       if (hf >= nhf) break;
       unsigned sg[2][2];   // sigmoids, four bf16 values each
 #pragma unroll
