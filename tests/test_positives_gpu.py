@@ -43,7 +43,7 @@ def test_one_pass_step(gpu, kind, batch, n, monkeypatch):
 
 
 @pytest.mark.parametrize("kind,batch", [("bf16", 20), ("bf16", 300), ("sim", 128), ("fp8", 64), ("fp8", 300)])
-@pytest.mark.parametrize("n", [8, 9, 257, 5000])
+@pytest.mark.parametrize("n", [8, 9, 257, 5000, 32761])     # (the most, 32,768, less two neighbours and five edges of the bf16 case)
 def test_three_kernel_step(gpu, kind, batch, n, monkeypatch):
     labels = crowded(n, batch, ROWS)
     make_case, bf16_case = H.make_case, K.bf16_case
