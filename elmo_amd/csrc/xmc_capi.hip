@@ -985,8 +985,8 @@ static int tiled_step_t(void* const* chunk_ptrs, int num_chunks, int rows_per_ch
       w, rows, tiles, glb, g_half, xT, lr, wd, sd, cs, saturate, kahan, kahan_type, nh, label0, live, sum, dp)
 #define XMC_LAUNCH_UPDATE_H(WTYPE, RMODE, KH)                                                                                  \
   do {                                                                                                                         \
-    if (halves == 1 && batch <= 32) XMC_LAUNCH_UPDATE_K(WTYPE, RMODE, 1, KH, 1);                                               \
-    else if (halves == 1 && batch <= 64) XMC_LAUNCH_UPDATE_K(WTYPE, RMODE, 1, KH, 2);                                          \
+    if (halves == 1 && batch <= 32 && !KH) XMC_LAUNCH_UPDATE_K(WTYPE, RMODE, 1, false, 1);                                     \
+    else if (halves == 1 && batch <= 64 && !KH) XMC_LAUNCH_UPDATE_K(WTYPE, RMODE, 1, false, 2);                                \
     else if (halves == 1) XMC_LAUNCH_UPDATE_K(WTYPE, RMODE, 1, KH, 4);                                                         \
     else if (halves == 2) XMC_LAUNCH_UPDATE_K(WTYPE, RMODE, 2, KH, 4);                                                         \
     else XMC_LAUNCH_UPDATE_K(WTYPE, RMODE, 4, KH, 4);                                                                          \
