@@ -72,6 +72,8 @@ def load():
     lib.xmc_debug_spin_limit.argtypes = [i32]
     lib.xmc_tiled_workspace_bytes_ex.restype = sz
     lib.xmc_tiled_workspace_bytes_ex.argtypes = [i32, i32, i32, i32]
+    lib.xmc_tiled_update_streams.restype = i32
+    lib.xmc_tiled_update_streams.argtypes = [i32, i32, i32, i32]
     lib.xmc_tiled_step.restype = i32
     lib.xmc_tiled_step.argtypes = [ctypes.POINTER(vp), i32, i32, i32, i32, vp, i32, i32, vp, i32, f32,
                                    ctypes.POINTER(ctypes.c_uint32), i32, i32, i32, vp, i32, i32, vp, vp, vp, vp, sz, vp]

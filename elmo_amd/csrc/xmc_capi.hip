@@ -806,6 +806,11 @@ int xmc_pass_on_error(const int32_t* error_word, int32_t* into_error, int32_t* i
 size_t xmc_tiled_error_offset(void) { return TW_ERR; }
 size_t xmc_tiled_sticky_error_offset(void) { return TW_ERR + 4; }
 
+int xmc_tiled_update_streams(int cus, int features, int batch, int tiles) {
+  if ((features != D && features != 1024) || batch <= 0 || batch > T_HALVES * BP || cus <= 0 || tiles <= 0) return XMC_ERR_SHAPE;
+  return tup_streams(cus, tiled_halves(batch), features, tiles);
+}
+
 int xmc_tiled_step(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, int rows_last_chunk, int weight_type,
                    const void* x_bf16, int batch, int features, const int32_t* labels_coo, int nnz, float lr,
                    const uint32_t* seeds, int round_mode, int quantize_x, int saturate, void* kahan, int kahan_type,
@@ -970,13 +975,7 @@ static int tiled_step_t(void* const* chunk_ptrs, int num_chunks, int rows_per_ch
         else tiled_gradx_kernel<W_E4M3, 2, DD><<<ggrid, 512, TgxGeom<W_E4M3, 2, DD>::LDS, stream>>>(w, rows, (int)rows_buf, rp, range, cs, spc, gsrc, g_half, live - h0 * BP, pdst, part_half);
       }
     }
-    const int nsub_u = tup_threads(halves) / 256;    // tiles a workgroup of the update kernel works on at a time
-    const int nfb = (DD / 64) / tup_csteps(halves, DD);
-    // streams of tiles: as many as the compute units hold at once, a multiple of eight (see the kernel's index map)
-    int ustreams = ((tiles + nsub_u - 1) / nsub_u + 7) / 8 * 8;
-    const int umost = di.cus * (halves == 1 ? 3 : 1) / nfb / 8 * 8;
-    if (ustreams > umost && umost > 0) ustreams = umost;
-    const int ugrid = tred_waves(DD) * halves / (tup_threads(halves) / 64) + nfb * ustreams;
+    const int ugrid = tred_waves(DD) * halves / (tup_threads(halves) / 64) + (DD / 64) / tup_csteps(halves, DD) * tup_streams(di.cus, halves, DD, tiles);
     const bool final_sum = c + nch == num_chunks;
     const TiledSum sum = {partial, part_half, nch, spc, range, rp, weight_type == W_BF16 ? 1 : 0, gx_total, batch,
                           final_sum ? (unsigned short*)grad_x_bf16 : nullptr, final_sum ? grad_x_f32 : nullptr};

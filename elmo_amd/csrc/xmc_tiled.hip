@@ -790,12 +790,32 @@ constexpr int tup_xbytes(int halves, int dd = D, int nks = BP / 32) { return tup
 constexpr int tup_threads(int halves) { return halves == 1 ? 256 : 512; }
 constexpr int tup_lds_bytes(int halves, int dd = D, int nks = BP / 32) { return halves * tup_xbytes(halves, dd, nks); }
 
-// Streams of tiles, as many as the compute units hold workgroups for, so that none starts when others are half done (four tiles a workgroup
-// before: 1,024 features, FP8 sr_fast, 46 K labels, batch 208 55 us a launch, now 48, 20 K, 448 62 / 53; bf16, 150 K, 256 189 / 180; one
-// batch half the same).
-// Launched with tup_threads(HALVES) threads and tup_lds(HALVES) bytes of LDS: four wavefronts per tile, so that a
-// compute unit runs at least eight wavefronts with one batch half (three workgroups) as with more (one workgroup of
-// eight wavefronts, two tiles at a time).
+// Streams of tiles of a launch over `tiles` tiles: a multiple of eight (see the kernel's index map), (dd / 64) / CS workgroups each.  A workgroup
+// loads its X^T operands once, so that it wants many tiles; but with one to five workgroups on a compute unit (registers and LDS of the
+// variant) streams that only just fill the device all end with the slowest, and a launch over many tiles is faster with more of them.
+// One batch half: three workgroups a compute unit, doubled up to twelve while a stream keeps five tiles.  Two or four: one, but three where
+// a stream keeps ten pairs of tiles and the operands are 64 KiB (96 with two halves of 768 features), and where streams in eights of one
+// workgroup each would leave compute units idle (768 features, four halves: 16 x 12 workgroups for 256).  us a step with weight decay,
+// the fewer / the more: 1,024 features, 670 K labels, batch 128, FP8 sr_fast 917 / 877, bf16 Philox 1674 / 1620, batch 256, e4m3 with
+// bf16 products, Philox 1942 / 1859;  768 features, batch 512, bf16 Philox, 670 K 3083 / 2897, 131 K 628 / 586.  Where it takes the fewer:
+// 1,024 features, 20 K, bf16 nearest, batch 256 88.7 / 91.1, 768 features, batch 256, Philox, 131 K 346 / 352, 670 K 1719 / 1730, batch 128,
+// 20 K, nearest 48.8 / 51.3.  (Four tiles a workgroup, before there were streams: the four cases in front 878, 1650, 1905, 3167.  What is slower
+// than then: 1,024 features, 670 K, batch 128, bf16 to nearest, 1294 instead of 1275.)
+inline int tup_streams(int cus, int halves, int dd, int tiles) {
+  const int nfb = dd / 64 / tup_csteps(halves, dd), at_once = tup_threads(halves) / 256, units = (tiles + at_once - 1) / at_once;
+  auto most = [&](int per_cu) { return cus * per_cu / nfb / 8 * 8; };
+  int per_cu = halves == 1 ? 3 : 1;
+  if (halves == 1) {
+    while (per_cu < 12 && units >= 5 * most(2 * per_cu)) per_cu *= 2;
+  } else if (most(1) * nfb < cus || (halves * tup_xbytes(halves, dd) <= 65536 && units >= 10 * most(3))) {
+    per_cu = 3;
+  }
+  const int all = (units + 7) / 8 * 8, m = most(per_cu);
+  return m > 0 && m < all ? m : all;
+}
+
+// Launched with tup_threads(HALVES) threads and tup_lds_bytes(HALVES, DD, NKS) bytes of LDS: four wavefronts per tile; with more than one
+// batch half eight wavefronts work on two tiles at a time.
 // HALVES (batch halves: 1, 2 or 4) and KAHAN (a compensated head may be present) are template parameters: with run-time
 // branches around the products the compiler issued every LDS operand read right in front of its matrix instruction.
 // NKS: K steps of 32 batch rows (of a half; 1, 2 or 4 with one half, 4 with a compensated head: twelve more variants of that, and the

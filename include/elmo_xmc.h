@@ -283,6 +283,12 @@ int xmc_tiled_step_ex(void* const* chunk_ptrs, int num_chunks, int rows_per_chun
                       int num_head, float weight_decay, float dropout_p, unsigned long long dropout_seed, void* grad_x_bf16,
                       float* grad_x_f32, float* loss_out, void* workspace, size_t workspace_bytes, void* stream);
 
+/* Diagnostics (no counterpart in the reference), host-only: streams of tiles that the update kernel of the three-kernel form is launched
+ * with on `cus` compute units, for a launch over `tiles` tiles of 64 label rows; each stream is 4 to 16 workgroups.  (With 768
+ * features, e4m3 weights, 129 to 256 batch rows and no compensated head another kernel does the update.)  XMC_ERR_SHAPE for what
+ * xmc_tiled_step does not take. */
+int xmc_tiled_update_streams(int cus, int features, int batch, int tiles);
+
 /* Byte offsets, inside the workspace of xmc_tiled_step, of its error word and its sticky error word (one int32 each; no
  * counterpart in the reference).  With 768 features, without a compensated head, a loss or weight decay, the step is one
  * persistent kernel; for batches of more than 64 rows the workgroups that share a tile sequence wait for one another as

@@ -194,3 +194,21 @@ def test_pass_on_error_rejects_bad_arguments_before_touching_the_device():
     assert lib.xmc_pass_on_error(None, P, P, None) == -1
     assert lib.xmc_pass_on_error(P, P, None, None) == -1 and lib.xmc_pass_on_error(P, None, P, None) == -1
     assert lib.xmc_pass_on_error(P + 2, P, P, None) == -3 and lib.xmc_pass_on_error(P, P, P + 1, None) == -3
+
+
+@pytest.mark.parametrize("features,batch,per_stream", [(768, 32, 4), (768, 128, 4), (768, 256, 4), (768, 512, 12),
+                                                       (1024, 64, 8), (1024, 128, 8), (1024, 256, 8), (1024, 512, 16)])
+def test_streams_of_the_update_fill_the_compute_units(features, batch, per_stream):
+    """Streams come in eights, no more than there are tiles for; from 131 K labels on their workgroups are whole rounds over 256
+    compute units, and over many tiles there are several rounds except where a workgroup's operands fill half of its LDS."""
+    streams = lambda tiles: _lib.load().xmc_tiled_update_streams(256, features, batch, tiles)
+    at_once = 1 if batch <= 128 else 2
+    for tiles in (1, 7, 8, 9, 40, 157, 313, 1000, 2048, 10470, 134000):
+        n = streams(tiles)
+        assert n % 8 == 0 and 0 < n < (tiles + at_once - 1) // at_once + 8
+        if tiles >= 2048:       # 131 K labels
+            assert n * per_stream % 256 == 0 and n * per_stream >= (768 if batch <= 128 else 256), (tiles, n)
+        if tiles >= 10470:
+            assert n * per_stream == (3072 if batch <= 128 else 256 if (features, batch) == (768, 256) else 768), (tiles, n)
+    for bad in ((0, features, batch, 1), (256, 512, batch, 1), (256, features, 513, 1), (256, features, 0, 1), (256, features, batch, 0)):
+        assert _lib.load().xmc_tiled_update_streams(*bad) == -2
