@@ -943,7 +943,7 @@ static int tiled_step_t(void* const* chunk_ptrs, int num_chunks, int rows_per_ch
           tile_ptr + (hh >> 1) * tp_stride + c * tiles_per_chunk, label0_seg, glb + hh * g_half, gbl + hh * g_half, g_half, live - hh * BP);
     }
     for (int hh = 0; !fp8_logits && hh < halves; hh++) {
-      if (hh * BP >= live && !loss_out) break;   // (a loss is summed over every launch's tiles)
+      if (hh * BP >= live) break;   // no batch rows: no G, nothing to add to the loss
       unsigned short* gl = glb + hh * g_half;
       unsigned short* gb = gbl + hh * g_half;
       const unsigned short* xh = xb + (size_t)hh * BP * DD;

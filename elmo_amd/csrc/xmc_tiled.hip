@@ -263,7 +263,8 @@ __global__ __launch_bounds__(512, 1) void tiled_logits_kernel(const void* w, int
 #pragma unroll
   for (int ks = 0; ks < DD / 32; ks++) xr[ks] = *(const bf16x8*)(xb + ((size_t)(v * (DD / 32) + ks) * 64 + lane) * 8);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // from here on the loop counts its own operations: nothing is in flight
-  const bool active = LOSS || 32 * (v >> 1) < live_rows;   // its K step of 32 batch rows has any
+  const bool active = 32 * (v >> 1) < live_rows;   // its K step of 32 batch rows has any
+  if (LOSS && !active && lane == 0) wsum[v] = 0.f;
   int it = 0, b0 = 0, b2 = NB - 1;   // it % NB, (it + NB - 1) % NB
   for (int st = blockIdx.x; st < nsub; st += gs, it++) {
     // younger than the loads of this sub-tile: the loads of the next one and the stores of up to two steps
@@ -281,7 +282,10 @@ __global__ __launch_bounds__(512, 1) void tiled_logits_kernel(const void* w, int
     const int buf = b0;
     b0 = b0 == NB - 1 ? 0 : b0 + 1;
     b2 = b2 == NB - 1 ? 0 : b2 + 1;
-    if (!active) continue;
+    if (!active) {
+      if (LOSS) __syncthreads();   // the one in front of the sum of the shares below
+      continue;
+    }
     floatx4 acc[2] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
     const unsigned abase = (unsigned)(buf * G::BUF + l16 * G::STRIDE + kg * (WT == W_BF16 ? 16 : 8));
     // the LDS reads run three K steps ahead of the MFMAs (everything unrolled: xr must stay in registers)

@@ -103,6 +103,31 @@ def test_nothing_is_read_of_rows_that_the_batch_does_not_have(gpu, kind, batch):
     assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
 
 
+@pytest.mark.parametrize("kind", ["bf16", "sim"])
+@pytest.mark.parametrize("batch", [16, 33, 257, 300])
+def test_a_loss_writes_no_more_than_its_shares(gpu, kind, batch):
+    """Rows that the batch does not have, whole halves among them, are left out with a loss as without: beyond its two shares a tile
+    it touches nothing of the workspace that the step without one leaves alone."""
+    import torch
+    from elmo_amd import ops
+    rows, d, tiles = 400, 1024, 7
+    gen = torch.Generator(device=gpu).manual_seed(batch)
+    w0 = (torch.randn(rows, d, generator=gen, device=gpu) * 0.02).to(torch.bfloat16 if kind == "bf16" else torch.float8_e4m3fn)
+    x = torch.randn(batch, d, generator=gen, device=gpu).to(torch.bfloat16)
+    labels = torch.tensor([[0, 0], [batch - 1, rows - 1], [batch // 2, 200]], dtype=torch.int32, device=gpu)
+    loss, out = torch.zeros(1, device=gpu), []
+    for loss_out in (None, loss):
+        w = w0.clone()
+        ws = torch.full((ops.tiled_workspace_bytes(1, rows, batch, d),), 255, dtype=torch.uint8, device=gpu)
+        g = ops.tiled_step([w], rows, "bf16" if kind == "bf16" else "e4m3", x, labels, 0.1, workspace=ws, loss_out=loss_out)
+        out.append((w.view(torch.uint8), g, ws != 255))
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
+    assert int((out[1][2] & ~out[0][2]).sum()) <= 2 * tiles * 4
+    z = (x.float() @ w0.float().t()).to(torch.bfloat16).double()
+    ref = z.clamp(min=0).sum() - z[labels[:, 0].long(), labels[:, 1].long()].sum() + torch.log1p(torch.exp(-z.abs())).sum()
+    assert abs(loss.item() - ref.item()) <= 1e-4 * abs(ref.item())      # (as in test_loss_over_four_halves)
+
+
 def test_loss_over_four_halves(gpu):
     """Ragged chunks and a batch that ends inside the third half: rows that pad either do not count."""
     import torch
