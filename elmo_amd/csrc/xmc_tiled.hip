@@ -16,10 +16,13 @@ enum WType { W_E4M3 = 0, W_BF16 = 1 };
 constexpr int T_SPLITS = 64;                       // most label ranges of the grad_X kernel
 // Label ranges (times four feature quarters: workgroups) of a grad_X launch over `rows` label rows.  A range writes the sums of all batch rows,
 // 512 KiB a batch half at 1,024 features, which the update's launch reads again; with few labels that costs more than the idle
-// compute units of fewer ranges.  s ranges take steps / s steps of 32 labels and s sums, least where s^2 is proportional to the steps:
-// 64 from 65 K labels on, 8 up to 1,024.  us a step, 64 ranges / with s^2 = 0.5, 1, 2 times the steps (1,024 features): FP8, batch 448,
-// 2,500 labels 72.7 / 72.9 68.9 69.0, 8 K 97.8 / 94.3 94.3 90.7, 20 K 141 / 149 139 137, 46 K 220 / 234 228 221;  batch 208, 8 K 52.6 / 53.0
-// 52.8 50.5;  bf16, batch 16, 8 K 39.0 / 35.1 37.3 37.8, 46 K 80.3 / 84.4 81.3 79.0;  batch 300, 8 K 95.5 / 94.5 95.7 92.0.
+// compute units of fewer ranges.  s ranges take steps / s steps of 32 labels and s sums, least where s^2 is proportional to the steps;
+// in eights, so 8 up to 1,024 rows and 64 from 50 K rows of a launch on (56^2 = 2 x 1,568).  us a step, 64 ranges / with s^2 = 0.5, 1, 2
+// times the steps, 1,024 features: FP8, batch 448, 2,500 labels 72.7 / 72.9 68.9 69.0, 8 K 97.8 / 94.3 94.3 90.7, 20 K 141 / 149 139 137,
+// 46 K 220 / 234 228 221;  batch 208, 8 K 52.6 / 53.0 52.8 50.5;  bf16, batch 16, 8 K 39.0 / 35.1 37.3 37.8, 46 K 80.3 / 84.4 81.3 79.0.
+// 768 features, 64 ranges / s^2 = 2, 3, 4 times the steps, geometric mean over weights and batches of 16 to 448: 3 K labels 1.082 / 1 1.008
+// 1.007, 8 K 1.028 / 1 0.963 0.965, 14 K 1.020 / 1 1.003 1.010, 27 K 1.023 / 1 1.014 1.022.  Several chunks share the ranges of a launch, none
+// across a boundary; 8 K labels in eight chunks, bf16, batch 128, 64 ranges / these (24) 34.3 / 34.3, batch 448 92.4 / 88.7.
 inline int tiled_splits(int rows) {
   const int steps = rows / 32;
   int s = 8;
@@ -643,7 +646,7 @@ template <int DD>
 __device__ __forceinline__ void tiled_reduce_wave(int widx, int half, int lane, const TiledSum& r, int cs, const DropoutParams& dp) {
   const floatx4* partial = r.partial + (size_t)half * r.part_half;
   const int spc = r.spc, range = r.range, bound = r.bound;
-  // (slot, fb, wavefront of the grad_X kernel's layout); eight loads in flight
+  // (slot, fb, wavefront of the grad_X kernel's layout)
   const int slot = widx >> 4, fb = (widx >> 2) & 3, wv = widx & 3;
   const int tid = wv * 64 + lane, l16 = lane & 15, kg = lane >> 4;
   constexpr int NN = DD / 256, SL = 8 * NN;   // blocks of 16 features per wavefront; slots per (split, feature quarter)
@@ -652,21 +655,27 @@ __device__ __forceinline__ void tiled_reduce_wave(int widx, int half, int lane, 
   floatx4 tot = {0.f, 0.f, 0.f, 0.f};
   const int row0 = BP * half + 16 * mb;
   if (row0 >= r.batch) return;
-  for (int ck = 0; ck < r.nchunks; ck++) {   // the chunks of the launch, each summed (and rounded) by itself
-    const int crows = min((ck + 1) * cs, bound) - ck * cs, splits = (crows + range - 1) / range;
-    const floatx4* pc = partial + (size_t)ck * spc * 4 * SL * 256;
-    floatx4 s = {0.f, 0.f, 0.f, 0.f};
-    int sp = 0;
-    for (; sp + 8 <= splits; sp += 8) {
-      floatx4 v[8];
+  // Every chunk but the last has spc ranges: all partials lie one behind the other, and eight loads are in flight whatever a chunk's number of
+  // ranges (a chunk's last one to seven were loaded one after the other before: 1,024 features, 8 K labels in eight chunks, three
+  // ranges each, batch 128 41.4 us a step, now 36.8).
+  const int last = (min(r.nchunks * cs, bound) - (r.nchunks - 1) * cs + range - 1) / range, n = (r.nchunks - 1) * spc + last;
+  floatx4 s = {0.f, 0.f, 0.f, 0.f};
+  int left = spc;   // ranges of the chunk that are not summed yet
+  for (int e0 = 0; e0 < n; e0 += 8) {
+    floatx4 v[8];
 #pragma unroll
-      for (int x = 0; x < 8; x++) v[x] = pc[(((size_t)(sp + x) * 4 + fb) * SL + slot) * 256 + tid];
+    for (int x = 0; x < 8; x++) v[x] = partial[(((size_t)min(e0 + x, n - 1) * 4 + fb) * SL + slot) * 256 + tid];
 #pragma unroll
-      for (int x = 0; x < 8; x++) s += v[x];
+    for (int x = 0; x < 8; x++) {
+      if (e0 + x >= n) break;
+      s += v[x];
+      if (--left == 0 || e0 + x == n - 1) {   // the chunks are rounded one by one
+#pragma unroll
+        for (int i = 0; i < 4; i++) tot[i] += r.round_bf16 ? bf16_rt(s[i]) : s[i];
+        s = floatx4{0.f, 0.f, 0.f, 0.f};
+        left = spc;
+      }
     }
-    for (; sp < splits; sp++) s += pc[(((size_t)sp * 4 + fb) * SL + slot) * 256 + tid];
-#pragma unroll
-    for (int i = 0; i < 4; i++) tot[i] += r.round_bf16 ? bf16_rt(s[i]) : s[i];
   }
 #pragma unroll
   for (int i = 0; i < 4; i++) {

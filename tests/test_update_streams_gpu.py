@@ -92,3 +92,28 @@ def test_compensated_head_that_ends_in_a_later_tile(gpu, features, batch, rows, 
     tot_g = C.e4m3_decode(new[0][:head]).astype(np.float64) + kt.float().cpu().numpy()
     tot_r = C.e4m3_decode(ref_codes[0][:head]).astype(np.float64) + ref_k
     assert np.abs(tot_g - tot_r).max() <= 2.0 ** -6 * np.abs(ref_k).max() + 2.0 ** -16
+
+
+@pytest.mark.parametrize("features,batch", [(768, 40), (768, 300), (1024, 200)])
+@pytest.mark.parametrize("last", [1, 70, 640])
+def test_short_last_chunk_of_a_launch(gpu, features, batch, last):
+    """Chunks that lie one behind the other share a launch and its ranges of grad_X, of which a short last chunk has fewer than the
+    others: the same step with a launch for every chunk gives the same weights, and grad_X up to a chunk's bf16 rounding."""
+    import torch
+    from elmo_amd import ops
+    rows, nc = 1024, 4
+    gen = torch.Generator(device=gpu).manual_seed(last + batch)
+    w0 = (torch.randn(rows * (nc - 1) + last, features, generator=gen, device=gpu) * 0.02).to(torch.bfloat16)
+    x = torch.randn(batch, features, generator=gen, device=gpu).to(torch.bfloat16)
+    labels = torch.tensor([[0, 0], [batch - 1, w0.shape[0] - 1], [batch // 2, rows]], dtype=torch.int32, device=gpu)
+    out = []
+    for together in (True, False):
+        w = w0.clone()
+        views = w.split(rows) if together else [v.clone() for v in reversed(w.split(rows))][::-1]
+        g, gf = ops.tiled_step(views, rows, "bf16", x, labels, 0.1, weight_decay=0.02, want_f32=True)
+        out.append((torch.cat([v.view(torch.int16) for v in views]), gf))
+    assert torch.equal(out[0][0], out[1][0])
+    # each of the four chunks' sums is rounded to bf16; another order of its fp32 sum moves a sum near a tie by one unit, 2^-8 of it
+    assert (out[0][1] - out[1][1]).abs().max() <= nc * 2.0 ** -8 * out[1][1].abs().max()
+    # and few are near one: the sums differ by some 2^-20 of their terms' sum, a tie comes every 2^-8 of the value
+    assert (out[0][1] != out[1][1]).float().mean() < 0.05
