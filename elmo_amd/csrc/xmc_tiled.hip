@@ -137,7 +137,7 @@ __device__ __forceinline__ void tiled_prep_x_thread(int i, const unsigned short*
 // 64-row tile and write the first key of each, the others (in front of the first segment only) prepare X.  Bound by latency.  Before,
 // the images of X and, for every pair, a rank sort and a search for each tile's first key were launches one behind the other, and the
 // logits kernels went through a tile's keys one by one for every wavefront (a third of all positives lies in the first tile).  us a
-// step, 1,024 features, then / now: FP8 sr_fast, 19,655 labels, batch 448, 9.6 positives a row 419 / 154, 46 K, 208, 5.2 195 / 131,
+// step, 1,024 features, then / with this alone: FP8 sr_fast, 19,655 labels, batch 448, 9.6 positives a row 419 / 154, 46 K, 208, 5.2 195 / 131,
 // 300 K, 96, 5 416 / 402; e4m3 with bf16 products, nearest, 8 K, 200, 36 451 / 74; bf16, nearest, 300 K, 256, 5 915 / 873.
 struct TiledPrep {
   const int* coo; int nnz, batch, label_base, label_count, rows_per_chunk, tiles_per_chunk, num_tiles, ptr_blocks, pairs;
@@ -215,12 +215,12 @@ __device__ __forceinline__ void t_store_g(const unsigned (&sg)[2], int r0, int r
 
 // Batch rows come in K steps of 32 (of the update's products).  Wavefronts of the logits kernels and of the grad_X kernel whose rows lie in
 // none that has any only take part in the loads, and the update takes zeros in place of their G, which is not written: a batch of 8
-// to 32 rows used to pay for 128.  us a step, 1,024 features, before / now: bf16, Philox, 16 K labels, batch 13 75 / 61, 245 K, 12
+// to 32 rows used to pay for 128.  us a step, 1,024 features, before / with this: bf16, Philox, 16 K labels, batch 13 75 / 61, 245 K, 12
 // 664 / 590; FP8, nearest, 120 K, 32 161 / 120; e4m3 with bf16 products, Philox, 92 K, 44 226 / 196.
 
 // Vector memory operations retire in order.  Per sub-tile a wavefront issues its loads of the sub-tile two steps ahead
 // (always, past the end they fetch the last sub-tile again into a buffer nobody reads, so that the count is the same in
-// every step) and then ten stores of G.  The wait at the top of a step leaves in flight what was issued after the
+// every step) and then, if its batch rows exist, three stores of G.  The wait at the top of a step leaves in flight what was issued after the
 // loads of the sub-tile it is about to read.
 template <int WT, bool LOSS, int DD>
 __global__ __launch_bounds__(512, 1) void tiled_logits_kernel(const void* w, int rows, int nsub, const unsigned short* xb,
@@ -692,9 +692,10 @@ __device__ __forceinline__ void tiled_reduce_wave(int widx, int half, int lane, 
   }
 }
 
-// ---- grad_W and the SGD update of one chunk, in place.  blockIdx = tile*4 + fb; wavefront w owns label rows 16w..16w+15
-//      of the tile and features 192fb.. (12 blocks of 16).  A^T[f][l] = sum_b X^T[f][b] G[l][b].  The rows of a feature
-//      block are permuted (row 4kg+e of block nn = 4c+q is feature 192fb + 64c + 16kg + 4q + e, see tiled_prep_x_thread)
+// ---- grad_W and the SGD update of one launch's chunks, in place.  A stream of tiles is one workgroup for every CS x 64 features (index
+//      map in the kernel); wavefront w of four owns label rows 16w..16w+15 of a tile and all of the workgroup's features (4 CS blocks of
+//      16).  A^T[f][l] = sum_b X^T[f][b] G[l][b].  The rows of a feature block are permuted (row 4kg+e of block 4c+q is feature
+//      64 (CS fb + c) + 16kg + 4q + e, see tiled_prep_x_thread)
 //      so that a lane ends up with 16 consecutive features of one label row per step c, and the four lanes of a row
 //      with 64 consecutive bytes.
 //        bf16 weights : a = bf16(A); t = w - lr*a; RTN: bf16(t);  SR: bits(t) + (philox(seed, l*768+f) & 0xFFFF), clear 16 bits
@@ -831,15 +832,17 @@ inline int tup_streams(int cus, int halves, int dd, int tiles) {
 // batch half eight wavefronts work on two tiles at a time.
 // HALVES (batch halves: 1, 2 or 4) and KAHAN (a compensated head may be present) are template parameters: with run-time
 // branches around the products the compiler issued every LDS operand read right in front of its matrix instruction.
-// NKS: K steps of 32 batch rows (of a half; 1, 2 or 4 with one half, 4 with a compensated head: twelve more variants of that, and the
-// dense logits of 131 K labels, batch 40, whose kernel lies in the same code object, took 27.1 instead of 26.4 us a call).
+// NKS: K steps of 32 batch rows (of a half; 1, 2 or 4 with one half; with a compensated head, which this form hardly ever has up to 64
+// rows, always 4).  us a step with weight decay, NKS / 4 with zeros: 768 features, batch 32, FP8 sr_fast, 131 K labels 95.5 / 106.5,
+// 670 K 519 / 539, 20 K 35.7 / 38.9, bf16 Philox, 131 K 200 / 212, nearest 135 / 139;  batch 64, FP8, 131 K 99.7 / 110;  1,024 features, batch
+// 32, 131 K, FP8 118 / 128, bf16 nearest 200 / 203, 670 K 1181 / 1170 (the one case that is slower).
 template <int WT, int MODE, int HALVES, bool KAHAN, int DD, int NKS>
 __global__ __launch_bounds__(HALVES == 1 ? 256 : 512, HALVES == 1 ? 3 : HALVES == 2 ? 2 : 1) void tiled_update_kernel(
     void* w, int rows, int ntiles, const unsigned short* glb, size_t g_half_stride, const unsigned short* xT, float lr, float wd, TiledSeeds seeds,
     int cs, int saturate, void* kahan, int kahan_type, int num_head, unsigned label0, int live_rows, TiledSum red, DropoutParams dp) {
   static_assert(!KAHAN || WT == W_E4M3, "the compensated head belongs to the FP8 layer");
   // the first workgroups sum the chunk's grad_X partials (384 wavefronts per batch half), the others update the weights
-  static_assert(NKS == BP / 32 || HALVES == 1, "a K step of the first half only");
+  static_assert(NKS == BP / 32 || HALVES == 1, "fewer K steps only with one half");
   constexpr int CS = tup_csteps(HALVES, DD), XB = tup_xbytes(HALVES, DD, NKS), NFB = (DD / 64) / CS, WAVES = tup_threads(HALVES) / 64;
   constexpr int TRED_WAVES = tred_waves(DD), RED_BLOCKS = TRED_WAVES * HALVES / WAVES;
   if ((int)blockIdx.x < RED_BLOCKS) {
@@ -867,8 +870,8 @@ __global__ __launch_bounds__(HALVES == 1 ? 256 : 512, HALVES == 1 ? 3 : HALVES =
     }
   }
   __syncthreads();
-  // The G rows and the weights of the next tile are loaded before the products of the current one: a wavefront waits
-  // for memory once per launch, not four times per tile.
+  // The G rows and the weights of the stream's next tile are loaded before the products of the current one: a wavefront waits for
+  // memory once a tile, for loads that were issued a tile ago.
   constexpr int WDW = WT == W_BF16 ? 8 : 4;   // dwords of 16 weights
   bf16x8 gf_n[HALVES][NKS];
   intx4 wr_n[CS][WDW / 4];

@@ -116,7 +116,7 @@ class XMCBCECHUNKEDLayer(nn.Module):
                        logits is computed inside the logits kernel and returned (one host synchronisation).  This is
                        the value the reference's _compute_loss is written to return (chunked.py:57-72); the reference
                        itself passes the weight chunk where the logits belong (chunked.py:109).  Such a step runs as three
-                       kernels per chunk: 1.4 to 2.5 times as long, and because its sums are taken in another order some
+                       kernels per chunk: 1.0 to 2.3 times as long, and because its sums are taken in another order some
                        weights (up to 15 in a million, measured) round differently than with skip_loss=True.
         '''
         assert embed.is_cuda and embed.dim() == 2 and embed.shape[1] == self.features

@@ -169,7 +169,7 @@ def test_dropout_quantize_rejects_bad_arguments_before_touching_the_device():
 
 
 def test_three_kernel_path_accepts_label_spaces_of_2_24_and_more():
-    """The sort key keeps 24 bits for the label; the tiled step takes larger label spaces in segments of whole
+    """The key of a positive keeps 24 bits for the label; the tiled step takes larger label spaces in segments of whole
     chunks, so 64 chunks of 262,272 rows (16,785,408 labels) pass the range check and fail only on the workspace size
     given here (no device is touched).  A single chunk of 2^24 rows, and the fused path at this size, are refused."""
     lib = _lib.load()

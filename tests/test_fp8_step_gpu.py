@@ -102,7 +102,7 @@ def test_duplicate_and_dense_positives(gpu):
 
 
 def test_many_positives_boundary_labels_and_ignored_entries(gpu):
-    """Close to the 32,768 pairs a step accepts (the sort and the descriptor search then use their largest LDS
+    """Close to the 32,768 pairs a step accepts (the launch that groups them by tile then uses its largest LDS
     footprint), with positives on the first and last label, on both sides of the chunk boundary and in every batch
     row; pairs whose row or label lies outside the batch or the label space are ignored."""
     nc, rows, batch = 2, 4096, 128
@@ -208,7 +208,7 @@ def test_step_replays_in_a_captured_graph(gpu):
 
 @pytest.mark.parametrize("nnz", [1, 63, 64, 65, 193, 1025, 4609])
 def test_sort_pads_the_positives_to_whole_blocks_only(gpu, nnz):
-    """Numbers of positives around the sort's block of 64 keys, in random order and with repetitions, against the oracle."""
+    """Numbers of positives around whole wavefronts of 64, from which the grouping by tile takes them, in random order and with repetitions, against the oracle."""
     case = H.make_case(2, 1040, 64, 90 + nnz)
     rng = np.random.default_rng(nnz)
     case["labels"] = np.stack([rng.integers(0, 64, nnz), rng.integers(0, 2 * 1040, nnz)], axis=1).astype(np.int32)

@@ -131,7 +131,8 @@ def test_bf16_layer_at_131k_labels_against_the_whole_oracle(gpu):
 
 def test_label_space_above_2_24_on_the_three_kernel_path(gpu):
     """16,785,408 labels (64 chunks of 262,272 rows, 12.9 GB of e4m3 weights), batch 32, true-FP8 arithmetic: the positives
-    are sorted in two segments of the label space (63 chunks + 1).  Positives on both sides of the segment boundary, at
+    are taken in two segments of the label space (63 chunks + 1).  (Plain steps of 768 features run as one kernel; with weight decay,
+    in three: test_three_kernel_gpu.py.)  Positives on both sides of the segment boundary, at
     label 2^24 and beyond and on the last label; lr = 0 is the identity, grad_X equals library GEMMs over all chunks,
     sampled rows (among them every row with a positive) equal the oracle after a real step."""
     import torch

@@ -177,7 +177,7 @@ def test_replays_of_a_captured_step_with_weight_decay(gpu):
 
 
 def test_label_space_above_2_24_with_weight_decay(gpu):
-    """The positives are sorted in two segments of the label space (63 chunks + 1): positives and sampled rows on both sides of
+    """The positives are taken in two segments of the label space (63 chunks + 1): positives and sampled rows on both sides of
     the segment boundary, at label 2^24 and at the end."""
     import torch
     from elmo_amd import ops

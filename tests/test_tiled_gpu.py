@@ -169,7 +169,7 @@ def test_bf16_layer_duplicates_and_no_positives(gpu):
 
 
 def test_bf16_layer_many_positives_over_four_halves(gpu):
-    """30,000 positives (close to the 32,768 a step accepts) spread over 512 batch rows, i.e. over both sorted lists, with
+    """30,000 positives (close to the 32,768 a step accepts) spread over 512 batch rows, i.e. over both lists (one for every 256 rows), with
     pairs on the first and last row of every half; entries outside the batch are ignored."""
     L, nc, batch = 2048, 2, 512
     x, w, _ = bf16_case(L, batch, 39)
