@@ -57,9 +57,11 @@ void fill_device_info(int dev) {
   cluster_set_lds_sim();
   cluster_set_lds_fp8();
   (void)hipFuncSetAttribute((const void*)cluster_prep_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, MAX_POS * 4);
-  (void)hipFuncSetAttribute((const void*)fp8_forward_kernel<1, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, FwdGeom<1>::LDS);
-  (void)hipFuncSetAttribute((const void*)fp8_forward_kernel<1, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, FwdGeom<1>::LDS);
-  (void)hipFuncSetAttribute((const void*)fp8_forward_kernel<2, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, FwdGeom<2>::LDS);
+  (void)hipFuncSetAttribute((const void*)fp8_forward_kernel<1, 1, false>, hipFuncAttributeMaxDynamicSharedMemorySize, FwdGeom<1>::LDS);
+  (void)hipFuncSetAttribute((const void*)fp8_forward_kernel<1, 4, false>, hipFuncAttributeMaxDynamicSharedMemorySize, FwdGeom<1>::LDS);
+  (void)hipFuncSetAttribute((const void*)fp8_forward_kernel<2, 1, false>, hipFuncAttributeMaxDynamicSharedMemorySize, FwdGeom<2>::LDS);
+  (void)hipFuncSetAttribute((const void*)fp8_forward_kernel<1, 1, true>, hipFuncAttributeMaxDynamicSharedMemorySize, FwdGeom<1, true>::LDS);
+  (void)hipFuncSetAttribute((const void*)fp8_forward_kernel<1, 4, true>, hipFuncAttributeMaxDynamicSharedMemorySize, FwdGeom<1, true>::LDS);
   (void)hipFuncSetAttribute((const void*)fp8_forward_select_kernel<0, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, SelGeom<4>::LDS);
   (void)hipFuncSetAttribute((const void*)fp8_forward_select_kernel<1, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, SelGeom<4>::LDS);
   (void)hipFuncSetAttribute((const void*)fp8_forward_select_kernel<0, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, SelGeom<8>::LDS);
@@ -173,6 +175,15 @@ void prep_x(const void* x_bf16, int batch, float scale_x, unsigned char* xq, hip
   prep_x_kernel<<<n / 256, 256, 0, stream>>>((const unsigned short*)x_bf16, batch, n, 1.0f / scale_x, xq);
 }
 
+// Whether the workgroups of the logits kernel convert X themselves instead of reading an image that a launch in front has written.
+// The launch is 3 us of the GPU, and what bounds small label spaces is the host's 4 us for it; the conversion takes a workgroup longer
+// the more rows it has, without loads of tiles on their way from 49 rows on.  us a call, image / conversion, by rows:
+//   1   131 K labels 20.0/17.9    40  30 K 12.6/9.9, 131 K 22.1/21.2, 300 K 40.9/40.0, 670 K 118.0/116.6    48  48 K 12.6/11.8
+//   64  2 K 12.0/9.4, 32 K 12.1/10.3, 48 K 13.0/13.7, 131 K 23.3/24.4
+//   100, 128  2 K 12.0/9.5 11.9/10.0 among others, but 24.5/25.0 24.6/26.0 alone
+bool forward_converts(int batch, long long tiles, int cus) {
+  return batch <= 48 || (batch <= FWD_CONV && tiles <= 4 * (long long)cus);
+}
 // The launches of the inference logits, shared by xmc_fp8_forward (operand images in the caller's workspace) and
 // xmc_fp8_forward_static (operand images in this device's copy of the static array); shapes are checked by the callers.
 int forward_launch(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, const void* x_bf16, int batch, float scale_w,
@@ -182,11 +193,14 @@ int forward_launch(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, 
   if (!(scale_w > 0.f) || !(scale_x > 0.f)) return XMC_ERR_SHAPE;
   DeviceInfo di = device_info();
   if (di.ok != 1) return XMC_ERR_DEVICE;
-  prep_x(x_bf16, batch, scale_x, xq, stream);
+  const bool conv = forward_converts(batch, (num_labels + FT - 1) / FT, di.cus);
+  if (!conv) prep_x(x_bf16, batch, scale_x, xq, stream);
   ForwardParams fp;
   for (int c = 0; c < MAX_CHUNKS; c++) fp.chunk[c] = c < num_chunks ? (const unsigned char*)chunk_ptrs[c] : nullptr;
   fp.rows_per_chunk = rows_per_chunk;
   fp.tiles_per_chunk = (rows_per_chunk + FT - 1) / FT;
+  fp.x = (const unsigned short*)x_bf16;
+  fp.inv_scale_x = 1.0f / scale_x;
   const int last_chunk = (int)((num_labels - 1) / rows_per_chunk);
   fp.tile_begin = 0;
   fp.tile_end = last_chunk * fp.tiles_per_chunk + (int)((num_labels - (long long)last_chunk * rows_per_chunk + FT - 1) / FT);
@@ -203,9 +217,11 @@ int forward_launch(void* const* chunk_ptrs, int num_chunks, int rows_per_chunk, 
   // 37.8/35.4 51.0/52.0, 131 K 22.4/22.4 27.5/27.7, 128 rows, 50 K 16.8/17.2: from 32 tiles for each compute unit on.  With more rows by no rule: 256 rows, 400 K 116/126, 500 K 200/193, 800 K 222/244, 1 M 413/386.
   const bool runs = batch <= BP && fp.tile_end >= 32 * di.cus;
   const int grid = fp.tile_end < di.cus ? fp.tile_end : di.cus;   // one workgroup fills the LDS of a compute unit
-  if (batch > BP) fp8_forward_kernel<2, 1><<<grid, FNT, FwdGeom<2>::LDS, stream>>>(fp);
-  else if (runs) fp8_forward_kernel<1, 4><<<grid, FNT, FwdGeom<1>::LDS, stream>>>(fp);
-  else fp8_forward_kernel<1, 1><<<grid, FNT, FwdGeom<1>::LDS, stream>>>(fp);
+  if (conv && runs) fp8_forward_kernel<1, 4, true><<<grid, FNT, FwdGeom<1, true>::LDS, stream>>>(fp);
+  else if (conv) fp8_forward_kernel<1, 1, true><<<grid, FNT, FwdGeom<1, true>::LDS, stream>>>(fp);
+  else if (batch > BP) fp8_forward_kernel<2, 1, false><<<grid, FNT, FwdGeom<2>::LDS, stream>>>(fp);
+  else if (runs) fp8_forward_kernel<1, 4, false><<<grid, FNT, FwdGeom<1>::LDS, stream>>>(fp);
+  else fp8_forward_kernel<1, 1, false><<<grid, FNT, FwdGeom<1>::LDS, stream>>>(fp);
   return launch_status();
 }
 
@@ -596,7 +612,7 @@ int xmc_fp8_forward_topk(void* const* chunk_ptrs, int num_chunks, int rows_per_c
     fp.tile_end = tile_end;
     fp.col0 = base;
     const int tiles = tile_end - tile_begin;
-    fp8_forward_kernel<1, 1><<<tiles < di.cus ? tiles : di.cus, FNT, FwdGeom<1>::LDS, stream>>>(fp);
+    fp8_forward_kernel<1, 1, false><<<tiles < di.cus ? tiles : di.cus, FNT, FwdGeom<1>::LDS, stream>>>(fp);
     int done = 0;
     if (n > 32768) {          // two workgroups per row
       if (have[0] < k || have[1] < k) {

@@ -13,9 +13,8 @@ __device__ __forceinline__ intx8 lds_read32(const unsigned char* q) {
   return intx8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
 }
 
-// Operand image of X for the inference kernels: e4m3(X / scale_x) in v_mfma 16x16x128 B-operand order,
-// [(w*2+nb)*6+ks][lane][32 bytes]; one thread per four features, rows at or past `batch` are zero.  (Converted by every
-// workgroup from X itself instead, without this launch: 9 us more per pass at batch 128.)
+// Operand image of X for the inference kernels (but for small batches, whose workgroups convert X themselves): e4m3(X / scale_x) in v_mfma 16x16x128 B-operand order,
+// [(w*2+nb)*6+ks][lane][32 bytes]; one thread per four features, rows at or past `batch` are zero.
 __global__ void prep_x_kernel(const unsigned short* x, int batch, int n, float inv_scale_x, unsigned char* xq) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
@@ -35,7 +34,9 @@ struct ForwardParams {
   const unsigned char* chunk[MAX_CHUNKS];
   int rows_per_chunk, tiles_per_chunk;
   int tile_begin, tile_end;
-  const unsigned char* xq;     // operand image of X
+  const unsigned char* xq;     // operand image of X, or
+  const unsigned short* x;     // X itself (FWD_CONV), bf16 [batch][768]
+  float inv_scale_x;
   float zscale;
   unsigned short* out;         // bf16 [batch][out_stride]
   long long out_stride;
@@ -48,11 +49,14 @@ constexpr int FT = 32;                    // labels per tile of the inference ke
 constexpr int FB = FT * WS;               // one tile in LDS (rows of 48 + 1 pieces of 16 bytes)
 constexpr int FNT = 512;                  // eight wavefronts of 32 batch rows: four per half of a tile's labels (128 rows), or eight (256)
 constexpr int ZS = FT * 2 + 16;           // LDS row stride of the staged logits [b][32 labels] bf16, bytes
+constexpr int FWD_CONV = 64;              // most batch rows whose X the workgroups of fp8_forward_kernel convert themselves
 // Geometry for up to HB x 128 batch rows
-template <int HB> struct FwdGeom {
+template <int HB, bool CONV = false> struct FwdGeom {
   static constexpr int BUF = HB == 1 ? 5 : 4;          // tile buffers in LDS, one workgroup to a compute unit
   static constexpr int ZB = HB * BP * ZS;              // a stage of logits
-  static constexpr int LDS = BUF * FB + 2 * ZB;
+  static constexpr int LDS = CONV ? 160 * 1024 : BUF * FB + 2 * ZB;
+  static constexpr int X = LDS - FWD_CONV * WS;        // (CONV) e4m3 X before the first tile; X as it comes lies in front of it
+  static_assert(!CONV || (BUF * FB + 2 * ZB <= LDS && X >= FWD_CONV * D * 2 && X % 16 == 0), "LDS budget");
 };
 constexpr int FWD_ROWS = 2 * BP;          // most batch rows of a launch
 
@@ -77,6 +81,33 @@ __device__ __forceinline__ void fwd_load_x(const unsigned char* xq_image, int w,
 #pragma unroll
     for (int ks = 0; ks < 6; ks++)
       xq[nb][ks] = *(const intx8*)(xq_image + ((size_t)((w * 2 + nb) * 6 + ks) * 64 + lane) * 32);
+}
+
+// X itself instead of its image, for up to FWD_CONV batch rows: straight to LDS as it comes, converted there, and read as the rows of
+// a tile are; it saves the launch in front.  Loops of a few instructions with all loads in flight: the first pass over code costs 1.5
+// to 2 clocks a byte (24 pieces of a thread unrolled were 10 KiB of it: 131 K labels, 40 rows 26.8 us a call), and a loop that loaded 16
+// rows while it converted 16 others had a miss of the L2 in every round (25.1; an image 22.1, as it is 21.2).  What X holds in LDS behind
+// the batch are logits of nobody.
+__device__ __forceinline__ void fwd_request_x(const unsigned short* x, int rows, unsigned raw, int v, int lane) {
+  const int pieces = rows * (D * 2 / 16);
+#pragma unroll 1
+  for (int c0 = v * 64; c0 < pieces; c0 += FNT) {
+    const unsigned ldsoff = __builtin_amdgcn_readfirstlane(raw + (unsigned)(c0 * 16));
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(ldsoff), "v"(min(c0 + lane, pieces - 1) * 16), "s"(x) : "memory", "m0");
+  }
+}
+__device__ __forceinline__ void fwd_convert_x(int rows, float inv_scale_x, const unsigned char* raw, unsigned char* img, int tid) {
+  constexpr int PR = D * 2 / 16;
+#pragma unroll 1
+  for (int ch = tid; ch < rows * PR; ch += FNT) {
+    const uint4 r = *(const uint4*)(raw + ch * 16);
+    auto val = [&](unsigned bits) { return clamp448(__uint_as_float(bits) * inv_scale_x); };
+    auto pack = [&](unsigned a, unsigned b) {
+      const int lo = __builtin_amdgcn_cvt_pk_fp8_f32(val(a << 16), val(a & 0xFFFF0000u), 0, false);
+      return (unsigned)__builtin_amdgcn_cvt_pk_fp8_f32(val(b << 16), val(b & 0xFFFF0000u), lo, true);
+    };
+    *(uint2*)(img + ch / PR * WS + ch % PR * 8) = uint2{pack(r.x, r.y), pack(r.z, r.w)};
+  }
 }
 
 // z[nb]: logits of 16 labels (tile rows from `rows` on) and batch rows 32w + 16nb ..  All operands are requested before the
@@ -121,22 +152,26 @@ __device__ __forceinline__ void fwd_wait(bool full) {
 // staged logits of the tile before (two stages in turn) leave as 16 consecutive bytes of a batch row per lane.
 // HBM bound: 131 K labels, batch 40 (101 MB in, 10 MB out) 20.9 us = 5.3 TB/s; the same loads without anything else take 17.2.
 // Two workgroups of four wavefronts with three buffers and three barriers per tile took 23.2; a batch that is no multiple of
-// 16 also cost a padded copy of X and a copy of the logits (42 us the call, 25 now).
+// 16 also cost a padded copy of X and a copy of the logits (42 us the call, 25 without).
+// CONV: the workgroups convert X themselves (up to FWD_CONV rows; forward_converts has the line): the call 25.3 / 24.1 us.
 // HB = 2: 129 to 256 batch rows from one pass over the weights, every wavefront with 32 rows and both halves of a tile.
 // us a call, two slices of 128 rows / now: 256 rows, 8 K labels 22.3 / 13.6, 131 K 54.6 / 39.6, 400 K 190 / 117, 1 M 569 / 414 (1.3 GB in
 // and out: 3.1 TB/s);  129 rows, 131 K 48.0 / 32.9, 400 K 160 / 88, 1 M 438 / 288.
 // RUN: consecutive tiles that a workgroup takes in a round (a power of two); what is left of the tiles is taken singly.
-template <int HB, int RUN>
+template <int HB, int RUN, bool CONV>
 __global__ __launch_bounds__(FNT, 2) void fp8_forward_kernel(const ForwardParams p) {
-  constexpr int FBUF = FwdGeom<HB>::BUF, ZB = FwdGeom<HB>::ZB;
+  typedef FwdGeom<HB, CONV> Geo;
+  constexpr int FBUF = Geo::BUF, ZB = Geo::ZB;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
   const int tid = threadIdx.x, v = __builtin_amdgcn_readfirstlane(tid >> 6), w = HB == 1 ? v & 3 : v, half0 = HB == 1 ? v >> 2 : 0;
   const int lane = tid & 63, l16 = lane & 15, kg = lane >> 4, nblocks = (int)gridDim.x;
   const unsigned lds0 = (unsigned)(size_t)(lds_u8*)lds_raw;
   const bool active = 32 * w < p.batch;   // (wave-uniform) a wavefront without batch rows only helps to load and store
   intx8 xq[2][6];
-  if (active) fwd_load_x(p.xq, w, lane, xq);
-  __builtin_amdgcn_s_waitcnt(0);
+  if constexpr (!CONV) {
+    if (active) fwd_load_x(p.xq, w, lane, xq);
+    __builtin_amdgcn_s_waitcnt(0);
+  }
   const int mine = (int)blockIdx.x, first = p.tile_begin + mine;
   const int rounds = RUN > 1 ? (p.tile_end - p.tile_begin) / (nblocks * RUN) : 0, in_runs = rounds * RUN;
   int ahead = first;                      // next tile to be requested
@@ -189,7 +224,34 @@ __global__ __launch_bounds__(FNT, 2) void fp8_forward_kernel(const ForwardParams
         for (int e = 0; e < s && e < nvalid; e++) orow[e] = zrow[e];
     }
   };
-  for (int k = 0; k < FBUF - 1; k++) issue(k);
+  int k0 = 0;
+  if constexpr (CONV) {
+    const int raw = Geo::X - ((p.batch + 15) & ~15) * (D * 2);
+    fwd_request_x(p.x, p.batch, lds0 + (unsigned)raw, v, lane);
+    int n = 0;   // tiles on their way into the buffers in front of X
+#pragma unroll 1
+    for (; k0 < FBUF - 1 && (k0 + 1) * FB <= raw; k0++) {
+      n += ahead < p.tile_end ? 1 : 0;
+      issue(k0);
+    }
+    static_assert(FT * 64 / FNT == 4, "loads of a tile");
+    if (n == 3) asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
+    else if (n == 2) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+    else if (n == 1) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    fwd_convert_x(p.batch, p.inv_scale_x, lds_raw + raw, lds_raw + Geo::X, tid);
+    __syncthreads();
+    if (active) {
+#pragma unroll
+      for (int nb = 0; nb < 2; nb++)
+#pragma unroll
+        for (int ks = 0; ks < 6; ks++) xq[nb][ks] = lds_read32(lds_raw + Geo::X + (32 * w + 16 * nb + l16) * WS + ks * 128 + kg * 32);
+    }
+    __syncthreads();   // X's places are free
+  }
+#pragma unroll 1
+  for (; k0 < FBUF - 1; k0++) issue(k0);
   int buf = 0, par = 0, t = first;
   for (; t < p.tile_end; t += nblocks) {
     unsigned char* stage = lds_raw + FBUF * FB;
@@ -250,7 +312,7 @@ template <int WAVES> struct SelGeom {
 // The rows' counters lie a cache line apart: next to each other 57 K atomics (670 K labels, batch 128, k = 100) on four lines
 // took 16 us where they came together.
 constexpr int SEL_COUNT_STRIDE = 32;
-static_assert(2 * SelGeom<4>::LDS <= 160 * 1024 && SelGeom<8>::LDS <= 160 * 1024 && FwdGeom<1>::LDS <= 160 * 1024 && FwdGeom<2>::LDS <= 160 * 1024, "LDS budget");
+static_assert(2 * SelGeom<4>::LDS <= 160 * 1024 && SelGeom<8>::LDS <= 160 * 1024, "LDS budget");
 
 struct SelectParams {
   const unsigned char* chunk[MAX_CHUNKS];
