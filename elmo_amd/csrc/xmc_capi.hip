@@ -4,6 +4,7 @@
 #include "xmc_fp8_forward.hip"
 #include "xmc_fp8_quad.hip"
 #include "xmc_fp8_role.hip"
+#include "xmc_fp8_small.hip"
 #include "xmc_tiled.hip"
 #include "xmc_cluster_aux.hip"
 #include "xmc_topk.hip"
@@ -53,6 +54,7 @@ void fill_device_info(int dev) {
   // opt in to the full 160 KiB of LDS once per device
   role_plain_set_lds();
   role_heavy_set_lds();
+  small_set_lds();
   cluster_set_lds_bf16();
   cluster_set_lds_sim();
   cluster_set_lds_fp8();
@@ -241,6 +243,20 @@ bool small_batch_one_pass(int batch, long long tiles, int round_mode, int cus) {
   if (batch > 64 || round_mode == XMC_ROUND_SR_PHILOX) return false;
   return tiles >= (round_mode == XMC_ROUND_RTN ? (batch <= 32 ? 6 : 20) : (batch <= 32 ? 32 : 64)) * (long long)cus;
 }
+// Whether a true-FP8 step without weight decay, dropout or a compensated head takes the two launches of xmc_fp8_small.hip, a workgroup for
+// every 32 labels and one to a compute unit at most.  What they gain is a launch and the latencies of the quads' exchange; what they lose
+// grows with the labels, 48 KiB of grad_X sums per 16 batch rows and workgroup, and with Philox, whose words take a workgroup longer than
+// the four of a quad.  us a step, fused kernel / this one, at 1 K, 2 K, 4 K, 6 K, 8 K labels:
+//   16 rows  sr_fast 14.2/10.0 14.4/10.5 14.5/11.9 16.1/13.9 16.5/15.7   nearest 14.2/10.2 14.3/9.9 14.4/11.5 15.7/13.5 16.0/15.3
+//            Philox 17.0/14.3 17.2/15.3 17.5/17.3 21.9/19.4 22.4/21.2
+//   32 rows  sr_fast 15.9/10.3 15.9/12.1 16.1/15.4 17.8/17.7 18.0/20.4   nearest 15.6/10.3 15.8/11.6 15.8/15.0 17.4/17.3 17.5/20.5
+//            Philox 18.8/15.5 18.9/17.3 19.2/20.7 23.7/23.0 24.1/24.2
+// (Workgroups that take several tiles one after the other, and sum: 8 K, 16 rows 15.9, 16 K 20.3/19.9 with the fused kernel, and half a
+// microsecond more with one tile each.)
+bool small_step(int batch, int nnz, long long tiles, int round_mode, int grid) {
+  const long long most = batch <= 16 ? 256 : round_mode == XMC_ROUND_SR_PHILOX ? 64 : 160;
+  return batch <= SM_BATCH && nnz <= SM_POS && tiles <= (most < grid ? most : grid);
+}
 // Its places in the fused step's workspace: the grad_X sums from WS_PARTIAL on (32 rows: as many bytes as the fused kernel's; 64 rows:
 // twice that, over the exchange ring and the descriptors, which this form does not use, and up to 14 MiB beyond: only workspaces of
 // xmc_workspace_bytes_ex hold them), then the first key of every tile.
@@ -419,6 +435,39 @@ static int fused_step(void* const* chunk_ptrs, int num_chunks, int rows_per_chun
     return cluster_step(chunk_ptrs, num_chunks, rows_per_chunk, rows_per_chunk, W_E4M3, x_bf16, batch, labels_coo, nnz, lr, seeds, round_mode, 1, 1,
                         dp, grad_x_bf16, grad_x_f32, at, true, di.cus, di.failure_word, stream);
   }
+  const int qgrid = grid / 32 * 32;   // whole quads on every XCD
+  if (qgrid < 32) return XMC_ERR_DEVICE;
+  const int small_per_chunk = (rows_per_chunk + SM_ROWS - 1) / SM_ROWS;
+  if (kahan_type == 0 && weight_decay == 0.f && dropout_p == 0.f &&
+      small_step(batch, nnz, (long long)num_chunks * small_per_chunk, round_mode, qgrid)) {
+    SmallParams p;
+    for (int c = 0; c < MAX_CHUNKS; c++) {
+      p.chunk[c] = c < num_chunks ? (unsigned char*)chunk_ptrs[c] : nullptr;
+      p.seed[c] = (c < num_chunks && seeds) ? (round_mode == XMC_ROUND_SR_FAST ? fast_seed(seeds[c]) : seeds[c]) : 0u;
+    }
+    p.rows_per_chunk = rows_per_chunk;
+    p.tiles_per_chunk = small_per_chunk;
+    p.num_tiles = num_chunks * small_per_chunk;
+    p.x = (const unsigned short*)x_bf16;
+    p.coo = (const int2*)labels_coo;
+    p.nnz = nnz;
+    p.batch = batch;
+    p.inv_scale_x = 1.0f / scale_x;
+    p.zscale = scale_w * scale_x;
+    p.lr_eff = lr / scale_w;
+    p.partial = (floatx4*)(ws + WS_PARTIAL);
+    p.flags = (int*)(ws + WS_FLAGS);
+    static_assert((size_t)MAX_WG * SM_BATCH * D * 4 <= WS_EXCH - WS_PARTIAL, "grad_X sums of a workgroup for every compute unit");
+    if (g_prof_start) (void)hipEventRecord(g_prof_start, stream);
+    // (as many workgroups as the fused kernel has: all of them record their XCD)
+    small_variant(round_mode, batch)<<<qgrid, SM_NT, SM_LDS, stream>>>(p);
+    if (g_prof_stop) (void)hipEventRecord(g_prof_stop, stream);
+    g_prof_start = g_prof_stop = nullptr;
+    const int blocks = batch / 16 * 48;
+    fp8_small_reduce_kernel<<<blocks, SM_RW * 64, 0, stream>>>(p.partial, p.num_tiles, blocks, scale_w, grad_x_f32, (unsigned short*)grad_x_bf16,
+                                                               p.flags, di.failure_word);
+    return launch_status();
+  }
   {
     QuadParams p;
     for (int c = 0; c < MAX_CHUNKS; c++) {
@@ -442,8 +491,6 @@ static int fused_step(void* const* chunk_ptrs, int num_chunks, int rows_per_chun
     p.lr_eff = lr / scale_w;
     p.wd_eff = weight_decay * scale_w;   // T = c - (lr / s) (A + wd s c) for codes c = W / s
     p.batch = batch;
-    int qgrid = grid / 32 * 32;   // whole quads on every XCD
-    if (qgrid < 32) return XMC_ERR_DEVICE;
     p.nquads = qgrid >> 2;
     // with a compensated head the tiles that hold its rows run first, as a launch of their own
     const int head_tiles = (num_head + TL - 1) / TL, rest_tiles = num_tiles - head_tiles;
