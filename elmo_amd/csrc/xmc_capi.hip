@@ -257,6 +257,21 @@ bool small_step(int batch, int nnz, long long tiles, int round_mode, int grid) {
   const long long most = batch <= 16 ? 256 : round_mode == XMC_ROUND_SR_PHILOX ? 64 : 160;
   return batch <= SM_BATCH && nnz <= SM_POS && tiles <= (most < grid ? most : grid);
 }
+// Quads of the fused kernel for a step's tiles, of `most` that the device has.  A quad leaves the sum of grad_X of all its tiles, 384 KiB at
+// 128 rows, and one without tiles leaves as much: written, and read again behind the kernel.  With few tiles those sums cost more than a
+// second tile for every quad (not with Philox and up to 96 rows, whose tiles are long and whose sums are short, and not where a quarter of
+// the device would do).  Whole numbers of quads on each XCD.  us a step, all quads / now, at 300, 1 K, 2 K, 4 K, 5 K labels:
+//   sr_fast  48 rows 16.9/13.7 18.3/14.3 18.5/15.9 18.7/17.8 20.1/18.8     128 rows 26.0/16.4 27.9/19.5 28.3/21.6 28.6/25.5 29.1/27.4
+//   Philox   64 rows 21.0/16.6 23.3/17.7 23.1/19.8 23.3/23.3 27.6/25.9     128 rows 26.8/19.2 30.1/21.6 31.5/25.7 32.1/30.9 34.4/32.6
+// (Two tiles a quad instead of one: 2 K labels, 48 rows 16.0/16.4, Philox 128 rows 25.0/26.3, but 96 rows 19.4/18.7, 128 rows 22.3/20.9; 4 K, Philox,
+// 64 rows 23.3/24.8.  Three on 48 quads instead of 64, 9 K: 48 rows 22.2/21.2, but 128 rows 30.3/30.6: above two as many quads as there are.)
+int fused_quads(int tiles, int batch, int round_mode, int most) {
+  if (tiles > 2 * most) return most;
+  const bool philox = round_mode == XMC_ROUND_SR_PHILOX;
+  const bool single = tiles <= most / 2 ? batch <= 48 || philox : tiles <= most && philox && batch <= 96;
+  const int q = ((single ? tiles : (tiles + 1) / 2) + 7) / 8 * 8;
+  return q < most ? q : most;
+}
 // Its places in the fused step's workspace: the grad_X sums from WS_PARTIAL on (32 rows: as many bytes as the fused kernel's; 64 rows:
 // twice that, over the exchange ring and the descriptors, which this form does not use, and up to 14 MiB beyond: only workspaces of
 // xmc_workspace_bytes_ex hold them), then the first key of every tile.
@@ -491,7 +506,9 @@ static int fused_step(void* const* chunk_ptrs, int num_chunks, int rows_per_chun
     p.lr_eff = lr / scale_w;
     p.wd_eff = weight_decay * scale_w;   // T = c - (lr / s) (A + wd s c) for codes c = W / s
     p.batch = batch;
-    p.nquads = qgrid >> 2;
+    // (the two launches of a step with a compensated head continue one another's sums)
+    p.nquads = kahan_type == 0 ? fused_quads(num_tiles, batch, round_mode, qgrid >> 2) : qgrid >> 2;
+    const int step_grid = 4 * p.nquads;
     // with a compensated head the tiles that hold its rows run first, as a launch of their own
     const int head_tiles = (num_head + TL - 1) / TL, rest_tiles = num_tiles - head_tiles;
     p.kahan = (unsigned char*)kahan;
@@ -514,16 +531,16 @@ static int fused_step(void* const* chunk_ptrs, int num_chunks, int rows_per_chun
     p.desc = desc + 2 * (size_t)p.nquads * p.kmax_head;
     if (head_tiles > 0) { p.cnt_base = QF_CNT2; p.acc_init = 1; }
     // the variants with the Philox recipe or a compensated head live in the library's second translation unit
-    if (kahan_type != 0) role_heavy_launch(round_mode, false, kahan_type, role_blocks(batch, false, kahan_type), qgrid, stream, ph);
+    if (kahan_type != 0) role_heavy_launch(round_mode, false, kahan_type, role_blocks(batch, false, kahan_type), step_grid, stream, ph);
     if (rest_tiles > 0) {
       const bool wd = weight_decay != 0.f;
       const int blocks = role_blocks(batch, wd, 0);
-      if (round_mode == XMC_ROUND_SR_PHILOX) role_heavy_launch(round_mode, wd, 0, blocks, qgrid, stream, p);
-      else role_plain_launch(round_mode, wd, blocks, qgrid, stream, p);
+      if (round_mode == XMC_ROUND_SR_PHILOX) role_heavy_launch(round_mode, wd, 0, blocks, step_grid, stream, p);
+      else role_plain_launch(round_mode, wd, blocks, step_grid, stream, p);
     }
     if (g_prof_stop) (void)hipEventRecord(g_prof_stop, stream);
     g_prof_start = g_prof_stop = nullptr;
-    reduce_gx_role_kernel<<<(batch + 15) / 16 * 48, 256, 0, stream>>>((const floatx4*)(ws + WS_PARTIAL), qgrid, scale_w, grad_x_f32,
+    reduce_gx_role_kernel<<<(batch + 15) / 16 * 48, 256, 0, stream>>>((const floatx4*)(ws + WS_PARTIAL), step_grid, scale_w, grad_x_f32,
                                                  (unsigned short*)grad_x_bf16, batch, (int*)(ws + WS_FLAGS), di.failure_word, dp);
   }
   return launch_status();

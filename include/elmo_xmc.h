@@ -335,7 +335,8 @@ int xmc_pass_on_error(const int32_t* error_word, int32_t* into_error, int32_t* i
 
 /* Diagnostics of the placement assumption of the fused kernel (no counterpart in the reference).  The kernel builds
  * quads out of workgroups g with equal g % 8 and expects them on one XCD; every workgroup records the XCC id it really
- * ran on.  xmc_step_workgroups: number of workgroups the fused kernel is launched with on the current device.
+ * ran on.  xmc_step_workgroups: the most workgroups the fused kernel is launched with on the current device (a step of few
+ * tiles takes fewer; the ids of the others are 0).
  * xmc_step_xcc_ids: copies the ids of the first `count` workgroups of the last step to host memory (synchronises).
  * xmc_quad_placement_check: host-only; number of quads whose four members recorded different ids (0 = fine) - the
  * comparison the device makes at the end of every step before it raises bit 1 of the error word. */
