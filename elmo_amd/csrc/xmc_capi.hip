@@ -272,6 +272,15 @@ int fused_quads(int tiles, int batch, int round_mode, int most) {
   const int q = ((single ? tiles : (tiles + 1) / 2) + 7) / 8 * 8;
   return q < most ? q : most;
 }
+// The same for the launch of a compensated head, whose tiles take twice as long and whose sums are read and written once more, by the launch
+// of the other tiles: a quad for a tile, from 65 tiles on as few as two each need.  us a step with a fifth of the labels compensated, bf16 terms,
+// sr_fast, all quads in both launches / now, at 8 K, 11 K, 16 K labels: 128 rows 45.9/40.7 47.9/44.3 50.2/49.3, 32 rows 28.5/27.4 29.8/29.2 31.0/31.0;
+// e5m2, nearest, 128 rows 45.0/39.8 47.1/43.4 49.4/48.2, 22 K 52.3/51.3, 30 K 55.8/54.8.
+int head_quads(int tiles, int most) {
+  if (tiles > 2 * most) return most;
+  const int q = ((tiles <= most ? tiles : (tiles + 1) / 2) + 7) / 8 * 8;
+  return q < most ? q : most;
+}
 // Its places in the fused step's workspace: the grad_X sums from WS_PARTIAL on (32 rows: as many bytes as the fused kernel's; 64 rows:
 // twice that, over the exchange ring and the descriptors, which this form does not use, and up to 14 MiB beyond: only workspaces of
 // xmc_workspace_bytes_ex hold them), then the first key of every tile.
@@ -506,18 +515,19 @@ static int fused_step(void* const* chunk_ptrs, int num_chunks, int rows_per_chun
     p.lr_eff = lr / scale_w;
     p.wd_eff = weight_decay * scale_w;   // T = c - (lr / s) (A + wd s c) for codes c = W / s
     p.batch = batch;
-    // (the two launches of a step with a compensated head continue one another's sums)
-    p.nquads = kahan_type == 0 ? fused_quads(num_tiles, batch, round_mode, qgrid >> 2) : qgrid >> 2;
-    const int step_grid = 4 * p.nquads;
     // with a compensated head the tiles that hold its rows run first, as a launch of their own
     const int head_tiles = (num_head + TL - 1) / TL, rest_tiles = num_tiles - head_tiles;
+    // (their quads' sums are continued by the quads of the other launch: at least as many)
+    p.nquads_head = head_quads(head_tiles, qgrid >> 2);
+    const int rest_quads = fused_quads(rest_tiles, batch, round_mode, qgrid >> 2);
+    p.nquads = rest_quads > p.nquads_head ? rest_quads : p.nquads_head;
     p.kahan = (unsigned char*)kahan;
     p.num_head = num_head;
     p.head_tiles = head_tiles;
-    p.kmax_head = (head_tiles + p.nquads - 1) / p.nquads;
+    p.kmax_head = head_tiles > 0 ? (head_tiles + p.nquads_head - 1) / p.nquads_head : 0;
     p.kmax = (rest_tiles + p.nquads - 1) / p.nquads;
     p.cnt_base = 0;
-    p.acc_init = 0;
+    p.acc_quads = 0;
     p.spin_limit = g_spin_limit.load(std::memory_order_relaxed);
     const int desc_blocks = (num_tiles + PREP_NT - 1) / PREP_NT;
     quad_prep_kernel<<<desc_blocks + (BP * (D / 4) + PREP_NT - 1) / PREP_NT, PREP_NT, (size_t)nnz * 4, stream>>>(
@@ -528,19 +538,19 @@ static int fused_step(void* const* chunk_ptrs, int num_chunks, int rows_per_chun
     ph.run_tiles = head_tiles;
     ph.kmax = p.kmax_head;
     p.run_tiles = rest_tiles;
-    p.desc = desc + 2 * (size_t)p.nquads * p.kmax_head;
-    if (head_tiles > 0) { p.cnt_base = QF_CNT2; p.acc_init = 1; }
+    p.desc = desc + 2 * (size_t)p.nquads_head * p.kmax_head;
+    if (head_tiles > 0) { p.cnt_base = QF_CNT2; p.acc_quads = p.nquads_head; }
     // the variants with the Philox recipe or a compensated head live in the library's second translation unit
-    if (kahan_type != 0) role_heavy_launch(round_mode, false, kahan_type, role_blocks(batch, false, kahan_type), step_grid, stream, ph);
+    if (kahan_type != 0) role_heavy_launch(round_mode, false, kahan_type, role_blocks(batch, false, kahan_type), 4 * p.nquads_head, stream, ph);
     if (rest_tiles > 0) {
       const bool wd = weight_decay != 0.f;
       const int blocks = role_blocks(batch, wd, 0);
-      if (round_mode == XMC_ROUND_SR_PHILOX) role_heavy_launch(round_mode, wd, 0, blocks, step_grid, stream, p);
-      else role_plain_launch(round_mode, wd, blocks, step_grid, stream, p);
+      if (round_mode == XMC_ROUND_SR_PHILOX) role_heavy_launch(round_mode, wd, 0, blocks, 4 * p.nquads, stream, p);
+      else role_plain_launch(round_mode, wd, blocks, 4 * p.nquads, stream, p);
     }
     if (g_prof_stop) (void)hipEventRecord(g_prof_stop, stream);
     g_prof_start = g_prof_stop = nullptr;
-    reduce_gx_role_kernel<<<(batch + 15) / 16 * 48, 256, 0, stream>>>((const floatx4*)(ws + WS_PARTIAL), step_grid, scale_w, grad_x_f32,
+    reduce_gx_role_kernel<<<(batch + 15) / 16 * 48, 256, 0, stream>>>((const floatx4*)(ws + WS_PARTIAL), 4 * p.nquads, scale_w, grad_x_f32,
                                                  (unsigned short*)grad_x_bf16, batch, (int*)(ws + WS_FLAGS), di.failure_word, dp);
   }
   return launch_status();

@@ -40,7 +40,7 @@ struct QuadParams {
   const unsigned* keys;               // positives grouped by tile: label*256 + batch_row
   const uint4* desc;                  // [nquads][kmax][2] tile descriptors written by quad_desc_prep_kernel: the tiles of
                                       // one quad are consecutive entries, in the order the quad walks them
-  int nquads;                         // quads of the step kernel's launch (grid / 4)
+  int nquads, nquads_head;            // quads of the step kernel's launch (grid / 4), and of the head's
   int kmax;                           // descriptor entries per quad = ceil(run_tiles / nquads)
   floatx4* partial;                   // [gridDim.x][24][256] per-workgroup grad_X partial sums
   unsigned char* exch;                // [nquads][QSLOTS][QG_BYTES] G exchange ring
@@ -55,7 +55,7 @@ struct QuadParams {
   unsigned char* kahan;               // [num_head, 768] bf16 or e5m2, or null
   int num_head, head_tiles, kmax_head;
   int cnt_base;                       // first of this launch's tiles-published counters in flags
-  int acc_init;                       // the grad_X partials continue from what the launch before left in `partial`
+  int acc_quads;                      // the grad_X partials of this many quads continue from what the launch before left in `partial`
   int spin_limit;                     // polls of a partner's counter before a workgroup gives up (QSPIN_LIMIT; a test aid
                                       // lowers it to exercise the give-up path)
 };
@@ -262,8 +262,8 @@ __global__ __launch_bounds__(PREP_NT) void quad_prep_kernel(const QuadParams p, 
     // counts from the head's end (the reference updates those rows through sliced tensors, so the offsets of its random
     // numbers restart there: chunked_head_kahan_fp8xmc_clf.py:130-131).
     const bool behind = t >= p.head_tiles;
-    const int tl = behind ? t - p.head_tiles : t, km = behind ? p.kmax : p.kmax_head;
-    const int slot = (behind ? p.nquads * p.kmax_head : 0) + (tl % p.nquads) * km + tl / p.nquads;
+    const int tl = behind ? t - p.head_tiles : t, km = behind ? p.kmax : p.kmax_head, nq = behind ? p.nquads : p.nquads_head;
+    const int slot = (behind ? p.nquads_head * p.kmax_head : 0) + (tl % nq) * km + tl / nq;
     const int row_rec = row0 - (behind && c == 0 ? p.num_head : 0);
     desc[2 * slot] = uint4{(unsigned)base, (unsigned)(base >> 32), (unsigned)min(TL, p.rows_per_chunk - row0), p.seed[c]};
     desc[2 * slot + 1] = uint4{(unsigned)p0, (unsigned)p1, (unsigned)row_rec, (unsigned)(c * p.rows_per_chunk + row0)};

@@ -664,7 +664,7 @@ __global__ __launch_bounds__(QNT, 1) void fp8_step_role_kernel(const QuadParams 
     for (int mb = 0; mb < 2 * NK; mb++)
 #pragma unroll
       for (int nn = 0; nn < 3; nn++)
-        acc2[mb][nn] = p.acc_init ? prev[(mb * 3 + nn) * 256 + s * 64 + lane] : floatx4{0.f, 0.f, 0.f, 0.f};
+        acc2[mb][nn] = quad < p.acc_quads ? prev[(mb * 3 + nn) * 256 + s * 64 + lane] : floatx4{0.f, 0.f, 0.f, 0.f};
   }
 
   // per-lane parts of the LDS addresses
