@@ -243,6 +243,26 @@ bool small_batch_one_pass(int batch, long long tiles, int round_mode, int cus) {
   if (batch > 64 || round_mode == XMC_ROUND_SR_PHILOX) return false;
   return tiles >= (round_mode == XMC_ROUND_RTN ? (batch <= 32 ? 6 : 20) : (batch <= 32 ? 32 : 64)) * (long long)cus;
 }
+// Clusters of the one-pass step for a step's tiles, of `most` that the device has.  Every workgroup leaves a sum of grad_X of 192 KiB (96 up to
+// 32 rows), written and read again behind the kernel: with fewer tiles than clusters, but not by much, half as many clusters with two tiles
+// each are faster, unless a second tile takes longer than the sums (Philox, FP8 logits in clusters of one).  us a step, a cluster for every
+// tile / for two, at 2 K, 3 K, 4 K, 5 K, 6.5 K, 8 K labels:
+//   32 rows   bf16, nearest 18.5/20.2 20.2/20.6 21.4/21.7 23.7/22.8 26.8/23.7 28.3/24.2   sr_fast 22.4/23.1 (4 K) 24.6/24.2 27.6/25.4 28.8/25.8
+//             e4m3 with bf16 products, nearest 17.4/18.5 19.5/19.4 21.0/20.1 22.4/21.0 24.3/22.1 27.2/23.1   Philox, either: 3 to 8 us slower
+//   64 rows   bf16, nearest 22.4/23.4 26.4/25.1 29.3/26.1 31.6/28.0 32.8/30.6 32.7/31.2   sr_fast 22.9/25.0 27.2/26.8 30.4/27.5 31.7/29.4 32.8/32.4 33.1/33.2
+//             e4m3 with bf16 products, nearest 22.2/22.8 25.4/24.4 28.0/25.4 31.7/27.3 33.3/29.0 34.6/31.0
+//   128 rows  bf16, nearest 29.8/27.6 33.2/29.8 35.7/32.2   sr_fast 29.4/28.7 33.3/30.4 35.6/32.9   Philox 32.2/34.4 37.3/36.5 38.8/37.7
+//             e4m3 with bf16 products, nearest 29.6/27.0 33.3/29.4 35.5/31.6   FP8 logits, sr_fast 25.6/26.7 and 33.1/31.0 (5 K)
+//   256 rows  bf16, 1 K, 1.6 K, 2 K nearest 30.9/29.0 33.4/31.5 35.3/33.3   Philox 31.8/32.1 34.7/33.9 36.8/35.6
+//             FP8 logits, 2 K, 4 K  nearest 31.2/29.6 36.1/34.5   sr_fast 31.2/30.4 36.4/35.0   Philox 33.8/35.6 39.2/40.0
+int one_pass_clusters(int tiles, int most, int c, int nbk, bool fp8, int round_mode) {
+  if (tiles > most) return most;
+  const bool philox = round_mode == XMC_ROUND_SR_PHILOX;
+  bool two = false;   // tiles for a cluster
+  if (c == 1) two = !philox && !fp8 && 16 * tiles > (nbk == 2 ? 9 : 5) * most;
+  else if (c == 2 || c == 4) two = philox ? !fp8 && 4 * tiles >= 3 * most : 8 * tiles >= (c == 2 ? 3 : 4) * most;
+  return two ? (tiles + 1) / 2 : tiles;
+}
 // Whether a true-FP8 step without weight decay, dropout or a compensated head takes the two launches of xmc_fp8_small.hip, a workgroup for
 // every 32 labels and one to a compute unit at most.  What they gain is a launch and the latencies of the quads' exchange; what they lose
 // grows with the labels, 48 KiB of grad_X sums per 16 batch rows and workgroup, and with Philox, whose words take a workgroup longer than
@@ -382,7 +402,7 @@ static int cluster_step(void* const* chunk_ptrs, int num_chunks, int rows_per_ch
     p.tpc64 = tpc64;
     p.ntiles = (nch - 1) * p.tpc + p.tpc_last;
     const int most = (cus < CLU_MAXWG ? cus : CLU_MAXWG) / 8 / c * 8;   // whole clusters on every XCD
-    p.nclusters = p.ntiles < most ? p.ntiles : most;
+    p.nclusters = one_pass_clusters(p.ntiles, most, c, nbk, fp8, round_mode);
     p.label0_seg = 0u;
     p.label0 = (unsigned)c0 * (unsigned)rows_per_chunk;
     p.xq = at.xq;

@@ -57,3 +57,42 @@ def test_compensated_head(gpu, nc, rows, head, batch):
         assert H.e4m3_ulp_distance(a, b).max() <= 1 and np.mean(a == b) > 0.998
     assert np.mean(terms.float().cpu().numpy() == ref_k) > 0.99      # (a term turns over with its weight)
     assert np.abs(gf.cpu().numpy() - ref_gx).max() <= 1e-3 * np.abs(ref_gx).max()
+
+
+@pytest.mark.parametrize("mode", ["rtn", "sr_philox"])
+@pytest.mark.parametrize("weights", ["bf16", "e4m3", "fp8"])
+@pytest.mark.parametrize("batch,labels", [
+    (20, 4600), (20, 4630), (20, 8192), (64, 2560), (64, 2570), (64, 8192),      # clusters of one
+    (100, 1504), (100, 1530), (100, 3072), (100, 4096), (100, 4128),             # of two
+    (200, 990), (200, 1024), (200, 1536), (200, 2048), (200, 4096)])             # of four
+@pytest.mark.parametrize("nc", [1, 3])
+def test_one_pass_step_with_half_the_clusters(gpu, nc, batch, labels, weights, mode):
+    """Either side of the lines from which on a cluster takes two tiles, against the same layer with chunks that go on in rows of zeros, whose
+    tiles are more than the clusters there are.  A row's update depends on no other row, so the weights agree to the bit.  Rows of zeros add
+    nothing to grad_X: the same fp32 sum in another grouping (2^-16 of its largest value); with bf16 weights the sum of a chunk is
+    rounded to bf16 by itself, where a neighbour may come out: 2^-8 of it, and the largest of three sums that partly cancel is taken to
+    be at most four times the largest of their total."""
+    import torch
+    from elmo_amd import ops
+    rows = labels // nc // 16 * 16
+    more = 9600 // nc // 16 * 16
+    g = torch.Generator(device=gpu).manual_seed(batch + labels)
+    dtype = torch.bfloat16 if weights == "bf16" else torch.float8_e4m3fn
+    chunks = [torch.randn(rows, 768, generator=g, device=gpu).mul_(0.05).to(dtype) for _ in range(nc)]
+    others = [torch.cat([c.float(), torch.zeros(more - rows, 768, device=gpu)]).to(dtype) for c in chunks]
+    x = torch.randn(batch, 768, generator=g, device=gpu).to(torch.bfloat16)
+    pos = torch.stack([torch.arange(5 * batch, device=gpu) % batch, torch.randint(0, nc * rows, (5 * batch,), generator=g, device=gpu)], 1).to(torch.int32)
+    pos_others = torch.stack([pos[:, 0], pos[:, 1] // rows * more + pos[:, 1] % rows], 1).contiguous()
+    kind, fp8 = "bf16" if weights == "bf16" else "e4m3", weights == "fp8"
+    out = []
+    for w, n, labs in ((chunks, rows, pos), (others, more, pos_others)):
+        ws = ops.alloc_tiled_workspace(nc, n, gpu, batch)
+        off = ops.tiled_error_offset()
+        ws[off + 8:].fill_(0x7F)
+        out.append(ops.tiled_step(w, n, kind, x, labs, 0.05, seeds=[3 + c for c in range(nc)], round_mode=mode, workspace=ws, want_f32=True,
+                                  quantize_x=fp8, saturate=fp8)[1])
+        assert int(ws[off:off + 4].view(torch.int32).item()) == 0
+    for a, b in zip(chunks, others):
+        assert torch.equal(a.view(torch.uint8), b[:rows].view(torch.uint8))
+    tol = (2 ** -16 if weights != "bf16" else 4 * nc * 2 ** -8) * out[1].abs().max().item()
+    assert (out[0] - out[1]).abs().max().item() <= tol
