@@ -177,6 +177,16 @@ void prep_x(const void* x_bf16, int batch, float scale_x, unsigned char* xq, hip
   prep_x_kernel<<<n / 256, 256, 0, stream>>>((const unsigned short*)x_bf16, batch, n, 1.0f / scale_x, xq);
 }
 
+// the inverse of s modulo n, for s coprime to n
+int tile_stride_inverse(int s, int n) {
+  long long r0 = n, r1 = s % n, t0 = 0, t1 = 1;
+  while (r1 != 0) {
+    const long long q = r0 / r1, r = r0 - q * r1, t = t0 - q * t1;
+    r0 = r1; r1 = r; t0 = t1; t1 = t;
+  }
+  return (int)(((t0 % n) + n) % n);
+}
+
 // Whether the workgroups of the logits kernel convert X themselves instead of reading an image that a launch in front has written.
 // The launch is 3 us of the GPU, and what bounds small label spaces is the host's 4 us for it; the conversion takes a workgroup longer
 // the more rows it has, without loads of tiles on their way from 49 rows on.  us a call, image / conversion, by rows:
@@ -386,7 +396,6 @@ static int cluster_step(void* const* chunk_ptrs, int num_chunks, int rows_per_ch
     const ClusterPrep pp = {labels_coo, nnz, batch, c0 * rows_per_chunk, nch * rows_per_chunk, pairs, rows_per_chunk, tpc64, nch * tpc64,
                             ptr_blocks, at.keys, at.tile_ptr, at.tp_stride, (const unsigned short*)x_bf16, bp, bf16 ? 0 : fp8 ? 2 : 1,
                             at.xq, at.xt, at.flags, c0 == 0 ? at.err : nullptr};   // (a failure in one segment stays visible behind the others)
-    cluster_prep_kernel<<<ptr_blocks * pairs + prep_blocks, PREP_NT, (size_t)nnz * 4, stream>>>(pp, dp);
     ClusterParams p;
     for (int k = 0; k < MAX_CHUNKS; k++) {
       p.chunk[k] = k < nch ? (unsigned char*)chunk_ptrs[c0 + k] : nullptr;
@@ -422,6 +431,19 @@ static int cluster_step(void* const* chunk_ptrs, int num_chunks, int rows_per_ch
     p.saturate = saturate;
     p.spin_limit = g_spin_limit.load(std::memory_order_relaxed);
     p.loads_behind = clu_loads_behind((long long)p.ntiles * tile_rows * (D * 2));
+    // Clusters of one with few positives prepare themselves (the products of a tile's number and an inverse are taken in 32 bits).  us a
+    // step, prepared by a launch in front / by themselves: 32 rows, bf16, nearest 2 K labels 18.4/15.7, 8 K 24.4/21.8, 131 K 73.0/70.2, 500 K 332/330,
+    // Philox, 2 K 24.2/21.4, 131 K 160.2/157.1; e4m3 with bf16 products, nearest, 2 K 17.8/15.2, 131 K 56.9/54.4; 64 rows, bf16, nearest, 2 K 22.2/20.6,
+    // 131 K 84.9/83.1, e4m3, Philox, 8 K 37.1/36.0, 500 K 580/580.
+    p.self = c == 1 && !fp8 && dp.p == 0.f && seg_chunks == num_chunks && nnz <= CLU_SELF_POS && p.tpc < 65536 &&
+             p.ntiles / p.nclusters < CLU_SELF_TILES;
+    p.nnz = nnz;
+    p.batch = batch;
+    p.perm_inv = tile_stride_inverse(p.perm, p.tpc);
+    p.perm_inv_last = tile_stride_inverse(p.perm_last, p.tpc_last);
+    p.coo = (const int2*)labels_coo;
+    p.x = (const unsigned char*)x_bf16;
+    if (!p.self) cluster_prep_kernel<<<ptr_blocks * pairs + prep_blocks, PREP_NT, (size_t)nnz * 4, stream>>>(pp, dp);
     if (profiled && g_prof_start) (void)hipEventRecord(g_prof_start, stream);
     var.fn<<<(p.nclusters + 7) / 8 * 8 * c, CLU_NT, var.lds, stream>>>(p);
     if (profiled) {

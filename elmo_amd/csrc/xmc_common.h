@@ -159,6 +159,16 @@ __device__ __forceinline__ float dropout_backward(float g, unsigned off, const D
   return dropout_keep(off, dp) ? g / dp.keep_scale : 0.f;
 }
 
+// The key of a positive: label*256 + (batch row - row0) for the batch rows row0..row0+255 that lie below `batch`;
+// 0xFFFFFFFF for every other entry and for labels outside the label space.  Labels are taken relative to label_base, and
+// those outside [label_base, label_base + label_count) are dropped: a label space of 2^24 labels and more is taken in
+// segments of whole chunks (a key keeps 24 bits for the label).
+__device__ __forceinline__ unsigned positive_key(int2 e, int batch, int row0, int label_base, int label_count) {
+  const int r = e.x - row0;
+  const long long lab = (long long)e.y - label_base;
+  return (r >= 0 && r < 256 && r + row0 < batch && e.y >= 0 && lab >= 0 && lab < label_count && lab < (1 << 24) - 1) ? (((unsigned)lab << 8) | (unsigned)r) : 0xFFFFFFFFu;
+}
+
 // Which of a wavefront's logits are positives.  The wavefront holds the logits of NLAB labels from label0 on and NROW batch rows from
 // row0 on (row0 as the keys count it), one of the two 16, as matrix results: lane l has labels 4 (l / 16).. + 3 of every sixteen and batch
 // row l % 16 of every sixteen; with ROWS4 label l % 16 and rows 4 (l / 16).. + 3.  Bit 4 n + e of a lane's result: its e-th label (row)

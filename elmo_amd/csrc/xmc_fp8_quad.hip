@@ -128,16 +128,6 @@ __device__ __forceinline__ QTile q_desc_full(q_cdesc* desc, int t) {
 }
 
 #ifndef XMC_HEAVY_TU   // the kernels below are compiled once, in the library's main translation unit
-// The key of a positive: label*256 + (batch row - row0) for the batch rows row0..row0+255 that lie below `batch`;
-// 0xFFFFFFFF for every other entry and for labels outside the label space.  Labels are taken relative to label_base, and
-// those outside [label_base, label_base + label_count) are dropped: a label space of 2^24 labels and more is taken in
-// segments of whole chunks (a key keeps 24 bits for the label).
-__device__ __forceinline__ unsigned positive_key(int2 e, int batch, int row0, int label_base, int label_count) {
-  const int r = e.x - row0;
-  const long long lab = (long long)e.y - label_base;
-  return (r >= 0 && r < 256 && r + row0 < batch && e.y >= 0 && lab >= 0 && lab < label_count && lab < (1 << 24) - 1) ? (((unsigned)lab << 8) | (unsigned)r) : 0xFFFFFFFFu;
-}
-
 // The positives of PREP_NT consecutive tiles, grouped by tile (the step kernels take a tile's in any order, repeated or not): keys
 // p0 .. p1-1 are those of tile t0 + tid.  The block reads all positives, counts those in front of its tiles and those in each of them,
 // and puts the latter behind one another.  Bound by latency: two passes over the positives, the second in LDS.  Until now they were
