@@ -257,6 +257,7 @@ bool small_batch_one_pass(int batch, long long tiles, int round_mode, int cus) {
 // 32 rows), written and read again behind the kernel: with fewer tiles than clusters, but not by much, half as many clusters with two tiles
 // each are faster, unless a second tile takes longer than the sums (Philox, FP8 logits in clusters of one).  us a step, a cluster for every
 // tile / for two, at 2 K, 3 K, 4 K, 5 K, 6.5 K, 8 K labels:
+//   (up to 64 rows with a launch in front that prepares X and the positives; without it both are 2 to 3 us less)
 //   32 rows   bf16, nearest 18.5/20.2 20.2/20.6 21.4/21.7 23.7/22.8 26.8/23.7 28.3/24.2   sr_fast 22.4/23.1 (4 K) 24.6/24.2 27.6/25.4 28.8/25.8
 //             e4m3 with bf16 products, nearest 17.4/18.5 19.5/19.4 21.0/20.1 22.4/21.0 24.3/22.1 27.2/23.1   Philox, either: 3 to 8 us slower
 //   64 rows   bf16, nearest 22.4/23.4 26.4/25.1 29.3/26.1 31.6/28.0 32.8/30.6 32.7/31.2   sr_fast 22.9/25.0 27.2/26.8 30.4/27.5 31.7/29.4 32.8/32.4 33.1/33.2

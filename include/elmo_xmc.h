@@ -135,7 +135,7 @@ int xmc_fp8_forward_wide(void* const* chunk_ptrs, int num_chunks, int rows_per_c
 
 /* xmc_fp8_forward without a workspace argument.  It has no counterpart in the reference: it is for callers that cannot
  * allocate device memory for a workspace (code under HIP graph capture, serving loops and harnesses that forbid
- * hipMalloc).  The operand image of X that xmc_fp8_forward keeps in the caller's workspace lives in a static device array
+ * hipMalloc).  The operand image of X that xmc_fp8_forward keeps in the caller's workspace (from 49 rows on) lives in a static device array
  * of the library instead (98,304 bytes per GPU, held until the process ends), so the limits are those of the array:
  * features == 768 and batch <= 128 (a multiple of 16); anything larger returns XMC_ERR_SHAPE.  The call allocates and
  * frees nothing.  Every call on a GPU uses that GPU's one array: calls that overlap on the same GPU (two streams, two
