@@ -144,6 +144,7 @@ __global__ __launch_bounds__(CLU_RW * 64) void cluster_reduce_kernel(const Clust
   __shared__ floatx4 sh[CLU_RW][64];
   const int pslot = r.nbk * 6 * 8 * 64;
   const int pos = blockIdx.x * 64 + lane, m = pos / pslot, q = pos - m * pslot;
+  if (16 * (m * r.nbk + (q >> 9) / 6) >= r.batch) return;   // (the same for the block's 64 positions: rows that are not there)
   auto sum_slots = [&](int s0, int s1) {
     floatx4 s = {0.f, 0.f, 0.f, 0.f};
     int k = s0;
