@@ -17,6 +17,8 @@ def compare(gpu, nc, rows, batch, mode, dropout=0.0):
     n = 9 * batch
     labels = torch.stack([torch.arange(n, device=gpu) % batch, torch.randint(0, nc * rows, (n,), generator=g, device=gpu)], 1)
     edges = [[batch - 1, nc * rows - 1], [0, 0], [0, 0], [0, rows - 1], [-1, 3], [0, nc * rows]]        # (the last two are ignored)
+    if nc * rows <= 8192 and batch <= 32:
+        edges += [[-1, 3]] * 4097        # (more pairs than the small step's kernel takes)
     labels = torch.cat([labels, torch.tensor(edges, device=gpu)]).to(torch.int32).contiguous()
     ws = ops.alloc_workspace(nc, rows, gpu)
     ws.view(torch.uint8)[: ops.step_sticky_error_offset()].fill_(0xFF)      # nothing of it is read before it is written

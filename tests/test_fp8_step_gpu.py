@@ -51,6 +51,12 @@ def check_rtn(case, device, **kw):
     return mism / total
 
 
+def off_the_small_step(labels):
+    """The same positives among more than 4,096 pairs, which small layers with up to 32 batch rows take the role kernel for: the rest lie
+    outside the batch and are ignored."""
+    return np.concatenate([labels, np.tile([[-1, 0]], (4097, 1))])
+
+
 @pytest.mark.parametrize("nc,rows,batch,seed", [
     (1, 64, 16, 11),          # a single tile
     (1, 16, 16, 12),          # a single ragged tile
@@ -61,6 +67,8 @@ def check_rtn(case, device, **kw):
 def test_rtn_parity_small(gpu, nc, rows, batch, seed):
     case = H.make_case(nc, rows, batch, seed)
     check_rtn(case, gpu)
+    if batch <= 32:
+        check_rtn(case, gpu, device_labels=off_the_small_step(case["labels"]))
 
 
 def test_quads_run_on_one_xcd_each(gpu):
@@ -99,6 +107,7 @@ def test_duplicate_and_dense_positives(gpu):
     extra = [(0, 0), (0, 0), (3, 0), (3, 5), (3, 5), (7, 63), (7, 64), (15, 127)] + [(b, 1) for b in range(16)]
     case = H.make_case(2, 64, 16, 31, extra_labels=extra)
     check_rtn(case, gpu)
+    check_rtn(case, gpu, device_labels=off_the_small_step(case["labels"]))
 
 
 def test_many_positives_boundary_labels_and_ignored_entries(gpu):
