@@ -8,11 +8,15 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("weights,mode", [("bf16", "rtn"), ("bf16", "sr_fast"), ("bf16", "sr_philox"), ("e4m3", "rtn"), ("e4m3", "sr_fast"), ("e4m3", "sr_philox"),
                                           ("fp8", "rtn"), ("fp8", "sr_fast"), ("fp8", "sr_philox")])
-@pytest.mark.parametrize("batch", [1, 16, 17, 33, 48, 65, 80, 81, 129, 144, 177, 193, 241, 257, 273, 385, 497])
-def test_neither_written_nor_read(gpu, batch, weights, mode):
+@pytest.mark.parametrize("batch,rows", [(b, 6016) for b in (1, 16, 17, 33, 48, 65, 80, 81, 129, 144, 177, 193, 241, 257, 273, 385, 497)] +
+                         [(b, 10256) for b in (129, 144, 145, 161, 177)])
+def test_neither_written_nor_read(gpu, batch, rows, weights, mode):
+    """Clusters of all sizes: of three, for 129 to 192 rows, from 7,680 labels on with FP8 logits and 10,240 otherwise."""
     import torch
     from elmo_amd import ops
-    rows = 6016
+    members = next(c for c, most in ((1, 64), (2, 128), (3 if rows >= (7680 if weights == "fp8" else 10240) else 4, 192), (4, 256), (6, 384), (8, 512))
+                   if batch <= most)
+    cap = 32 if batch <= 32 else 64 * members       # rows that the cluster of this batch holds
     g = torch.Generator(device=gpu).manual_seed(batch)
     w0 = torch.randn(rows, 768, generator=g, device=gpu).mul_(0.05).to(torch.bfloat16 if weights == "bf16" else torch.float8_e4m3fn)
     x = torch.randn(512, 768, generator=g, device=gpu).to(torch.bfloat16)
@@ -37,7 +41,6 @@ def test_neither_written_nor_read(gpu, batch, weights, mode):
     used = step(batch, None, x[:batch], ws)
     for got in (poisoned, used):
         assert torch.equal(got[0], fresh[0]) and torch.equal(got[1], fresh[1])
-    cap = next(c for c in (32, 64, 128, 192, 256, 384, 512) if c >= batch)   # rows that the cluster of this batch holds
     padded = torch.zeros(cap, 768, device=gpu, dtype=torch.bfloat16)
     padded[:batch] = x[:batch]
     whole = step(cap, 0, padded)
