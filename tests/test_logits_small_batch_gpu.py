@@ -28,3 +28,20 @@ def test_logits(gpu, nc, rows, labels, batch):
     want = ops.fp8_forward(chunks, torch.cat([nan, x[batch:]]), labels, workspace=ws)[:batch]
     got = ops.fp8_forward(chunks, nan, labels, workspace=ws)
     assert torch.equal(got.contiguous().view(torch.int16), want.contiguous().view(torch.int16))
+
+
+@pytest.mark.parametrize("batch", [1, 16, 17, 32, 33, 48])
+def test_logits_in_runs_of_tiles(gpu, batch):
+    """From 32 tiles of 32 labels a compute unit on, up to 48 rows: runs of four tiles, with one to three of a workgroup's first tiles loaded beside
+    X; a ragged end, the last round's tiles taken singly.  Rows of a larger batch read the image."""
+    import torch
+    from elmo_amd import _lib, ops
+    nc, rows, labels = 2, 133136, 266263
+    assert nc * rows // 32 > 32 * _lib.load().xmc_step_workgroups()
+    g = torch.Generator(device=gpu).manual_seed(batch)
+    chunks = [torch.randn(rows, 768, generator=g, device=gpu).mul_(0.05).to(torch.float8_e4m3fn) for _ in range(nc)]
+    x = torch.randn(80, 768, generator=g, device=gpu).to(torch.bfloat16)
+    ws = ops.alloc_workspace(nc, rows, gpu)
+    want = ops.fp8_forward(chunks, x, labels, 0.5, 0.37, workspace=ws)[:batch]
+    got = ops.fp8_forward(chunks, x[:batch].contiguous(), labels, 0.5, 0.37, workspace=ws)
+    assert torch.equal(got.contiguous().view(torch.int16), want.contiguous().view(torch.int16))
