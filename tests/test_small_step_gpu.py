@@ -7,6 +7,7 @@ import pytest
 
 import helpers as H
 from oracle import step as O
+from test_fp8_step_gpu import check_rtn
 
 pytestmark = pytest.mark.gpu
 
@@ -56,3 +57,46 @@ def test_positives(gpu, batch):
     for a, b in zip(w1, codes):
         assert H.e4m3_ulp_distance(a, b).max() <= 1 and np.mean(a == b) > 0.998
     assert np.abs(f1.cpu().numpy() - gx).max() <= 1e-3 * np.abs(gx).max()
+
+
+@pytest.mark.parametrize("nc,rows,batch", [(1, 16, 16), (1, 48, 32), (33, 32, 16), (64, 16, 32), (2, 2576, 16), (5, 1024, 32), (1, 8192, 16)])
+def test_against_the_oracle(gpu, nc, rows, batch):
+    """One tile, partial tiles, many chunks, the most tiles of either batch."""
+    check_rtn(H.make_case(nc, rows, batch, 23 * nc + rows + batch), gpu)
+
+
+@pytest.mark.parametrize("mode", ["rtn", "sr_fast", "sr_philox"])
+@pytest.mark.parametrize("batch", [16, 32])
+def test_infinities_nan_and_the_largest_weights(gpu, batch, mode):
+    """Weights at e4m3's largest values and NaN, embeddings that saturate, vanish or are no numbers: the same bits as the fused kernel's, and
+    what is not finite in grad_X in the same places."""
+    import torch
+    from elmo_amd import ops
+    nc, rows = 2, 80                                     # (chunks end in the middle of a tile)
+    g = torch.Generator(device=gpu).manual_seed(batch)
+    w0 = [torch.randn(rows, 768, generator=g, device=gpu).mul_(0.05).to(torch.float8_e4m3fn) for _ in range(nc)]
+    w0[0].view(torch.uint8)[3, ::2] = 0x7E              # 448
+    w0[0].view(torch.uint8)[4, ::3] = 0xFE              # -448
+    x0 = torch.randn(batch, 768, generator=g, device=gpu)
+    x0[0, :6] = torch.tensor([1e30, -1e30, 500.0, 2 ** -9, 1e-30, -0.0], device=gpu)
+    special = x0.clone()
+    special[1, 7], special[2, 8], special[batch - 1, 9] = float("inf"), -float("inf"), float("nan")
+    pos = torch.stack([torch.arange(5 * batch, device=gpu) % batch, torch.randint(0, nc * rows, (5 * batch,), generator=g, device=gpu)], 1).to(torch.int32)
+    ignored = torch.tensor([[-1, 0]], dtype=torch.int32, device=gpu)
+    ws = ops.alloc_workspace(nc, rows, gpu)
+    for x in (x0, special):
+        for code in (0x30, 0x7F):                        # 0.5, NaN: in the last row of a chunk
+            out = []
+            for extra in (0, 4097):
+                w = [c.clone() for c in w0]
+                w[1].view(torch.uint8)[rows - 1, 5] = code
+                labels = torch.cat([pos, ignored.expand(extra, 2)]).contiguous()
+                _, gf = ops.fp8_step(w, x.to(torch.bfloat16), labels, 40.0, seeds=[7, 12], round_mode=mode, workspace=ws, want_f32=True)
+                assert ops.step_error_word(ws, nc, rows) == 0
+                out.append((torch.cat([c.view(torch.uint8) for c in w]), gf))
+            (w1, f1), (w2, f2) = out
+            assert torch.equal(w1, w2)
+            assert bool(((w1 & 0x7F) == 0x7E).any())     # some updates saturate
+            assert torch.equal(torch.isfinite(f1), torch.isfinite(f2))
+            fin = torch.isfinite(f2)
+            assert (f1 - f2)[fin].abs().max().item() <= 2 ** -16 * f2[fin].abs().max().item()
