@@ -193,6 +193,8 @@ int tile_stride_inverse(int s, int n) {
 //   1   131 K labels 20.0/17.9    40  30 K 12.6/9.9, 131 K 22.1/21.2, 300 K 40.9/40.0, 670 K 118.0/116.6    48  48 K 12.6/11.8
 //   64  2 K 12.0/9.4, 32 K 12.1/10.3, 48 K 13.0/13.7, 131 K 23.3/24.4
 //   100, 128  2 K 12.0/9.5 11.9/10.0 among others, but 24.5/25.0 24.6/26.0 alone
+// Where no host is in the way (replays of a graph) the launch is cheaper, and 57 to 64 rows a little slower without it: 2 K labels, 48 rows
+// 6.5/6.2, 56 6.5/6.4, 64 6.5/6.8, 30 K, 64 10.0/10.5; waited for alone, 2 K, 64 23.4/22.2, 30 K 26.1/25.5.
 bool forward_converts(int batch, long long tiles, int cus) {
   return batch <= 48 || (batch <= FWD_CONV && tiles <= 4 * (long long)cus);
 }
@@ -266,6 +268,8 @@ bool small_batch_one_pass(int batch, long long tiles, int round_mode, int cus) {
 //             e4m3 with bf16 products, nearest 29.6/27.0 33.3/29.4 35.5/31.6   FP8 logits, sr_fast 25.6/26.7 and 33.1/31.0 (5 K)
 //   256 rows  bf16, 1 K, 1.6 K, 2 K nearest 30.9/29.0 33.4/31.5 35.3/33.3   Philox 31.8/32.1 34.7/33.9 36.8/35.6
 //             FP8 logits, 2 K, 4 K  nearest 31.2/29.6 36.1/34.5   sr_fast 31.2/30.4 36.4/35.0   Philox 33.8/35.6 39.2/40.0
+// (Two tiles each of fewer clusters were measured for no more tiles than clusters, and in clusters of one, two and four: elsewhere as many
+// clusters as there are, or as tiles.)
 int one_pass_clusters(int tiles, int most, int c, int nbk, bool fp8, int round_mode) {
   if (tiles > most) return most;
   const bool philox = round_mode == XMC_ROUND_SR_PHILOX;
@@ -277,11 +281,16 @@ int one_pass_clusters(int tiles, int most, int c, int nbk, bool fp8, int round_m
 // Whether a true-FP8 step without weight decay, dropout or a compensated head takes the two launches of xmc_fp8_small.hip, a workgroup for
 // every 32 labels and one to a compute unit at most.  What they gain is a launch and the latencies of the quads' exchange; what they lose
 // grows with the labels, 48 KiB of grad_X sums per 16 batch rows and workgroup, and with Philox, whose words take a workgroup longer than
-// the four of a quad.  us a step, fused kernel / this one, at 1 K, 2 K, 4 K, 6 K, 8 K labels:
-//   16 rows  sr_fast 14.2/10.0 14.4/10.5 14.5/11.9 16.1/13.9 16.5/15.7   nearest 14.2/10.2 14.3/9.9 14.4/11.5 15.7/13.5 16.0/15.3
-//            Philox 17.0/14.3 17.2/15.3 17.5/17.3 21.9/19.4 22.4/21.2
-//   32 rows  sr_fast 15.9/10.3 15.9/12.1 16.1/15.4 17.8/17.7 18.0/20.4   nearest 15.6/10.3 15.8/11.6 15.8/15.0 17.4/17.3 17.5/20.5
-//            Philox 18.8/15.5 18.9/17.3 19.2/20.7 23.7/23.0 24.1/24.2
+// the four of a quad.  us a step in replays of a graph, five positives a row, fused kernel / this one, at 1 K, 2 K, 4 K, 6 K, 8 K labels:
+//   16 rows  sr_fast 12.7/8.9 13.2/9.9 15.0/12.1 15.6/14.1 16.1/16.0   nearest 12.4/8.7 13.1/9.6 14.5/11.7 15.2/13.8 15.7/15.7
+//            Philox 15.5/14.4 16.2/15.4 17.3/17.6 21.4/19.9 21.9/21.4
+//   32 rows  sr_fast 12.9/10.6 14.1/12.3 15.8/15.7 17.1/18.4 17.9/21.2   nearest 12.9/10.2 13.9/11.9 15.6/15.3 16.5/17.9 17.4/21.0
+//            Philox 15.9/15.8 16.8/17.6 19.1/20.9 22.6/23.7 23.7/24.9
+// Launched from the host it gains up to two more, a launch less: waited for alone, 32 rows, 5 K 32.1/31.5 (16.5/17.3 in a graph), Philox, 2 K 32.3/31.8,
+// 6 K 38.0/37.5.  With more positives the launch that the fused kernel has in front takes longer: 5, 36, 128 a row, sr_fast, 16 rows, 4 K 14.9/12.0
+// 15.6/12.2 16.6/12.6, 8 K 16.2/16.1 17.0/16.1 17.8/16.6, 32 rows, 1 K 12.9/10.6 13.5/10.9 17.1/11.8, 5 K 16.5/17.3 17.4/17.4 19.7/18.4, Philox, 2 K 16.8/17.6 17.6/17.9
+// 20.4/18.8: at SM_POS, all that SM_BATCH rows have at 128 each, this form has gained.  (Eight pairs of a thread requested together instead of one
+// behind the other: 32 rows, 128 a row 0.2 to 0.5 faster, 36 a row and 64 a row of 16 rows 0.1 to 0.5 slower.)
 // (Workgroups that take several tiles one after the other, and sum: 8 K, 16 rows 15.9, 16 K 20.3/19.9 with the fused kernel, and half a
 // microsecond more with one tile each.)
 bool small_step(int batch, int nnz, long long tiles, int round_mode, int grid) {
@@ -290,8 +299,8 @@ bool small_step(int batch, int nnz, long long tiles, int round_mode, int grid) {
 }
 // Quads of the fused kernel for a step's tiles, of `most` that the device has.  A quad leaves the sum of grad_X of all its tiles, 384 KiB at
 // 128 rows, and one without tiles leaves as much: written, and read again behind the kernel.  With few tiles those sums cost more than a
-// second tile for every quad (not with Philox and up to 96 rows, whose tiles are long and whose sums are short, and not where a quarter of
-// the device would do).  Whole numbers of quads on each XCD.  us a step, all quads / now, at 300, 1 K, 2 K, 4 K, 5 K labels:
+// second tile for every quad, but where sums are short or tiles long: a quad for every tile with up to 48 rows or Philox up to half as many tiles
+// as quads, with Philox and up to 96 rows up to as many.  Whole numbers of quads on each XCD.  us a step, all quads / now, at 300, 1 K, 2 K, 4 K, 5 K labels:
 //   sr_fast  48 rows 16.9/13.7 18.3/14.3 18.5/15.9 18.7/17.8 20.1/18.8     128 rows 26.0/16.4 27.9/19.5 28.3/21.6 28.6/25.5 29.1/27.4
 //   Philox   64 rows 21.0/16.6 23.3/17.7 23.1/19.8 23.3/23.3 27.6/25.9     128 rows 26.8/19.2 30.1/21.6 31.5/25.7 32.1/30.9 34.4/32.6
 // (Two tiles a quad instead of one: 2 K labels, 48 rows 16.0/16.4, Philox 128 rows 25.0/26.3, but 96 rows 19.4/18.7, 128 rows 22.3/20.9; 4 K, Philox,

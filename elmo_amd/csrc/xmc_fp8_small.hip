@@ -7,7 +7,8 @@
 // one of memory (X, weights and positives are requested together), those of four short stages with a barrier behind each, and the
 // first pass over the kernel's code.  The step of xmc_fp8_role.hip, whose quads share a tile, is a launch more and a chain of an
 // exchange longer; its tiles leave a 64th of the sums of grad_X, this one's a sum of 48 KiB per 16 batch rows and 32 labels, which
-// is why it is not for large label spaces or batches (small_step).  4 K labels, 16 rows, sr_fast: 12.0 us a step, 14.5 in three launches;
+// is why it is not for large label spaces or batches (small_step).  4 K labels, 16 rows, sr_fast: 12.0 us a step in replays of a graph, 14.1 in three
+// launches of all quads; launched from the host, 15.7 a pass among others, where the host is what bounds it (18.4), 33 waited for alone (35);
 // traced 8.5 and 4.1 (4.1, 7.2 and 3.2 of the three).  64 labels to a workgroup would halve the sums and double the update's vector work.
 //
 // Reference semantics: as xmc_fp8_role.hip; the weights are the same to the bit (same operands in the same order into the same
@@ -18,7 +19,7 @@ namespace xmc {
 
 constexpr int SM_ROWS = 32;                  // label rows of a workgroup
 constexpr int SM_BATCH = 32;                 // most batch rows
-constexpr int SM_POS = 4096;                 // most positives: every workgroup reads all of them
+constexpr int SM_POS = 4096;                 // most positives: every workgroup reads all of them (small_step has what they cost)
 constexpr int SM_NT = 512;
 constexpr int SM_XBS = D * 2 + 16;           // LDS row stride of X in bf16
 constexpr int SM_GS = 80;                    // LDS row stride of G, 32 bf16 values

@@ -135,7 +135,8 @@ int xmc_fp8_forward_wide(void* const* chunk_ptrs, int num_chunks, int rows_per_c
 
 /* xmc_fp8_forward without a workspace argument.  It has no counterpart in the reference: it is for callers that cannot
  * allocate device memory for a workspace (code under HIP graph capture, serving loops and harnesses that forbid
- * hipMalloc).  The operand image of X that xmc_fp8_forward keeps in the caller's workspace (from 49 rows on) lives in a static device array
+ * hipMalloc).  The operand image of X that xmc_fp8_forward keeps in the caller's workspace (for more than 64 rows, and for 49 to 64 of
+ * more than 128 labels per compute unit; fewer need none) lives in a static device array
  * of the library instead (98,304 bytes per GPU, held until the process ends), so the limits are those of the array:
  * features == 768 and batch <= 128 (a multiple of 16); anything larger returns XMC_ERR_SHAPE.  The call allocates and
  * frees nothing.  Every call on a GPU uses that GPU's one array: calls that overlap on the same GPU (two streams, two
@@ -339,7 +340,8 @@ int xmc_pass_on_error(const int32_t* error_word, int32_t* into_error, int32_t* i
  * tiles takes fewer; the ids of the others are 0).
  * xmc_step_xcc_ids: copies the ids of the first `count` workgroups of the last step to host memory (synchronises).
  * xmc_quad_placement_check: host-only; number of quads whose four members recorded different ids (0 = fine) - the
- * comparison the device makes at the end of every step before it raises bit 1 of the error word. */
+ * comparison the device makes at the end of every step of the fused kernel before it raises bit 1 of the error word.  (Steps of small
+ * label spaces and batches exchange nothing between workgroups: they record the ids and compare none.) */
 int xmc_step_workgroups(void);
 int xmc_step_xcc_ids(const void* workspace, int32_t* ids_host, int count, void* stream);
 int xmc_quad_placement_check(const int32_t* xcc_ids_host, int num_workgroups);
