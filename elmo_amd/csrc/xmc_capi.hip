@@ -286,7 +286,7 @@ int one_pass_clusters(int tiles, int most, int c, int nbk, bool fp8, int round_m
 //            Philox 15.5/14.4 16.2/15.4 17.3/17.6 21.4/19.9 21.9/21.4
 //   32 rows  sr_fast 12.9/10.6 14.1/12.3 15.8/15.7 17.1/18.4 17.9/21.2   nearest 12.9/10.2 13.9/11.9 15.6/15.3 16.5/17.9 17.4/21.0
 //            Philox 15.9/15.8 16.8/17.6 19.1/20.9 22.6/23.7 23.7/24.9
-// Launched from the host it gains up to two more, a launch less: waited for alone, 32 rows, 5 K 32.1/31.5 (16.5/17.3 in a graph), Philox, 2 K 32.3/31.8,
+// Launched from the host it gains 1.1 to 1.4 more, a launch less: waited for alone, 32 rows, 5 K 32.1/31.5 (16.5/17.3 in a graph), Philox, 2 K 32.3/31.8,
 // 6 K 38.0/37.5.  With more positives the launch that the fused kernel has in front takes longer: 5, 36, 128 a row, sr_fast, 16 rows, 4 K 14.9/12.0
 // 15.6/12.2 16.6/12.6, 8 K 16.2/16.1 17.0/16.1 17.8/16.6, 32 rows, 1 K 12.9/10.6 13.5/10.9 17.1/11.8, 5 K 16.5/17.3 17.4/17.4 19.7/18.4, Philox, 2 K 16.8/17.6 17.6/17.9
 // 20.4/18.8: at SM_POS, all that SM_BATCH rows have at 128 each, this form has gained.  (Eight pairs of a thread requested together instead of one
