@@ -300,15 +300,15 @@ bool small_step(int batch, int nnz, long long tiles, int round_mode, int grid) {
 // Quads of the fused kernel for a step's tiles, of `most` that the device has.  A quad leaves the sum of grad_X of all its tiles, 384 KiB at
 // 128 rows, and one without tiles leaves as much: written, and read again behind the kernel.  With few tiles those sums cost more than a
 // second tile for every quad, but where sums are short or tiles long: a quad for every tile with up to 48 rows or Philox up to half as many tiles
-// as quads, with Philox and up to 96 rows up to as many.  Whole numbers of quads on each XCD.  us a step, all quads / now, at 300, 1 K, 2 K, 4 K, 5 K labels:
+// as quads, with up to 16 rows (32 with decay, 96 with Philox) up to as many.  Whole numbers of quads on each XCD.  us a step, all quads / now, at 300, 1 K, 2 K, 4 K, 5 K labels:
 //   sr_fast  48 rows 16.9/13.7 18.3/14.3 18.5/15.9 18.7/17.8 20.1/18.8     128 rows 26.0/16.4 27.9/19.5 28.3/21.6 28.6/25.5 29.1/27.4
 //   Philox   64 rows 21.0/16.6 23.3/17.7 23.1/19.8 23.3/23.3 27.6/25.9     128 rows 26.8/19.2 30.1/21.6 31.5/25.7 32.1/30.9 34.4/32.6
 // (Two tiles a quad instead of one: 2 K labels, 48 rows 16.0/16.4, Philox 128 rows 25.0/26.3, but 96 rows 19.4/18.7, 128 rows 22.3/20.9; 4 K, Philox,
-// 64 rows 23.3/24.8.  Three on 48 quads instead of 64, 9 K: 48 rows 22.2/21.2, but 128 rows 30.3/30.6: above two as many quads as there are.)
-int fused_quads(int tiles, int batch, int round_mode, int most) {
+// 64 rows 23.3/24.8; 16 rows, 2.6 K labels, dropout, sr_fast 15.6/16.0, more than SM_POS pairs 16.6/17.1, decay 17.2/18.4, 32 rows, 4 K, decay 19.0/19.5.  Three on 48 quads instead of 64, 9 K: 48 rows 22.2/21.2, but 128 rows 30.3/30.6: above two as many quads as there are.)
+int fused_quads(int tiles, int batch, int round_mode, bool decay, int most) {
   if (tiles > 2 * most) return most;
   const bool philox = round_mode == XMC_ROUND_SR_PHILOX;
-  const bool single = tiles <= most / 2 ? batch <= 48 || philox : tiles <= most && philox && batch <= 96;
+  const bool single = tiles <= most / 2 ? batch <= 48 || philox : tiles <= most && batch <= (philox ? 96 : decay ? 32 : 16);
   const int q = ((single ? tiles : (tiles + 1) / 2) + 7) / 8 * 8;
   return q < most ? q : most;
 }
@@ -571,7 +571,7 @@ static int fused_step(void* const* chunk_ptrs, int num_chunks, int rows_per_chun
     const int head_tiles = (num_head + TL - 1) / TL, rest_tiles = num_tiles - head_tiles;
     // (their quads' sums are continued by the quads of the other launch: at least as many)
     p.nquads_head = head_quads(head_tiles, qgrid >> 2);
-    const int rest_quads = fused_quads(rest_tiles, batch, round_mode, qgrid >> 2);
+    const int rest_quads = fused_quads(rest_tiles, batch, round_mode, weight_decay != 0.f, qgrid >> 2);
     p.nquads = rest_quads > p.nquads_head ? rest_quads : p.nquads_head;
     p.kahan = (unsigned char*)kahan;
     p.num_head = num_head;

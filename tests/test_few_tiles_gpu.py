@@ -35,6 +35,27 @@ def test_step(gpu, nc, rows, batch):
     assert lib.xmc_quad_placement_check(ids, n) == 0
 
 
+@pytest.mark.parametrize("tiles,batch,mode,decay,quads", [
+    (32, 48, "rtn", 0.0, 32), (33, 16, "rtn", 0.0, 40), (64, 16, "sr_fast", 0.0, 64), (65, 16, "rtn", 0.0, 40), (64, 32, "sr_fast", 0.0, 32), (64, 32, "sr_fast", 0.01, 64),
+    (57, 48, "rtn", 0.01, 32), (57, 96, "sr_philox", 0.0, 64), (57, 112, "sr_philox", 0.01, 32), (128, 128, "rtn", 0.0, 64), (129, 16, "rtn", 0.0, 64)])
+def test_quads(gpu, tiles, batch, mode, decay, quads):
+    """How many quads a step of few tiles takes: one for every tile where that is faster (the figures stand beside the rule)."""
+    import ctypes
+    import torch
+    from elmo_amd import _lib, ops
+    lib = _lib.load()
+    n = lib.xmc_step_workgroups()
+    if n != 256:
+        pytest.skip("the quads of a whole device")
+    case = H.make_case(1, 64 * tiles - 16, batch, tiles + batch, extra_labels=[[-1, 0]] * 4097)     # (more pairs than the small step takes)
+    chunks, x, labels = H.to_device_case(case, gpu)
+    ws = ops.alloc_workspace(1, 64 * tiles - 16, gpu)
+    ops.fp8_step(chunks, x, labels, 0.05, seeds=[3], round_mode=mode, workspace=ws, weight_decay=decay)
+    ids = (ctypes.c_int32 * n)()
+    _lib.check(lib.xmc_step_xcc_ids(ws.data_ptr(), ids, n, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)), "xmc_step_xcc_ids")
+    assert 8 * sum(v != 0 for v in ids) == 7 * 4 * quads      # (an eighth ran on XCD 0, the others did not run)
+
+
 @pytest.mark.parametrize("batch", [32, 128])
 @pytest.mark.parametrize("nc,rows,head", [(1, 64, 40), (1, 640, 640), (1, 1040, 70), (1, 4160, 4160), (2, 2080, 520), (2, 4160, 4128), (1, 8256, 100), (2, 8256, 8240)])
 def test_compensated_head(gpu, nc, rows, head, batch):
