@@ -282,13 +282,13 @@ int one_pass_clusters(int tiles, int most, int c, int nbk, bool fp8, int round_m
 // every 32 labels and one to a compute unit at most.  What they gain is a launch and the latencies of the quads' exchange; what they lose
 // grows with the labels, 48 KiB of grad_X sums per 16 batch rows and workgroup, and with Philox, whose words take a workgroup longer than
 // the four of a quad.  us a step in replays of a graph, five positives a row, fused kernel / this one, at 1 K, 2 K, 4 K, 6 K, 8 K labels:
-//   16 rows  sr_fast 12.7/8.9 13.2/9.9 15.0/12.1 15.6/14.1 16.1/16.0   nearest 12.4/8.7 13.1/9.6 14.5/11.7 15.2/13.8 15.7/15.7
+//   16 rows  sr_fast 12.7/8.9 13.2/9.9 14.4/12.1 15.6/14.1 16.1/16.0   nearest 12.4/8.7 13.1/9.6 14.2/11.7 15.2/13.8 15.7/15.7
 //            Philox 15.5/14.4 16.2/15.4 17.3/17.6 21.4/19.9 21.9/21.4
 //   32 rows  sr_fast 12.9/10.6 14.1/12.3 15.8/15.7 17.1/18.4 17.9/21.2   nearest 12.9/10.2 13.9/11.9 15.6/15.3 16.5/17.9 17.4/21.0
 //            Philox 15.9/15.8 16.8/17.6 19.1/20.9 22.6/23.7 23.7/24.9
 // Launched from the host it gains 1.1 to 1.4 more, a launch less: waited for alone, 32 rows, 5 K 32.1/31.5 (16.5/17.3 in a graph), Philox, 2 K 32.3/31.8,
-// 6 K 38.0/37.5.  With more positives the launch that the fused kernel has in front takes longer: 5, 36, 128 a row, sr_fast, 16 rows, 4 K 14.9/12.0
-// 15.6/12.2 16.6/12.6, 8 K 16.2/16.1 17.0/16.1 17.8/16.6, 32 rows, 1 K 12.9/10.6 13.5/10.9 17.1/11.8, 5 K 16.5/17.3 17.4/17.4 19.7/18.4, Philox, 2 K 16.8/17.6 17.6/17.9
+// 6 K 38.0/37.5.  With more positives the launch that the fused kernel has in front takes longer: 5, 36, 128 a row, sr_fast, 16 rows, 4 K 14.4/12.1
+// 14.9/12.2 15.6/12.7, 8 K 16.2/16.1 17.0/16.1 17.8/16.6, 32 rows, 1 K 12.9/10.6 13.5/10.9 17.1/11.8, 5 K 16.5/17.3 17.4/17.4 19.7/18.4, Philox, 2 K 16.8/17.6 17.6/17.9
 // 20.4/18.8: at SM_POS, all that SM_BATCH rows have at 128 each, this form has gained.  (Eight pairs of a thread requested together instead of one
 // behind the other: 32 rows, 128 a row 0.2 to 0.5 faster, 36 a row and 64 a row of 16 rows 0.1 to 0.5 slower.)
 // (Workgroups that take several tiles one after the other, and sum: 8 K, 16 rows 15.9, 16 K 20.3/19.9 with the fused kernel, and half a
